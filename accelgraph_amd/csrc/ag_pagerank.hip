@@ -742,6 +742,244 @@ __global__ __launch_bounds__(AG_FIN_WG) void pr_ddf_finish(PullGeom G, PrCtl C, 
     pr_close(C, iter, red);
 }
 
+// ---------------------------------------------------------------- data-driven, full pull in edge order
+//
+// The same full pull on an unblocked plan, every row of in-degree <= AG_DD_SEQ_MAX summed in
+// the reference's sequential order (so the run equals the sequential restatement bit for bit),
+// longer rows in the worklist form's workgroup tree. A row's serial chain of additions is the
+// only serial work: its ids and contributions are loaded a chunk ahead, and the chain itself
+// takes one instruction per in-edge (16-lane rows: a DPP broadcast folded into the add; 64-lane
+// rows: a lane read and an add; a workgroup's rows: LDS values, staged by all its lanes).
+// Bound by those chains and the gathers. RMAT-19 (8 M in-edges): 75 us an iteration, where
+// the worklists took 370 (nearly every vertex stays listed until the end of a run, so marking
+// the out-neighbours, 16 lanes along a hub's 30 K out-edges, cost more than it saved).
+
+// rows up to this in-degree are summed in edge order; longer rows in a lane-strided tree
+#define AG_DD_SEQ_MAX 8192u
+#define AG_DD_CHUNK (4u * AG_WG)   // in-edges of a workgroup's row staged at a time
+
+// Sum of c over a row of more than AG_DD_SEQ_MAX in-edges [b, e) by a workgroup: four lane
+// accumulators, 16 loads in flight, then a fixed tree. Valid in thread 0. `load` reads the
+// contribution of a source.
+template <class F>
+__device__ __forceinline__ float dd_tree_sum(const uint32_t *src, uint32_t b, uint32_t e, F load,
+                                             float *s_red)
+{
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t j = b + threadIdx.x;
+    for (; j + 15u * AG_WG < e; j += 16u * AG_WG) {
+        uint32_t id[16];
+        float x[16];
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; u++)
+            id[u] = src[j + u * AG_WG];
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; u++)
+            x[u] = load(id[u]);
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; u++)
+            a[u & 3u] = __fadd_rn(a[u & 3u], x[u]);
+    }
+    for (; j + 3u * AG_WG < e; j += 4u * AG_WG) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++)
+            a[u] = __fadd_rn(a[u], load(src[j + u * AG_WG]));
+    }
+    for (; j < e; j += AG_WG)
+        a[0] = __fadd_rn(a[0], load(src[j]));
+    return block_reduce<float, AG_WG>(__fadd_rn(__fadd_rn(a[0], a[1]), __fadd_rn(a[2], a[3])),
+                                      s_red);
+}
+
+// s + the 16 values of a row of lanes, lane 0's first: the same sum in each of the 16 lanes.
+template <int L = 0>
+__device__ __forceinline__ float dd_add16(float s, float x)
+{
+    if constexpr (L < 16) {
+        // DPP row_newbcast: lane L of the row of 16, in every lane of the row
+        const int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xF, 0xF, true);
+        return dd_add16<L + 1>(__fadd_rn(s, __int_as_float(y)), x);
+    } else {
+        return s;
+    }
+}
+
+// s + the 64 values of a wavefront, lane 0's first.
+template <int L = 0>
+__device__ __forceinline__ float dd_add64(float s, float x)
+{
+    if constexpr (L < 64)
+        return dd_add64<L + 1>(
+            __fadd_rn(s, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), L))), x);
+    else
+        return s;
+}
+
+// One row [lo, hi) per W lanes (16 or 64) in edge order: |c| of its in-edges, and whether one of
+// them carries a sign. Four loads of W in-edges are in flight, the next four's ids behind them.
+// Padding adds +0 to a sum that is never -0.
+template <uint32_t W>
+__device__ __forceinline__ DdAcc dd_lane_row(const uint32_t *src, const float *c, uint32_t lo,
+                                             uint32_t hi, uint32_t lane)
+{
+    float s = 0.0f;
+    uint32_t any = 0u, id[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; u++)
+        id[u] = lo + u * W + lane < hi ? ld_stream(&src[lo + u * W + lane]) : 0u;
+    for (uint32_t j0 = lo; j0 < hi; j0 += 4u * W) {
+        float x[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++)
+            x[u] = j0 + u * W + lane < hi ? c[id[u]] : 0.0f;
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t j = j0 + (4u + u) * W + lane;
+            id[u] = j < hi ? ld_stream(&src[j]) : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            if (j0 + u * W < hi) {   // the same for every lane of the row
+                any |= __float_as_uint(x[u]);
+                if constexpr (W == 16u)
+                    s = dd_add16(s, fabsf(x[u]));
+                else
+                    s = dd_add64(s, fabsf(x[u]));
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t m = W / 2u; m >= 1u; m >>= 1)
+        any |= (uint32_t)__shfl_xor((int)any, (int)m, (int)W);
+    return DdAcc(s, (any >> 31) ? 1.0f : 0.0f);
+}
+
+// A row [lo, hi) of at most AG_DD_SEQ_MAX in-edges by a workgroup, in edge order: all lanes stage
+// the next chunk of |c| in one half of s_vals while the first wavefront adds the other half.
+// Valid in the first wavefront; ends on a barrier.
+__device__ __forceinline__ DdAcc dd_wg_row(const uint32_t *src, const float *c, uint32_t lo,
+                                           uint32_t hi, float *s_vals)
+{
+    const uint32_t tid = threadIdx.x;
+    float s = 0.0f, x[4];
+    uint32_t any = 0u, id[4], h = 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; u++)
+        id[u] = lo + u * AG_WG + tid < hi ? ld_stream(&src[lo + u * AG_WG + tid]) : 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; u++)
+        x[u] = lo + u * AG_WG + tid < hi ? c[id[u]] : 0.0f;
+    for (uint32_t j0 = lo; j0 < hi; j0 += AG_DD_CHUNK, h ^= AG_DD_CHUNK) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            s_vals[h + u * AG_WG + tid] = fabsf(x[u]);
+            any |= __float_as_uint(x[u]);
+        }
+        __syncthreads();
+        const uint32_t n0 = j0 + AG_DD_CHUNK;
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++)
+            id[u] = n0 + u * AG_WG + tid < hi ? ld_stream(&src[n0 + u * AG_WG + tid]) : 0u;
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++)
+            x[u] = n0 + u * AG_WG + tid < hi ? c[id[u]] : 0.0f;
+        if (tid < AG_WAVE) {
+            // whole groups of 16: the padding adds +0
+            const uint32_t cnt = hi - j0 < AG_DD_CHUNK ? hi - j0 : AG_DD_CHUNK;
+            for (uint32_t q = 0; q < cnt; q += 16u) {
+                float v[16];
+#pragma unroll
+                for (uint32_t u = 0; u < 16u; u++)
+                    v[u] = s_vals[h + q + u];
+#pragma unroll
+                for (uint32_t u = 0; u < 16u; u++)
+                    s = __fadd_rn(s, v[u]);
+            }
+        }
+    }
+    const int f = __syncthreads_or((int)(any >> 31));
+    return DdAcc(s, f ? 1.0f : 0.0f);
+}
+
+// Work items, heaviest first: BLOCK and HUB rows (a workgroup each), WAVE rows (a wavefront
+// each), GROUP16 rows (16 lanes each), THREAD tiles (a lane per row, from LDS).
+__global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF32Args A)
+{
+    __shared__ float s_vals[AG_TILE_NNZ_MAX];
+    __shared__ float s_wave[AG_WG / AG_WAVE];
+    static_assert(2u * AG_DD_CHUNK <= AG_TILE_NNZ_MAX, "both halves of a staged row");
+    const PrState *st = C.st;
+    if (*(volatile const uint32_t *)&st->done)
+        return;
+    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
+    Red red{};
+    const PrDdPol p = dd_policy(iter, A);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t r_grp = G.bin_row[AG_BIN_GROUP16], r_wav = G.bin_row[AG_BIN_WAVE];
+    const uint32_t r_big = G.bin_row[AG_BIN_BLOCK], r_end = G.bin_row[AG_NBINS];
+    const uint32_t n_big = r_end - r_big;
+    const uint32_t n_wav = n_big + (r_big - r_wav + AG_WG / AG_WAVE - 1u) / (AG_WG / AG_WAVE);
+    const uint32_t n_grp = n_wav + (r_wav - r_grp + AG_WG / 16u - 1u) / (AG_WG / 16u);
+    const uint32_t total = n_grp + (G.slot_blk0[AG_NSLOTS] - G.slot_blk0[AG_NSLOTS - 1]);
+    for (uint32_t it = blockIdx.x; it < total; it += gridDim.x) {
+        if (it < n_big) {
+            const uint32_t row = r_big + it, lo = G.off[row], hi = G.off[row + 1];
+            DdAcc acc;
+            if (hi - lo > AG_DD_SEQ_MAX) {
+                uint32_t any = 0u;
+                const float s = dd_tree_sum(G.src, lo, hi, [&](uint32_t v) {
+                    const float x = p.cin[v];
+                    any |= __float_as_uint(x);
+                    return fabsf(x);
+                }, s_wave);
+                const int f = __syncthreads_or((int)(any >> 31));
+                acc = DdAcc(s, f ? 1.0f : 0.0f);
+            } else {
+                acc = dd_wg_row(G.src, p.cin, lo, hi, s_vals);
+            }
+            if (tid == 0)
+                p.finish(row, acc, red);
+        } else if (it < n_wav) {
+            const uint32_t row = r_wav + (it - n_big) * (AG_WG / AG_WAVE) + tid / AG_WAVE;
+            if (row < r_big) {
+                const uint32_t lane = tid % AG_WAVE;
+                const DdAcc acc = dd_lane_row<AG_WAVE>(G.src, p.cin, G.off[row], G.off[row + 1],
+                                                       lane);
+                if (lane == 0)
+                    p.finish(row, acc, red);
+            }
+        } else if (it < n_grp) {
+            const uint32_t row = r_grp + (it - n_wav) * (AG_WG / 16u) + tid / 16u;
+            if (row < r_wav) {
+                const uint32_t lane = tid % 16u;
+                const DdAcc acc = dd_lane_row<16u>(G.src, p.cin, G.off[row], G.off[row + 1], lane);
+                if (lane == 0)
+                    p.finish(row, acc, red);
+            }
+        } else {
+            // the signed contributions of a tile's in-edges, then a lane per row
+            const uint32_t tile = it - n_grp;
+            const uint32_t r0 = G.tile_row[tile], r1 = G.tile_row[tile + 1];
+            const uint32_t e0 = G.off[r0];
+            stage_edges(G.src, e0, G.off[r1] - e0, PrF32Pol<float, float>{p.cin}, s_vals);
+            __syncthreads();
+            for (uint32_t r = r0 + tid; r < r1; r += AG_WG) {
+                const uint32_t b = G.off[r] - e0, e = G.off[r + 1] - e0;
+                float s = 0.0f;
+                uint32_t any = 0u;
+                for (uint32_t q = b; q < e; q++) {
+                    const float x = s_vals[q];
+                    any |= __float_as_uint(x);
+                    s = __fadd_rn(s, fabsf(x));
+                }
+                p.finish(r, DdAcc(s, (any >> 31) ? 1.0f : 0.0f), red);
+            }
+            __syncthreads();   // s_vals is reused by this workgroup's next item
+        }
+    }
+    pr_store_partial(C, red);
+}
+
 // ---------------------------------------------------------------- push direction
 //
 // pageRankPushGraphCSR (pageRank.c:1111-1272) and pageRankPushFixedPointGraphCSR
@@ -817,6 +1055,7 @@ __global__ __launch_bounds__(AG_FIN_WG) void pr_plain_finish(PrCtl C)
 
 // ---------------------------------------------------------------- data-driven pull
 //
+// The worklist form (user starts on unblocked plans, and user starts whose signs are taken).
 // pageRankDataDrivenPullGraphCSR (pageRank.c:2810-2969): every vertex starts on the worklist;
 // per iteration the contributions rank/out_degree are those of the iteration's start
 // (:2870-2876), each listed vertex sums its in-edges, adds |delta|/N to the error, and only
@@ -834,8 +1073,6 @@ __global__ __launch_bounds__(AG_FIN_WG) void pr_plain_finish(PrCtl C)
 // sequential restatement bit for bit; longer rows take a fixed lane-strided tree order.
 
 #define AG_DD_LANES 16u
-// rows up to this in-degree are summed in edge order; longer rows in a lane-strided tree
-#define AG_DD_SEQ_MAX 8192u
 
 __global__ __launch_bounds__(AG_WG) void pr_dd_gather_kernel(PrCtl C, PrF32Args A, uint32_t n,
                                                              const uint32_t *off,
@@ -855,23 +1092,12 @@ __global__ __launch_bounds__(AG_WG) void pr_dd_gather_kernel(PrCtl C, PrF32Args 
     const uint32_t hubs = *(volatile const uint32_t *)&st->dd_hubs[iter & 1u];
     const float *c = (const float *)A.c32[0];
     Red red{};
-    // hub rows (in-degree > AG_DD_SEQ_MAX), listed from the far end: one workgroup each, four
-    // independent lane accumulators (a fixed order, so the sum is deterministic)
+    // hub rows (in-degree > AG_DD_SEQ_MAX), listed from the far end: one workgroup each, in a
+    // fixed order, so the sum is deterministic
     for (uint32_t h = blockIdx.x; h < hubs; h += gridDim.x) {
         const uint32_t v = queue[n - 1u - h];
         const uint32_t b = off[v], e = off[v + 1];
-        float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-        uint32_t j = b + threadIdx.x;
-        for (; j + 3u * AG_WG < e; j += 4u * AG_WG) {
-            a0 = __fadd_rn(a0, c[src[j]]);
-            a1 = __fadd_rn(a1, c[src[j + AG_WG]]);
-            a2 = __fadd_rn(a2, c[src[j + 2u * AG_WG]]);
-            a3 = __fadd_rn(a3, c[src[j + 3u * AG_WG]]);
-        }
-        for (; j < e; j += AG_WG)
-            a0 = __fadd_rn(a0, c[src[j]]);
-        const float sum = block_reduce<float, AG_WG>(__fadd_rn(__fadd_rn(a0, a1),
-                                                               __fadd_rn(a2, a3)), s_red);
+        const float sum = dd_tree_sum(src, b, e, [&](uint32_t u) { return c[u]; }, s_red);
         if (threadIdx.x == 0) {
             const float nw = __fadd_rn(A.base, __fmul_rn(A.damp, sum));
             const double err = (double)fabsf(__fsub_rn(nw, A.rank[v]));
@@ -1247,11 +1473,15 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     if (o.direction == AG_DIR_DATA_DRIVEN && kc != 0)
         return ag_set_error(AG_ERR_UNSUPPORTED,
                             "the data-driven pull takes FP32 with f32 storage only");
-    // the data-driven pull keeps explicit worklists on unblocked plans (edge-order sums) and
-    // runs as a full pull with sign-bit lists on source-blocked plans. The sign bit is free
-    // only while every contribution is >= +0, i.e. from a start vector without negative
-    // entries, -0 or NaN (ranks stay positive from there); other user starts keep worklists.
-    bool dd_lists = o.direction == AG_DIR_DATA_DRIVEN && g->blk.bits == 0;
+    // the data-driven pull runs as a full pull with sign-bit lists: in edge order on unblocked
+    // plans, in the pull's order on source-blocked ones. The sign bit is free only while every
+    // contribution is >= +0, i.e. from a start vector without negative entries, -0 or NaN
+    // (ranks stay positive from there); other user starts keep explicit worklists. So do all
+    // user starts on unblocked plans: a restart from nearly converged ranks lists few vertices
+    // after its first iteration, which an iteration over every row cannot use (from the
+    // built-in starts nearly every vertex stays listed until the end of the run).
+    bool dd_lists = o.direction == AG_DIR_DATA_DRIVEN && g->blk.bits == 0 &&
+                    o.init == AG_INIT_USER;
     if (o.direction == AG_DIR_DATA_DRIVEN && !dd_lists && o.init == AG_INIT_USER &&
         o.init_ranks) {
         for (uint32_t v = 0; v < g->n && !dd_lists; v++) {
@@ -1488,6 +1718,13 @@ int ag_pr_launch_iteration(ag_pr_session *s)
         const BlockGeom B = ag_make_block_geom(g);
         const BlockGeom &B1 = B;
         AG_PR_LAUNCH_BLOCKED(pr_ddf_blk_kernel, pr_ddf_cmb_kernel, pr_ddf_finish);
+        AG_HIP(hipGetLastError());
+        return AG_OK;
+    }
+    if (s->o.direction == AG_DIR_DATA_DRIVEN && !s->dd_queue[0]) {
+        C.nparts = ag_pull_grid(g, AG_TILE_NNZ_MAX * 4u);
+        pr_dds_kernel<<<C.nparts, block, 0, stream>>>(G, C, A);
+        pr_plain_finish<<<1, fin, 0, stream>>>(C);
         AG_HIP(hipGetLastError());
         return AG_OK;
     }

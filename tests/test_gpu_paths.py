@@ -1,0 +1,61 @@
+"""Kernels that a size, type or option selects, at the sizes where the selection or a tile ends."""
+import numpy as np
+import pytest
+
+import accelgraph_amd as ag
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+# in-degrees at the ends of the row classes, of a lane group's and a workgroup's chunks, and of
+# the rows summed in edge order (8192)
+EDGE_DEGREES = [0, 1, 15, 16, 17, 63, 64, 65, 128, 129, 255, 256, 257, 1023, 1024, 1025, 2047,
+                2048, 2049, 3072, 4096, 4097, 8191, 8192]
+
+
+def graph_with_degrees(degrees, n=20011, seed=3):
+    """Row i has degrees[i] in-edges from distinct sources; a sparse random part keeps ranks
+    moving for a while."""
+    rng = np.random.default_rng(seed)
+    src = [rng.choice(np.arange(len(degrees), n), d, replace=False) for d in degrees]
+    dst = [np.full(d, i) for i, d in enumerate(degrees)]
+    src.append(rng.integers(0, n, 4 * n))
+    dst.append(rng.integers(len(degrees), n, 4 * n))
+    return ag.Graph.from_edges(np.concatenate(src), np.concatenate(dst), n=n)
+
+
+@pytest.mark.parametrize("init", [ag.INIT_REFERENCE, ag.INIT_UNIFORM])
+def test_data_driven_row_classes(device, init):
+    """From a built-in start the data-driven pull evaluates every row in edge order: the
+    sequential oracle's run bit for bit at every row class's ends, and the run that the same
+    start gives as a user start (explicit worklists)."""
+    g = graph_with_degrees(EDGE_DEGREES)
+    dg = device.upload(g)
+    kw = dict(direction=ag.DIR_DATA_DRIVEN, max_iterations=200, epsilon=1e-5, scaled=True)
+    run = dg.pagerank(init=init, **kw)
+    ref = oracle.pagerank_dd_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, g.edges_idx,
+                                  g.out_degree, g.fwd_dest, init=init, max_iterations=200,
+                                  epsilon=1e-5)
+    assert run.iterations == ref.iterations and run.executed > 5
+    np.testing.assert_array_equal(run.hist_active, ref.hist_active)
+    np.testing.assert_array_equal(run.scaled.view(np.uint32), ref.scaled.view(np.uint32))
+    np.testing.assert_allclose(run.hist_err, ref.hist_err, rtol=1e-9, atol=1e-15)
+    start = np.full(g.n, 1.0 if init == ag.INIT_UNIFORM else np.float32(1) - np.float32(0.85),
+                    np.float32)
+    lists = dg.pagerank(init_ranks=start, **kw)
+    np.testing.assert_array_equal(run.scaled.view(np.uint32), lists.scaled.view(np.uint32))
+    np.testing.assert_array_equal(run.hist_active, lists.hist_active)
+    dg.close()
+
+
+@pytest.mark.parametrize("degree", [8193, 12288, 12289, 18000])
+def test_data_driven_long_rows(device, degree):
+    """Rows above 8192 in-edges take one fixed tree in both forms of the data-driven pull."""
+    g = graph_with_degrees([degree, 3])
+    dg = device.upload(g)
+    kw = dict(direction=ag.DIR_DATA_DRIVEN, max_iterations=60, epsilon=1e-5, scaled=True)
+    run = dg.pagerank(init=ag.INIT_UNIFORM, **kw)
+    lists = dg.pagerank(init_ranks=np.ones(g.n, np.float32), **kw)
+    np.testing.assert_array_equal(run.scaled.view(np.uint32), lists.scaled.view(np.uint32))
+    np.testing.assert_array_equal(run.hist_active, lists.hist_active)
+    dg.close()
