@@ -20,6 +20,8 @@
 #endif
 static_assert(AG_PB_ROWS >= 2u && AG_PB_ROWS <= 65536u, "push bins use 16-bit local row ids");
 
+#define AG_LANE_MAX 64u    // rows of a tile with at most this many elements: a lane each
+
 struct ag_device {
     int ordinal;
     hipStream_t stream;
@@ -52,6 +54,8 @@ struct ag_dgraph {
     int wq_user;         // wq came from ag_graph_set_fixed_weights
     uint32_t *outdeg;    // [n]
     uint32_t *tile_row;  // [n_tiles+1]
+    uint4 *rt;           // [n_rt] row tiles of the regular schedule (PullGeom::rt)
+    uint32_t n_rt, n_heavy;
     uint32_t *seg_row, *seg_lo, *seg_hi;  // [n_segs]
     uint32_t *hub_seg0;  // [n_hubs+1]
     uint64_t *hub_part;    // [n_segs] 8-byte partial sums (float or u64 bits)
@@ -95,6 +99,10 @@ struct PullGeom {
     const uint32_t *seg_hi;
     const uint32_t *hub_seg0;
     uint64_t *hub_part;
+    const uint4 *rt;         // [n_rt] row tiles {first row, end row, first in-edge, end}
+    uint32_t n_rt;
+    uint32_t n_heavy;        // items of slot_blk0 before the row tiles (hub segments, block rows)
+    uint32_t lane_max;       // rows of a tile up to this in-degree are summed by one lane
     uint32_t n;
     uint32_t n_hubs;
     uint32_t seq_hubs;       // plan in reference order: a hub row is one segment, added by one
@@ -145,6 +153,9 @@ void ag_block_geom_skip_hot(const ag_dgraph *g, BlockGeom &B);
 // number of work items. Per CU: the plan's wg_per_cu, else default_per_cu, never more than
 // LDS allows.
 uint32_t ag_pull_grid(const ag_dgraph *g, uint32_t lds_bytes, uint32_t default_per_cu = 4u);
+
+// The same for the regular schedule in row tiles.
+uint32_t ag_tile_grid(const ag_dgraph *g, uint32_t lds_bytes);
 
 // Device-side iteration state of a PageRank session.
 struct PrState {

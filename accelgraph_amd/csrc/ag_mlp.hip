@@ -368,7 +368,9 @@ struct NbrDegPol {
     {
         return __uint2float_rn(off[s + 1] - off[s]);
     }
-    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &) const
+    using Pre = NoPre;
+    __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
+    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &, Pre = Pre{}) const
     {
         const uint32_t d = off[r + 1] - off[r];
         feat[(size_t)r * MLP_FSTRIDE + 2] = d ? log1pf(__fdiv_rn(sum, __uint2float_rn(d))) : 0.0f;
@@ -801,7 +803,7 @@ static int compute_features(ag_dgraph *g, const float *r1, const float *r2, floa
     feat_local_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, g->off, g->outdeg, r1, r2, feat);
     PullGeom G = ag_make_geom(g);
     NbrDegPol pol{g->off, feat};
-    const uint32_t grid = ag_pull_grid(g, AG_TILE_NNZ_MAX * 4u);
+    const uint32_t grid = ag_tile_grid(g, AG_TILE_NNZ_MAX * 4u);
     pull_kernel<NbrDegPol><<<grid, AG_WG, 0, s>>>(G, pol);
     if (g->n_hubs)
         pull_finish_kernel<NbrDegPol><<<1, AG_FIN_WG, 0, s>>>(G, pol);

@@ -181,6 +181,16 @@ __device__ __forceinline__ void pr_close(const PrCtl &C, uint32_t iter, Red red)
         pr_control(C, iter, t.err, t.active);
 }
 
+// What a row's update reads of the row itself, loaded ahead of its sum.
+struct RankPre {
+    float old;
+    uint32_t od;
+};
+__device__ __forceinline__ RankPre rank_pre(const float *rank, const uint32_t *outdeg, uint32_t r)
+{
+    return RankPre{__builtin_nontemporal_load(&rank[r]), __builtin_nontemporal_load(&outdeg[r])};
+}
+
 // ---------------------------------------------------------------- FP32 policy
 
 template <typename RT, typename WT>
@@ -196,16 +206,20 @@ struct PrF32Pol {
     __device__ __forceinline__ float edge(uint32_t, uint32_t s) const { return ld_f32(cin[s]); }
     // the same term from a stored contribution already in hand (hot-segment LDS copy)
     __device__ __forceinline__ float edge_val(uint32_t, RT v) const { return ld_f32(v); }
-    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &red) const
+    using Pre = RankPre;
+    __device__ __forceinline__ Pre pre(uint32_t r) const { return rank_pre(rank, outdeg, r); }
+    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &red, const Pre &q) const
     {
         const float nw = __fadd_rn(base, __fmul_rn(damp, sum));
-        const float old = __builtin_nontemporal_load(&rank[r]);
         __builtin_nontemporal_store(nw, &rank[r]);
-        const double e = (double)fabsf(__fsub_rn(nw, old));
+        const double e = (double)fabsf(__fsub_rn(nw, q.old));
         red.err += __ddiv_rn(e, dn);
         red.active += (e >= eps) ? 1u : 0u;
-        const uint32_t od = __builtin_nontemporal_load(&outdeg[r]);
-        cout[r] = st_from_f32<WT>(od ? __fdiv_rn(nw, __uint2float_rn(od)) : 0.0f);
+        cout[r] = st_from_f32<WT>(q.od ? __fdiv_rn(nw, __uint2float_rn(q.od)) : 0.0f);
+    }
+    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &red) const
+    {
+        finish(r, sum, red, pre(r));
     }
 };
 
@@ -247,15 +261,18 @@ template <typename HT>
 __device__ __forceinline__ void pr_f32_main(const PullGeom &G, const PrCtl &C,
                                             const PrF32Args &A, bool mixed)
 {
-    __shared__ float s_vals[AG_TILE_NNZ_MAX];
+    using LP = PrF32Pol<float, float>;   // every storage sums in FP32
+    AG_TILE_LDS(LP, tile);
     __shared__ float s_wave[AG_WG / AG_WAVE];
     const PrState *st = C.st;
     if (*(volatile const uint32_t *)&st->done)
         return;
     const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pr_f32_dispatch<HT>(st, iter, A, mixed,
-                        [&](const auto &p) { pull_items(G, p, red, s_vals, s_wave); });
+    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) {
+        using P = std::remove_cv_t<std::remove_reference_t<decltype(p)>>;
+        pull_items(G, p, red, TileLds<P>{tile.vals, tile.lsum, tile.lng, tile.cnt}, s_wave);
+    });
     pr_store_partial(C, red);
 }
 
@@ -463,16 +480,20 @@ struct PrFixPol {
     double dn, eps;
 
     __device__ __forceinline__ uint64_t edge(uint32_t, uint32_t s) const { return (uint64_t)cin[s]; }
-    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red) const
+    using Pre = RankPre;
+    __device__ __forceinline__ Pre pre(uint32_t r) const { return rank_pre(rank, outdeg, r); }
+    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red, const Pre &x) const
     {
         const float nw = fix_update<BITS>(base, damp, q);
-        const float old = __builtin_nontemporal_load(&rank[r]);
         __builtin_nontemporal_store(nw, &rank[r]);
-        const double e = (double)fabsf(__fsub_rn(nw, old));
+        const double e = (double)fabsf(__fsub_rn(nw, x.old));
         red.err += __ddiv_rn(e, dn);
         red.active += (e >= eps) ? 1u : 0u;
-        const uint32_t od = __builtin_nontemporal_load(&outdeg[r]);
-        cout[r] = od ? fix_encode<BITS>(__fdiv_rn(nw, __uint2float_rn(od))) : (CT)0;
+        cout[r] = x.od ? fix_encode<BITS>(__fdiv_rn(nw, __uint2float_rn(x.od))) : (CT)0;
+    }
+    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red) const
+    {
+        finish(r, q, red, pre(r));
     }
 };
 
@@ -535,18 +556,22 @@ struct PrQuantPol {
     double dn, eps;
 
     __device__ __forceinline__ uint64_t edge(uint32_t, uint32_t s) const { return (uint64_t)codes[s]; }
-    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red) const
+    using Pre = RankPre;
+    __device__ __forceinline__ Pre pre(uint32_t r) const { return rank_pre(rank, outdeg, r); }
+    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red, const Pre &x) const
     {
         const float nw = __fadd_rn(base, __fmul_rn(damp, __fmul_rn(scale, __ull2float_rn(q))));
-        const float old = __builtin_nontemporal_load(&rank[r]);
         __builtin_nontemporal_store(nw, &rank[r]);
-        const double e = (double)fabsf(__fsub_rn(nw, old));
+        const double e = (double)fabsf(__fsub_rn(nw, x.old));
         red.err += __ddiv_rn(e, dn);
         red.active += (e >= eps) ? 1u : 0u;
-        const uint32_t od = __builtin_nontemporal_load(&outdeg[r]);
-        const float c = od ? __fdiv_rn(nw, __uint2float_rn(od)) : 0.0f;
+        const float c = x.od ? __fdiv_rn(nw, __uint2float_rn(x.od)) : 0.0f;
         cf[r] = c;
         red.cmax = max(red.cmax, quant_max_bits(c));
+    }
+    __device__ __forceinline__ void finish(uint32_t r, uint64_t q, Red &red) const
+    {
+        finish(r, q, red, pre(r));
     }
 };
 
@@ -595,14 +620,15 @@ __global__ __launch_bounds__(AG_WG) void pr_quant_init_max(uint32_t n, const flo
 template <int KC>
 __global__ __launch_bounds__(AG_WG) void pr_int_kernel(PullGeom G, PrCtl C, PrF32Args A)
 {
-    __shared__ uint64_t s_vals[AG_TILE_NNZ_MAX];
+    using P = decltype(int_policy<KC>(C.st, 0u, A));
+    AG_TILE_LDS(P, tile);
     __shared__ uint64_t s_wave[AG_WG / AG_WAVE];
     const PrState *st = C.st;
     if (*(volatile const uint32_t *)&st->done)
         return;
     const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pull_items(G, int_policy<KC>(st, iter, A), red, s_vals, s_wave);
+    pull_items(G, int_policy<KC>(st, iter, A), red, tile, s_wave);
     pr_store_partial(C, red);
 }
 
@@ -1786,7 +1812,7 @@ int ag_pr_launch_iteration(ag_pr_session *s)
         AG_HIP(hipGetLastError());
         return AG_OK;
     }
-    const uint32_t grid = ag_pull_grid(g, lds);
+    const uint32_t grid = ag_tile_grid(g, lds);
     C.nparts = grid;
     switch (s->kind_code) {
     case 0: AG_PR_LAUNCH_REGULAR(pr_f32_kernel, pr_f32_finish); break;

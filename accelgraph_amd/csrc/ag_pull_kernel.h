@@ -129,6 +129,10 @@ __device__ __forceinline__ uint32_t ld_stream(const uint32_t *p)
     return __builtin_nontemporal_load(p);
 }
 
+#define AG_LONG_MAX 64u    // longer rows of one tile: at most AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1)
+static_assert(AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1u) < AG_LONG_MAX,
+              "the long rows of a full tile must fit the tile's LDS list");
+
 #define AG_UNROLL 4
 // Partials per lane in flight when a combine tile is staged in LDS: 8 of 8 bytes (the
 // fixed-point and quantised kinds, 4 workgroups per CU for their LDS; RMAT-25 fixed-32
@@ -144,30 +148,33 @@ __device__ __forceinline__ uint32_t ld_stream(const uint32_t *p)
 #define AG_TILE_UNROLL 16
 
 // Lane-strided partial sum of in-edges lo, lo+S, ... < hi. Each round issues the source-id
-// loads of AG_UNROLL elements, then their gathers, all predicated, so a lane has up to
-// AG_UNROLL independent gathers in flight and a short row costs one round trip, not one per
-// element. Accumulators combine in a fixed tree.
-template <class P, uint32_t S>
+// loads of U elements, then their gathers, all predicated, so a lane has up to U independent
+// gathers in flight and a short row costs one round trip, not one per element. Four accumulators
+// take the elements in turn and combine in a fixed tree, whatever U is. Workgroup rows take 16
+// loads a lane (4096 in-edges a round, as an LDS
+// tile): RMAT-18 SpMV 25.4 -> 22.1 us, RMAT-20 81.7 -> 77.9 us against 4.
+template <class P, uint32_t S, int U = AG_UNROLL>
 __device__ __forceinline__ typename P::Acc strided_sum(const PullGeom &G, const P &pol,
                                                         uint32_t lo, uint32_t hi)
 {
     using Acc = typename P::Acc;
+    static_assert(U % AG_UNROLL == 0, "the accumulators take turns");
     Acc a[AG_UNROLL];
 #pragma unroll
     for (int u = 0; u < AG_UNROLL; u++)
         a[u] = Acc(0);
-    for (uint32_t j = lo; j < hi; j += AG_UNROLL * S) {
-        uint32_t sidx[AG_UNROLL];
+    for (uint32_t j = lo; j < hi; j += U * S) {
+        uint32_t sidx[U];
 #pragma unroll
-        for (int u = 0; u < AG_UNROLL; u++) {
+        for (int u = 0; u < U; u++) {
             const uint32_t jj = j + u * S;
             sidx[u] = jj < hi ? ld_stream(&G.src[jj]) : 0u;
         }
 #pragma unroll
-        for (int u = 0; u < AG_UNROLL; u++) {
+        for (int u = 0; u < U; u++) {
             const uint32_t jj = j + u * S;
             if (jj < hi)
-                a[u] = a[u] + pol.edge(jj, sidx[u]);
+                a[u % AG_UNROLL] = a[u % AG_UNROLL] + pol.edge(jj, sidx[u]);
         }
     }
     return (a[0] + a[1]) + (a[2] + a[3]);
@@ -179,7 +186,7 @@ __device__ __forceinline__ void pull_hub_segment(const PullGeom &G, const P &pol
 {
     using Acc = typename P::Acc;
     const uint32_t lo = G.seg_lo[s], hi = G.seg_hi[s];
-    Acc acc = strided_sum<P, AG_WG>(G, pol, lo + threadIdx.x, hi);
+    Acc acc = strided_sum<P, AG_WG, AG_TILE_UNROLL>(G, pol, lo + threadIdx.x, hi);
     acc = block_reduce<Acc, AG_WG>(acc, s_wave);
     if (threadIdx.x == 0)
         G.hub_part[s] = acc_bits<Acc>(acc);
@@ -213,13 +220,13 @@ __device__ __forceinline__ void pull_hub_segment_seq(const PullGeom &G, const P 
         G.hub_part[s] = acc_bits<Acc>(acc);
 }
 
-template <class P>
+template <class P, int U = AG_TILE_UNROLL>
 __device__ __forceinline__ void pull_block_row(const PullGeom &G, const P &pol, uint32_t row,
                                                Red &red, typename P::Acc *s_wave)
 {
     using Acc = typename P::Acc;
     const uint32_t lo = G.off[row], hi = G.off[row + 1];
-    Acc acc = strided_sum<P, AG_WG>(G, pol, lo + threadIdx.x, hi);
+    Acc acc = strided_sum<P, AG_WG, U>(G, pol, lo + threadIdx.x, hi);
     acc = block_reduce<Acc, AG_WG>(acc, s_wave);
     if (threadIdx.x == 0)
         pol.finish(row, acc, red);
@@ -317,22 +324,183 @@ __device__ __forceinline__ void pull_one_item(const PullGeom &G, const P &pol, u
         pull_thread_tile(G, pol, it - G.slot_blk0[4], red, s_vals);
 }
 
-// All work items of one workgroup of the persistent grid.
+// ---------------------------------------------------------------- row tiles
+//
+// The regular schedule hands the rows of the bins up to G.rt_row1 to the workgroups as tiles of
+// consecutive rows (at most AG_TILE_NNZ_MAX in-edges, see ag_row_tiles), whatever their bin: a
+// tile's ids and then its values are gathered with up to 16 loads in flight a lane and staged in
+// LDS, rows of at most lane_max in-edges are summed by one lane in stream order, longer ones by a
+// wavefront, and every row is finished by a lane of its own, so the loads and stores of the
+// update are coalesced. The next tile's ids, and this tile's row bounds and update operands, are
+// in flight while the values arrive: a tile costs one dependent round of loads.
+// A group of lanes per row, four gathers in flight each and a chain of four dependent loads a
+// row (offsets, ids, values, update operands), left the chip waiting. SpMV before -> with row
+// tiles: RMAT-16 9.4 -> 7.0 us, RMAT-18 28 -> 22, RMAT-20 102 -> 78 (0.2 T in-edges/s, the L2
+// request rate that also bounds the blocked pass 1), Erdos-Renyi 300 K rows 29.5 -> 25.
+
+// Update operands of a policy whose update reads nothing of the row.
+struct NoPre {
+};
+
+struct RowTile {
+    uint32_t r0, r1, e0, e1;
+};
+
+template <class P>
+struct TileLds {
+    typename P::Acc *vals;                     // [AG_TILE_NNZ_MAX]
+    typename P::Acc *lsum;                     // [AG_LONG_MAX] sums of the long rows
+    uint32_t *lng;                             // [AG_WG / AG_WAVE][AG_LONG_MAX] each wavefront's
+    uint32_t *cnt;                             // [AG_WG / AG_WAVE]
+};
+
+#define AG_TILE_LDS(P, T)                                             \
+    __shared__ typename P::Acc T##_vals[AG_TILE_NNZ_MAX];             \
+    __shared__ typename P::Acc T##_lsum[AG_LONG_MAX];                 \
+    __shared__ uint32_t T##_lng[AG_WG / AG_WAVE * AG_LONG_MAX];       \
+    __shared__ uint32_t T##_cnt[AG_WG / AG_WAVE];                     \
+    const TileLds<P> T{T##_vals, T##_lsum, T##_lng, T##_cnt}
+
+__device__ __forceinline__ RowTile row_tile_at(const PullGeom &G, uint32_t i)
+{
+    RowTile t{};
+    if (i < G.n_rt) {
+        const uint4 v = G.rt[i];
+        t = RowTile{v.x, v.y, v.z, v.w};
+    }
+    return t;
+}
+
+// A row's values s_vals[b, e) in element order, the first one starting the sum.
+template <typename Acc>
+__device__ __forceinline__ Acc lane_sum(const Acc *s_vals, uint32_t b, uint32_t e)
+{
+    if (e == b)
+        return Acc(0);
+    Acc acc = s_vals[b];
+    uint32_t q = b + 1;
+    for (; q + 4u <= e; q += 4u) {
+        const Acc v0 = s_vals[q], v1 = s_vals[q + 1], v2 = s_vals[q + 2], v3 = s_vals[q + 3];
+        acc = acc + v0;
+        acc = acc + v1;
+        acc = acc + v2;
+        acc = acc + v3;
+    }
+    for (; q < e; q++)
+        acc = acc + s_vals[q];
+    return acc;
+}
+
+template <class P>
+__device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, uint32_t i,
+                                               uint32_t step, Red &red, const TileLds<P> &L)
+{
+    using Acc = typename P::Acc;
+    const uint32_t tid = threadIdx.x, wave = tid / AG_WAVE, lane = tid % AG_WAVE;
+    RowTile cur = row_tile_at(G, i), nxt = row_tile_at(G, i + step);
+    uint32_t w[AG_TILE_UNROLL];
+#pragma unroll
+    for (int u = 0; u < AG_TILE_UNROLL; u++) {
+        const uint32_t j = cur.e0 + tid + u * AG_WG;
+        w[u] = j < cur.e1 ? ld_stream(&G.src[j]) : 0u;
+    }
+    while (cur.r1 > cur.r0) {
+        // this lane's first row: bounds and update operands
+        uint32_t r = cur.r0 + tid, b = 0, e = 0;
+        typename P::Pre pre{};
+        if (r < cur.r1) {
+            b = G.off[r];
+            e = G.off[r + 1];
+            pre = pol.pre(r);
+        }
+#pragma unroll
+        for (int u = 0; u < AG_TILE_UNROLL; u++) {
+            const uint32_t j = cur.e0 + tid + u * AG_WG;
+            if (j < cur.e1)
+                L.vals[j - cur.e0] = pol.edge(j, w[u]);
+        }
+        i += step;
+        const RowTile nn = row_tile_at(G, i + step);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < AG_TILE_UNROLL; u++) {
+            const uint32_t j = nxt.e0 + tid + u * AG_WG;
+            w[u] = j < nxt.e1 ? ld_stream(&G.src[j]) : 0u;   // in flight during the sums
+        }
+        uint32_t nl = 0;   // this wavefront's long rows
+        for (uint32_t q0 = cur.r0 + wave * AG_WAVE; q0 < cur.r1; q0 += AG_WG) {
+            const uint32_t rn = r + AG_WG;
+            uint32_t bn = 0, en = 0;
+            typename P::Pre pn{};
+            if (rn < cur.r1) {
+                bn = G.off[rn];
+                en = G.off[rn + 1];
+                pn = pol.pre(rn);
+            }
+            const bool is_long = r < cur.r1 && e - b > G.lane_max;
+            const uint64_t mask = __ballot(is_long);
+            if (is_long)
+                L.lng[wave * AG_LONG_MAX + nl +
+                      __builtin_popcountll(mask & ((1ull << lane) - 1ull))] = r;
+            else if (r < cur.r1)
+                pol.finish(r, lane_sum(L.vals, b - cur.e0, e - cur.e0), red, pre);
+            nl += (uint32_t)__builtin_popcountll(mask);
+            r = rn;
+            b = bn;
+            e = en;
+            pre = pn;
+        }
+        if (lane == 0)
+            L.cnt[wave] = nl;
+        __syncthreads();
+        // the long rows in wavefront order: the k-th one belongs to the same lane in every run
+        static_assert(AG_WG / AG_WAVE == 4, "four wavefronts' lists");
+        const uint32_t c0 = L.cnt[0], c1 = c0 + L.cnt[1], c2 = c1 + L.cnt[2], c3 = c2 + L.cnt[3];
+        if (c3) {
+            const auto row_of = [&](uint32_t k) {
+                const uint32_t *l = L.lng;
+                return k < c0 ? l[k] : k < c1 ? l[AG_LONG_MAX + k - c0]
+                             : k < c2 ? l[2u * AG_LONG_MAX + k - c1]
+                                      : l[3u * AG_LONG_MAX + k - c2];
+            };
+            uint32_t mine = 0;
+            if (tid < c3) {
+                mine = row_of(tid);
+                pre = pol.pre(mine);
+            }
+            for (uint32_t k = wave; k < c3; k += AG_WG / AG_WAVE) {
+                const uint32_t row = row_of(k);
+                const uint32_t lo = G.off[row] - cur.e0, hi = G.off[row + 1] - cur.e0;
+                Acc acc = Acc(0);
+                for (uint32_t q = lo + lane; q < hi; q += AG_WAVE)
+                    acc = acc + L.vals[q];
+                acc = group_reduce<Acc, AG_WAVE>(acc);
+                if (lane == 0)
+                    L.lsum[k] = acc;
+            }
+            __syncthreads();
+            if (tid < c3)
+                pol.finish(mine, L.lsum[tid], red, pre);
+        }
+        __syncthreads();   // the LDS is reused by the next tile
+        cur = nxt;
+        nxt = nn;
+    }
+}
+
+// All work items of one workgroup of the persistent grid: the items above the row tiles (hub
+// segments and workgroup rows), then tiles.
 template <class P>
 __device__ __forceinline__ void pull_items(const PullGeom &G, const P &pol, Red &red,
-                                           typename P::Acc *s_vals, typename P::Acc *s_wave)
+                                           const TileLds<P> &L, typename P::Acc *s_wave)
 {
-    const uint32_t total = G.slot_blk0[AG_NSLOTS];
-    for (uint32_t it = blockIdx.x; it < total; it += gridDim.x)
-        pull_one_item(G, pol, it, red, s_vals, s_wave);
+    uint32_t it = blockIdx.x;
+    for (; it < G.n_heavy; it += gridDim.x)
+        pull_one_item(G, pol, it, red, L.vals, s_wave);
+    pull_row_tiles(G, pol, it - G.n_heavy, gridDim.x, red, L);
 }
 
 // ---------------------------------------------------------------- source-blocked pull
-
-#define AG_LANE_MAX 64u    // rows of a tile with at most this many elements: a lane each
-#define AG_LONG_MAX 64u    // longer rows of one tile: at most AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1)
-static_assert(AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1u) < AG_LONG_MAX,
-              "the long rows of a full tile must fit the tile's LDS list");
 
 // First pass: a virtual row's sum is stored as its partial; the update waits for the combine.
 template <class P>
@@ -814,7 +982,7 @@ __device__ __forceinline__ void pull_combine_items(const BlockGeom &B, const P &
     for (uint32_t i = blockIdx.x; i < end; i += gridDim.x) {
         const uint32_t first = B.c_item[2 * i], kind = B.c_item[2 * i + 1] & 15u;
         if (kind != AG_ITEM_CTILE) {
-            pull_block_row(B.C, cp, first, red, s_wave);
+            pull_block_row<CombPol<P>, AG_UNROLL>(B.C, cp, first, red, s_wave);
             continue;
         }
         const uint32_t r0 = B.ct_row[2 * first], r1 = B.ct_row[2 * first + 1];
@@ -876,10 +1044,10 @@ __device__ __forceinline__ void pull_hub_finish(const PullGeom &G, const P &pol,
 template <class P>
 __global__ __launch_bounds__(AG_WG) void pull_kernel(PullGeom G, P pol)
 {
-    __shared__ typename P::Acc s_vals[AG_TILE_NNZ_MAX];
+    AG_TILE_LDS(P, tile);
     __shared__ typename P::Acc s_wave[AG_WG / AG_WAVE];
     Red red{};
-    pull_items(G, pol, red, s_vals, s_wave);
+    pull_items(G, pol, red, tile, s_wave);
 }
 
 // Plain source-blocked pull (SpMV): pass 1 with `pol` reading per-edge data in virtual-row

@@ -13,6 +13,10 @@
 #include <time.h>
 #include <unistd.h>
 
+#include <algorithm>
+#include <new>
+#include <vector>
+
 #include "ag_internal.h"
 #include "ag_fixed_dev.h"
 
@@ -224,7 +228,7 @@ extern "C" int ag_graph_free(ag_dgraph *g)
     (void)hipSetDevice(g->dev->ordinal);
     (void)hipStreamSynchronize(g->dev->stream);
     ag_ppr_free_ws(g);
-    void *ptrs[] = {g->d2o, g->off, g->src, g->w, g->wq, g->outdeg, g->tile_row, g->seg_row,
+    void *ptrs[] = {g->d2o, g->off, g->src, g->w, g->wq, g->outdeg, g->tile_row, g->rt, g->seg_row,
                     g->seg_lo, g->seg_hi, g->hub_seg0, g->hub_part, g->vec_a, g->vec_b,
                     g->blk.voff, g->blk.vsrc, g->blk.vw, g->blk.item, g->blk.coff, g->blk.cidx,
                     g->blk.lpos, g->blk.ct_row, g->blk.ct_start, g->blk.ct_pre, g->blk.c_item,
@@ -252,6 +256,10 @@ PullGeom ag_make_geom(const ag_dgraph *g)
     G.seg_hi = g->seg_hi;
     G.hub_seg0 = g->hub_seg0;
     G.hub_part = g->hub_part;
+    G.rt = g->rt;
+    G.n_rt = g->n_rt;
+    G.n_heavy = g->n_heavy;
+    G.lane_max = g->params.thread_max_deg > AG_LANE_MAX ? g->params.thread_max_deg : AG_LANE_MAX;
     G.n = g->n;
     G.n_hubs = g->n_hubs;
     G.seq_hubs = g->params.fp32_order == AG_ORDER_REFERENCE ? 1u : 0u;
@@ -346,6 +354,60 @@ uint32_t ag_pull_grid(const ag_dgraph *g, uint32_t lds_bytes, uint32_t default_p
     return grid < g->total_blocks ? grid : g->total_blocks;
 }
 
+uint32_t ag_tile_grid(const ag_dgraph *g, uint32_t lds_bytes)
+{
+    const uint32_t grid = g->dev->num_cus * wg_per_cu(g, lds_bytes), items = g->n_heavy + g->n_rt;
+    return grid < items ? grid : items;
+}
+
+// Cuts the rows of the bins whose rows fit a tile into row tiles. A tile holds
+// at most `nnz` in-edges (one row may hold more, up to AG_TILE_NNZ_MAX) and `rows` rows: as few
+// as let the resident workgroups finish in as many rounds as full tiles would need, so that
+// small graphs still give every CU work (RMAT-12: 256 in-edges a tile) and the last round is
+// not nearly empty.
+static int cut_row_tiles(ag_dgraph *g, const uint32_t *off, std::vector<uint4> &rt)
+{
+    const ag_plan_params &q = g->params;
+    // bins are ordered by degree: the first bin whose rows may exceed a tile ends the tiles
+    const uint32_t max_deg[] = {q.thread_max_deg, q.group16_max_deg, q.wave_max_deg};
+    int bins = 0;
+    while (bins < 3 && max_deg[bins] <= AG_TILE_NNZ_MAX)
+        bins++;
+    const uint32_t row1 = g->bin_row[bins];
+    const uint64_t m1 = g->n ? off[row1] : 0u;
+    g->n_heavy = g->slot_blk0[AG_NSLOTS - bins];   // slots run from the heaviest bin down
+    const uint64_t slots = (uint64_t)g->dev->num_cus * (q.wg_per_cu ? q.wg_per_cu : 4u);
+    const uint64_t items = m1 / AG_TILE_NNZ_MAX + row1 / AG_TILE_ROWS_MAX + g->n_heavy + 1u;
+    const uint64_t rounds = (items + slots - 1) / slots;
+    try {
+        const uint64_t budget = slots * rounds, room = budget - g->n_heavy;
+        uint64_t nnz = (m1 + room - 1u) / room;   // items covers n_heavy: room > 0
+        for (nnz = nnz < AG_WG ? AG_WG : nnz;; nnz += nnz / 8u) {
+            nnz = nnz < q.tile_nnz ? nnz : q.tile_nnz;
+            const uint32_t rows = q.tile_rows < nnz ? q.tile_rows
+                                                    : nnz < AG_WG ? AG_WG : (uint32_t)nnz;
+            const bool last_try = nnz == q.tile_nnz;
+            rt.clear();
+            uint32_t r = 0;
+            while (r < row1 && (last_try || rt.size() + g->n_heavy < budget)) {
+                const uint32_t last = row1 - r < rows ? row1 : r + rows;
+                // the last row end within nnz in-edges (off is their prefix sum), a row at least
+                const uint64_t lim = (uint64_t)off[r] + nnz;
+                uint32_t e = (uint32_t)(std::upper_bound(off + r + 1, off + last + 1, lim) - off);
+                e = e - 1u > r ? e - 1u : r + 1u;
+                rt.push_back(make_uint4(r, e, off[r], off[e]));
+                r = e;
+            }
+            if (r >= row1)
+                break;
+        }
+    } catch (const std::bad_alloc &) {
+        return ag_set_error(AG_ERR_OOM, "host allocation failed");
+    }
+    g->n_rt = (uint32_t)rt.size();
+    return AG_OK;
+}
+
 // vec_a / vec_b: two scratch arrays of `bytes` each, used to permute SpMV/gather vectors
 // between original and device order.
 int ag_ensure_vec(ag_dgraph *g, size_t bytes)
@@ -417,6 +479,9 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
     if (st == AG_OK && plan.w) st = dev_upload(g, &g->w, plan.w, plan.m);
     if (st == AG_OK) st = dev_upload(g, &g->outdeg, plan.outdeg, plan.n);
     if (st == AG_OK) st = dev_upload(g, &g->tile_row, plan.tile_row, (size_t)plan.n_tiles + 1);
+    std::vector<uint4> rt;   // outlives its copy: freed after the wait below
+    if (st == AG_OK) st = cut_row_tiles(g, plan.off, rt);
+    if (st == AG_OK) st = dev_upload(g, &g->rt, rt.data(), rt.size());
     if (st == AG_OK) st = dev_upload(g, &g->seg_row, plan.seg_row, plan.n_segs);
     if (st == AG_OK) st = dev_upload(g, &g->seg_lo, plan.seg_lo, plan.n_segs);
     if (st == AG_OK) st = dev_upload(g, &g->seg_hi, plan.seg_hi, plan.n_segs);

@@ -38,7 +38,12 @@ struct SpmvF32Pol {
     {
         return __fmul_rn(xs, WEIGHTED ? __builtin_nontemporal_load(&w[j]) : 0.0001f);
     }
-    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &) const { y[r] = sum; }
+    using Pre = NoPre;
+    __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
+    __device__ __forceinline__ void finish(uint32_t r, float sum, Red &, Pre = Pre{}) const
+    {
+        y[r] = sum;
+    }
 };
 
 // Hot pass of the FP32 SpMV (see pull_hot_items): x gathered from LDS copies of its hot
@@ -66,7 +71,12 @@ struct SpmvFixPol {
             (uint64_t)xq[s] * (uint64_t)(WEIGHTED ? __builtin_nontemporal_load(&wq[j]) : wconst);
         return (uint64_t)(uint32_t)(wide >> 16);
     }
-    __device__ __forceinline__ void finish(uint32_t r, uint64_t sum, Red &) const { y[r] = sum; }
+    using Pre = NoPre;
+    __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
+    __device__ __forceinline__ void finish(uint32_t r, uint64_t sum, Red &, Pre = Pre{}) const
+    {
+        y[r] = sum;
+    }
 };
 
 template <typename T>
@@ -152,7 +162,12 @@ struct Gather {
     const VT *v;
     A *out;
     __device__ __forceinline__ A edge(uint32_t, uint32_t s) const { return (A)v[s]; }
-    __device__ __forceinline__ void finish(uint32_t r, A sum, Red &) const { out[r] = sum; }
+    using Pre = NoPre;
+    __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
+    __device__ __forceinline__ void finish(uint32_t r, A sum, Red &, Pre = Pre{}) const
+    {
+        out[r] = sum;
+    }
 };
 
 } // namespace
@@ -170,7 +185,7 @@ static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps, double *avg_ms)
         AG_HIP(hipEventCreate(&e1));
         AG_HIP(hipEventRecord(e0, stream));
     }
-    const uint32_t grid = ag_pull_grid(g, AG_TILE_NNZ_MAX * (uint32_t)sizeof(typename P::Acc));
+    const uint32_t grid = ag_tile_grid(g, AG_TILE_NNZ_MAX * (uint32_t)sizeof(typename P::Acc));
     for (uint32_t i = 0; i < reps && g->total_blocks; i++) {
         pull_kernel<P><<<grid, AG_WG, 0, stream>>>(G, pol);
         if (g->n_hubs)

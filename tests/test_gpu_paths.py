@@ -59,3 +59,43 @@ def test_data_driven_long_rows(device, degree):
     np.testing.assert_array_equal(run.scaled.view(np.uint32), lists.scaled.view(np.uint32))
     np.testing.assert_array_equal(run.hist_active, lists.hist_active)
     dg.close()
+
+
+TILE_PLANS = {"default": {}, "few-workgroups": dict(wg_per_cu=1), "small-tiles": dict(tile_nnz=64),
+              # rows above 64 in-edges in the thread bin: still one lane, in stream order
+              "long-lanes": dict(thread_max_deg=200, group16_max_deg=300),
+              # wave rows that need not fit a tile are left to their groups of lanes
+              "wide-waves": dict(wave_max_deg=6000, block_max_deg=6001),
+              "wide-groups": dict(group16_max_deg=5000, wave_max_deg=5001, block_max_deg=5002)}
+
+
+@pytest.mark.parametrize("pname", list(TILE_PLANS))
+@pytest.mark.parametrize("n", [20011, 700_001])
+def test_row_tiles(device, pname, n):
+    """The regular schedule's row tiles at the ends of the row classes, of a tile's in-edges and
+    rows and with as many rounds as one workgroup per CU needs: fixed point exact, FP32 rows
+    summed by one lane equal to the sequential sum, the others within a reordered sum's bound."""
+    degrees = EDGE_DEGREES + [4095, 6000, 6001, 9000, 16384, 16385]
+    degrees = [d for d in degrees if d < n - len(degrees)]
+    g = graph_with_degrees(degrees, n)
+    p = TILE_PLANS[pname]
+    dg = device.upload(g, params=ag.plan_params(src_block_bits=ag.SRC_BLOCK_OFF, **p))
+    rng = np.random.default_rng(11)
+    xq = rng.integers(0, 1 << 20, n, dtype=np.uint32)
+    yq, _ = dg.spmv_fixed(xq)
+    wc = int(oracle.fixed_encode(32, np.array([0.0001], np.float32))[0])
+    np.testing.assert_array_equal(
+        yq, oracle.spmv_fixed(g.inv_idx, g.in_degree, g.inv_src, None, wc, xq))
+    x = rng.random(n, dtype=np.float32)
+    y, _ = dg.spmv(x)
+    ref = oracle.spmv_f32(g.inv_idx, g.in_degree, g.inv_src, None, x)
+    lane = g.in_degree <= max(64, p.get("thread_max_deg", 0))
+    if pname not in ("wide-groups",):
+        np.testing.assert_array_equal(y[lane].view(np.uint32), ref[lane].view(np.uint32))
+    d = g.in_degree.astype(np.float64)
+    assert np.all(np.abs(y.astype(np.float64) - ref) <= 2 * d * 2.0 ** -24 * np.abs(ref))
+    run = dg.pagerank(kind=ag.KIND_FIXED32, max_iterations=6, stop_rule=ag.STOP_NONE)
+    want = oracle.pagerank_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, kind=32,
+                                max_iterations=6, stop_rule=2)
+    np.testing.assert_array_equal(run.ranks.view(np.uint32), want.ranks.view(np.uint32))
+    dg.close()
