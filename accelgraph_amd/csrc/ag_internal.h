@@ -9,17 +9,6 @@
 #include "../host/ag_plan.h"
 
 #define AG_MAX_EVENTS 2
-// Push bins (ag_push.h): rows per bin (the LDS row array of phase 2, and 16-bit local row
-// ids) and slots per multi-row bin (one workgroup's work); a row with more in-edges than
-// AG_PB_SLOTS is a bin by itself.
-#ifndef AG_PB_ROWS
-#define AG_PB_ROWS 4096u
-#endif
-#ifndef AG_PB_SLOTS
-#define AG_PB_SLOTS 131072u
-#endif
-static_assert(AG_PB_ROWS >= 2u && AG_PB_ROWS <= 65536u, "push bins use 16-bit local row ids");
-
 #define AG_LANE_MAX 64u    // rows of a tile with at most this many elements: a lane each
 
 struct ag_device {
@@ -66,18 +55,9 @@ struct ag_dgraph {
     uint32_t *btick;     // [2 * AG_NXCD] pass-1 ticket counters (BlockGeom::tick), zeroed
     uint32_t bdyn;       // pass-1 tiles handed out by ticket (BlockGeom::dyn)
     uint32_t *vwq;       // [blk.mb] FloatToFixed32(vw), built on the first fixed SpMV
-    // forward CSR in device row ids (out-edges), built on the first push / data-driven run
+    // forward CSR in device row ids (out-edges), built on the first run with worklists
     uint32_t *fwd_off;   // [n+1]
-    uint32_t *fwd_src;   // [m] source of every out-edge (row id of the forward CSR)
     uint32_t *fwd_dst;   // [m] destination, ascending within a row
-    float *fwd_w;        // [m] weight of every out-edge (null for an unweighted graph)
-    // push bins (ag_graph_push_bins): ranges of destination rows, and the slot of every
-    // out-edge in the bin buffer (bins in row order, forward order inside a bin)
-    uint32_t pb_nbins;
-    uint32_t *pb_row;    // [pb_nbins+1] first row of every bin (one allocation with pb_off)
-    uint32_t *pb_off;    // [pb_nbins+1] first slot of every bin
-    uint32_t *pb_pos;    // [m] slot of every out-edge
-    uint16_t *pb_dst;    // [m] row of every slot minus its bin's first row
     // scratch for permuted vectors (x, y) of SpMV / gather, sized lazily
     void *vec_a;
     void *vec_b;
@@ -189,7 +169,6 @@ struct ag_pr_session {
     float *rank;
     void *c[2];
     void *c16[2];
-    void *push_vals;            // push: the bin buffer, one value per out-edge slot [m]
     uint32_t *dd_queue[2];      // data-driven pull: worklists by iteration parity
     uint8_t *dd_flag;           // data-driven pull: next-worklist marks [n rounded up to 4]
     double *fin_part;
@@ -206,12 +185,9 @@ struct ag_pr_session {
 // Enqueue one PageRank iteration of a session (main + finish kernel).
 int ag_pr_launch_iteration(ag_pr_session *s);
 
-// Builds g->fwd_off / fwd_src / fwd_dst (the forward CSR in device row ids) from the uploaded
-// inverse CSR, once; later calls return at once.
+// Builds g->fwd_off / fwd_dst (the forward CSR in device row ids) from the uploaded inverse CSR,
+// once; later calls return at once.
 int ag_graph_forward(ag_dgraph *g);
-
-// Builds g->pb_* (push bins and slots, after the forward CSR), once; later calls return at once.
-int ag_graph_push_bins(ag_dgraph *g);
 
 int ag_set_error(int status, const char *fmt, ...);
 int ag_hip_fail(hipError_t e, const char *what, const char *file, int line);

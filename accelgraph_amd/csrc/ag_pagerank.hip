@@ -34,7 +34,6 @@
 #include "ag_internal.h"
 #include "ag_fixed_dev.h"
 #include "ag_pull_kernel.h"
-#include "ag_push.h"
 
 // Accumulator of the data-driven pull on a source-blocked plan: the FP32 sum of the in-edges
 // and whether any in-neighbour took a new rank in the previous iteration (0 or 1, reduced
@@ -1006,69 +1005,6 @@ __global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF3
     pr_store_partial(C, red);
 }
 
-// ---------------------------------------------------------------- push direction
-//
-// pageRankPushGraphCSR (pageRank.c:1111-1272) and pageRankPushFixedPointGraphCSR
-// (:1992-2117) keep the pull's host loop and form next[u] by scattering every source's
-// contribution along its out-edges. Here the scatter is propagation-blocked (ag_push.h):
-// phase 1 copies every out-edge's source contribution into its bin slot, phase 2 adds each
-// bin's slots per row in LDS and applies the kind's update to every row of the bin, then the
-// one-workgroup finish closes the iteration. Fixed-point sums are exact u64 sums, equal to
-// the pull's bit for bit; FP32 sums take the LDS atomics' order (a hub row's bin: a fixed
-// tree), which may differ from run to run (FP32 bar).
-
-template <int KC>
-struct PushVal {
-    using T = typename FixT<KC>::T;
-    using A = unsigned long long;
-};
-template <>
-struct PushVal<0> {
-    using T = float;
-    using A = float;
-};
-
-template <int KC>
-__global__ __launch_bounds__(AG_WG) void pr_push_scatter_kernel(PrCtl C, PrF32Args A, uint32_t m,
-                                                                const uint32_t *fsrc,
-                                                                const uint32_t *pos, void *vals)
-{
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    using VT = typename PushVal<KC>::T;
-    const VT *c = (const VT *)A.c32[(*(volatile const uint32_t *)&st->iter) & 1u];
-    pb_scatter(m, pos, (VT *)vals,
-               [&](uint32_t j) { return c[__builtin_nontemporal_load(&fsrc[j])]; });
-}
-
-template <int KC>
-__global__ __launch_bounds__(AG_WG) void pr_push_bins_kernel(PrCtl C, PrF32Args A, PushBins P,
-                                                             const void *vals)
-{
-    using VT = typename PushVal<KC>::T;
-    using AT = typename PushVal<KC>::A;
-    __shared__ AT s_acc[AG_PB_ROWS];
-    __shared__ AT s_wave[AG_WG / AG_WAVE];
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
-    Red red{};
-    if constexpr (KC == 0) {
-        const uint32_t rd = iter & 1u, wr = rd ^ 1u;
-        const PrF32Pol<float, float> p{(const float *)A.c32[rd], (float *)A.c32[wr], A.rank,
-                                       A.outdeg, A.base, A.damp, A.dn, A.eps};
-        pb_bins(P, (const VT *)vals, s_acc, s_wave,
-                [&](uint32_t r, float sum) { p.finish(r, sum, red); });
-    } else {
-        const PrFixPol<KC> p = fix_policy<KC>(iter, A);
-        pb_bins(P, (const VT *)vals, s_acc, s_wave,
-                [&](uint32_t r, AT sum) { p.finish(r, (uint64_t)sum, red); });
-    }
-    pr_store_partial(C, red);
-}
-
 // Closes an iteration whose every row was updated by the preceding launch.
 __global__ __launch_bounds__(AG_FIN_WG) void pr_plain_finish(PrCtl C)
 {
@@ -1398,7 +1334,7 @@ static void session_free(ag_pr_session *s)
     (void)hipSetDevice(s->g->dev->ordinal);
     (void)hipStreamSynchronize(s->g->dev->stream);
     void *ptrs[] = {s->st, s->part_err, s->part_act, s->part_cmax, s->hist_err, s->hist_act,
-                    s->rank, s->c[0], s->c[1], s->c16[0], s->c16[1], s->push_vals, s->dd_queue[0],
+                    s->rank, s->c[0], s->c[1], s->c16[0], s->c16[1], s->dd_queue[0],
                     s->dd_queue[1], s->dd_flag, s->fin_part, s->fin_sum, s->user};
     for (void *p : ptrs)
         if (p)
@@ -1522,8 +1458,8 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
         return ag_set_error(AG_ERR_INVALID, "bad init mode or missing init_ranks");
     if (!(o.epsilon >= 0.0))
         return ag_set_error(AG_ERR_INVALID, "epsilon must be >= 0");
-    if (o.direction == AG_DIR_PUSH || dd_lists) {
-        const int fst = dd_lists ? ag_graph_forward(g) : ag_graph_push_bins(g);
+    if (dd_lists) {
+        const int fst = ag_graph_forward(g);
         if (fst != AG_OK)
             return fst;
     }
@@ -1564,8 +1500,6 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
         AG_TRY(salloc(s, &s->c16[0], (size_t)n * 2));
         AG_TRY(salloc(s, &s->c16[1], (size_t)n * 2));
     }
-    if (o.direction == AG_DIR_PUSH)   // one contribution per out-edge slot, stored as c[]
-        AG_TRY(salloc(s, &s->push_vals, (size_t)g->m * celem));
     if (dd_lists) {
         AG_TRY(salloc(s, (void **)&s->dd_queue[0], (size_t)n * sizeof(uint32_t)));
         AG_TRY(salloc(s, (void **)&s->dd_queue[1], (size_t)n * sizeof(uint32_t)));
@@ -1687,6 +1621,14 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
         AG_PR_LAUNCH_BLOCKED(BLK, CMB, FIN);                                 \
     } while (0)
 
+// The push (pageRankPushGraphCSR, pageRank.c:1111-1272; pageRankPushFixedPointGraphCSR,
+// :1992-2117) adds every contribution into its destinations' sums: the pull's sums, and the same
+// ranks. It runs the pull's kernels, whose first pass on a source-blocked plan is a push of each
+// source block's pre-added pieces into their rows' slots. Scattering along the out-edges measured
+// slower in every form: RMAT-22 FP32 1036 us an iteration with binned stores and LDS float adds
+// (0.2 T/s over the chip, and 27 bytes of HBM writes per 4-byte store), against 270 us; with
+// memory atomics 33 ms on RMAT-25. The pull's order is also closer to 64 bits (RMAT-22, 10
+// iterations: 6e-8 against 3e-6) and the same on every run.
 int ag_pr_launch_iteration(ag_pr_session *s)
 {
     ag_dgraph *g = s->g;
@@ -1718,28 +1660,6 @@ int ag_pr_launch_iteration(ag_pr_session *s)
     A.eps = s->o.epsilon;
     const uint32_t lds = (s->kind_code >= 8) ? AG_TILE_NNZ_MAX * 8u : AG_TILE_NNZ_MAX * 4u;
     dim3 block(AG_WG), fin(AG_FIN_WG);
-    if (s->o.direction == AG_DIR_PUSH) {
-        const uint32_t gs = (g->dev->num_cus * 16u + AG_NXCD - 1u) / AG_NXCD * AG_NXCD;
-        const uint32_t gu = ag_quant_grid(g);
-        const PushBins P{g->pb_nbins, g->pb_row, g->pb_off, g->pb_pos, g->pb_dst};
-        C.nparts = gu;
-        switch (s->kind_code) {
-#define AG_PUSH(KC)                                                                              \
-    pr_push_scatter_kernel<KC><<<gs, block, 0, stream>>>(C, A, g->m, g->fwd_src, g->pb_pos,    \
-                                                         s->push_vals);                         \
-    pr_push_bins_kernel<KC><<<gu, block, 0, stream>>>(C, A, P, s->push_vals);                  \
-    break
-        case 0: AG_PUSH(0);
-        case 64: AG_PUSH(64);
-        case 32: AG_PUSH(32);
-        case 16: AG_PUSH(16);
-        default: AG_PUSH(8);
-#undef AG_PUSH
-        }
-        pr_plain_finish<<<1, fin, 0, stream>>>(C);
-        AG_HIP(hipGetLastError());
-        return AG_OK;
-    }
     if (s->o.direction == AG_DIR_DATA_DRIVEN && blocked && !s->dd_queue[0]) {
         const BlockGeom B = ag_make_block_geom(g);
         const BlockGeom &B1 = B;

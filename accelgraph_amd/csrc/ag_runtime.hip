@@ -233,8 +233,7 @@ extern "C" int ag_graph_free(ag_dgraph *g)
                     g->blk.voff, g->blk.vsrc, g->blk.vw, g->blk.item, g->blk.coff, g->blk.cidx,
                     g->blk.lpos, g->blk.ct_row, g->blk.ct_start, g->blk.ct_pre, g->blk.c_item,
                     g->blk.hgrp, g->blk.vsp, g->blk.tbase,
-                    g->vpart, g->btick, g->vwq, g->fwd_off, g->fwd_src, g->fwd_dst,
-                    g->fwd_w, g->pb_row, g->pb_pos, g->pb_dst};
+                    g->vpart, g->btick, g->vwq, g->fwd_off, g->fwd_dst};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);

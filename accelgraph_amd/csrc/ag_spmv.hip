@@ -7,8 +7,8 @@
 // SCALEF = 16 (FixedPoint/cu/cu_sum_kernel_control.sv:155-164, FixedPoint/pkg/
 // globals_cu_pkg.sv:37). Each call computes y = A x once per repetition (the RTL overwrites
 // y every run). Unweighted graphs use the constant weight 0.0001f (SPMV.c:1206). The push
-// forms (SPMV.c:752-848, 1017-1136) scatter along the forward CSR and accumulate across
-// repetitions, as the reference's output is never cleared there.
+// forms (SPMV.c:752-848, 1017-1136) accumulate across repetitions, as the reference's output is
+// never cleared there.
 //
 // The raw gather is the sum kernel itself (cu_PageRank/CSR/PULL/*/cu/cu_sum_kernel_control.sv)
 // on caller-supplied per-vertex values; it exists so the gather arithmetic can be checked
@@ -19,7 +19,6 @@
 #include "ag_internal.h"
 #include "ag_fixed_dev.h"
 #include "ag_pull_kernel.h"
-#include "ag_push.h"
 
 namespace {
 
@@ -95,53 +94,53 @@ __global__ void permute_out_kernel(uint32_t n, const T *dev, const uint32_t *d2o
         orig[d2o[r]] = dev[r];
 }
 
-// SpMV push (SPMV.c:752-848, 1017-1136): every source adds w * x[src] into its out-edges'
-// destinations. The reference never clears the output between iterations, so repetitions
-// accumulate (y = reps * A x). Propagation-blocked (ag_push.h): phase 1 writes every
-// out-edge's product into its bin slot, phase 2 adds each bin's slots per row in LDS and adds
-// the row's sum to y. FP32: binary32 products, summed in the LDS atomics' order (a hub row's
-// bin: a fixed tree). Fixed point: Q32.32 x and weights, MULFixed64V1 products, exact u64 sums.
-template <bool WEIGHTED>
-__global__ __launch_bounds__(AG_WG) void spmv_push_scatter_kernel(uint32_t m, const uint32_t *fsrc,
-                                                                  const uint32_t *pos,
-                                                                  const float *fw, const float *x,
-                                                                  float *vals)
-{
-    pb_scatter(m, pos, vals, [&](uint32_t j) {
-        const float w = WEIGHTED ? __builtin_nontemporal_load(&fw[j]) : 0.0001f;
-        return __fmul_rn(w, x[__builtin_nontemporal_load(&fsrc[j])]);
-    });
-}
+// SpMV push (SPMV.c:752-848, 1017-1136): the reference adds w * x[src] into every out-edge's
+// destination and never clears the output between iterations, so repetitions accumulate
+// (y = reps * A x). The products' sums are the pull's, so the push is the pull with an update
+// that adds to y: RMAT-22 997 -> 261 us (FP32) and 1073 -> 317 us (Q32.32) a product, RMAT-16
+// 175 -> 7.4 us, against scattering into bins and adding those in LDS. FP32: binary32 products,
+// added in the pull's order. Fixed point: Q32.32 x and weights, MULFixed64V1 products, exact u64
+// sums.
+template <typename A>
+struct AddTo {
+    A *y;
+    using Pre = A;
+    __device__ __forceinline__ A pre(uint32_t r) const { return y[r]; }
+    __device__ __forceinline__ void finish(uint32_t r, A sum, Red &, A old) const
+    {
+        y[r] = old + sum;
+    }
+    __device__ __forceinline__ void finish(uint32_t r, A sum, Red &red) const
+    {
+        finish(r, sum, red, pre(r));
+    }
+};
 
 template <bool WEIGHTED>
-__global__ __launch_bounds__(AG_WG) void spmv_push_fixed_scatter_kernel(
-    uint32_t m, const uint32_t *fsrc, const uint32_t *pos, const float *fw, const uint64_t *xq,
-    uint64_t wc, uint64_t *vals)
-{
-    pb_scatter(m, pos, vals, [&](uint32_t j) {
-        const uint64_t w =
-            WEIGHTED ? ag_dev_double_to_fixed64((double)__builtin_nontemporal_load(&fw[j])) : wc;
-        return ag_dev_mul_fixed64(w, xq[__builtin_nontemporal_load(&fsrc[j])]);
-    });
-}
+struct SpmvPushPol : AddTo<float> {
+    using Acc = float;
+    SpmvF32Pol<WEIGHTED> p;
+    __device__ __forceinline__ float edge(uint32_t j, uint32_t s) const { return p.edge(j, s); }
+    __device__ __forceinline__ float edge_val(uint32_t j, float xs) const
+    {
+        return p.edge_val(j, xs);
+    }
+};
 
-__global__ __launch_bounds__(AG_WG) void spmv_push_bins_kernel(PushBins P, const float *vals,
-                                                               float *y)
-{
-    __shared__ float s_acc[AG_PB_ROWS];
-    __shared__ float s_wave[AG_WG / AG_WAVE];
-    pb_bins(P, vals, s_acc, s_wave, [&](uint32_t r, float sum) { y[r] = y[r] + sum; });
-}
-
-__global__ __launch_bounds__(AG_WG) void spmv_push_fixed_bins_kernel(PushBins P,
-                                                                     const uint64_t *vals,
-                                                                     uint64_t *y)
-{
-    __shared__ unsigned long long s_acc[AG_PB_ROWS];
-    __shared__ unsigned long long s_wave[AG_WG / AG_WAVE];
-    pb_bins(P, vals, s_acc, s_wave,
-            [&](uint32_t r, unsigned long long sum) { y[r] += (uint64_t)sum; });
-}
+template <bool WEIGHTED>
+struct SpmvPushFixPol : AddTo<uint64_t> {
+    using Acc = uint64_t;
+    const uint64_t *xq;
+    const float *w;
+    uint64_t wconst;
+    __device__ __forceinline__ uint64_t edge(uint32_t j, uint32_t s) const
+    {
+        const uint64_t wq =
+            WEIGHTED ? ag_dev_double_to_fixed64((double)__builtin_nontemporal_load(&w[j]))
+                     : wconst;
+        return ag_dev_mul_fixed64(wq, xq[s]);
+    }
+};
 
 __global__ __launch_bounds__(AG_WG) void zero_u32_kernel(uint32_t *p, uint32_t count)
 {
@@ -209,7 +208,7 @@ static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps, double *avg_ms)
     return st;
 }
 
-// The hot pass of a blocked SpMV: FP32 only (the fixed-point form gathers everything in
+// The hot pass of a blocked SpMV pull: FP32 only (the fixed-point form gathers everything in
 // pass 1). Returns whether it was launched.
 template <class P>
 static bool spmv_hot_launch(const ag_dgraph *, const BlockGeom &, const P &, hipStream_t)
@@ -419,51 +418,18 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
     return ag_wait_stream(g->dev);
 }
 
-// reps propagation-blocked push passes into yd (ywords u32 words, zeroed first) through a
-// bin buffer of m values of vbytes each, timed with HIP events. launch(p1, p2, vals) enqueues
-// one pass with phase-1 and phase-2 grids p1 and p2.
-template <class L>
-static int run_push(ag_dgraph *g, uint32_t reps, double *avg_ms, void *yd, uint32_t ywords,
-                    size_t vbytes, const L &launch)
+// Clears y and runs `reps` accumulating passes: pv reads per-edge data in virtual-row order, pu
+// in regular order.
+template <class P>
+static int run_push(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps, double *avg_ms)
 {
-    hipStream_t stream = g->dev->stream;
-    void *vals = NULL;
-    AG_HIP(hipMalloc(&vals, (g->m ? g->m : 1u) * vbytes));
-    const uint32_t zb = (ywords + AG_WG - 1) / AG_WG;
-    zero_u32_kernel<<<zb < 4096u ? (zb ? zb : 1u) : 4096u, AG_WG, 0, stream>>>((uint32_t *)yd,
-                                                                               ywords);
-    hipEvent_t e0 = NULL, e1 = NULL;
-    hipError_t e = hipSuccess;
-    if (avg_ms) {
-        e = hipEventCreate(&e0);
-        if (e == hipSuccess)
-            e = hipEventCreate(&e1);
-        if (e == hipSuccess)
-            e = hipEventRecord(e0, stream);
-    }
-    const uint32_t p1 = (g->dev->num_cus * 16u + AG_NXCD - 1u) / AG_NXCD * AG_NXCD;
-    const uint32_t p2 = g->pb_nbins < g->dev->num_cus * 8u ? g->pb_nbins : g->dev->num_cus * 8u;
-    for (uint32_t i = 0; e == hipSuccess && i < reps && g->m; i++)
-        launch(p1, p2, vals);
-    if (e == hipSuccess)
-        e = hipGetLastError();
-    if (e == hipSuccess && avg_ms)
-        e = hipEventRecord(e1, stream);
-    int st = (e == hipSuccess) ? ag_wait_stream(g->dev) : ag_hip_fail(e, "push launch", __FILE__, __LINE__);
-    if (st == AG_OK && avg_ms) {
-        float ms = 0.0f;
-        e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess)
-            st = ag_hip_fail(e, "hipEventElapsedTime", __FILE__, __LINE__);
-        *avg_ms = reps ? (double)ms / reps : 0.0;
-    }
-    if (e0)
-        (void)hipEventDestroy(e0);
-    if (e1)
-        (void)hipEventDestroy(e1);
-    (void)hipStreamSynchronize(stream);
-    (void)hipFree(vals);
-    return st;
+    const uint32_t words = (uint32_t)(sizeof(*pu.y) / 4u) * g->n;
+    const uint32_t zb = (words + AG_WG - 1) / AG_WG;
+    zero_u32_kernel<<<zb < 4096u ? zb : 4096u, AG_WG, 0, g->dev->stream>>>((uint32_t *)pu.y,
+                                                                           words);
+    AG_HIP(hipGetLastError());
+    return g->blk.bits ? run_pull_blocked(g, pv, pu, reps, avg_ms)
+                       : run_pull(g, pu, reps, avg_ms);
 }
 
 extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t reps, double *avg_ms)
@@ -476,9 +442,7 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     if (n == 0)
         return AG_OK;
     AG_HIP(hipSetDevice(g->dev->ordinal));
-    int st = ag_graph_push_bins(g);
-    if (st == AG_OK)
-        st = ag_ensure_vec(g, (size_t)n * sizeof(uint64_t));
+    int st = ag_ensure_vec(g, (size_t)n * sizeof(uint64_t));
     if (st != AG_OK)
         return st;
     hipStream_t stream = g->dev->stream;
@@ -489,18 +453,10 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     AG_HIP(hipMemcpyAsync(xo, x, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
-    const uint32_t m = g->m;
-    const float *fw = g->fwd_w;
-    const PushBins P{g->pb_nbins, g->pb_row, g->pb_off, g->pb_pos, g->pb_dst};
-    st = run_push(g, reps, avg_ms, yd, n, sizeof(float), [&](uint32_t p1, uint32_t p2, void *v) {
-        if (fw)
-            spmv_push_scatter_kernel<true><<<p1, AG_WG, 0, stream>>>(m, g->fwd_src, g->pb_pos, fw,
-                                                                     xd, (float *)v);
-        else
-            spmv_push_scatter_kernel<false><<<p1, AG_WG, 0, stream>>>(m, g->fwd_src, g->pb_pos,
-                                                                      NULL, xd, (float *)v);
-        spmv_push_bins_kernel<<<p2, AG_WG, 0, stream>>>(P, (const float *)v, yd);
-    });
+    st = g->w ? run_push(g, SpmvPushPol<true>{{yd}, {xd, g->blk.vw, NULL}},
+                         SpmvPushPol<true>{{yd}, {xd, g->w, NULL}}, reps, avg_ms)
+              : run_push(g, SpmvPushPol<false>{{yd}, {xd, NULL, NULL}},
+                         SpmvPushPol<false>{{yd}, {xd, NULL, NULL}}, reps, avg_ms);
     if (st != AG_OK)
         return st;
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
@@ -520,9 +476,7 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     if (n == 0)
         return AG_OK;
     AG_HIP(hipSetDevice(g->dev->ordinal));
-    int st = ag_graph_push_bins(g);
-    if (st == AG_OK)
-        st = ag_ensure_vec(g, (size_t)n * sizeof(uint64_t) * 2);
+    int st = ag_ensure_vec(g, (size_t)n * sizeof(uint64_t) * 2);
     if (st != AG_OK)
         return st;
     hipStream_t stream = g->dev->stream;
@@ -533,20 +487,11 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     AG_HIP(hipMemcpyAsync(xo, xq, (size_t)n * sizeof(uint64_t), hipMemcpyHostToDevice, stream));
     permute_in_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
-    const uint32_t m = g->m;
-    const float *fw = g->fwd_w;
     const uint64_t wc = DoubleToFixed64((double)0.0001f);   // SPMV.c:1080
-    const PushBins P{g->pb_nbins, g->pb_row, g->pb_off, g->pb_pos, g->pb_dst};
-    st = run_push(g, reps, avg_ms, yd, 2u * n, sizeof(uint64_t),
-                  [&](uint32_t p1, uint32_t p2, void *v) {
-        if (fw)
-            spmv_push_fixed_scatter_kernel<true><<<p1, AG_WG, 0, stream>>>(
-                m, g->fwd_src, g->pb_pos, fw, xd, 0ull, (uint64_t *)v);
-        else
-            spmv_push_fixed_scatter_kernel<false><<<p1, AG_WG, 0, stream>>>(
-                m, g->fwd_src, g->pb_pos, NULL, xd, wc, (uint64_t *)v);
-        spmv_push_fixed_bins_kernel<<<p2, AG_WG, 0, stream>>>(P, (const uint64_t *)v, yd);
-    });
+    st = g->w ? run_push(g, SpmvPushFixPol<true>{{yd}, xd, g->blk.vw, 0u},
+                         SpmvPushFixPol<true>{{yd}, xd, g->w, 0u}, reps, avg_ms)
+              : run_push(g, SpmvPushFixPol<false>{{yd}, xd, NULL, wc},
+                         SpmvPushFixPol<false>{{yd}, xd, NULL, wc}, reps, avg_ms);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);

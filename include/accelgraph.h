@@ -251,12 +251,9 @@ typedef struct ag_pr_options {
 
 /* Direction of the sum (pageRankGraphCSR's pushpull codes, pageRank.c:874-939):
  *   PULL         gather over in-edges (codes 0, 2, 4, 9-13)
- *   PUSH         scatter every contribution along the out-edges, then update every vertex
- *                (codes 1 and 3, pageRank.c:1111-1272, 1992-2117), propagation-blocked: each
- *                out-edge writes its source's contribution to a slot of its destination's
- *                bin, and each bin's slots are added per row in LDS; AG_KIND_F32 with f32
- *                storage or a fixed-point kind. FP32 sums take the LDS atomics' order;
- *                fixed-point sums are exact and equal the pull's
+ *   PUSH         every source adds its contribution along its out-edges, then every vertex is
+ *                updated (codes 1 and 3, pageRank.c:1111-1272, 1992-2117): the pull's sums, taken
+ *                by the pull's kernels; AG_KIND_F32 with f32 storage or a fixed-point kind
  *   DATA_DRIVEN  pull over a worklist (code 6, pageRank.c:2810-2969): only listed vertices
  *                gather; a vertex whose |delta| >= epsilon takes its new rank and lists its
  *                out-neighbours for the next iteration, others keep their rank; AG_KIND_F32
@@ -265,8 +262,7 @@ typedef struct ag_pr_options {
  *                order on unblocked plans, in the pull's order on source-blocked ones. User
  *                starts on unblocked plans, and user starts with negative entries, keep
  *                explicit worklists
- * PUSH, and DATA_DRIVEN with worklists, build the graph's forward CSR on the device on first
- * use. */
+ * DATA_DRIVEN with worklists builds the graph's forward CSR on the device on first use. */
 enum { AG_DIR_PULL = 0, AG_DIR_PUSH = 1, AG_DIR_DATA_DRIVEN = 2 };
 
 void ag_pr_options_default(ag_pr_options *o);
@@ -324,12 +320,11 @@ int ag_spmv_pull_noalloc(ag_dgraph *g, const float *x, float *y);
 int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *x_q, uint64_t *y_q,
                        uint32_t repetitions, double *avg_kernel_ms);
 /* Push forms (SPMVPushGraphCSR / SPMVPushFixedPointGraphCSR, SPMV.c:752-848, 1017-1136):
- * every source adds w*x[src] to its out-neighbours (propagation-blocked, as the PageRank push).
- * As in the reference the output is not cleared between repetitions, so y = the sum of
- * `repetitions` products (0 repetitions: y = 0). FP32: binary32 products, each repetition's
- * row sum added in the LDS atomics' order, then added to y. Fixed point: x_q and y_q in Q32.32
- * (DoubleToFixed64), weights DoubleToFixed64(w) (0.0001f unweighted), products MULFixed64V1,
- * exact u64 sums. The forward CSR and the push bins are built on the device on first use. */
+ * every source adds w*x[src] to its out-neighbours. As in the reference the output is not
+ * cleared between repetitions, so y = the sum of `repetitions` products (0 repetitions: y = 0).
+ * FP32: binary32 products, each repetition's row sum added in the pull's order, then added to y.
+ * Fixed point: x_q and y_q in Q32.32 (DoubleToFixed64), weights DoubleToFixed64(w) (0.0001f
+ * unweighted), products MULFixed64V1, exact u64 sums. */
 int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t repetitions,
                  double *avg_kernel_ms);
 int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *x_q, uint64_t *y_q, uint32_t repetitions,
