@@ -30,6 +30,8 @@
 // one partial per piece, pass 2 adds each row's partials in block order and finishes the row.
 #pragma once
 
+#include <type_traits>
+
 #include "ag_internal.h"
 
 #define AG_WAVE 64
@@ -128,6 +130,38 @@ __device__ __forceinline__ uint32_t ld_stream(const uint32_t *p)
 {
     return __builtin_nontemporal_load(p);
 }
+
+// Update operands of a policy whose update reads nothing of the row, and the per-edge data of a
+// policy without any.
+struct NoPre {
+};
+
+// Per-edge data (SpMV weights) that a tile loads with its source ids, a tile ahead of the gathers
+// that multiply by it: P::Edge, P::edge_pre(j) and P::edge_at(s, data) of policies that have any.
+// Loaded with the gathers instead, the weights took the place of gathers in flight: weighted
+// SpMV RMAT-22 422 us, RMAT-20 122, Erdos-Renyi 300 K 39; a tile ahead 307, 99 and 29.
+template <class P, class = void>
+struct EdgeOf {
+    using T = NoPre;
+    static __device__ __forceinline__ T load(const P &, uint32_t) { return T{}; }
+    template <class TT>
+    static __device__ __forceinline__ typename P::Acc term(const TT &tt, const P &pol, uint32_t j,
+                                                           uint32_t s, T)
+    {
+        return tt.term(pol, j, s);
+    }
+};
+template <class P>
+struct EdgeOf<P, std::void_t<typename P::Edge>> {
+    using T = typename P::Edge;
+    static __device__ __forceinline__ T load(const P &pol, uint32_t j) { return pol.edge_pre(j); }
+    template <class TT>
+    static __device__ __forceinline__ typename P::Acc term(const TT &, const P &pol, uint32_t,
+                                                           uint32_t s, T e)
+    {
+        return pol.edge_at(s, e);   // policies with per-edge data keep no LDS table
+    }
+};
 
 #define AG_LONG_MAX 64u    // longer rows of one tile: at most AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1)
 static_assert(AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1u) < AG_LONG_MAX,
@@ -324,6 +358,27 @@ __device__ __forceinline__ void pull_one_item(const PullGeom &G, const P &pol, u
         pull_thread_tile(G, pol, it - G.slot_blk0[4], red, s_vals);
 }
 
+// Where a first-pass gather reads edge j's term from (source s): the policy's own gather
+// (NoTop), or, for the sources [base, base + n) of an LDS copy of that part of the
+// contribution vector, the copy (TopTab). Both give the same value.
+struct NoTop {
+    template <class P>
+    __device__ __forceinline__ typename P::Acc term(const P &pol, uint32_t j, uint32_t s) const
+    {
+        return pol.edge(j, s);
+    }
+};
+template <typename RT>
+struct TopTab {
+    const RT *tab;
+    uint32_t base;
+    template <class P>
+    __device__ __forceinline__ typename P::Acc term(const P &pol, uint32_t j, uint32_t s) const
+    {
+        return s >= base ? pol.edge_val(j, tab[s - base]) : pol.edge(j, s);
+    }
+};
+
 // ---------------------------------------------------------------- row tiles
 //
 // The regular schedule hands the rows of the bins up to G.rt_row1 to the workgroups as tiles of
@@ -337,10 +392,6 @@ __device__ __forceinline__ void pull_one_item(const PullGeom &G, const P &pol, u
 // row (offsets, ids, values, update operands), left the chip waiting. SpMV before -> with row
 // tiles: RMAT-16 9.4 -> 7.0 us, RMAT-18 28 -> 22, RMAT-20 102 -> 78 (0.2 T in-edges/s, the L2
 // request rate that also bounds the blocked pass 1), Erdos-Renyi 300 K rows 29.5 -> 25.
-
-// Update operands of a policy whose update reads nothing of the row.
-struct NoPre {
-};
 
 struct RowTile {
     uint32_t r0, r1, e0, e1;
@@ -397,13 +448,19 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, 
 {
     using Acc = typename P::Acc;
     const uint32_t tid = threadIdx.x, wave = tid / AG_WAVE, lane = tid % AG_WAVE;
+    using ED = EdgeOf<P>;
     RowTile cur = row_tile_at(G, i), nxt = row_tile_at(G, i + step);
     uint32_t w[AG_TILE_UNROLL];
+    typename ED::T ed[AG_TILE_UNROLL];
+    const auto load_ids = [&](const RowTile &t) {
 #pragma unroll
-    for (int u = 0; u < AG_TILE_UNROLL; u++) {
-        const uint32_t j = cur.e0 + tid + u * AG_WG;
-        w[u] = j < cur.e1 ? ld_stream(&G.src[j]) : 0u;
-    }
+        for (int u = 0; u < AG_TILE_UNROLL; u++) {
+            const uint32_t j = t.e0 + tid + u * AG_WG;
+            w[u] = j < t.e1 ? ld_stream(&G.src[j]) : 0u;
+            ed[u] = j < t.e1 ? ED::load(pol, j) : typename ED::T{};
+        }
+    };
+    load_ids(cur);
     while (cur.r1 > cur.r0) {
         // this lane's first row: bounds and update operands
         uint32_t r = cur.r0 + tid, b = 0, e = 0;
@@ -417,16 +474,12 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, 
         for (int u = 0; u < AG_TILE_UNROLL; u++) {
             const uint32_t j = cur.e0 + tid + u * AG_WG;
             if (j < cur.e1)
-                L.vals[j - cur.e0] = pol.edge(j, w[u]);
+                L.vals[j - cur.e0] = ED::term(NoTop(), pol, j, w[u], ed[u]);
         }
         i += step;
         const RowTile nn = row_tile_at(G, i + step);
         __syncthreads();
-#pragma unroll
-        for (int u = 0; u < AG_TILE_UNROLL; u++) {
-            const uint32_t j = nxt.e0 + tid + u * AG_WG;
-            w[u] = j < nxt.e1 ? ld_stream(&G.src[j]) : 0u;   // in flight during the sums
-        }
+        load_ids(nxt);   // in flight during the sums
         uint32_t nl = 0;   // this wavefront's long rows
         for (uint32_t q0 = cur.r0 + wave * AG_WAVE; q0 < cur.r1; q0 += AG_WG) {
             const uint32_t rn = r + AG_WG;
@@ -524,27 +577,6 @@ struct CombPol {
     __device__ __forceinline__ void finish(uint32_t r, Acc acc, Red &red) const
     {
         base.finish(r, acc, red);
-    }
-};
-
-// Where a first-pass gather reads edge j's term from (source s): the policy's own gather
-// (NoTop), or, for the sources [base, base + n) of an LDS copy of that part of the
-// contribution vector, the copy (TopTab). Both give the same value.
-struct NoTop {
-    template <class P>
-    __device__ __forceinline__ typename P::Acc term(const P &pol, uint32_t j, uint32_t s) const
-    {
-        return pol.edge(j, s);
-    }
-};
-template <typename RT>
-struct TopTab {
-    const RT *tab;
-    uint32_t base;
-    template <class P>
-    __device__ __forceinline__ typename P::Acc term(const P &pol, uint32_t j, uint32_t s) const
-    {
-        return s >= base ? pol.edge_val(j, tab[s - base]) : pol.edge(j, s);
     }
 };
 
@@ -714,14 +746,18 @@ __device__ __forceinline__ SortedTile sorted_tile_at(const BlockGeom &B, uint32_
 static_assert(AG_TILE_NNZ_MAX <= AG_TILE_UNROLL * AG_WG,
               "a lane holds all of its ids of a sorted tile at once");
 
-// The packed ids of a sorted tile, AG_TILE_UNROLL per lane: the whole tile.
-__device__ __forceinline__ void load_sorted_ids(const uint32_t *vsp, const SortedTile &t,
-                                                uint32_t (&w)[AG_TILE_UNROLL])
+// The packed ids and per-edge data of a sorted tile, AG_TILE_UNROLL per lane: the whole tile.
+template <class P>
+__device__ __forceinline__ void load_sorted_ids(const uint32_t *vsp, const P &pol,
+                                                const SortedTile &t,
+                                                uint32_t (&w)[AG_TILE_UNROLL],
+                                                typename EdgeOf<P>::T (&ed)[AG_TILE_UNROLL])
 {
 #pragma unroll
     for (int u = 0; u < AG_TILE_UNROLL; u++) {
         const uint32_t kk = threadIdx.x + u * AG_WG;
         w[u] = kk < t.nnz ? ld_stream(&vsp[t.e0 + kk]) : 0u;
+        ed[u] = kk < t.nnz ? EdgeOf<P>::load(pol, t.e0 + kk) : typename EdgeOf<P>::T{};
     }
 }
 
@@ -759,7 +795,8 @@ __device__ __forceinline__ void pull_sorted_items(const PullGeom &U, const Block
     }
     SortedTile cur = sorted_tile_at(B, i, end);
     uint32_t w[AG_TILE_UNROLL];
-    load_sorted_ids(B.vsp, cur, w);
+    typename EdgeOf<P>::T ed[AG_TILE_UNROLL];
+    load_sorted_ids(B.vsp, pol, cur, w, ed);
     uint32_t k = 0;
     while (cur.valid) {
         uint32_t next = 0;
@@ -773,7 +810,8 @@ __device__ __forceinline__ void pull_sorted_items(const PullGeom &U, const Block
                 const uint32_t kk = tid + u * AG_WG;
                 if (kk < cur.nnz) {
                     const uint32_t pos = w[u] >> bits;   // < nnz: a permutation of the tile
-                    s_vals[pos] = tt.term(pp, cur.e0 + kk, cur.base + (w[u] & mask));
+                    s_vals[pos] = EdgeOf<P>::term(tt, pol, cur.e0 + kk, cur.base + (w[u] & mask),
+                                                  ed[u]);
                 }
             }
         }
@@ -787,7 +825,7 @@ __device__ __forceinline__ void pull_sorted_items(const PullGeom &U, const Block
         __syncthreads();
         i = B.dyn ? lo + L.ticket[k] : i + step;
         const SortedTile nxt = sorted_tile_at(B, i, end);
-        load_sorted_ids(B.vsp, nxt, w);   // in flight while this tile's rows are summed
+        load_sorted_ids(B.vsp, pol, nxt, w, ed);   // in flight while this tile's rows are summed
         if (!cur.reg) {
             if (cur.nnz == cur.last - cur.first) {   // single edges: partials in order
                 for (uint32_t q = tid; q < cur.nnz; q += AG_WG)
@@ -1051,9 +1089,11 @@ __global__ __launch_bounds__(AG_WG) void pull_kernel(PullGeom G, P pol)
 }
 
 // Plain source-blocked pull (SpMV): pass 1 with `pol` reading per-edge data in virtual-row
-// order and `upol` in regular order for the unblocked rows, then the combine pass.
+// order and `upol` in regular order for the unblocked rows, then the combine pass. Four wavefronts
+// a SIMD: the weights a tile ahead took 137 registers and with them a workgroup per CU (a spill
+// of 8-12 bytes at 128).
 template <class P, class PU>
-__global__ __launch_bounds__(AG_WG) void pull_blocked_kernel(PullGeom U, BlockGeom B, P pol,
+__global__ __launch_bounds__(AG_WG, 4) void pull_blocked_kernel(PullGeom U, BlockGeom B, P pol,
                                                              PU upol)
 {
     __shared__ typename P::Acc s_vals[AG_TILE_NNZ_MAX];

@@ -22,9 +22,22 @@
 
 namespace {
 
+// Per-edge data of the weighted policies (EdgeOf); the unweighted ones have none.
+template <bool WEIGHTED, typename T>
+struct EdgeData {
+};
+template <typename T>
+struct EdgeData<true, T> {
+    using Edge = T;
+};
+
 template <bool WEIGHTED>
-struct SpmvF32Pol {
+struct SpmvF32Pol : EdgeData<WEIGHTED, float> {
     using Acc = float;
+    __device__ __host__ SpmvF32Pol(const float *x_, const float *w_, float *y_)
+        : x(x_), w(w_), y(y_)
+    {
+    }
     const float *x;     // device order
     const float *w;     // [m] or null
     float *y;           // device order
@@ -36,6 +49,14 @@ struct SpmvF32Pol {
     __device__ __forceinline__ float edge_val(uint32_t j, float xs) const
     {
         return __fmul_rn(xs, WEIGHTED ? __builtin_nontemporal_load(&w[j]) : 0.0001f);
+    }
+    __device__ __forceinline__ float edge_pre(uint32_t j) const
+    {
+        return __builtin_nontemporal_load(&w[j]);
+    }
+    __device__ __forceinline__ float edge_at(uint32_t s, float wj) const
+    {
+        return __fmul_rn(x[s], wj);
     }
     using Pre = NoPre;
     __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
@@ -58,17 +79,28 @@ __global__ __launch_bounds__(AG_WG) void spmv_hot_kernel(BlockGeom B, SpmvF32Pol
 }
 
 template <bool WEIGHTED>
-struct SpmvFixPol {
+struct SpmvFixPol : EdgeData<WEIGHTED, uint32_t> {
     using Acc = uint64_t;
+    __device__ __host__ SpmvFixPol(const uint32_t *xq_, const uint32_t *wq_, uint32_t wc,
+                                   uint64_t *y_)
+        : xq(xq_), wq(wq_), wconst(wc), y(y_)
+    {
+    }
     const uint32_t *xq;
     const uint32_t *wq;
     uint32_t wconst;
     uint64_t *y;
     __device__ __forceinline__ uint64_t edge(uint32_t j, uint32_t s) const
     {
-        const uint64_t wide =
-            (uint64_t)xq[s] * (uint64_t)(WEIGHTED ? __builtin_nontemporal_load(&wq[j]) : wconst);
-        return (uint64_t)(uint32_t)(wide >> 16);
+        return edge_at(s, WEIGHTED ? __builtin_nontemporal_load(&wq[j]) : wconst);
+    }
+    __device__ __forceinline__ uint32_t edge_pre(uint32_t j) const
+    {
+        return __builtin_nontemporal_load(&wq[j]);
+    }
+    __device__ __forceinline__ uint64_t edge_at(uint32_t s, uint32_t w) const
+    {
+        return (uint64_t)(uint32_t)(((uint64_t)xq[s] * (uint64_t)w) >> 16);
     }
     using Pre = NoPre;
     __device__ __forceinline__ Pre pre(uint32_t) const { return Pre{}; }
@@ -117,9 +149,14 @@ struct AddTo {
 };
 
 template <bool WEIGHTED>
-struct SpmvPushPol : AddTo<float> {
+struct SpmvPushPol : AddTo<float>, EdgeData<WEIGHTED, float> {
     using Acc = float;
     SpmvF32Pol<WEIGHTED> p;
+    __device__ __forceinline__ float edge_pre(uint32_t j) const { return p.edge_pre(j); }
+    __device__ __forceinline__ float edge_at(uint32_t s, float wj) const
+    {
+        return p.edge_at(s, wj);
+    }
     __device__ __forceinline__ float edge(uint32_t j, uint32_t s) const { return p.edge(j, s); }
     __device__ __forceinline__ float edge_val(uint32_t j, float xs) const
     {
@@ -128,17 +165,23 @@ struct SpmvPushPol : AddTo<float> {
 };
 
 template <bool WEIGHTED>
-struct SpmvPushFixPol : AddTo<uint64_t> {
+struct SpmvPushFixPol : AddTo<uint64_t>, EdgeData<WEIGHTED, float> {
     using Acc = uint64_t;
     const uint64_t *xq;
     const float *w;
     uint64_t wconst;
     __device__ __forceinline__ uint64_t edge(uint32_t j, uint32_t s) const
     {
-        const uint64_t wq =
-            WEIGHTED ? ag_dev_double_to_fixed64((double)__builtin_nontemporal_load(&w[j]))
-                     : wconst;
-        return ag_dev_mul_fixed64(wq, xq[s]);
+        return WEIGHTED ? edge_at(s, __builtin_nontemporal_load(&w[j]))
+                        : ag_dev_mul_fixed64(wconst, xq[s]);
+    }
+    __device__ __forceinline__ float edge_pre(uint32_t j) const
+    {
+        return __builtin_nontemporal_load(&w[j]);
+    }
+    __device__ __forceinline__ uint64_t edge_at(uint32_t s, float wj) const
+    {
+        return ag_dev_mul_fixed64(ag_dev_double_to_fixed64((double)wj), xq[s]);
     }
 };
 
@@ -453,10 +496,10 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     AG_HIP(hipMemcpyAsync(xo, x, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
-    st = g->w ? run_push(g, SpmvPushPol<true>{{yd}, {xd, g->blk.vw, NULL}},
-                         SpmvPushPol<true>{{yd}, {xd, g->w, NULL}}, reps, avg_ms)
-              : run_push(g, SpmvPushPol<false>{{yd}, {xd, NULL, NULL}},
-                         SpmvPushPol<false>{{yd}, {xd, NULL, NULL}}, reps, avg_ms);
+    st = g->w ? run_push(g, SpmvPushPol<true>{{yd}, {}, {xd, g->blk.vw, NULL}},
+                         SpmvPushPol<true>{{yd}, {}, {xd, g->w, NULL}}, reps, avg_ms)
+              : run_push(g, SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}},
+                         SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}}, reps, avg_ms);
     if (st != AG_OK)
         return st;
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
@@ -488,10 +531,10 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     permute_in_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
     const uint64_t wc = DoubleToFixed64((double)0.0001f);   // SPMV.c:1080
-    st = g->w ? run_push(g, SpmvPushFixPol<true>{{yd}, xd, g->blk.vw, 0u},
-                         SpmvPushFixPol<true>{{yd}, xd, g->w, 0u}, reps, avg_ms)
-              : run_push(g, SpmvPushFixPol<false>{{yd}, xd, NULL, wc},
-                         SpmvPushFixPol<false>{{yd}, xd, NULL, wc}, reps, avg_ms);
+    st = g->w ? run_push(g, SpmvPushFixPol<true>{{yd}, {}, xd, g->blk.vw, 0u},
+                         SpmvPushFixPol<true>{{yd}, {}, xd, g->w, 0u}, reps, avg_ms)
+              : run_push(g, SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc},
+                         SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc}, reps, avg_ms);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);

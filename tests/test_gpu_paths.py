@@ -99,3 +99,25 @@ def test_row_tiles(device, pname, n):
                                 max_iterations=6, stop_rule=2)
     np.testing.assert_array_equal(run.ranks.view(np.uint32), want.ranks.view(np.uint32))
     dg.close()
+
+
+@pytest.mark.parametrize("plan", [{}, dict(src_block_bits=10), dict(src_block_bits=9, piece_nnz=1),
+                                  dict(src_block_bits=10, tile_sort=ag.SORT_OFF)])
+@pytest.mark.parametrize("form", ["pull", "push"])
+def test_weighted_tiles(device, plan, form):
+    """Per-edge weights loaded a tile ahead of the gathers: every edge meets its own weight in
+    regular and first-pass tiles, full and partly filled (fixed point exact)."""
+    g = graph_with_degrees(EDGE_DEGREES + [16385])
+    rng = np.random.default_rng(2)
+    g.set_weights(rng.random(g.m, dtype=np.float32))
+    dg = device.upload(g, weights=True, params=ag.plan_params(**plan))
+    if form == "pull":
+        xq = rng.integers(0, 1 << 20, g.n, dtype=np.uint32)
+        wq = oracle.fixed_encode(32, g.inv_weight).astype(np.uint32)
+        want = oracle.spmv_fixed(g.inv_idx, g.in_degree, g.inv_src, wq, 0, xq)
+        np.testing.assert_array_equal(dg.spmv_fixed(xq)[0], want)
+    else:
+        xq = rng.integers(0, 1 << 34, g.n, dtype=np.uint64)
+        want = oracle.spmv_push_fixed(g.edges_idx, g.out_degree, g.fwd_dest, g.fwd_weight, xq, 3)
+        np.testing.assert_array_equal(dg.spmv_push_fixed(xq, 3)[0], want)
+    dg.close()
