@@ -124,6 +124,7 @@ struct BlockGeom {
     const uint32_t *vsp;
     const uint32_t *tbase;
     uint32_t sbits;
+    uint32_t has_reg;        // pass 1 has AG_ITEM_REG items: it finishes the unblocked rows
 };
 
 // Points pass 1 of B past the hot-segment tiles (when the hot pass runs before it).
@@ -159,7 +160,7 @@ struct ag_pr_session {
     ag_pr_options o;
     uint32_t kind_code;         // 0 f32, 1 bf16, 2 f16, 64/32/16/8
     size_t celem;               // bytes per stored contribution
-    PrState *st;                // device
+    PrState *st;                // device [2], by iteration parity
     PrState *st_host;           // pinned
     double *part_err;
     uint32_t *part_act;
@@ -175,15 +176,13 @@ struct ag_pr_session {
     double *fin_sum;
     float *user;
     uint32_t enqueued;
-    hipEvent_t *ev;             // per-launch events when record_history (max_iterations + 1)
+    uint64_t *hist_t;           // device clock per iteration when record_history (start, end)
+    hipEvent_t loop_ev;         // before the first iteration when record_history
+    uint32_t nparts;            // partials of one iteration's launches
     hipEvent_t step_ev[2];
     uint32_t step_launches;
-    uint32_t ev_count;
     struct timespec t0;  // wall clock at ag_pr_begin
 };
-
-// Enqueue one PageRank iteration of a session (main + finish kernel).
-int ag_pr_launch_iteration(ag_pr_session *s);
 
 // Builds g->fwd_off / fwd_dst (the forward CSR in device row ids) from the uploaded inverse CSR,
 // once; later calls return at once.

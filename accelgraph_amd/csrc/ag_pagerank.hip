@@ -9,13 +9,14 @@
 // and finally rank[v] /= N with an FP64 sum (:1079-1085).
 //
 // One iteration is either
-//   regular:        pr_*_kernel (gather + update for every row) then pr_*_finish, or
+//   regular:        pr_*_kernel (gather + update for every row), then pr_*_hubs where rows are
+//                   cut into segments, or
 //   source-blocked: pr_*_blk_kernel (per-block partial sums, XCD-sliced) then pr_*_cmb_kernel
-//                   (partials added per row in block order + update) then pr_*_finish.
+//                   (partials added per row in block order + update).
 // The update is fused into the launch that completes a row's sum: the damping update, the
 // per-workgroup L1 / active partials and the next iteration's contribution; `next` never
-// exists in memory. Contributions ping-pong between two buffers by iteration parity. The
-// one-workgroup finish kernel adds the per-workgroup partials in a fixed order, records the
+// exists in memory. Contributions ping-pong between two buffers by iteration parity. The first
+// launch of the next iteration adds the per-workgroup partials in a fixed order, records the
 // iteration's error and active count, decides the 16-bit -> FP32 refinement and sets a done
 // flag that turns every later launch into a no-op, so many iterations can be queued without
 // a host round trip per iteration.
@@ -23,7 +24,7 @@
 // Fixed-point variants (pageRank.c:1276-1990) gather u64/u32/u16/u8 contributions into an
 // exact u64 sum (wraps modulo 2^64) and convert with the formats of fixedPoint.h. Quantised
 // variants (pageRank.c:2119-2676) gather u32/u16/u8 codes of a per-iteration scale into an
-// exact u64 sum; a small pr_quant_kernel after each finish writes the next codes.
+// exact u64 sum; a small pr_quant_kernel after each iteration writes the next codes.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -94,32 +95,77 @@ __device__ __forceinline__ _Float16 st_from_f32<_Float16>(float x) { return (_Fl
 
 // ---------------------------------------------------------------- iteration control
 
+// An iteration is closed -- its partials added, its error recorded, the stop and the refinement
+// decided -- by the first kernel of the next one: every workgroup adds the partials itself, in the
+// same order, while its first loads are in flight, and workgroup 0 writes the outcome. The launch
+// boundary orders it, and the state is kept twice (by iteration parity) so that no launch reads
+// what it writes. A launch of its own for this took 4 us of an RMAT-12 iteration's 14, and a HIP
+// event per iteration for the history 6 more: the start and end are read off the device clock.
+// The last iteration of a step is closed by pr_close_kernel, so a poll finds everything settled.
 struct PrCtl {
-    PrState *st;
-    double *part_err;      // [nparts] per-workgroup partials of the main launch
-    uint32_t *part_act;    // [nparts]
-    uint32_t *part_cmax;   // [nparts] quantised kinds only (else null): largest contribution
-    double *hist_err;      // [max_iterations]
-    uint32_t *hist_act;    // [max_iterations]
-    uint32_t nparts;       // partials of all passes of one iteration
-    uint32_t part_base;    // first partial of this launch's workgroups
+    PrState *st;             // [2]: iteration `it` reads st[it & 1], writes st[(it + 1) & 1]
+    double *part_err;        // [nparts] per-workgroup partials of iteration `it`
+    uint32_t *part_act;      // [nparts]
+    const double *prev_err;  // those of iteration it - 1
+    const uint32_t *prev_act;
+    uint32_t *part_cmax;     // [nparts] quantised kinds only (else null): largest contribution
+    double *hist_err;        // [max_iterations]
+    uint32_t *hist_act;      // [max_iterations]
+    uint64_t *hist_t;        // [2 * max_iterations] device clock at an iteration's start and end
+    uint32_t it;             // the iteration being launched
+    uint32_t pending;        // iteration it - 1 is still to be closed
+    uint32_t nparts;         // partials of all passes of one iteration
+    uint32_t part_base;      // first partial of this launch's workgroups
     uint32_t stop_rule;
-    uint32_t mixed;        // 16-bit storage with f32 refinement
+    uint32_t mixed;          // 16-bit storage with f32 refinement
     double l1_tol;
     double refine_l1;
+    double dn;               // vertices: the error is the sum of |delta| over this
 };
 
-// Record iteration `iter` and decide whether the run stops (one thread of the finish kernel).
-__device__ __forceinline__ void pr_control(const PrCtl &C, uint32_t iter, double E, uint32_t A)
+// The part of the state that iterations hand on, field by field (it stays in registers).
+struct PrRun {
+    uint32_t iter, done, stop_iter, last_active, stall, qmax_bits;
+    int32_t refine_iter;
+    float qscale;
+    double last_err, best_err;
+};
+
+__device__ __forceinline__ PrRun pr_load(const PrState *p)
 {
-    PrState *st = C.st;
-    C.hist_err[iter] = E;
-    C.hist_act[iter] = A;
+    return PrRun{p->iter, p->done, p->stop_iter, p->last_active, p->stall, p->qmax_bits,
+                 p->refine_iter, p->qscale, p->last_err, p->best_err};
+}
+
+__device__ __forceinline__ void pr_save(PrState *p, const PrRun &S)
+{
+    p->iter = S.iter;
+    p->done = S.done;
+    p->stop_iter = S.stop_iter;
+    p->last_active = S.last_active;
+    p->stall = S.stall;
+    p->qmax_bits = S.qmax_bits;
+    p->refine_iter = S.refine_iter;
+    p->qscale = S.qscale;
+    p->last_err = S.last_err;
+    p->best_err = S.best_err;
+}
+
+// State S after iteration `iter` with |delta| sum `sum` and active count A: whether the run
+// stops. `writer` also records the iteration.
+__device__ __forceinline__ void pr_control(const PrCtl &C, PrRun &S, uint32_t iter, double sum,
+                                           uint32_t A, bool writer)
+{
+    const double E = __ddiv_rn(sum, C.dn);
+    if (writer) {
+        C.hist_err[iter] = E;
+        C.hist_act[iter] = A;
+    }
     bool can_stop = true;
     if (C.mixed) {
-        const int32_t ri = st->refine_iter;
+        const int32_t ri = S.refine_iter;
         if (ri < 0) {
-            refine_decide(st, iter, E, C.refine_l1);
+            refine_decide(S, iter, E, C.refine_l1);
             can_stop = false;
         } else {
             can_stop = (int32_t)iter >= ri + 1;
@@ -131,53 +177,139 @@ __device__ __forceinline__ void pr_control(const PrCtl &C, uint32_t iter, double
     else if (C.stop_rule == AG_STOP_L1)
         stop = (E <= C.l1_tol);
     if (can_stop && stop) {
-        st->done = 1;
-        st->stop_iter = iter;
+        S.done = 1;
+        S.stop_iter = iter;
     }
-    st->last_err = E;
-    st->last_active = A;
-    st->iter = iter + 1;
+    S.last_err = E;
+    S.last_active = A;
+    S.iter = iter + 1;
 }
 
-// Per-workgroup partials of the main launch (plain stores; read after the launch boundary).
+// Sums of an error term and a count per lane over an NT-lane workgroup, the same in every lane.
+template <uint32_t NT>
+__device__ __forceinline__ void block_sum_all(double &e, uint32_t &a)
+{
+    __shared__ double s_e[NT / AG_WAVE];
+    __shared__ uint32_t s_a[NT / AG_WAVE];
+#pragma unroll
+    for (int m = AG_WAVE / 2; m >= 1; m >>= 1) {
+        e = e + __shfl_xor(e, m, AG_WAVE);
+        a = a + __shfl_xor(a, m, AG_WAVE);
+    }
+    if ((threadIdx.x & (AG_WAVE - 1)) == 0) {
+        s_e[threadIdx.x / AG_WAVE] = e;
+        s_a[threadIdx.x / AG_WAVE] = a;
+    }
+    __syncthreads();
+    e = s_e[0];
+    a = s_a[0];
+#pragma unroll
+    for (uint32_t k = 1; k < NT / AG_WAVE; k++) {
+        e = e + s_e[k];
+        a = a + s_a[k];
+    }
+}
+
+// First step of an iteration's first kernel, in two halves: the constructor loads the state and
+// (up to four a lane) the previous iteration's partials, the call makes S the state with every
+// earlier iteration closed. False when the run has stopped (the same in every workgroup).
+struct PrAhead {
+    PrRun S;
+    double e[4];
+    uint32_t a[4];
+    bool run;
+
+    __device__ __forceinline__ explicit PrAhead(const PrCtl &C) : run(false)
+    {
+        S = pr_load(&C.st[C.it & 1u]);
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t i = threadIdx.x + u * AG_WG;
+            const bool in = C.pending && i < C.nparts;
+            e[u] = in ? C.prev_err[i] : 0.0;
+            a[u] = in ? C.prev_act[i] : 0u;
+        }
+    }
+    __device__ __forceinline__ bool operator()(const PrCtl &C)
+    {
+        const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+        const bool was_done = S.done != 0u;
+        if (!was_done && C.pending) {
+            double E = (e[0] + e[1]) + (e[2] + e[3]);
+            uint32_t A = (a[0] + a[1]) + (a[2] + a[3]);
+            for (uint32_t i = threadIdx.x + 4u * AG_WG; i < C.nparts; i += AG_WG) {
+                E += C.prev_err[i];
+                A += C.prev_act[i];
+            }
+            block_sum_all<AG_WG>(E, A);
+            pr_control(C, S, C.it - 1u, E, A, writer);
+        }
+        if (writer) {
+            pr_save(&C.st[(C.it + 1u) & 1u], S);
+            if (C.hist_t && !was_done) {
+                const uint64_t t = wall_clock64();
+                if (C.pending)
+                    C.hist_t[2u * (C.it - 1u) + 1u] = t;
+                C.hist_t[2u * C.it] = t;
+            }
+        }
+        run = !S.done;
+        return run;
+    }
+};
+
+__device__ __forceinline__ bool pr_open(const PrCtl &C, PrRun &S)
+{
+    PrAhead open(C);
+    const bool run = open(C);
+    S = open.S;
+    return run;
+}
+
+// The state an iteration's later kernels see (written by its first).
+__device__ __forceinline__ const PrState *pr_now(const PrCtl &C)
+{
+    return C.st + ((C.it + 1u) & 1u);
+}
+
+// Closes iteration it - 1 after the last launch of a step; iteration `it` then finds nothing
+// pending. One workgroup.
+__global__ __launch_bounds__(AG_WG) void pr_close_kernel(PrCtl C)
+{
+    PrRun S = pr_load(&C.st[C.it & 1u]);
+    if (S.done)
+        return;
+    double E = 0.0;
+    uint32_t A = 0u;
+    for (uint32_t i = threadIdx.x; i < C.nparts; i += AG_WG) {
+        E += C.prev_err[i];
+        A += C.prev_act[i];
+    }
+    block_sum_all<AG_WG>(E, A);
+    if (threadIdx.x == 0) {
+        pr_control(C, S, C.it - 1u, E, A, true);
+        pr_save(&C.st[C.it & 1u], S);
+        if (C.hist_t)
+            C.hist_t[2u * (C.it - 1u) + 1u] = wall_clock64();
+    }
+}
+
+// Per-workgroup partials of a launch (plain stores; read after the launch boundary).
+template <uint32_t NT = AG_WG>
 __device__ __forceinline__ void pr_store_partial(const PrCtl &C, Red red)
 {
-    __shared__ double s_e[AG_WG / AG_WAVE];
-    __shared__ uint32_t s_a[AG_WG / AG_WAVE];
-    Red t = block_reduce_red<AG_WG>(red, s_e, s_a);
+    __shared__ uint32_t s_m[NT / AG_WAVE];
+    __syncthreads();   // the sums of the opening step may still be read
+    block_sum_all<NT>(red.err, red.active);
     if (C.part_cmax) {
-        const uint32_t m = block_max_u32<AG_WG>(red.cmax, s_a);
+        const uint32_t m = block_max_u32<NT>(red.cmax, s_m);
         if (threadIdx.x == 0)
             C.part_cmax[C.part_base + blockIdx.x] = m;
     }
     if (threadIdx.x == 0) {
-        C.part_err[C.part_base + blockIdx.x] = t.err;
-        C.part_act[C.part_base + blockIdx.x] = t.active;
+        C.part_err[C.part_base + blockIdx.x] = red.err;
+        C.part_act[C.part_base + blockIdx.x] = red.active;
     }
-}
-
-// Finish kernel tail: hub rows already folded into `red`; add the main launch's partials in
-// index order and close the iteration.
-__device__ __forceinline__ void pr_close(const PrCtl &C, uint32_t iter, Red red)
-{
-    __shared__ double s_e[AG_FIN_WG / AG_WAVE];
-    __shared__ uint32_t s_a[AG_FIN_WG / AG_WAVE];
-    uint32_t mx = red.cmax;
-    for (uint32_t i = threadIdx.x; i < C.nparts; i += AG_FIN_WG) {
-        red.err += C.part_err[i];
-        red.active += C.part_act[i];
-        if (C.part_cmax)
-            mx = max(mx, C.part_cmax[i]);
-    }
-    Red t = block_reduce_red<AG_FIN_WG>(red, s_e, s_a);
-    if (C.part_cmax) {
-        // the quantiser of the next iteration reads this (after the launch boundary)
-        mx = block_max_u32<AG_FIN_WG>(mx, s_a);
-        if (threadIdx.x == 0)
-            C.st->qmax_bits = mx;
-    }
-    if (threadIdx.x == 0)
-        pr_control(C, iter, t.err, t.active);
 }
 
 // What a row's update reads of the row itself, loaded ahead of its sum.
@@ -200,7 +332,7 @@ struct PrF32Pol {
     float *rank;
     const uint32_t *outdeg;
     float base, damp;
-    double dn, eps;
+    double eps;
 
     __device__ __forceinline__ float edge(uint32_t, uint32_t s) const { return ld_f32(cin[s]); }
     // the same term from a stored contribution already in hand (hot-segment LDS copy)
@@ -212,7 +344,7 @@ struct PrF32Pol {
         const float nw = __fadd_rn(base, __fmul_rn(damp, sum));
         __builtin_nontemporal_store(nw, &rank[r]);
         const double e = (double)fabsf(__fsub_rn(nw, q.old));
-        red.err += __ddiv_rn(e, dn);
+        red.err += e;
         red.active += (e >= eps) ? 1u : 0u;
         cout[r] = st_from_f32<WT>(q.od ? __fdiv_rn(nw, __uint2float_rn(q.od)) : 0.0f);
     }
@@ -228,32 +360,31 @@ struct PrF32Args {
     float *rank;
     const uint32_t *outdeg;
     float base, damp;
-    double dn, eps;
+    double eps;
 };
 
 // Runs `body(policy)` with the policy of this iteration's storage mode.
 template <typename HT, class F>
-__device__ __forceinline__ void pr_f32_dispatch(const PrState *st, uint32_t iter,
-                                                const PrF32Args &A, bool mixed, F &&body)
+__device__ __forceinline__ void pr_f32_dispatch(int32_t ri, uint32_t iter, const PrF32Args &A,
+                                                bool mixed, F &&body)
 {
     const uint32_t rd = iter & 1u, wr = rd ^ 1u;
     if (!mixed) {
         body(PrF32Pol<float, float>{(const float *)A.c32[rd], (float *)A.c32[wr], A.rank,
-                                    A.outdeg, A.base, A.damp, A.dn, A.eps});
+                                    A.outdeg, A.base, A.damp, A.eps});
         return;
     }
-    const int32_t ri = *(volatile const int32_t *)&st->refine_iter;
     const bool wf32 = ri >= 0 && (int32_t)iter >= ri;
     const bool rf32 = ri >= 0 && (int32_t)iter >= ri + 1;
     if (rf32)
         body(PrF32Pol<float, float>{(const float *)A.c32[rd], (float *)A.c32[wr], A.rank,
-                                    A.outdeg, A.base, A.damp, A.dn, A.eps});
+                                    A.outdeg, A.base, A.damp, A.eps});
     else if (wf32)
         body(PrF32Pol<HT, float>{(const HT *)A.c16[rd], (float *)A.c32[wr], A.rank, A.outdeg,
-                                 A.base, A.damp, A.dn, A.eps});
+                                 A.base, A.damp, A.eps});
     else
         body(PrF32Pol<HT, HT>{(const HT *)A.c16[rd], (HT *)A.c16[wr], A.rank, A.outdeg, A.base,
-                              A.damp, A.dn, A.eps});
+                              A.damp, A.eps});
 }
 
 template <typename HT>
@@ -263,29 +394,44 @@ __device__ __forceinline__ void pr_f32_main(const PullGeom &G, const PrCtl &C,
     using LP = PrF32Pol<float, float>;   // every storage sums in FP32
     AG_TILE_LDS(LP, tile);
     __shared__ float s_wave[AG_WG / AG_WAVE];
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
+    TileAhead<LP> ahead;
+    ahead.load(G, LP{});
     Red red{};
-    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) {
-        using P = std::remove_cv_t<std::remove_reference_t<decltype(p)>>;
-        pull_items(G, p, red, TileLds<P>{tile.vals, tile.lsum, tile.lng, tile.cnt}, s_wave);
+    if (!mixed) {
+        // the previous iteration is closed while the first tile's values arrive
+        PrAhead open(C);
+        pr_f32_dispatch<HT>(0, C.it, A, false, [&](auto p) {
+            using P = decltype(p);
+            pull_items(G, p, red, TileLds<P>{tile.vals, tile.lsum, tile.lng, tile.cnt}, s_wave,
+                       ahead, false, [&](P &) { return open(C); });
+        });
+        if (open.run)
+            pr_store_partial(C, red);
+        return;
+    }
+    PrRun S;   // the storage to read depends on it
+    if (!pr_open(C, S))
+        return;
+    pr_f32_dispatch<HT>(S.refine_iter, C.it, A, mixed, [&](auto p) {
+        using P = decltype(p);
+        pull_items(G, p, red, TileLds<P>{tile.vals, tile.lsum, tile.lng, tile.cnt}, s_wave, ahead,
+                   true, [](P &) { return true; });
     });
     pr_store_partial(C, red);
 }
 
+// Hub rows of a regular iteration, after its segments (one workgroup, one more partial).
 template <typename HT>
-__device__ __forceinline__ void pr_f32_fin(const PullGeom &G, const PrCtl &C,
-                                           const PrF32Args &A, bool mixed)
+__device__ __forceinline__ void pr_f32_hubs(const PullGeom &G, const PrCtl &C,
+                                            const PrF32Args &A, bool mixed)
 {
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    const PrState *st = pr_now(C);
+    if (st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) { pull_hub_finish(G, p, red); });
-    pr_close(C, iter, red);
+    pr_f32_dispatch<HT>(st->refine_iter, C.it, A, mixed,
+                        [&](const auto &p) { pull_hub_finish(G, p, red); });
+    pr_store_partial<AG_FIN_WG>(C, red);
 }
 
 // Source-blocked iteration: pass 1 (partials of the blocked rows, full update of the others),
@@ -301,12 +447,11 @@ __device__ __forceinline__ void pr_f32_blk(const PullGeom &U, const BlockGeom &B
     __shared__ float s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
     __shared__ float s_top[AG_TOP_IDS];
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    PrRun S;
+    if (!pr_open(C, S))
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) {
+    pr_f32_dispatch<HT>(S.refine_iter, C.it, A, mixed, [&](const auto &p) {
         using RT = std::remove_cv_t<std::remove_pointer_t<decltype(p.cin)>>;
         static_assert(sizeof(RT) <= sizeof(float), "the table holds 4-byte contributions");
         if (B.top0 < B.n_src) {
@@ -320,7 +465,8 @@ __device__ __forceinline__ void pr_f32_blk(const PullGeom &U, const BlockGeom &B
             pull_blocked_items(U, B, p, p, red, s_vals, s_wave, L);
         }
     });
-    pr_store_partial(C, red);
+    if (C.part_err)
+        pr_store_partial(C, red);
 }
 
 template <typename HT>
@@ -330,12 +476,11 @@ __device__ __forceinline__ void pr_f32_cmb(const BlockGeom &B, const PrCtl &C,
     __shared__ float s_vals[AG_TILE_NNZ_MAX];
     __shared__ float s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    const PrState *st = pr_now(C);
+    if (st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) {
+    pr_f32_dispatch<HT>(st->refine_iter, C.it, A, mixed, [&](const auto &p) {
         pull_combine_items(B, p, red, s_vals, s_wave, L);
     });
     pr_store_partial(C, red);
@@ -351,11 +496,10 @@ __device__ __forceinline__ void pr_f32_hot(const BlockGeom &B, const PrCtl &C,
     __shared__ float s_vals[AG_HOT_NNZ];
     __shared__ uint32_t s_long[AG_LONG_MAX];
     __shared__ uint32_t s_nlong;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    PrRun S;
+    if (!pr_open(C, S))
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
-    pr_f32_dispatch<HT>(st, iter, A, mixed, [&](const auto &p) {
+    pr_f32_dispatch<HT>(S.refine_iter, C.it, A, mixed, [&](const auto &p) {
         pull_hot_items(B, p, p.cin, s_tab, s_vals, s_long, &s_nlong);
     });
 }
@@ -413,17 +557,17 @@ __global__ __launch_bounds__(AG_WG) void pr_f16_kernel(PullGeom G, PrCtl C, PrF3
 {
     pr_f32_main<_Float16>(G, C, A, true);
 }
-__global__ __launch_bounds__(AG_FIN_WG) void pr_f32_finish(PullGeom G, PrCtl C, PrF32Args A)
+__global__ __launch_bounds__(AG_FIN_WG) void pr_f32_hubs(PullGeom G, PrCtl C, PrF32Args A)
 {
-    pr_f32_fin<float>(G, C, A, false);
+    pr_f32_hubs<float>(G, C, A, false);
 }
-__global__ __launch_bounds__(AG_FIN_WG) void pr_bf16_finish(PullGeom G, PrCtl C, PrF32Args A)
+__global__ __launch_bounds__(AG_FIN_WG) void pr_bf16_hubs(PullGeom G, PrCtl C, PrF32Args A)
 {
-    pr_f32_fin<bf16s>(G, C, A, true);
+    pr_f32_hubs<bf16s>(G, C, A, true);
 }
-__global__ __launch_bounds__(AG_FIN_WG) void pr_f16_finish(PullGeom G, PrCtl C, PrF32Args A)
+__global__ __launch_bounds__(AG_FIN_WG) void pr_f16_hubs(PullGeom G, PrCtl C, PrF32Args A)
 {
-    pr_f32_fin<_Float16>(G, C, A, true);
+    pr_f32_hubs<_Float16>(G, C, A, true);
 }
 
 // ---------------------------------------------------------------- fixed-point policy
@@ -476,7 +620,7 @@ struct PrFixPol {
     float *rank;
     const uint32_t *outdeg;
     float base, damp;
-    double dn, eps;
+    double eps;
 
     __device__ __forceinline__ uint64_t edge(uint32_t, uint32_t s) const { return (uint64_t)cin[s]; }
     using Pre = RankPre;
@@ -486,7 +630,7 @@ struct PrFixPol {
         const float nw = fix_update<BITS>(base, damp, q);
         __builtin_nontemporal_store(nw, &rank[r]);
         const double e = (double)fabsf(__fsub_rn(nw, x.old));
-        red.err += __ddiv_rn(e, dn);
+        red.err += e;
         red.active += (e >= eps) ? 1u : 0u;
         cout[r] = x.od ? fix_encode<BITS>(__fdiv_rn(nw, __uint2float_rn(x.od))) : (CT)0;
     }
@@ -502,7 +646,7 @@ __device__ __forceinline__ PrFixPol<BITS> fix_policy(uint32_t iter, const PrF32A
     using CT = typename FixT<BITS>::T;
     const uint32_t rd = iter & 1u, wr = rd ^ 1u;
     return PrFixPol<BITS>{(const CT *)A.c32[rd], (CT *)A.c32[wr], A.rank, A.outdeg, A.base,
-                          A.damp, A.dn, A.eps};
+                          A.damp, A.eps};
 }
 
 // ---------------------------------------------------------------- quantised policy
@@ -510,8 +654,8 @@ __device__ __forceinline__ PrFixPol<BITS> fix_policy(uint32_t iter, const PrF32A
 // pageRankPullQuant{32,16,8}BitGraphCSR (pageRank.c:2119-2676): per iteration the f32
 // contributions get a scale from their maximum (zero point 0), are quantised to B-bit codes,
 // the codes are summed exactly in u64 and the update is base + damp * (scale * (float)sum).
-// Here the update writes the f32 contributions and a per-workgroup maximum, the finish kernel
-// reduces the maximum, and pr_quant_kernel writes the codes the next gather reads; the u64
+// Here the update writes the f32 contributions and a per-workgroup maximum, and pr_quant_kernel
+// reduces the maximum and writes the codes the next gather reads; the u64
 // sums are exact, so any summation order gives the same ranks. The quantiser (the reference's
 // quantization.h is not in its tree) is defined as
 //   scale = mx > 0 ? (float)((double)mx / (2^B - 1)) : 1     mx = largest finite c >= 0
@@ -552,7 +696,7 @@ struct PrQuantPol {
     float *rank;
     const uint32_t *outdeg;
     float base, damp, scale;
-    double dn, eps;
+    double eps;
 
     __device__ __forceinline__ uint64_t edge(uint32_t, uint32_t s) const { return (uint64_t)codes[s]; }
     using Pre = RankPre;
@@ -562,7 +706,7 @@ struct PrQuantPol {
         const float nw = __fadd_rn(base, __fmul_rn(damp, __fmul_rn(scale, __ull2float_rn(q))));
         __builtin_nontemporal_store(nw, &rank[r]);
         const double e = (double)fabsf(__fsub_rn(nw, x.old));
-        red.err += __ddiv_rn(e, dn);
+        red.err += e;
         red.active += (e >= eps) ? 1u : 0u;
         const float c = x.od ? __fdiv_rn(nw, __uint2float_rn(x.od)) : 0.0f;
         cf[r] = c;
@@ -576,26 +720,41 @@ struct PrQuantPol {
 
 // Integer-sum policies: KC = 64/32/16/8 fixed point, 100 + B quantised B-bit codes.
 template <int KC>
-__device__ __forceinline__ auto int_policy(const PrState *st, uint32_t iter, const PrF32Args &A)
+__device__ __forceinline__ auto int_policy(float scale, uint32_t iter, const PrF32Args &A)
 {
     if constexpr (KC > 100) {
         using CT = typename FixT<KC - 100>::T;
-        const float scale = *(volatile const float *)&st->qscale;
         return PrQuantPol<KC - 100>{(const CT *)A.c32[1], (float *)A.c32[0], A.rank, A.outdeg,
-                                    A.base, A.damp, scale, A.dn, A.eps};
+                                    A.base, A.damp, scale, A.eps};
     } else {
         return fix_policy<KC>(iter, A);
     }
 }
 
 // Codes of the next iteration from its f32 contributions; records the scale they use.
+// The maximum is over the iteration's `nparts` partials (none: st->qmax_bits, of the start).
 template <int BITS>
 __global__ __launch_bounds__(AG_WG) void pr_quant_kernel(uint32_t n, PrState *st, const float *cf,
-                                                         typename FixT<BITS>::T *codes)
+                                                         typename FixT<BITS>::T *codes,
+                                                         const uint32_t *part_cmax,
+                                                         uint32_t nparts)
 {
-    if (*(volatile const uint32_t *)&st->done)
+    __shared__ uint32_t s_w[AG_WG / AG_WAVE];
+    if (st->done)
         return;
-    const float scale = quant_scale<BITS>(*(volatile const uint32_t *)&st->qmax_bits);
+    uint32_t mx = nparts ? 0u : st->qmax_bits;
+    for (uint32_t i = threadIdx.x; i < nparts; i += AG_WG)
+        mx = max(mx, part_cmax[i]);
+#pragma unroll
+    for (int m = AG_WAVE / 2; m >= 1; m >>= 1)
+        mx = max(mx, (uint32_t)__shfl_xor(mx, m, AG_WAVE));
+    if (threadIdx.x % AG_WAVE == 0)
+        s_w[threadIdx.x / AG_WAVE] = mx;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < AG_WG / AG_WAVE; k++)
+        mx = max(mx, s_w[k]);
+    const float scale = quant_scale<BITS>(mx);
     const double inv = __ddiv_rn(1.0, (double)scale);
     for (uint32_t v = blockIdx.x * AG_WG + threadIdx.x; v < n; v += gridDim.x * AG_WG)
         codes[v] = quant_code<BITS>(cf[v], inv);
@@ -619,16 +778,22 @@ __global__ __launch_bounds__(AG_WG) void pr_quant_init_max(uint32_t n, const flo
 template <int KC>
 __global__ __launch_bounds__(AG_WG) void pr_int_kernel(PullGeom G, PrCtl C, PrF32Args A)
 {
-    using P = decltype(int_policy<KC>(C.st, 0u, A));
+    using P = decltype(int_policy<KC>(0.0f, 0u, A));
     AG_TILE_LDS(P, tile);
     __shared__ uint64_t s_wave[AG_WG / AG_WAVE];
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
+    TileAhead<P> ahead;
+    ahead.load(G, P{});
     Red red{};
-    pull_items(G, int_policy<KC>(st, iter, A), red, tile, s_wave);
-    pr_store_partial(C, red);
+    PrAhead open(C);   // as in pr_f32_main
+    P pol = int_policy<KC>(0.0f, C.it, A);
+    pull_items(G, pol, red, tile, s_wave, ahead, false, [&](P &p) {
+        const bool run = open(C);
+        if constexpr (KC > 100)
+            p.scale = open.S.qscale;
+        return run;
+    });
+    if (open.run)
+        pr_store_partial(C, red);
 }
 
 template <int KC>
@@ -638,14 +803,14 @@ __global__ __launch_bounds__(AG_WG) void pr_int_blk_kernel(PullGeom U, BlockGeom
     __shared__ uint64_t s_vals[AG_TILE_NNZ_MAX];
     __shared__ uint64_t s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    PrRun S;
+    if (!pr_open(C, S))
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    const auto p = int_policy<KC>(st, iter, A);
+    const auto p = int_policy<KC>(S.qscale, C.it, A);
     pull_blocked_items(U, B, p, p, red, s_vals, s_wave, L);
-    pr_store_partial(C, red);
+    if (C.part_err)
+        pr_store_partial(C, red);
 }
 
 template <int KC>
@@ -654,25 +819,23 @@ __global__ __launch_bounds__(AG_WG) void pr_int_cmb_kernel(BlockGeom B, PrCtl C,
     __shared__ uint64_t s_vals[AG_TILE_NNZ_MAX];
     __shared__ uint64_t s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    const PrState *st = pr_now(C);
+    if (st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pull_combine_items(B, int_policy<KC>(st, iter, A), red, s_vals, s_wave, L);
+    pull_combine_items(B, int_policy<KC>(st->qscale, C.it, A), red, s_vals, s_wave, L);
     pr_store_partial(C, red);
 }
 
 template <int KC>
-__global__ __launch_bounds__(AG_FIN_WG) void pr_int_finish(PullGeom G, PrCtl C, PrF32Args A)
+__global__ __launch_bounds__(AG_FIN_WG) void pr_int_hubs(PullGeom G, PrCtl C, PrF32Args A)
 {
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    const PrState *st = pr_now(C);
+    if (st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pull_hub_finish(G, int_policy<KC>(st, iter, A), red);
-    pr_close(C, iter, red);
+    pull_hub_finish(G, int_policy<KC>(st->qscale, C.it, A), red);
+    pr_store_partial<AG_FIN_WG>(C, red);
 }
 
 // ---------------------------------------------------------------- data-driven, full pull
@@ -692,7 +855,7 @@ struct PrDdPol {
     float *rank;
     const uint32_t *outdeg;
     float base, damp;
-    double dn, eps;
+    double eps;
     bool all_listed;      // the first iteration lists every vertex
 
     __device__ __forceinline__ DdAcc edge(uint32_t, uint32_t s) const
@@ -706,7 +869,7 @@ struct PrDdPol {
         float rk = __builtin_nontemporal_load(&rank[r]);
         const double e = (double)fabsf(__fsub_rn(nw, rk));
         if (all_listed || acc.f > 0.0f)
-            red.err += __ddiv_rn(e, dn);
+            red.err += e;
         const bool upd = e >= eps;
         if (upd) {
             rk = nw;
@@ -723,7 +886,7 @@ __device__ __forceinline__ PrDdPol dd_policy(uint32_t iter, const PrF32Args &A)
 {
     const uint32_t rd = iter & 1u, wr = rd ^ 1u;
     return PrDdPol{(const float *)A.c32[rd], (float *)A.c32[wr], A.rank, A.outdeg, A.base,
-                   A.damp, A.dn, A.eps, iter == 0};
+                   A.damp, A.eps, iter == 0};
 }
 
 __global__ __launch_bounds__(AG_WG) void pr_ddf_blk_kernel(PullGeom U, BlockGeom B, PrCtl C,
@@ -732,14 +895,14 @@ __global__ __launch_bounds__(AG_WG) void pr_ddf_blk_kernel(PullGeom U, BlockGeom
     __shared__ DdAcc s_vals[AG_TILE_NNZ_MAX];
     __shared__ DdAcc s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    PrRun S;
+    if (!pr_open(C, S))
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    const PrDdPol p = dd_policy(iter, A);
+    const PrDdPol p = dd_policy(C.it, A);
     pull_blocked_items(U, B, p, p, red, s_vals, s_wave, L);
-    pr_store_partial(C, red);
+    if (C.part_err)
+        pr_store_partial(C, red);
 }
 
 __global__ __launch_bounds__(AG_WG) void pr_ddf_cmb_kernel(BlockGeom B, PrCtl C, PrF32Args A)
@@ -747,24 +910,12 @@ __global__ __launch_bounds__(AG_WG) void pr_ddf_cmb_kernel(BlockGeom B, PrCtl C,
     __shared__ DdAcc s_vals[AG_TILE_NNZ_MAX];
     __shared__ DdAcc s_wave[AG_WG / AG_WAVE];
     __shared__ BlkLds L;
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    const PrState *st = pr_now(C);
+    if (st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    pull_combine_items(B, dd_policy(iter, A), red, s_vals, s_wave, L);
+    pull_combine_items(B, dd_policy(C.it, A), red, s_vals, s_wave, L);
     pr_store_partial(C, red);
-}
-
-__global__ __launch_bounds__(AG_FIN_WG) void pr_ddf_finish(PullGeom G, PrCtl C, PrF32Args A)
-{
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
-    Red red{};
-    pull_hub_finish(G, dd_policy(iter, A), red);
-    pr_close(C, iter, red);
 }
 
 // ---------------------------------------------------------------- data-driven, full pull in edge order
@@ -933,12 +1084,11 @@ __global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF3
     __shared__ float s_vals[AG_TILE_NNZ_MAX];
     __shared__ float s_wave[AG_WG / AG_WAVE];
     static_assert(2u * AG_DD_CHUNK <= AG_TILE_NNZ_MAX, "both halves of a staged row");
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
+    PrRun S;
+    if (!pr_open(C, S))
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
     Red red{};
-    const PrDdPol p = dd_policy(iter, A);
+    const PrDdPol p = dd_policy(C.it, A);
     const uint32_t tid = threadIdx.x;
     const uint32_t r_grp = G.bin_row[AG_BIN_GROUP16], r_wav = G.bin_row[AG_BIN_WAVE];
     const uint32_t r_big = G.bin_row[AG_BIN_BLOCK], r_end = G.bin_row[AG_NBINS];
@@ -1005,16 +1155,6 @@ __global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF3
     pr_store_partial(C, red);
 }
 
-// Closes an iteration whose every row was updated by the preceding launch.
-__global__ __launch_bounds__(AG_FIN_WG) void pr_plain_finish(PrCtl C)
-{
-    const PrState *st = C.st;
-    if (*(volatile const uint32_t *)&st->done)
-        return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
-    pr_close(C, iter, Red{});
-}
-
 // ---------------------------------------------------------------- data-driven pull
 //
 // The worklist form (user starts on unblocked plans, and user starts whose signs are taken).
@@ -1053,6 +1193,8 @@ __global__ __launch_bounds__(AG_WG) void pr_dd_gather_kernel(PrCtl C, PrF32Args 
     const uint32_t cnt = *(volatile const uint32_t *)&st->dd_count[iter & 1u];
     const uint32_t hubs = *(volatile const uint32_t *)&st->dd_hubs[iter & 1u];
     const float *c = (const float *)A.c32[0];
+    if (C.hist_t && blockIdx.x == 0 && threadIdx.x == 0)
+        C.hist_t[2u * C.it] = wall_clock64();
     Red red{};
     // hub rows (in-degree > AG_DD_SEQ_MAX), listed from the far end: one workgroup each, in a
     // fixed order, so the sum is deterministic
@@ -1063,7 +1205,7 @@ __global__ __launch_bounds__(AG_WG) void pr_dd_gather_kernel(PrCtl C, PrF32Args 
         if (threadIdx.x == 0) {
             const float nw = __fadd_rn(A.base, __fmul_rn(A.damp, sum));
             const double err = (double)fabsf(__fsub_rn(nw, A.rank[v]));
-            red.err += __ddiv_rn(err, A.dn);
+            red.err += err;
             s_upd = err >= A.eps ? 1u : 0u;
             if (s_upd) {
                 A.rank[v] = nw;
@@ -1097,7 +1239,7 @@ __global__ __launch_bounds__(AG_WG) void pr_dd_gather_kernel(PrCtl C, PrF32Args 
         const double err = (double)fabsf(__fsub_rn(nw, old));
         const bool upd = err >= A.eps;
         if (lane == 0) {
-            red.err += __ddiv_rn(err, A.dn);
+            red.err += err;
             if (upd) {
                 A.rank[v] = nw;
                 red.active += 1u;
@@ -1202,18 +1344,29 @@ __global__ __launch_bounds__(AG_WG) void pr_dd_compact_kernel(PrState *st, uint3
     }
 }
 
-// Finish of a data-driven iteration: closes it and clears the consumed worklist's length,
-// which the compaction of the next iteration fills again.
-__global__ __launch_bounds__(AG_FIN_WG) void pr_dd_finish(PrCtl C)
+// Finish of a data-driven iteration: closes it in place and clears the consumed worklist's
+// length, which the compaction of the next iteration fills again. Worklist runs keep their state
+// in st[0] alone: every kernel reads the lists' lengths there.
+__global__ __launch_bounds__(AG_WG) void pr_dd_finish(PrCtl C)
 {
     PrState *st = C.st;
     if (*(volatile const uint32_t *)&st->done)
         return;
-    const uint32_t iter = *(volatile const uint32_t *)&st->iter;
-    pr_close(C, iter, Red{});
+    double E = 0.0;
+    uint32_t A = 0u;
+    for (uint32_t i = threadIdx.x; i < C.nparts; i += AG_WG) {
+        E += C.part_err[i];
+        A += C.part_act[i];
+    }
+    block_sum_all<AG_WG>(E, A);
     if (threadIdx.x == 0) {
-        st->dd_count[iter & 1u] = 0u;
-        st->dd_hubs[iter & 1u] = 0u;
+        PrRun S = pr_load(st);
+        pr_control(C, S, C.it, E, A, true);
+        pr_save(st, S);
+        st->dd_count[C.it & 1u] = 0u;
+        st->dd_hubs[C.it & 1u] = 0u;
+        if (C.hist_t)
+            C.hist_t[2u * C.it + 1u] = wall_clock64();
     }
 }
 
@@ -1333,7 +1486,7 @@ static void session_free(ag_pr_session *s)
         return;
     (void)hipSetDevice(s->g->dev->ordinal);
     (void)hipStreamSynchronize(s->g->dev->stream);
-    void *ptrs[] = {s->st, s->part_err, s->part_act, s->part_cmax, s->hist_err, s->hist_act,
+    void *ptrs[] = {s->st, s->part_err, s->part_act, s->part_cmax, s->hist_err, s->hist_act, s->hist_t,
                     s->rank, s->c[0], s->c[1], s->c16[0], s->c16[1], s->dd_queue[0],
                     s->dd_queue[1], s->dd_flag, s->fin_part, s->fin_sum, s->user};
     for (void *p : ptrs)
@@ -1341,11 +1494,8 @@ static void session_free(ag_pr_session *s)
             (void)hipFree(p);
     if (s->st_host)
         (void)hipHostFree(s->st_host);
-    if (s->ev) {
-        for (uint32_t i = 0; i < s->ev_count; i++)
-            (void)hipEventDestroy(s->ev[i]);
-        free(s->ev);
-    }
+    if (s->loop_ev)
+        (void)hipEventDestroy(s->loop_ev);
     if (s->step_ev[0])
         (void)hipEventDestroy(s->step_ev[0]);
     if (s->step_ev[1])
@@ -1376,22 +1526,27 @@ static uint32_t ag_quant_grid(const ag_dgraph *g)
     return need < 1u ? 1u : need < cap ? need : cap;
 }
 
-// Codes of the next iteration (quantised kinds), after the iteration's finish kernel.
-static void ag_launch_quant(ag_pr_session *s)
+// Codes of the next iteration (quantised kinds), after an iteration's last kernel: from the
+// maximum of its nparts partials, into state `slot`, which the next iteration reads.
+static void ag_launch_quant(ag_pr_session *s, uint32_t slot, uint32_t nparts)
 {
     ag_dgraph *g = s->g;
     hipStream_t stream = g->dev->stream;
     const uint32_t grid = ag_quant_grid(g);
     const float *cf = (const float *)s->c[0];
+    PrState *st = s->st + slot;
     switch (s->kind_code) {
     case 132:
-        pr_quant_kernel<32><<<grid, AG_WG, 0, stream>>>(g->n, s->st, cf, (uint32_t *)s->c[1]);
+        pr_quant_kernel<32><<<grid, AG_WG, 0, stream>>>(g->n, st, cf, (uint32_t *)s->c[1],
+                                                           s->part_cmax, nparts);
         break;
     case 116:
-        pr_quant_kernel<16><<<grid, AG_WG, 0, stream>>>(g->n, s->st, cf, (uint16_t *)s->c[1]);
+        pr_quant_kernel<16><<<grid, AG_WG, 0, stream>>>(g->n, st, cf, (uint16_t *)s->c[1],
+                                                           s->part_cmax, nparts);
         break;
     default:
-        pr_quant_kernel<8><<<grid, AG_WG, 0, stream>>>(g->n, s->st, cf, (uint8_t *)s->c[1]);
+        pr_quant_kernel<8><<<grid, AG_WG, 0, stream>>>(g->n, st, cf, (uint8_t *)s->c[1],
+                                                           s->part_cmax, nparts);
         break;
     }
 }
@@ -1479,7 +1634,7 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     const uint32_t nblk = ag_pr_max_parts(g);
     const uint32_t fblk = (n + AG_WG - 1) / AG_WG ? (n + AG_WG - 1) / AG_WG : 1;
 
-    AG_TRY(salloc(s, (void **)&s->st, sizeof(PrState)));
+    AG_TRY(salloc(s, (void **)&s->st, 2 * sizeof(PrState)));
     {
         hipError_t e = hipHostMalloc((void **)&s->st_host, sizeof(PrState), hipHostMallocDefault);
         if (e != hipSuccess) {
@@ -1487,12 +1642,14 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
             return ag_hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
         }
     }
-    AG_TRY(salloc(s, (void **)&s->part_err, (size_t)nblk * sizeof(double)));
-    AG_TRY(salloc(s, (void **)&s->part_act, (size_t)nblk * sizeof(uint32_t)));
+    AG_TRY(salloc(s, (void **)&s->part_err, (size_t)nblk * 2 * sizeof(double)));
+    AG_TRY(salloc(s, (void **)&s->part_act, (size_t)nblk * 2 * sizeof(uint32_t)));
     if (kc > 100)
         AG_TRY(salloc(s, (void **)&s->part_cmax, (size_t)nblk * sizeof(uint32_t)));
     AG_TRY(salloc(s, (void **)&s->hist_err, (size_t)maxit * sizeof(double)));
     AG_TRY(salloc(s, (void **)&s->hist_act, (size_t)maxit * sizeof(uint32_t)));
+    if (o.record_history)
+        AG_TRY(salloc(s, (void **)&s->hist_t, (size_t)maxit * 2 * sizeof(uint64_t)));
     AG_TRY(salloc(s, (void **)&s->rank, (size_t)n * sizeof(float)));
     AG_TRY(salloc(s, &s->c[0], (size_t)n * celem));
     AG_TRY(salloc(s, &s->c[1], (size_t)n * celem));
@@ -1535,7 +1692,7 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
         if (kc > 100) {
             pr_quant_init_max<<<ag_quant_grid(g), AG_WG, 0, stream>>>(n, (const float *)s->c[0],
                                                                      s->st);
-            ag_launch_quant(s);
+            ag_launch_quant(s, 0u, 0u);
         }
         if (s->dd_queue[0]) {
             // data-driven pull: every vertex starts listed
@@ -1550,26 +1707,12 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
             return ag_hip_fail(e, "pr_init_kernel launch", __FILE__, __LINE__);
         }
     }
-    if (o.record_history) {
-        s->ev_count = maxit + 1;
-        s->ev = (hipEvent_t *)calloc(s->ev_count, sizeof(hipEvent_t));
-        if (!s->ev) {
-            session_free(s);
-            return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        }
-        for (uint32_t i = 0; i < s->ev_count; i++) {
-            hipError_t e = hipEventCreate(&s->ev[i]);
-            if (e != hipSuccess) {
-                s->ev_count = i;
-                session_free(s);
-                return ag_hip_fail(e, "hipEventCreate", __FILE__, __LINE__);
-            }
-        }
-    }
     {
         hipError_t e = hipEventCreate(&s->step_ev[0]);
         if (e == hipSuccess)
             e = hipEventCreate(&s->step_ev[1]);
+        if (e == hipSuccess && o.record_history)
+            e = hipEventCreate(&s->loop_ev);
         if (e != hipSuccess) {
             session_free(s);
             return ag_hip_fail(e, "hipEventCreate", __FILE__, __LINE__);
@@ -1579,10 +1722,13 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     return AG_OK;
 }
 
-#define AG_PR_LAUNCH_REGULAR(MAIN, FIN)                      \
+#define AG_PR_LAUNCH_REGULAR(MAIN, HUBS)                     \
     do {                                                     \
         MAIN<<<grid, block, 0, stream>>>(G, C, A);           \
-        FIN<<<1, fin, 0, stream>>>(G, C, A);                 \
+        if (g->n_hubs) {                                     \
+            C.part_base = grid;                              \
+            HUBS<<<1, fin, 0, stream>>>(G, C, A);            \
+        }                                                    \
     } while (0)
 
 // Default resident workgroups per CU of the two blocked passes (plan wg_per_cu overrides
@@ -1593,33 +1739,67 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
 #endif
 #define AG_COMBINE_PER_CU 8u
 
-#define AG_PR_LAUNCH_BLOCKED(BLK, CMB, FIN)                                  \
+// Pass 1 leaves partials only where it finishes rows itself (the unblocked ones).
+#define AG_PR_LAUNCH_BLOCKED(BLK, CMB)                                       \
     do {                                                                     \
         static const uint32_t res1 = ag_resident_per_cu(BLK);               \
         static const uint32_t res2 = ag_resident_per_cu(CMB);               \
-        const uint32_t g1 = ag_blocked_grid(g, res1, AG_PASS1_PER_CU);                    \
-        const uint32_t g2 = ag_blocked_grid(g, res2, AG_COMBINE_PER_CU);                    \
-        C.nparts = g1 + g2;                                                  \
-        C.part_base = 0;                                                     \
-        BLK<<<g1, block, 0, stream>>>(G, B1, C, A);                          \
-        C.part_base = g1;                                                    \
+        const uint32_t g1 = ag_blocked_grid(g, res1, AG_PASS1_PER_CU);      \
+        const uint32_t g2 = ag_blocked_grid(g, res2, AG_COMBINE_PER_CU);    \
+        const uint32_t p1 = B.has_reg ? g1 : 0u;                             \
+        C.nparts = p1 + g2;                                                  \
+        PrCtl C1 = C;                                                        \
+        if (!p1)                                                             \
+            C1.part_err = nullptr;                                           \
+        BLK<<<g1, block, 0, stream>>>(G, B1, C1, A);                         \
+        C.part_base = p1;                                                    \
         CMB<<<g2, block, 0, stream>>>(B, C, A);                              \
-        FIN<<<1, fin, 0, stream>>>(G, C, A);                                 \
     } while (0)
 
 // The FP32 kinds (any contribution storage) first gather the hot-segment tiles from LDS
-// (when the plan has hot segments); pass 1 then skips them.
+// (when the plan has hot segments); pass 1 then skips them. Both close the previous iteration
+// (to the same state), the hot pass reads the clock.
 #define AG_HOT_PER_CU 2u
-#define AG_PR_LAUNCH_BLOCKED_HOT(HOT, BLK, CMB, FIN)                         \
+#define AG_PR_LAUNCH_BLOCKED_HOT(HOT, BLK, CMB)                              \
     do {                                                                     \
         if (g->blk.n_hgrp) {                                                 \
             static const uint32_t resh = ag_resident_per_cu(HOT);           \
+            static const uint32_t resc = ag_resident_per_cu(CMB);           \
             const uint32_t gh = ag_blocked_grid(g, resh, AG_HOT_PER_CU);    \
+            static const uint32_t resb = ag_resident_per_cu(BLK);           \
+            C.nparts = (B.has_reg ? ag_blocked_grid(g, resb, AG_PASS1_PER_CU) : 0u) + \
+                       ag_blocked_grid(g, resc, AG_COMBINE_PER_CU);          \
             HOT<<<gh, block, 0, stream>>>(B, C, A);                          \
             ag_block_geom_skip_hot(g, B1);                                   \
+            C.hist_t = nullptr;                                              \
         }                                                                    \
-        AG_PR_LAUNCH_BLOCKED(BLK, CMB, FIN);                                 \
+        AG_PR_LAUNCH_BLOCKED(BLK, CMB);                                      \
     } while (0)
+
+// Control block of the iteration about to be enqueued (number s->enqueued).
+static PrCtl pr_ctl(const ag_pr_session *s, bool pending)
+{
+    const uint32_t it = s->enqueued, cap = ag_pr_max_parts(s->g);
+    PrCtl C;
+    memset(&C, 0, sizeof(C));
+    C.st = s->st;
+    C.part_err = s->part_err + (size_t)(it & 1u) * cap;
+    C.part_act = s->part_act + (size_t)(it & 1u) * cap;
+    C.prev_err = s->part_err + (size_t)((it & 1u) ^ 1u) * cap;
+    C.prev_act = s->part_act + (size_t)((it & 1u) ^ 1u) * cap;
+    C.part_cmax = s->kind_code > 100 ? s->part_cmax : nullptr;
+    C.hist_err = s->hist_err;
+    C.hist_act = s->hist_act;
+    C.hist_t = s->hist_t;
+    C.it = it;
+    C.pending = pending ? 1u : 0u;
+    C.stop_rule = s->o.stop_rule;
+    C.mixed = (s->kind_code == 1 || s->kind_code == 2) ? 1u : 0u;
+    C.l1_tol = s->o.l1_tolerance;
+    C.refine_l1 = s->o.refine_l1;
+    C.dn = (double)s->g->n;
+    return C;
+}
 
 // The push (pageRankPushGraphCSR, pageRank.c:1111-1272; pageRankPushFixedPointGraphCSR,
 // :1992-2117) adds every contribution into its destinations' sums: the pull's sums, and the same
@@ -1629,24 +1809,13 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
 // (0.2 T/s over the chip, and 27 bytes of HBM writes per 4-byte store), against 270 us; with
 // memory atomics 33 ms on RMAT-25. The pull's order is also closer to 64 bits (RMAT-22, 10
 // iterations: 6e-8 against 3e-6) and the same on every run.
-int ag_pr_launch_iteration(ag_pr_session *s)
+static int pr_launch_iteration(ag_pr_session *s, bool pending)
 {
     ag_dgraph *g = s->g;
     hipStream_t stream = g->dev->stream;
     const bool blocked = g->blk.bits != 0;
     PullGeom G = blocked ? ag_make_unblocked_geom(g) : ag_make_geom(g);
-    PrCtl C;
-    C.st = s->st;
-    C.part_err = s->part_err;
-    C.part_act = s->part_act;
-    C.part_cmax = s->kind_code > 100 ? s->part_cmax : nullptr;
-    C.hist_err = s->hist_err;
-    C.hist_act = s->hist_act;
-    C.part_base = 0;
-    C.stop_rule = s->o.stop_rule;
-    C.mixed = (s->kind_code == 1 || s->kind_code == 2) ? 1u : 0u;
-    C.l1_tol = s->o.l1_tolerance;
-    C.refine_l1 = s->o.refine_l1;
+    PrCtl C = pr_ctl(s, pending);
     PrF32Args A;
     A.c32[0] = s->c[0];
     A.c32[1] = s->c[1];
@@ -1656,21 +1825,21 @@ int ag_pr_launch_iteration(ag_pr_session *s)
     A.outdeg = g->outdeg;
     A.base = pr_base();
     A.damp = pr_damp();
-    A.dn = (double)g->n;
     A.eps = s->o.epsilon;
     const uint32_t lds = (s->kind_code >= 8) ? AG_TILE_NNZ_MAX * 8u : AG_TILE_NNZ_MAX * 4u;
     dim3 block(AG_WG), fin(AG_FIN_WG);
     if (s->o.direction == AG_DIR_DATA_DRIVEN && blocked && !s->dd_queue[0]) {
         const BlockGeom B = ag_make_block_geom(g);
         const BlockGeom &B1 = B;
-        AG_PR_LAUNCH_BLOCKED(pr_ddf_blk_kernel, pr_ddf_cmb_kernel, pr_ddf_finish);
+        AG_PR_LAUNCH_BLOCKED(pr_ddf_blk_kernel, pr_ddf_cmb_kernel);
+        s->nparts = C.nparts;
         AG_HIP(hipGetLastError());
         return AG_OK;
     }
     if (s->o.direction == AG_DIR_DATA_DRIVEN && !s->dd_queue[0]) {
         C.nparts = ag_pull_grid(g, AG_TILE_NNZ_MAX * 4u);
         pr_dds_kernel<<<C.nparts, block, 0, stream>>>(G, C, A);
-        pr_plain_finish<<<1, fin, 0, stream>>>(C);
+        s->nparts = C.nparts;
         AG_HIP(hipGetLastError());
         return AG_OK;
     }
@@ -1685,7 +1854,7 @@ int ag_pr_launch_iteration(ag_pr_session *s)
         pr_dd_compact_kernel<<<gq, block, 0, stream>>>(s->st, g->n, g->off, s->dd_flag,
                                                        s->dd_queue[(it & 1u) ^ 1u],
                                                        (it & 1u) ^ 1u);
-        pr_dd_finish<<<1, fin, 0, stream>>>(C);
+        pr_dd_finish<<<1, block, 0, stream>>>(C);
         AG_HIP(hipGetLastError());
         return AG_OK;
     }
@@ -1694,60 +1863,59 @@ int ag_pr_launch_iteration(ag_pr_session *s)
         BlockGeom B1 = B;   // pass 1: past the hot tiles when the hot pass gathers them
         switch (s->kind_code) {
         case 0:
-            AG_PR_LAUNCH_BLOCKED_HOT(pr_f32_hot_kernel, pr_f32_blk_kernel, pr_f32_cmb_kernel,
-                                     pr_f32_finish);
+            AG_PR_LAUNCH_BLOCKED_HOT(pr_f32_hot_kernel, pr_f32_blk_kernel, pr_f32_cmb_kernel);
             break;
         case 1:
-            AG_PR_LAUNCH_BLOCKED_HOT(pr_bf16_hot_kernel, pr_bf16_blk_kernel, pr_bf16_cmb_kernel,
-                                     pr_bf16_finish);
+            AG_PR_LAUNCH_BLOCKED_HOT(pr_bf16_hot_kernel, pr_bf16_blk_kernel, pr_bf16_cmb_kernel);
             break;
         case 2:
-            AG_PR_LAUNCH_BLOCKED_HOT(pr_f16_hot_kernel, pr_f16_blk_kernel, pr_f16_cmb_kernel,
-                                     pr_f16_finish);
+            AG_PR_LAUNCH_BLOCKED_HOT(pr_f16_hot_kernel, pr_f16_blk_kernel, pr_f16_cmb_kernel);
             break;
         case 64:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<64>, pr_int_cmb_kernel<64>, pr_int_finish<64>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<64>, pr_int_cmb_kernel<64>);
             break;
         case 32:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<32>, pr_int_cmb_kernel<32>, pr_int_finish<32>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<32>, pr_int_cmb_kernel<32>);
             break;
         case 16:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<16>, pr_int_cmb_kernel<16>, pr_int_finish<16>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<16>, pr_int_cmb_kernel<16>);
             break;
         case 8:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<8>, pr_int_cmb_kernel<8>, pr_int_finish<8>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<8>, pr_int_cmb_kernel<8>);
             break;
         case 132:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<132>, pr_int_cmb_kernel<132>, pr_int_finish<132>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<132>, pr_int_cmb_kernel<132>);
             break;
         case 116:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<116>, pr_int_cmb_kernel<116>, pr_int_finish<116>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<116>, pr_int_cmb_kernel<116>);
             break;
         default:
-            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<108>, pr_int_cmb_kernel<108>, pr_int_finish<108>);
+            AG_PR_LAUNCH_BLOCKED(pr_int_blk_kernel<108>, pr_int_cmb_kernel<108>);
             break;
         }
+        s->nparts = C.nparts;
         if (s->kind_code > 100)
-            ag_launch_quant(s);
+            ag_launch_quant(s, (C.it + 1u) & 1u, C.nparts);
         AG_HIP(hipGetLastError());
         return AG_OK;
     }
     const uint32_t grid = ag_tile_grid(g, lds);
-    C.nparts = grid;
+    C.nparts = grid + (g->n_hubs ? 1u : 0u);
+    s->nparts = C.nparts;
     switch (s->kind_code) {
-    case 0: AG_PR_LAUNCH_REGULAR(pr_f32_kernel, pr_f32_finish); break;
-    case 1: AG_PR_LAUNCH_REGULAR(pr_bf16_kernel, pr_bf16_finish); break;
-    case 2: AG_PR_LAUNCH_REGULAR(pr_f16_kernel, pr_f16_finish); break;
-    case 64: AG_PR_LAUNCH_REGULAR(pr_int_kernel<64>, pr_int_finish<64>); break;
-    case 32: AG_PR_LAUNCH_REGULAR(pr_int_kernel<32>, pr_int_finish<32>); break;
-    case 16: AG_PR_LAUNCH_REGULAR(pr_int_kernel<16>, pr_int_finish<16>); break;
-    case 8: AG_PR_LAUNCH_REGULAR(pr_int_kernel<8>, pr_int_finish<8>); break;
-    case 132: AG_PR_LAUNCH_REGULAR(pr_int_kernel<132>, pr_int_finish<132>); break;
-    case 116: AG_PR_LAUNCH_REGULAR(pr_int_kernel<116>, pr_int_finish<116>); break;
-    default: AG_PR_LAUNCH_REGULAR(pr_int_kernel<108>, pr_int_finish<108>); break;
+    case 0: AG_PR_LAUNCH_REGULAR(pr_f32_kernel, pr_f32_hubs); break;
+    case 1: AG_PR_LAUNCH_REGULAR(pr_bf16_kernel, pr_bf16_hubs); break;
+    case 2: AG_PR_LAUNCH_REGULAR(pr_f16_kernel, pr_f16_hubs); break;
+    case 64: AG_PR_LAUNCH_REGULAR(pr_int_kernel<64>, pr_int_hubs<64>); break;
+    case 32: AG_PR_LAUNCH_REGULAR(pr_int_kernel<32>, pr_int_hubs<32>); break;
+    case 16: AG_PR_LAUNCH_REGULAR(pr_int_kernel<16>, pr_int_hubs<16>); break;
+    case 8: AG_PR_LAUNCH_REGULAR(pr_int_kernel<8>, pr_int_hubs<8>); break;
+    case 132: AG_PR_LAUNCH_REGULAR(pr_int_kernel<132>, pr_int_hubs<132>); break;
+    case 116: AG_PR_LAUNCH_REGULAR(pr_int_kernel<116>, pr_int_hubs<116>); break;
+    default: AG_PR_LAUNCH_REGULAR(pr_int_kernel<108>, pr_int_hubs<108>); break;
     }
     if (s->kind_code > 100)
-        ag_launch_quant(s);
+        ag_launch_quant(s, (C.it + 1u) & 1u, C.nparts);
     AG_HIP(hipGetLastError());
     return AG_OK;
 }
@@ -1768,17 +1936,21 @@ extern "C" int ag_pr_step(ag_pr_session *s, uint32_t iterations)
     if (s->g->total_blocks == 0)
         return AG_OK;
     AG_HIP(hipEventRecord(s->step_ev[0], stream));
+    if (s->o.record_history && s->enqueued == 0)
+        AG_HIP(hipEventRecord(s->loop_ev, stream));
     for (uint32_t i = 0; i < iterations && s->enqueued < maxit; i++) {
-        if (s->ev)
-            AG_HIP(hipEventRecord(s->ev[s->enqueued], stream));
-        int st = ag_pr_launch_iteration(s);
+        int st = pr_launch_iteration(s, i > 0);
         if (st != AG_OK)
             return st;
         s->enqueued++;
         s->step_launches++;
     }
-    if (s->ev)
-        AG_HIP(hipEventRecord(s->ev[s->enqueued], stream));
+    if (s->step_launches && !s->dd_queue[0]) {
+        PrCtl C = pr_ctl(s, true);
+        C.nparts = s->nparts;
+        pr_close_kernel<<<1, AG_WG, 0, stream>>>(C);
+        AG_HIP(hipGetLastError());
+    }
     AG_HIP(hipEventRecord(s->step_ev[1], stream));
     return AG_OK;
 }
@@ -1812,8 +1984,9 @@ extern "C" int ag_pr_poll(ag_pr_session *s, ag_pr_result *res)
     if (!s)
         return ag_set_error(AG_ERR_INVALID, "session is null");
     AG_HIP(hipSetDevice(s->g->dev->ordinal));
-    AG_HIP(hipMemcpyAsync(s->st_host, s->st, sizeof(PrState), hipMemcpyDeviceToHost,
-                          s->g->dev->stream));
+    // worklist runs keep their state in st[0], the others where the next iteration reads it
+    AG_HIP(hipMemcpyAsync(s->st_host, s->st + (s->dd_queue[0] ? 0u : s->enqueued & 1u),
+                          sizeof(PrState), hipMemcpyDeviceToHost, s->g->dev->stream));
     int st = ag_wait_stream(s->g->dev);
     if (st != AG_OK)
         return st;
@@ -1860,13 +2033,20 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
         AG_HIP(hipMemcpy(active, s->hist_act, (size_t)k * sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (error)
         AG_HIP(hipMemcpy(error, s->hist_err, (size_t)k * sizeof(double), hipMemcpyDeviceToHost));
-    if (iter_ms) {
-        for (uint32_t i = 0; i < k; i++) {
-            float ms = 0.0f;
-            if (s->ev && i + 1 < s->ev_count && i + 1 <= s->enqueued)
-                AG_HIP(hipEventElapsedTime(&ms, s->ev[i], s->ev[i + 1]));
-            iter_ms[i] = ms;
-        }
+    if (iter_ms)
+        memset(iter_ms, 0, (size_t)k * sizeof(float));
+    if (iter_ms && s->hist_t) {
+        int khz = 0;   // the device clock ticks at a constant rate
+        AG_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, s->g->dev->ordinal));
+        uint64_t *t = (uint64_t *)malloc((size_t)k * 2 * sizeof(uint64_t));
+        if (!t)
+            return ag_set_error(AG_ERR_OOM, "host allocation failed");
+        hipError_t e = hipMemcpy(t, s->hist_t, (size_t)k * 2 * sizeof(uint64_t),
+                                 hipMemcpyDeviceToHost);
+        for (uint32_t i = 0; e == hipSuccess && khz > 0 && i < k; i++)
+            iter_ms[i] = (float)((double)(t[2 * i + 1] - t[2 * i]) / (double)khz);
+        free(t);
+        AG_HIP(e);
     }
     return AG_OK;
 }
@@ -1929,8 +2109,8 @@ extern "C" int ag_pr_end(ag_pr_session *s, float *ranks_out, ag_pr_result *res)
         *res = r;
         res->rank_sum = sum;
         float ms = 0.0f;
-        if (s->ev && s->enqueued > 0) {
-            if (hipEventElapsedTime(&ms, s->ev[0], s->ev[s->enqueued]) != hipSuccess)
+        if (s->loop_ev && s->enqueued > 0) {
+            if (hipEventElapsedTime(&ms, s->loop_ev, s->step_ev[1]) != hipSuccess)
                 ms = 0.0f;
         }
         res->loop_ms = ms;

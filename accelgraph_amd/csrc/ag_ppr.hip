@@ -420,7 +420,7 @@ __global__ __launch_bounds__(AG_FIN_WG) void ppr_finish_kernel(PullGeom G, PprAr
     if (C.storage != AG_STORE_F32) {
         const int32_t ri = st->refine_iter;
         if (ri < 0) {
-            refine_decide(st, iter, E, C.refine_l1);
+            refine_decide(*st, iter, E, C.refine_l1);
             can_stop = false;
         } else {
             can_stop = (int32_t)iter >= ri + 1;

@@ -20,8 +20,8 @@
 // The main kernel runs a persistent grid (compute units x resident workgroups); workgroup b
 // takes items b, b + grid, b + 2*grid, ... so the heavy items spread over the whole chip first.
 // No atomics on global memory: hub partials and per-workgroup reductions go to plain arrays
-// that a one-workgroup finish kernel reads after the launch boundary, in a fixed order, so
-// every result is deterministic from run to run. Lane partials use four independent
+// that are added after the launch boundary, in a fixed order, so every result is
+// deterministic from run to run. Lane partials use four independent
 // accumulators (memory-level parallelism) combined in a fixed tree.
 //
 // Source-blocked graphs (the second half of this file) replace the gather by two passes over
@@ -442,16 +442,56 @@ __device__ __forceinline__ Acc lane_sum(const Acc *s_vals, uint32_t b, uint32_t 
     return acc;
 }
 
+// A workgroup's tile, with its ids and per-edge data loaded (or on their way), and the next one.
 template <class P>
-__device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, uint32_t i,
-                                               uint32_t step, Red &red, const TileLds<P> &L)
+struct TileAhead {
+    uint32_t i;             // of the next tile
+    RowTile cur, nxt;
+    uint32_t w[AG_TILE_UNROLL];
+    typename EdgeOf<P>::T ed[AG_TILE_UNROLL];
+
+    __device__ __forceinline__ void load_ids(const PullGeom &G, const P &pol, const RowTile &t)
+    {
+#pragma unroll
+        for (int u = 0; u < AG_TILE_UNROLL; u++) {
+            const uint32_t j = t.e0 + threadIdx.x + u * AG_WG;
+            w[u] = j < t.e1 ? ld_stream(&G.src[j]) : 0u;
+            ed[u] = j < t.e1 ? EdgeOf<P>::load(pol, j) : typename EdgeOf<P>::T{};
+        }
+    }
+    // The workgroup's first tile: items n_heavy + b, n_heavy + b + grid, ... are its tiles.
+    __device__ __forceinline__ void load(const PullGeom &G, const P &pol)
+    {
+        const uint32_t h = G.n_heavy, b = blockIdx.x, g = gridDim.x;
+        const uint32_t first = b < h ? b + (h - b + g - 1u) / g * g - h : b - h;
+        cur = row_tile_at(G, first);
+        nxt = row_tile_at(G, first + g);
+        i = first + g;
+        load_ids(G, pol, cur);
+    }
+};
+
+// T: TileAhead of a policy with the same per-edge data. Unless `opened`, open(pol) is called once,
+// when the first tile's values have been gathered (its own loads are then in flight with them);
+// false ends the launch with nothing written.
+template <class P, class T, class OPEN>
+__device__ __forceinline__ void pull_row_tiles(const PullGeom &G, P &pol, Red &red,
+                                               const TileLds<P> &L, T &ahead, bool opened,
+                                               OPEN open)
 {
     using Acc = typename P::Acc;
     const uint32_t tid = threadIdx.x, wave = tid / AG_WAVE, lane = tid % AG_WAVE;
+    const uint32_t step = gridDim.x;
     using ED = EdgeOf<P>;
-    RowTile cur = row_tile_at(G, i), nxt = row_tile_at(G, i + step);
+    uint32_t i = ahead.i;
+    RowTile cur = ahead.cur, nxt = ahead.nxt;
     uint32_t w[AG_TILE_UNROLL];
     typename ED::T ed[AG_TILE_UNROLL];
+#pragma unroll
+    for (int u = 0; u < AG_TILE_UNROLL; u++) {
+        w[u] = ahead.w[u];
+        ed[u] = ahead.ed[u];
+    }
     const auto load_ids = [&](const RowTile &t) {
 #pragma unroll
         for (int u = 0; u < AG_TILE_UNROLL; u++) {
@@ -460,7 +500,6 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, 
             ed[u] = j < t.e1 ? ED::load(pol, j) : typename ED::T{};
         }
     };
-    load_ids(cur);
     while (cur.r1 > cur.r0) {
         // this lane's first row: bounds and update operands
         uint32_t r = cur.r0 + tid, b = 0, e = 0;
@@ -477,7 +516,12 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, 
                 L.vals[j - cur.e0] = ED::term(NoTop(), pol, j, w[u], ed[u]);
         }
         i += step;
-        const RowTile nn = row_tile_at(G, i + step);
+        const RowTile nn = row_tile_at(G, i);
+        if (!opened) {
+            if (!open(pol))
+                return;
+            opened = true;
+        }
         __syncthreads();
         load_ids(nxt);   // in flight during the sums
         uint32_t nl = 0;   // this wavefront's long rows
@@ -539,18 +583,25 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, const P &pol, 
         cur = nxt;
         nxt = nn;
     }
+    if (!opened)   // no tile for this workgroup
+        open(pol);
 }
 
 // All work items of one workgroup of the persistent grid: the items above the row tiles (hub
-// segments and workgroup rows), then tiles.
-template <class P>
-__device__ __forceinline__ void pull_items(const PullGeom &G, const P &pol, Red &red,
-                                           const TileLds<P> &L, typename P::Acc *s_wave)
+// segments and workgroup rows), then tiles; `open` as in pull_row_tiles, before the first item.
+template <class P, class T, class OPEN>
+__device__ __forceinline__ void pull_items(const PullGeom &G, P &pol, Red &red,
+                                           const TileLds<P> &L, typename P::Acc *s_wave, T &ahead,
+                                           bool opened, OPEN open)
 {
-    uint32_t it = blockIdx.x;
-    for (; it < G.n_heavy; it += gridDim.x)
+    if (!opened && blockIdx.x < G.n_heavy) {
+        if (!open(pol))
+            return;
+        opened = true;
+    }
+    for (uint32_t it = blockIdx.x; it < G.n_heavy; it += gridDim.x)
         pull_one_item(G, pol, it, red, L.vals, s_wave);
-    pull_row_tiles(G, pol, it - G.n_heavy, gridDim.x, red, L);
+    pull_row_tiles(G, pol, red, L, ahead, opened, open);
 }
 
 // ---------------------------------------------------------------- source-blocked pull
@@ -1085,7 +1136,9 @@ __global__ __launch_bounds__(AG_WG) void pull_kernel(PullGeom G, P pol)
     AG_TILE_LDS(P, tile);
     __shared__ typename P::Acc s_wave[AG_WG / AG_WAVE];
     Red red{};
-    pull_items(G, pol, red, tile, s_wave);
+    TileAhead<P> ahead;
+    ahead.load(G, pol);
+    pull_items(G, pol, red, tile, s_wave, ahead, true, [](P &) { return true; });
 }
 
 // Plain source-blocked pull (SpMV): pass 1 with `pol` reading per-edge data in virtual-row
@@ -1120,18 +1173,19 @@ __global__ __launch_bounds__(AG_FIN_WG) void pull_finish_kernel(PullGeom G, P po
     pull_hub_finish(G, pol, red);
 }
 
-// Storage switch of the 16-bit contribution phase (one thread): switch to f32 contributions
-// from iteration iter + 1 once the L1 delta E is at most refine_l1, or once E has not improved
-// on its best value by 1% for three iterations (the 16-bit rounding floor has been reached).
-__device__ __forceinline__ void refine_decide(PrState *st, uint32_t iter, double E,
-                                              double refine_l1)
+// Storage switch of the 16-bit contribution phase (st: best_err, stall, refine_iter): switch to
+// f32 contributions from iteration iter + 1 once the L1 delta E is at most refine_l1, or once E
+// has not improved on its best value by 1% for three iterations (the 16-bit rounding floor has
+// been reached).
+template <class S>
+__device__ __forceinline__ void refine_decide(S &st, uint32_t iter, double E, double refine_l1)
 {
-    if (iter == 0 || E < 0.99 * st->best_err) {
-        st->best_err = E;
-        st->stall = 0;
+    if (iter == 0 || E < 0.99 * st.best_err) {
+        st.best_err = E;
+        st.stall = 0;
     } else {
-        st->stall++;
+        st.stall++;
     }
-    if (E <= refine_l1 || st->stall >= 3)
-        st->refine_iter = (int32_t)iter + 1;
+    if (E <= refine_l1 || st.stall >= 3)
+        st.refine_iter = (int32_t)iter + 1;
 }

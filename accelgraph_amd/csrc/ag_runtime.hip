@@ -314,6 +314,7 @@ BlockGeom ag_make_block_geom(const ag_dgraph *g)
     K.vsp = B.vsp;
     K.tbase = B.tbase;
     K.sbits = B.bits && B.sorted ? B.bits : 0u;
+    K.has_reg = B.r_slot_blk0[AG_NSLOTS] ? 1u : 0u;
     return K;
 }
 

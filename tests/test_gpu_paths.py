@@ -121,3 +121,34 @@ def test_weighted_tiles(device, plan, form):
         want = oracle.spmv_push_fixed(g.edges_idx, g.out_degree, g.fwd_dest, g.fwd_weight, xq, 3)
         np.testing.assert_array_equal(dg.spmv_push_fixed(xq, 3)[0], want)
     dg.close()
+
+
+STEP_RUNS = [dict(kind=ag.KIND_F32), dict(kind=ag.KIND_F32, storage=ag.STORE_BF16, refine_l1=1e-2),
+             dict(kind=ag.KIND_FIXED32), dict(kind=ag.KIND_QUANT16),
+             dict(kind=ag.KIND_F32, direction=ag.DIR_DATA_DRIVEN)]
+
+
+@pytest.mark.parametrize("plan", [{}, dict(src_block_bits=8), dict(src_block_bits=8, blocked_min_bin=1),
+                                  dict(src_block_bits=8, hot_segments=16),
+                                  dict(thread_max_deg=2, group16_max_deg=6, wave_max_deg=20,
+                                       block_max_deg=60, segment_nnz=256)])
+@pytest.mark.parametrize("run", range(len(STEP_RUNS)))
+def test_steps_of_any_length(device, plan, run):
+    """An iteration is closed by the next one's first launch, or at the end of its step: the same
+    run however many iterations a step queues, past the stop included, with a time for each."""
+    g = ag.Graph.rmat(11)
+    dg = device.upload(g, params=ag.plan_params(**plan))
+    want = None
+    for chunk in (32, 1, 2, 3, 7):
+        r = dg.pagerank(chunk=chunk, max_iterations=90, epsilon=1e-4, **STEP_RUNS[run])
+        if want is None:
+            want = r
+            assert 5 < r.executed < 90 and r.hist_active[-1] == 0
+        assert (r.iterations, r.executed, r.refine_iteration) == (
+            want.iterations, want.executed, want.refine_iteration)
+        np.testing.assert_array_equal(r.ranks.view(np.uint32), want.ranks.view(np.uint32))
+        np.testing.assert_array_equal(r.hist_active, want.hist_active)
+        np.testing.assert_allclose(r.hist_err, want.hist_err, rtol=1e-12)
+        assert r.hist_ms.size == r.executed and np.all(r.hist_ms > 0) and np.all(r.hist_ms < 50)
+        assert abs(r.error_total - want.error_total) <= 1e-12 * want.error_total
+    dg.close()
