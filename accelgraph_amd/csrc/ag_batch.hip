@@ -76,6 +76,8 @@ struct ag_batch {
     uint32_t *h_order;        // graphs by decreasing edge count
     BatchCfg *cfg_host;       // pinned
     uint32_t *ndone_host;     // pinned
+    double *err_host;         // [G] pinned, then iters_host
+    uint32_t *iters_host;     // [G] pinned
     hipGraph_t graph;
     hipGraphExec_t exec;
     uint32_t exec_maxit;      // iterations of the captured solve (0: none)
@@ -298,6 +300,8 @@ extern "C" int ag_batch_free(ag_batch *b)
         (void)hipHostFree(b->cfg_host);
     if (b->ndone_host)
         (void)hipHostFree(b->ndone_host);
+    if (b->err_host)
+        (void)hipHostFree(b->err_host);
     free(b->h_graphs);
     free(b->h_off);
     free(b->h_order);
@@ -533,6 +537,10 @@ extern "C" int ag_batch_upload(ag_device *dev, uint32_t G, const uint32_t *vert_
         he = hipHostMalloc((void **)&b->cfg_host, sizeof(BatchCfg), hipHostMallocDefault);
         if (he == hipSuccess)
             he = hipHostMalloc((void **)&b->ndone_host, sizeof(uint32_t), hipHostMallocDefault);
+        if (he == hipSuccess)
+            he = hipHostMalloc((void **)&b->err_host, (size_t)(G ? G : 1) * 12u,
+                               hipHostMallocDefault);
+        b->iters_host = (uint32_t *)(b->err_host + G);
         if (he != hipSuccess)
             st = ag_hip_fail(he, "hipHostMalloc", __FILE__, __LINE__);
     }
@@ -682,16 +690,26 @@ extern "C" int ag_batch_pagerank(ag_batch *b, const ag_batch_options *opts, floa
     }
     if (he == hipSuccess && st == AG_OK)
         he = hipEventRecord(e1, s);
-    if (he == hipSuccess && st == AG_OK && ranks_out && b->total_n)
-        he = hipMemcpyAsync(ranks_out, b->a.out, (size_t)b->total_n * sizeof(float),
+    if (st == AG_OK && he != hipSuccess)
+        st = ag_hip_fail(he, "batch launch", __FILE__, __LINE__);
+    // the counts and errors into pinned memory, then the ranks: one wait for all
+    if (st == AG_OK) {
+        he = hipMemcpyAsync(b->err_host, b->a.err, (size_t)b->G * sizeof(double),
                             hipMemcpyDeviceToHost, s);
-    if (he == hipSuccess && st == AG_OK && iterations)
-        he = hipMemcpyAsync(iterations, b->a.iters, (size_t)b->G * sizeof(uint32_t),
-                            hipMemcpyDeviceToHost, s);
-    if (he == hipSuccess && st == AG_OK && error)
-        he = hipMemcpyAsync(error, b->a.err, (size_t)b->G * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (st == AG_OK)
-        st = (he == hipSuccess) ? ag_wait_stream(b->dev) : ag_hip_fail(he, "batch launch", __FILE__, __LINE__);
+        if (he == hipSuccess)
+            he = hipMemcpyAsync(b->iters_host, b->a.iters, (size_t)b->G * sizeof(uint32_t),
+                                hipMemcpyDeviceToHost, s);
+        if (he != hipSuccess)
+            st = ag_hip_fail(he, "batch results", __FILE__, __LINE__);
+    }
+    if (st == AG_OK && ranks_out)
+        st = ag_copy_out(b->dev, ranks_out, b->a.out, (size_t)b->total_n * sizeof(float));
+    if (st == AG_OK && (!ranks_out || b->total_n == 0))
+        st = ag_wait_stream(b->dev);
+    if (st == AG_OK && iterations)
+        memcpy(iterations, b->iters_host, (size_t)b->G * sizeof(uint32_t));
+    if (st == AG_OK && error)
+        memcpy(error, b->err_host, (size_t)b->G * sizeof(double));
     if (st == AG_OK && device_ms) {
         float ms = 0.0f;
         he = hipEventElapsedTime(&ms, e0, e1);

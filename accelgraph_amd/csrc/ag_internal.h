@@ -9,6 +9,8 @@
 #include "../host/ag_plan.h"
 
 #define AG_MAX_EVENTS 2
+#define AG_STAGE_SLOTS 4u
+#define AG_STAGE_BYTES ((size_t)4 << 20)
 #define AG_LANE_MAX 64u    // rows of a tile with at most this many elements: a lane each
 
 struct ag_device {
@@ -19,6 +21,27 @@ struct ag_device {
     uint32_t live_graphs;   // graphs uploaded on this device and not yet freed
     uint32_t num_cus;       // compute units (persistent-grid sizing)
     void *scratch;          // this device's copy of the ag_spmv_pull_noalloc scratch array
+    // pinned ring of the staged transfers (ag_copy_in / ag_copy_out), allocated on first use
+    char *stage;                        // [AG_STAGE_SLOTS][AG_STAGE_BYTES]
+    hipEvent_t stage_ev[AG_STAGE_SLOTS];   // the last transfer through each slot
+    uint32_t stage_used;                // slots whose event has been recorded (bit mask)
+    uint32_t stage_next;                // slot of the next transfer
+    hipEvent_t time_ev[2];              // a call's timed launches
+};
+
+// Buffers that ended sessions of a graph hand back for the next one to take (every PageRank call
+// begins and ends a session): at most AG_PARK_BYTES of device memory, one pinned block and one
+// set of events. Freed with the graph, or when an allocation fails.
+#define AG_PARK_BLOCKS 8u
+#define AG_PARK_BYTES ((size_t)1 << 30)
+#define AG_PIN_BYTES ((size_t)64 << 10)
+struct ag_parked {
+    void *dev[AG_PARK_BLOCKS];
+    size_t bytes[AG_PARK_BLOCKS];
+    uint32_t n_dev;
+    void *pin;               // [AG_PIN_BYTES]
+    hipEvent_t ev[3];
+    uint32_t has_ev;
 };
 
 // Device-resident graph: the plan arrays in HBM plus launch geometry.
@@ -64,6 +87,7 @@ struct ag_dgraph {
     size_t vec_bytes;
     // personalised PageRank: buffers and the captured solve, kept between calls
     struct ag_ppr_ws *ppr;
+    struct ag_parked parked;   // buffers of ended PageRank sessions
 };
 
 // Frees g->ppr (ag_ppr.hip).
@@ -161,7 +185,11 @@ struct ag_pr_session {
     uint32_t kind_code;         // 0 f32, 1 bf16, 2 f16, 64/32/16/8
     size_t celem;               // bytes per stored contribution
     PrState *st;                // device [2], by iteration parity
-    PrState *st_host;           // pinned
+    PrState *st_host;           // pinned, the start of pin
+    void *pin;                  // [AG_PIN_BYTES] state and history on their way to the caller
+    void *blk[AG_PARK_BLOCKS];  // this session's device allocations
+    size_t blk_bytes[AG_PARK_BLOCKS];
+    uint32_t n_blk;
     double *part_err;
     uint32_t *part_act;
     uint32_t *part_cmax;        // quantised kinds: per-workgroup largest contribution bits
@@ -176,8 +204,10 @@ struct ag_pr_session {
     double *fin_sum;
     float *user;
     uint32_t enqueued;
-    uint64_t *hist_t;           // device clock per iteration when record_history (start, end)
-    hipEvent_t loop_ev;         // before the first iteration when record_history
+    uint64_t *hist_t;           // device clock per iteration when record_history (start, end);
+                                // hist_err, it and hist_act are one run of memory
+    size_t hist_bytes;          // of hist_bytes bytes
+    hipEvent_t loop_ev;         // before the first iteration
     uint32_t nparts;            // partials of one iteration's launches
     hipEvent_t step_ev[2];
     uint32_t step_launches;
@@ -191,6 +221,13 @@ int ag_graph_forward(ag_dgraph *g);
 int ag_set_error(int status, const char *fmt, ...);
 int ag_hip_fail(hipError_t e, const char *what, const char *file, int line);
 int ag_wait_stream(ag_device *dev);
+// Host -> device copy on the device's stream, through the pinned ring: `host` may be reused on
+// return. Memory that is pinned already is copied straight (then it may not, before a wait).
+int ag_copy_in(ag_device *dev, void *dst, const void *host, size_t bytes);
+// Device -> host copy after the work on the device's stream; done on return.
+int ag_copy_out(ag_device *dev, void *host, const void *src, size_t bytes);
+// Frees the parked buffers of a graph.
+void ag_parked_free(ag_dgraph *g);
 
 #define AG_HIP(call)                                                   \
     do {                                                               \

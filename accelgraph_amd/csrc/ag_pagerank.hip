@@ -1408,18 +1408,14 @@ __global__ void pr_init_kernel(uint32_t n, uint32_t kind, uint32_t init, float b
 // out[d2o[r]] = rank[r] / N (pageRank.c:1083); per-workgroup FP64 partial sums
 __global__ __launch_bounds__(AG_WG) void pr_finalize_kernel(uint32_t n, const float *rank,
                                                              const uint32_t *d2o, float *out_orig,
-                                                             float *scaled_orig, double *part)
+                                                             double *part)
 {
     __shared__ double s_wave[AG_WG / AG_WAVE];
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     double v = 0.0;
-    if (r < n) {
-        float x = rank[r];
-        float y = __fdiv_rn(x, __uint2float_rn(n));
+    for (uint64_t r = blockIdx.x * AG_WG + threadIdx.x; r < n; r += gridDim.x * AG_WG) {
+        const float y = __fdiv_rn(rank[r], __uint2float_rn(n));
         out_orig[d2o[r]] = y;
-        if (scaled_orig)
-            scaled_orig[d2o[r]] = x;
-        v = (double)y;
+        v += (double)y;
     }
     v = block_reduce<double, AG_WG>(v, s_wave);
     if (threadIdx.x == 0)
@@ -1480,33 +1476,85 @@ static uint32_t ag_pr_max_parts(const ag_dgraph *g)
     return 2u * g->dev->num_cus * 32u + AG_NXCD;
 }
 
+void ag_parked_free(ag_dgraph *g)
+{
+    ag_parked &P = g->parked;
+    for (uint32_t i = 0; i < P.n_dev; i++)
+        (void)hipFree(P.dev[i]);
+    if (P.pin)
+        (void)hipHostFree(P.pin);
+    for (uint32_t i = 0; P.has_ev && i < 3u; i++)
+        (void)hipEventDestroy(P.ev[i]);
+    memset(&P, 0, sizeof(P));
+}
+
+// Ends a session: its buffers go back to the graph (nothing of it is on the stream any more), or
+// are freed where the graph keeps enough.
 static void session_free(ag_pr_session *s)
 {
     if (!s)
         return;
     (void)hipSetDevice(s->g->dev->ordinal);
     (void)hipStreamSynchronize(s->g->dev->stream);
-    void *ptrs[] = {s->st, s->part_err, s->part_act, s->part_cmax, s->hist_err, s->hist_act, s->hist_t,
-                    s->rank, s->c[0], s->c[1], s->c16[0], s->c16[1], s->dd_queue[0],
-                    s->dd_queue[1], s->dd_flag, s->fin_part, s->fin_sum, s->user};
-    for (void *p : ptrs)
-        if (p)
-            (void)hipFree(p);
-    if (s->st_host)
-        (void)hipHostFree(s->st_host);
-    if (s->loop_ev)
-        (void)hipEventDestroy(s->loop_ev);
-    if (s->step_ev[0])
-        (void)hipEventDestroy(s->step_ev[0]);
-    if (s->step_ev[1])
-        (void)hipEventDestroy(s->step_ev[1]);
+    ag_parked &P = s->g->parked;
+    size_t kept = 0;
+    for (uint32_t i = 0; i < P.n_dev; i++)
+        kept += P.bytes[i];
+    for (uint32_t i = 0; i < s->n_blk; i++) {
+        if (P.n_dev < AG_PARK_BLOCKS && kept + s->blk_bytes[i] <= AG_PARK_BYTES) {
+            kept += s->blk_bytes[i];
+            P.bytes[P.n_dev] = s->blk_bytes[i];
+            P.dev[P.n_dev++] = s->blk[i];
+        } else {
+            (void)hipFree(s->blk[i]);
+        }
+    }
+    if (s->pin && !P.pin)
+        P.pin = s->pin;
+    else if (s->pin)
+        (void)hipHostFree(s->pin);
+    hipEvent_t ev[3] = {s->step_ev[0], s->step_ev[1], s->loop_ev};
+    if (ev[0] && ev[1] && ev[2] && !P.has_ev) {
+        memcpy(P.ev, ev, sizeof(ev));
+        P.has_ev = 1u;
+    } else {
+        for (hipEvent_t e : ev)
+            if (e)
+                (void)hipEventDestroy(e);
+    }
     free(s);
 }
 
+// A device buffer of the session: the graph's smallest parked one that is large enough and at
+// most twice as large, or a new one.
 static int salloc(ag_pr_session *s, void **p, size_t bytes)
 {
-    AG_HIP(hipMalloc(p, bytes ? bytes : 8));
-    (void)s;
+    ag_parked &P = s->g->parked;
+    bytes = bytes ? bytes : 8;
+    uint32_t best = P.n_dev;
+    for (uint32_t i = 0; i < P.n_dev; i++)
+        if (P.bytes[i] >= bytes && P.bytes[i] / 2u <= bytes + 4096u &&
+            (best == P.n_dev || P.bytes[i] < P.bytes[best]))
+            best = i;
+    if (s->n_blk >= AG_PARK_BLOCKS)
+        return ag_set_error(AG_ERR_OOM, "too many session buffers");
+    if (best < P.n_dev) {
+        *p = P.dev[best];
+        s->blk_bytes[s->n_blk] = P.bytes[best];
+        P.n_dev--;
+        P.dev[best] = P.dev[P.n_dev];
+        P.bytes[best] = P.bytes[P.n_dev];
+    } else {
+        hipError_t e = hipMalloc(p, bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            ag_parked_free(s->g);
+            e = hipMalloc(p, bytes);
+        }
+        AG_HIP(e);
+        s->blk_bytes[s->n_blk] = bytes;
+    }
+    s->blk[s->n_blk++] = *p;
     return AG_OK;
 }
 
@@ -1518,6 +1566,13 @@ static int salloc(ag_pr_session *s, void **p, size_t bytes)
             return ag_st_;          \
         }                           \
     } while (0)
+
+// Workgroups of the finalisation: few enough that one workgroup adds their partials quickly.
+static uint32_t pr_final_grid(uint32_t n)
+{
+    const uint32_t need = (n + AG_WG - 1u) / AG_WG;
+    return need < 1u ? 1u : need < 2048u ? need : 2048u;
+}
 
 static uint32_t ag_quant_grid(const ag_dgraph *g)
 {
@@ -1632,24 +1687,41 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     const uint32_t n = g->n;
     const uint32_t maxit = o.max_iterations ? o.max_iterations : 1;
     const uint32_t nblk = ag_pr_max_parts(g);
-    const uint32_t fblk = (n + AG_WG - 1) / AG_WG ? (n + AG_WG - 1) / AG_WG : 1;
-
-    AG_TRY(salloc(s, (void **)&s->st, 2 * sizeof(PrState)));
+    const uint32_t fblk = pr_final_grid(n);
     {
-        hipError_t e = hipHostMalloc((void **)&s->st_host, sizeof(PrState), hipHostMallocDefault);
+        // everything small in one buffer; the history last, in one run
+        const size_t part = (size_t)nblk * 2u;
+        const size_t sizes[] = {2 * sizeof(PrState), part * sizeof(double), sizeof(double),
+                                (size_t)fblk * sizeof(double), part * sizeof(uint32_t),
+                                kc > 100 ? nblk * sizeof(uint32_t) : 0u};
+        size_t at[7] = {0};
+        for (int k = 0; k < 6; k++)
+            at[k + 1] = (at[k] + sizes[k] + 255u) & ~(size_t)255u;
+        char *ctl = NULL;
+        const size_t clocks = o.record_history ? 2u * (size_t)maxit : 0u;
+        s->hist_bytes = (size_t)maxit * 12u + clocks * 8u;
+        AG_TRY(salloc(s, (void **)&ctl, at[6] + s->hist_bytes));
+        s->st = (PrState *)(ctl + at[0]);
+        s->part_err = (double *)(ctl + at[1]);
+        s->fin_sum = (double *)(ctl + at[2]);
+        s->fin_part = (double *)(ctl + at[3]);
+        s->part_act = (uint32_t *)(ctl + at[4]);
+        s->part_cmax = (uint32_t *)(ctl + at[5]);
+        s->hist_err = (double *)(ctl + at[6]);
+        s->hist_t = (uint64_t *)(s->hist_err + maxit);
+        s->hist_act = (uint32_t *)(s->hist_t + clocks);
+    }
+    if (g->parked.pin) {
+        s->pin = g->parked.pin;
+        g->parked.pin = NULL;
+    } else {
+        hipError_t e = hipHostMalloc(&s->pin, AG_PIN_BYTES, hipHostMallocDefault);
         if (e != hipSuccess) {
             session_free(s);
             return ag_hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
         }
     }
-    AG_TRY(salloc(s, (void **)&s->part_err, (size_t)nblk * 2 * sizeof(double)));
-    AG_TRY(salloc(s, (void **)&s->part_act, (size_t)nblk * 2 * sizeof(uint32_t)));
-    if (kc > 100)
-        AG_TRY(salloc(s, (void **)&s->part_cmax, (size_t)nblk * sizeof(uint32_t)));
-    AG_TRY(salloc(s, (void **)&s->hist_err, (size_t)maxit * sizeof(double)));
-    AG_TRY(salloc(s, (void **)&s->hist_act, (size_t)maxit * sizeof(uint32_t)));
-    if (o.record_history)
-        AG_TRY(salloc(s, (void **)&s->hist_t, (size_t)maxit * 2 * sizeof(uint64_t)));
+    s->st_host = (PrState *)s->pin;
     AG_TRY(salloc(s, (void **)&s->rank, (size_t)n * sizeof(float)));
     AG_TRY(salloc(s, &s->c[0], (size_t)n * celem));
     AG_TRY(salloc(s, &s->c[1], (size_t)n * celem));
@@ -1662,8 +1734,6 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
         AG_TRY(salloc(s, (void **)&s->dd_queue[1], (size_t)n * sizeof(uint32_t)));
         AG_TRY(salloc(s, (void **)&s->dd_flag, (size_t)(n + 3u) / 4u * 4u));
     }
-    AG_TRY(salloc(s, (void **)&s->fin_part, (size_t)fblk * sizeof(double)));
-    AG_TRY(salloc(s, (void **)&s->fin_sum, sizeof(double)));
 
     PrState init_st;
     memset(&init_st, 0, sizeof(init_st));
@@ -1678,12 +1748,7 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     }
     if (o.init == AG_INIT_USER && n) {
         AG_TRY(salloc(s, (void **)&s->user, (size_t)n * sizeof(float)));
-        hipError_t e = hipMemcpyAsync(s->user, o.init_ranks, (size_t)n * sizeof(float),
-                                      hipMemcpyHostToDevice, stream);
-        if (e != hipSuccess) {
-            session_free(s);
-            return ag_hip_fail(e, "init ranks upload", __FILE__, __LINE__);
-        }
+        AG_TRY(ag_copy_in(g->dev, s->user, o.init_ranks, (size_t)n * sizeof(float)));
     }
     if (n) {
         void *c0 = (kc == 1 || kc == 2) ? s->c16[0] : s->c[0];
@@ -1707,11 +1772,16 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
             return ag_hip_fail(e, "pr_init_kernel launch", __FILE__, __LINE__);
         }
     }
-    {
+    if (g->parked.has_ev) {
+        s->step_ev[0] = g->parked.ev[0];
+        s->step_ev[1] = g->parked.ev[1];
+        s->loop_ev = g->parked.ev[2];
+        g->parked.has_ev = 0u;
+    } else {
         hipError_t e = hipEventCreate(&s->step_ev[0]);
         if (e == hipSuccess)
             e = hipEventCreate(&s->step_ev[1]);
-        if (e == hipSuccess && o.record_history)
+        if (e == hipSuccess)
             e = hipEventCreate(&s->loop_ev);
         if (e != hipSuccess) {
             session_free(s);
@@ -1790,7 +1860,7 @@ static PrCtl pr_ctl(const ag_pr_session *s, bool pending)
     C.part_cmax = s->kind_code > 100 ? s->part_cmax : nullptr;
     C.hist_err = s->hist_err;
     C.hist_act = s->hist_act;
-    C.hist_t = s->hist_t;
+    C.hist_t = s->o.record_history ? s->hist_t : nullptr;
     C.it = it;
     C.pending = pending ? 1u : 0u;
     C.stop_rule = s->o.stop_rule;
@@ -1979,14 +2049,19 @@ static void fill_result(const ag_pr_session *s, const PrState *st, ag_pr_result 
     r->refine_iteration = st->refine_iter;
 }
 
+// The state after the last step: where the next iteration reads it, st[0] for worklist runs.
+static const PrState *pr_settled(const ag_pr_session *s)
+{
+    return s->st + (s->dd_queue[0] ? 0u : s->enqueued & 1u);
+}
+
 extern "C" int ag_pr_poll(ag_pr_session *s, ag_pr_result *res)
 {
     if (!s)
         return ag_set_error(AG_ERR_INVALID, "session is null");
     AG_HIP(hipSetDevice(s->g->dev->ordinal));
-    // worklist runs keep their state in st[0], the others where the next iteration reads it
-    AG_HIP(hipMemcpyAsync(s->st_host, s->st + (s->dd_queue[0] ? 0u : s->enqueued & 1u),
-                          sizeof(PrState), hipMemcpyDeviceToHost, s->g->dev->stream));
+    AG_HIP(hipMemcpyAsync(s->st_host, pr_settled(s), sizeof(PrState), hipMemcpyDeviceToHost,
+                          s->g->dev->stream));
     int st = ag_wait_stream(s->g->dev);
     if (st != AG_OK)
         return st;
@@ -2019,6 +2094,12 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
     if (!s || !rows)
         return ag_set_error(AG_ERR_INVALID, "null argument");
     AG_HIP(hipSetDevice(s->g->dev->ordinal));
+    // short histories come with the state, in one transfer to the session's pinned block
+    const size_t all = s->hist_bytes, head = 256u;
+    const bool with_state = all + head <= AG_PIN_BYTES;
+    if (with_state)
+        AG_HIP(hipMemcpyAsync((char *)s->pin + head, s->hist_err, all, hipMemcpyDeviceToHost,
+                              s->g->dev->stream));
     ag_pr_result r;
     int st = ag_pr_poll(s, &r);
     if (st != AG_OK)
@@ -2029,26 +2110,38 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
     *rows = k;
     if (k == 0)
         return AG_OK;
-    if (active)
-        AG_HIP(hipMemcpy(active, s->hist_act, (size_t)k * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (error)
-        AG_HIP(hipMemcpy(error, s->hist_err, (size_t)k * sizeof(double), hipMemcpyDeviceToHost));
-    if (iter_ms)
-        memset(iter_ms, 0, (size_t)k * sizeof(float));
-    if (iter_ms && s->hist_t) {
-        int khz = 0;   // the device clock ticks at a constant rate
-        AG_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, s->g->dev->ordinal));
-        uint64_t *t = (uint64_t *)malloc((size_t)k * 2 * sizeof(uint64_t));
-        if (!t)
+    char *buf = NULL;
+    if (!with_state) {
+        buf = (char *)malloc(all);
+        if (!buf)
             return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        hipError_t e = hipMemcpy(t, s->hist_t, (size_t)k * 2 * sizeof(uint64_t),
-                                 hipMemcpyDeviceToHost);
-        for (uint32_t i = 0; e == hipSuccess && khz > 0 && i < k; i++)
-            iter_ms[i] = (float)((double)(t[2 * i + 1] - t[2 * i]) / (double)khz);
-        free(t);
-        AG_HIP(e);
+        st = ag_copy_out(s->g->dev, buf, s->hist_err, all);
+        if (st != AG_OK) {
+            free(buf);
+            return st;
+        }
     }
-    return AG_OK;
+    const char *h = with_state ? (const char *)s->pin + head : buf;
+    const double *he = (const double *)h;
+    const uint64_t *ht = (const uint64_t *)(h + ((const char *)s->hist_t - (const char *)s->hist_err));
+    const uint32_t *ha = (const uint32_t *)(h + ((const char *)s->hist_act - (const char *)s->hist_err));
+    if (active)
+        memcpy(active, ha, (size_t)k * sizeof(uint32_t));
+    if (error)
+        memcpy(error, he, (size_t)k * sizeof(double));
+    if (iter_ms) {
+        int khz = 0;   // the device clock ticks at a constant rate
+        const hipError_t e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate,
+                                                   s->g->dev->ordinal);
+        if (e != hipSuccess)
+            st = ag_hip_fail(e, "hipDeviceGetAttribute(clock rate)", __FILE__, __LINE__);
+        for (uint32_t i = 0; i < k; i++)
+            iter_ms[i] = s->o.record_history && khz > 0
+                             ? (float)((double)(ht[2 * i + 1] - ht[2 * i]) / (double)khz)
+                             : 0.0f;
+    }
+    free(buf);
+    return st;
 }
 
 extern "C" int ag_pr_read_scaled(ag_pr_session *s, float *scaled_out)
@@ -2065,9 +2158,7 @@ extern "C" int ag_pr_read_scaled(ag_pr_session *s, float *scaled_out)
     scaled_copy_kernel<<<(g->n + AG_WG - 1) / AG_WG, AG_WG, 0, g->dev->stream>>>(
         g->n, s->rank, g->d2o, (float *)g->vec_a);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(scaled_out, g->vec_a, (size_t)g->n * sizeof(float),
-                          hipMemcpyDeviceToHost, g->dev->stream));
-    return ag_wait_stream(g->dev);
+    return ag_copy_out(g->dev, scaled_out, g->vec_a, (size_t)g->n * sizeof(float));
 }
 
 extern "C" int ag_pr_end(ag_pr_session *s, float *ranks_out, ag_pr_result *res)
@@ -2079,37 +2170,41 @@ extern "C" int ag_pr_end(ag_pr_session *s, float *ranks_out, ag_pr_result *res)
     hipError_t e = hipSetDevice(g->dev->ordinal);
     if (e != hipSuccess)
         st = ag_hip_fail(e, "hipSetDevice", __FILE__, __LINE__);
+    // the state, the ranks and their sum, one wait for all
+    double *sum = (double *)((char *)s->pin + sizeof(PrState));
+    *sum = 0.0;
+    if (st == AG_OK) {
+        e = hipMemcpyAsync(s->st_host, pr_settled(s), sizeof(PrState), hipMemcpyDeviceToHost,
+                           g->dev->stream);
+        if (e != hipSuccess)
+            st = ag_hip_fail(e, "state copy", __FILE__, __LINE__);
+    }
+    if (st == AG_OK && g->n)
+        st = ag_ensure_vec(g, (size_t)g->n * sizeof(uint64_t));
+    if (st == AG_OK && g->n) {
+        const uint32_t fblk = pr_final_grid(g->n);
+        pr_finalize_kernel<<<fblk, AG_WG, 0, g->dev->stream>>>(g->n, s->rank, g->d2o,
+                                                               (float *)g->vec_a, s->fin_part);
+        sum_partials_kernel<<<1, AG_WG, 0, g->dev->stream>>>(s->fin_part, fblk, s->fin_sum);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(sum, s->fin_sum, sizeof(double), hipMemcpyDeviceToHost,
+                               g->dev->stream);
+        if (e != hipSuccess)
+            st = ag_hip_fail(e, "finalize", __FILE__, __LINE__);
+        if (st == AG_OK && ranks_out)
+            st = ag_copy_out(g->dev, ranks_out, g->vec_a, (size_t)g->n * sizeof(float));
+    }
+    if (st == AG_OK && (!ranks_out || !g->n))
+        st = ag_wait_stream(g->dev);
     ag_pr_result r;
     if (st == AG_OK)
-        st = ag_pr_poll(s, &r);
-    double sum = 0.0;
-    if (st == AG_OK && g->n) {
-        st = ag_ensure_vec(g, (size_t)g->n * sizeof(uint64_t));
-        const uint32_t fblk = (g->n + AG_WG - 1) / AG_WG;
-        if (st == AG_OK) {
-            pr_finalize_kernel<<<fblk, AG_WG, 0, g->dev->stream>>>(
-                g->n, s->rank, g->d2o, (float *)g->vec_a, NULL, s->fin_part);
-            sum_partials_kernel<<<1, AG_WG, 0, g->dev->stream>>>(s->fin_part, fblk, s->fin_sum);
-            e = hipGetLastError();
-            if (e == hipSuccess && ranks_out)
-                e = hipMemcpyAsync(ranks_out, g->vec_a, (size_t)g->n * sizeof(float),
-                                   hipMemcpyDeviceToHost, g->dev->stream);
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(&s->st_host->last_err, s->fin_sum, sizeof(double),
-                                   hipMemcpyDeviceToHost, g->dev->stream);
-            if (e != hipSuccess)
-                st = ag_hip_fail(e, "finalize", __FILE__, __LINE__);
-            if (st == AG_OK)
-                st = ag_wait_stream(g->dev);
-            if (st == AG_OK)
-                sum = s->st_host->last_err;
-        }
-    }
+        fill_result(s, s->st_host, &r);
     if (st == AG_OK && res) {
         *res = r;
-        res->rank_sum = sum;
+        res->rank_sum = *sum;
         float ms = 0.0f;
-        if (s->loop_ev && s->enqueued > 0) {
+        if (s->o.record_history && s->enqueued > 0) {
             if (hipEventElapsedTime(&ms, s->loop_ev, s->step_ev[1]) != hipSuccess)
                 ms = 0.0f;
         }

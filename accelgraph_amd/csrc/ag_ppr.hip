@@ -493,6 +493,7 @@ struct ag_ppr_ws {
     PprConf *conf;
     PrState *st_host;          // pinned
     PprConf *conf_host;        // pinned
+    uint32_t *o2d;             // [n] host: device row of every vertex
     hipGraph_t graph;
     hipGraphExec_t exec;
     uint32_t exec_maxit;       // iterations in the captured solve (0: none captured)
@@ -518,6 +519,7 @@ void ag_ppr_free_ws(ag_dgraph *g)
         (void)hipHostFree(w->st_host);
     if (w->conf_host)
         (void)hipHostFree(w->conf_host);
+    free(w->o2d);
     free(w);
     g->ppr = NULL;
 }
@@ -531,8 +533,15 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
         w = (ag_ppr_ws *)calloc(1, sizeof(ag_ppr_ws));
         if (!w)
             return ag_set_error(AG_ERR_OOM, "host allocation failed");
+        w->o2d = (uint32_t *)malloc((size_t)g->n * sizeof(uint32_t));
+        if (!w->o2d) {
+            free(w);
+            return ag_set_error(AG_ERR_OOM, "host allocation failed");
+        }
         g->ppr = w;
         w->n = g->n;
+        for (uint32_t r = 0; r < g->n; r++)
+            w->o2d[g->h_d2o[r]] = r;
         // 16-lane groups with up to 16 contribution lines in flight per lane: as many
         // workgroups per CU as fit, up to 8
         w->grid_max = ag_pull_grid(g, PPR_GROUPS * PPR_GL * 16u + PPR_GROUPS * PPR_W * 8u, 8u);
@@ -674,17 +683,9 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
     memset(conf, 0, sizeof(*conf));
     for (uint32_t c = 0; c < PPR_W; c++)
         conf->seed[c] = AG_PPR_UNIFORM;
-    {
-        uint32_t *o2d = (uint32_t *)malloc((size_t)n * sizeof(uint32_t));
-        if (!o2d)
-            return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        for (uint32_t r = 0; r < n; r++)
-            o2d[g->h_d2o[r]] = r;
-        for (uint32_t c = 0; c < k; c++)
-            if (seeds[c] != AG_PPR_UNIFORM)
-                conf->seed[c] = o2d[seeds[c]];
-        free(o2d);
-    }
+    for (uint32_t c = 0; c < k; c++)
+        if (seeds[c] != AG_PPR_UNIFORM)
+            conf->seed[c] = w->o2d[seeds[c]];
     conf->k = k;
     {
         // every scaled rank is at most N (the mass of a column never exceeds N), so a
@@ -787,11 +788,10 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         ppr_out_kernel<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(n, k, w->rank, g->d2o,
                                                                      (float)n, outd);
         e = hipGetLastError();
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(ranks_out, outd, tot * sizeof(float), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess && col_error)
-            e = hipMemcpyAsync(col_error, w->colerr, (size_t)k * sizeof(double), hipMemcpyDeviceToHost, s);
-        st = (e == hipSuccess) ? ag_wait_stream(g->dev) : ag_hip_fail(e, "PPR output", __FILE__, __LINE__);
+        st = (e == hipSuccess) ? ag_copy_out(g->dev, ranks_out, outd, tot * sizeof(float))
+                               : ag_hip_fail(e, "PPR output", __FILE__, __LINE__);
+        if (st == AG_OK && col_error)
+            st = ag_copy_out(g->dev, col_error, w->colerr, (size_t)k * sizeof(double));
     }
     if (e0)
         (void)hipEventDestroy(e0);

@@ -214,41 +214,34 @@ struct Gather {
 
 } // namespace
 
-// Timed launches of one pull policy `reps` times; *avg_ms is the mean launch duration from
-// HIP events on the device stream.
+// Launches of one pull policy `reps` times between the device's two timing events (read by
+// timed_ms once the call has waited).
 template <class P>
-static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps, double *avg_ms)
+static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps)
 {
     hipStream_t stream = g->dev->stream;
     PullGeom G = ag_make_geom(g);
-    hipEvent_t e0 = NULL, e1 = NULL;
-    if (avg_ms) {
-        AG_HIP(hipEventCreate(&e0));
-        AG_HIP(hipEventCreate(&e1));
-        AG_HIP(hipEventRecord(e0, stream));
-    }
+    AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
     const uint32_t grid = ag_tile_grid(g, AG_TILE_NNZ_MAX * (uint32_t)sizeof(typename P::Acc));
     for (uint32_t i = 0; i < reps && g->total_blocks; i++) {
         pull_kernel<P><<<grid, AG_WG, 0, stream>>>(G, pol);
         if (g->n_hubs)
             pull_finish_kernel<P><<<1, AG_FIN_WG, 0, stream>>>(G, pol);
     }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && avg_ms)
-        e = hipEventRecord(e1, stream);
-    int st = (e == hipSuccess) ? ag_wait_stream(g->dev) : ag_hip_fail(e, "pull launch", __FILE__, __LINE__);
-    if (st == AG_OK && avg_ms) {
-        float ms = 0.0f;
-        e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess)
-            st = ag_hip_fail(e, "hipEventElapsedTime", __FILE__, __LINE__);
-        *avg_ms = reps ? (double)ms / reps : 0.0;
-    }
-    if (e0)
-        (void)hipEventDestroy(e0);
-    if (e1)
-        (void)hipEventDestroy(e1);
-    return st;
+    AG_HIP(hipGetLastError());
+    AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
+    return AG_OK;
+}
+
+// Mean duration of the timed launches; the stream has been waited for.
+static int timed_ms(const ag_dgraph *g, uint32_t reps, double *avg_ms)
+{
+    if (!avg_ms)
+        return AG_OK;
+    float ms = 0.0f;
+    AG_HIP(hipEventElapsedTime(&ms, g->dev->time_ev[0], g->dev->time_ev[1]));
+    *avg_ms = reps ? (double)ms / reps : 0.0;
+    return AG_OK;
 }
 
 // The hot pass of a blocked SpMV pull: FP32 only (the fixed-point form gathers everything in
@@ -273,8 +266,7 @@ static bool spmv_hot_launch(const ag_dgraph *g, const BlockGeom &B,
 // regular order (unblocked rows); the hot pass (FP32), pass 1 then the combine pass per
 // repetition.
 template <class P>
-static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps,
-                            double *avg_ms)
+static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps)
 {
     hipStream_t stream = g->dev->stream;
     const PullGeom U = ag_make_unblocked_geom(g);
@@ -283,67 +275,60 @@ static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t rep
     static const uint32_t res1 = ag_resident_per_cu(pull_blocked_kernel<P, P>);
     static const uint32_t res2 = ag_resident_per_cu(pull_combine_kernel<P>);
     const uint32_t g1 = ag_blocked_grid(g, res1, 4u), g2 = ag_blocked_grid(g, res2, 8u);
-    hipEvent_t e0 = NULL, e1 = NULL;
-    if (avg_ms) {
-        AG_HIP(hipEventCreate(&e0));
-        AG_HIP(hipEventCreate(&e1));
-        AG_HIP(hipEventRecord(e0, stream));
-    }
+    AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
     for (uint32_t i = 0; i < reps; i++) {
         if (spmv_hot_launch(g, B, pv, stream))
             ag_block_geom_skip_hot(g, B1);
         pull_blocked_kernel<P, P><<<g1, AG_WG, 0, stream>>>(U, B1, pv, pu);
         pull_combine_kernel<P><<<g2, AG_WG, 0, stream>>>(B, pu);
     }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && avg_ms)
-        e = hipEventRecord(e1, stream);
-    int st = (e == hipSuccess) ? ag_wait_stream(g->dev)
-                               : ag_hip_fail(e, "blocked pull launch", __FILE__, __LINE__);
-    if (st == AG_OK && avg_ms) {
-        float ms = 0.0f;
-        e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess)
-            st = ag_hip_fail(e, "hipEventElapsedTime", __FILE__, __LINE__);
-        *avg_ms = reps ? (double)ms / reps : 0.0;
-    }
-    if (e0)
-        (void)hipEventDestroy(e0);
-    if (e1)
-        (void)hipEventDestroy(e1);
-    return st;
+    AG_HIP(hipGetLastError());
+    AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
+    return AG_OK;
 }
 
 // One FP32 SpMV on device buffers: x (host, original order) -> xo -> permuted into xd (device
 // order) -> y in device order into yd -> permuted back into xo -> y (host). yd may be xo (x
 // in original order is dead once permuted), never xd.
+// `staged`: x and y go through the pinned ring (which its first use allocates).
 static int spmv_f32_device(ag_dgraph *g, const float *x, float *y, float *xo, float *xd,
-                           float *yd, uint32_t reps, double *avg_ms)
+                           float *yd, uint32_t reps, double *avg_ms, bool staged)
 {
     const uint32_t n = g->n;
     hipStream_t stream = g->dev->stream;
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMemcpyAsync(xo, x, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
+    const size_t nb = (size_t)n * sizeof(float);
+    int st = AG_OK;
+    if (staged)
+        st = ag_copy_in(g->dev, xo, x, nb);
+    else
+        AG_HIP(hipMemcpyAsync(xo, x, nb, hipMemcpyHostToDevice, stream));
+    if (st != AG_OK)
+        return st;
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
-    int st;
     if (g->blk.bits && g->w)
         st = run_pull_blocked(g, SpmvF32Pol<true>{xd, g->blk.vw, yd},
-                              SpmvF32Pol<true>{xd, g->w, yd}, reps, avg_ms);
+                              SpmvF32Pol<true>{xd, g->w, yd}, reps);
     else if (g->blk.bits)
         st = run_pull_blocked(g, SpmvF32Pol<false>{xd, NULL, yd}, SpmvF32Pol<false>{xd, NULL, yd},
-                              reps, avg_ms);
+                              reps);
     else if (g->w)
-        st = run_pull(g, SpmvF32Pol<true>{xd, g->w, yd}, reps, avg_ms);
+        st = run_pull(g, SpmvF32Pol<true>{xd, g->w, yd}, reps);
     else
-        st = run_pull(g, SpmvF32Pol<false>{xd, NULL, yd}, reps, avg_ms);
+        st = run_pull(g, SpmvF32Pol<false>{xd, NULL, yd}, reps);
     if (st != AG_OK)
         return st;
     float *yo = (yd == xo) ? xd : xo;   // y in original order
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, yo);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(y, yo, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    return ag_wait_stream(g->dev);
+    if (staged) {
+        st = ag_copy_out(g->dev, y, yo, nb);
+    } else {
+        AG_HIP(hipMemcpyAsync(y, yo, nb, hipMemcpyDeviceToHost, stream));
+        st = ag_wait_stream(g->dev);
+    }
+    return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
 extern "C" int ag_spmv_pull(ag_dgraph *g, const float *x, float *y, uint32_t reps, double *avg_ms)
@@ -364,7 +349,7 @@ extern "C" int ag_spmv_pull(ag_dgraph *g, const float *x, float *y, uint32_t rep
     float *xo = (float *)g->vec_a;                    // x, original order (then y original)
     float *xd = (float *)g->vec_b;                    // x, device order
     float *yd = (float *)((char *)g->vec_b + (size_t)n * sizeof(float));  // y, device order
-    return spmv_f32_device(g, x, y, xo, xd, yd, reps, avg_ms);
+    return spmv_f32_device(g, x, y, xo, xd, yd, reps, avg_ms, true);
 }
 
 extern "C" int ag_spmv_pull_noalloc(ag_dgraph *g, const float *x, float *y)
@@ -388,7 +373,7 @@ extern "C" int ag_spmv_pull_noalloc(ag_dgraph *g, const float *x, float *y)
     // x in device order, then y in original order
     float *a = (float *)g->dev->scratch;
     float *b = a + n;
-    return spmv_f32_device(g, x, y, a, b, a, 1, NULL);
+    return spmv_f32_device(g, x, y, a, b, a, 1, NULL, false);
 }
 
 static uint32_t host_fixed32(float x)
@@ -439,40 +424,42 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
     uint32_t *xd = (uint32_t *)g->vec_b;
     uint64_t *yd = (uint64_t *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMemcpyAsync(xo, xq, (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
+    st = ag_copy_in(g->dev, xo, xq, (size_t)n * sizeof(uint32_t));
+    if (st != AG_OK)
+        return st;
     permute_in_kernel<uint32_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
     const uint32_t wc = host_fixed32(0.0001f);
     if (blocked && g->wq)
         st = run_pull_blocked(g, SpmvFixPol<true>{xd, g->vwq, 0u, yd},
-                              SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps, avg_ms);
+                              SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps);
     else if (blocked)
         st = run_pull_blocked(g, SpmvFixPol<false>{xd, NULL, wc, yd},
-                              SpmvFixPol<false>{xd, NULL, wc, yd}, reps, avg_ms);
+                              SpmvFixPol<false>{xd, NULL, wc, yd}, reps);
     else if (g->wq)
-        st = run_pull(g, SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps, avg_ms);
+        st = run_pull(g, SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps);
     else
-        st = run_pull(g, SpmvFixPol<false>{xd, NULL, wc, yd}, reps, avg_ms);
+        st = run_pull(g, SpmvFixPol<false>{xd, NULL, wc, yd}, reps);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, yo);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(yq, yo, (size_t)n * sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    return ag_wait_stream(g->dev);
+    st = ag_copy_out(g->dev, yq, yo, (size_t)n * sizeof(uint64_t));
+    return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
 // Clears y and runs `reps` accumulating passes: pv reads per-edge data in virtual-row order, pu
 // in regular order.
 template <class P>
-static int run_push(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps, double *avg_ms)
+static int run_push(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps)
 {
     const uint32_t words = (uint32_t)(sizeof(*pu.y) / 4u) * g->n;
     const uint32_t zb = (words + AG_WG - 1) / AG_WG;
     zero_u32_kernel<<<zb < 4096u ? zb : 4096u, AG_WG, 0, g->dev->stream>>>((uint32_t *)pu.y,
                                                                            words);
     AG_HIP(hipGetLastError());
-    return g->blk.bits ? run_pull_blocked(g, pv, pu, reps, avg_ms)
-                       : run_pull(g, pu, reps, avg_ms);
+    return g->blk.bits ? run_pull_blocked(g, pv, pu, reps)
+                       : run_pull(g, pu, reps);
 }
 
 extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t reps, double *avg_ms)
@@ -493,19 +480,21 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     float *xd = (float *)g->vec_b;
     float *yd = (float *)((char *)g->vec_b + (size_t)n * sizeof(float));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMemcpyAsync(xo, x, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
+    st = ag_copy_in(g->dev, xo, x, (size_t)n * sizeof(float));
+    if (st != AG_OK)
+        return st;
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
     st = g->w ? run_push(g, SpmvPushPol<true>{{yd}, {}, {xd, g->blk.vw, NULL}},
-                         SpmvPushPol<true>{{yd}, {}, {xd, g->w, NULL}}, reps, avg_ms)
+                         SpmvPushPol<true>{{yd}, {}, {xd, g->w, NULL}}, reps)
               : run_push(g, SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}},
-                         SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}}, reps, avg_ms);
+                         SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}}, reps);
     if (st != AG_OK)
         return st;
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(y, xo, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    return ag_wait_stream(g->dev);
+    st = ag_copy_out(g->dev, y, xo, (size_t)n * sizeof(float));
+    return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
 extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq, uint32_t reps,
@@ -527,20 +516,22 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     uint64_t *xd = (uint64_t *)g->vec_b;
     uint64_t *yd = (uint64_t *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMemcpyAsync(xo, xq, (size_t)n * sizeof(uint64_t), hipMemcpyHostToDevice, stream));
+    st = ag_copy_in(g->dev, xo, xq, (size_t)n * sizeof(uint64_t));
+    if (st != AG_OK)
+        return st;
     permute_in_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
     const uint64_t wc = DoubleToFixed64((double)0.0001f);   // SPMV.c:1080
     st = g->w ? run_push(g, SpmvPushFixPol<true>{{yd}, {}, xd, g->blk.vw, 0u},
-                         SpmvPushFixPol<true>{{yd}, {}, xd, g->w, 0u}, reps, avg_ms)
+                         SpmvPushFixPol<true>{{yd}, {}, xd, g->w, 0u}, reps)
               : run_push(g, SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc},
-                         SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc}, reps, avg_ms);
+                         SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc}, reps);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(yq, xo, (size_t)n * sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
-    return ag_wait_stream(g->dev);
+    st = ag_copy_out(g->dev, yq, xo, (size_t)n * sizeof(uint64_t));
+    return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
 template <typename VT, typename A>
@@ -556,16 +547,17 @@ static int gather_typed(ag_dgraph *g, const void *values, void *out)
     VT *vd = (VT *)g->vec_b;
     A *ad = (A *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMemcpyAsync(vo, values, (size_t)n * sizeof(VT), hipMemcpyHostToDevice, stream));
+    st = ag_copy_in(g->dev, vo, values, (size_t)n * sizeof(VT));
+    if (st != AG_OK)
+        return st;
     permute_in_kernel<VT><<<blk, AG_WG, 0, stream>>>(n, vo, g->d2o, vd);
     AG_HIP(hipGetLastError());
-    st = run_pull(g, Gather<VT, A>{vd, ad}, 1, NULL);
+    st = run_pull(g, Gather<VT, A>{vd, ad}, 1);
     if (st != AG_OK)
         return st;
     permute_out_kernel<A><<<blk, AG_WG, 0, stream>>>(n, ad, g->d2o, ao);
     AG_HIP(hipGetLastError());
-    AG_HIP(hipMemcpyAsync(out, ao, (size_t)n * sizeof(A), hipMemcpyDeviceToHost, stream));
-    return ag_wait_stream(g->dev);
+    return ag_copy_out(g->dev, out, ao, (size_t)n * sizeof(A));
 }
 
 extern "C" int ag_pull_gather(ag_dgraph *g, uint32_t type, const void *values, void *out)

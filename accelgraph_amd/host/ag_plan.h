@@ -154,6 +154,9 @@ int ag_plan_build(uint32_t n, uint32_t m, const uint32_t *out_degree,
 void ag_plan_free(ag_plan *plan);
 int ag_plan_params_check(const ag_plan_params *p, const char **err);
 
+/* memcpy on all cores (par_copy.c). */
+void ag_par_copy(void *dst, const void *src, size_t bytes);
+
 #ifdef __cplusplus
 }
 #endif

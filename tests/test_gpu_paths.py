@@ -152,3 +152,52 @@ def test_steps_of_any_length(device, plan, run):
         assert r.hist_ms.size == r.executed and np.all(r.hist_ms > 0) and np.all(r.hist_ms < 50)
         assert abs(r.error_total - want.error_total) <= 1e-12 * want.error_total
     dg.close()
+
+
+@pytest.mark.parametrize("n", [1, 1000, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 4 * (1 << 20) + 3,
+                               5 * (1 << 20) + 7])
+def test_staged_transfers(device, n):
+    """Vectors of less than, exactly and more than one 4 MB chunk of the pinned ring, and of more
+    chunks than it has: every value arrives at its place both ways, call after call."""
+    chain = np.arange(n - 1, dtype=np.uint32)
+    g = ag.Graph.from_edges(chain, chain + 1, n=n)
+    dg = device.upload(g)
+    rng = np.random.default_rng(n)
+    for _ in range(2):
+        v = rng.random(n, dtype=np.float32)
+        want = np.concatenate([[np.float32(0)], v[:-1]]).astype(np.float32)
+        np.testing.assert_array_equal(dg.gather(v, ag.GATHER_F32), want)
+        q = rng.integers(0, 1 << 62, n, dtype=np.uint64)
+        np.testing.assert_array_equal(dg.gather(q, ag.GATHER_U64),
+                                      np.concatenate([np.zeros(1, np.uint64), q[:-1]]))
+    dg.close()
+
+
+def test_sessions_reuse_parked_buffers(device):
+    """Sessions of different kinds, lengths and overlapping lifetimes on one graph take the buffers
+    that earlier ones left: the results are those of a fresh graph."""
+    g = ag.Graph.rmat(12)
+    dg = device.upload(g)
+    runs = [dict(kind=ag.KIND_FIXED64), dict(kind=ag.KIND_FIXED8), dict(), dict(max_iterations=300),
+            dict(storage=ag.STORE_F16), dict(kind=ag.KIND_QUANT8),
+            dict(direction=ag.DIR_DATA_DRIVEN), dict(history=False),
+            dict(max_iterations=4000, stop_rule=ag.STOP_L1, l1_tolerance=1e-7)]
+    for kw in runs + runs[::-1]:
+        fresh = device.upload(g)
+        want = fresh.pagerank(**dict(kw))
+        fresh.close()
+        got = dg.pagerank(**dict(kw))
+        np.testing.assert_array_equal(got.ranks.view(np.uint32), want.ranks.view(np.uint32))
+        np.testing.assert_array_equal(got.hist_active, want.hist_active)
+    a = dg.session(max_iterations=30, stop_rule=ag.STOP_NONE)
+    a.step(10)
+    b = dg.session(max_iterations=30, stop_rule=ag.STOP_NONE, kind=ag.KIND_FIXED32)
+    b.step(30)
+    rb, _ = b.end()
+    a.step(20)
+    ra, _ = a.end()
+    np.testing.assert_array_equal(
+        ra, dg.pagerank(max_iterations=30, stop_rule=ag.STOP_NONE).ranks)
+    np.testing.assert_array_equal(
+        rb, dg.pagerank(max_iterations=30, stop_rule=ag.STOP_NONE, kind=ag.KIND_FIXED32).ranks)
+    dg.close()
