@@ -221,6 +221,7 @@ int ag_graph_forward(ag_dgraph *g);
 int ag_set_error(int status, const char *fmt, ...);
 int ag_hip_fail(hipError_t e, const char *what, const char *file, int line);
 int ag_wait_stream(ag_device *dev);
+int ag_wait_event(ag_device *dev, hipEvent_t ev);
 // Host -> device copy on the device's stream, through the pinned ring: `host` may be reused on
 // return. Memory that is pinned already is copied straight (then it may not, before a wait).
 int ag_copy_in(ag_device *dev, void *dst, const void *host, size_t bytes);

@@ -1,16 +1,16 @@
 // ag_ppr.hip -- 64-column personalised PageRank pull.
 //
-// The plain iteration of pageRank.c:942-1109 applied to 64 rank vectors at once, each with
-// its own restart vector. Contributions are stored vertex-major, 64 per vertex, so an in-edge
-// gathers one contiguous 128-byte line (BF16/FP16) or 256-byte line (FP32): a group of 16
-// lanes (four columns per lane, 8-byte or 16-byte loads) reads it with one coalesced load, and
-// a group keeps the lines of 16 in-edges in flight at once, their source ids fetched by one
-// coalesced load and passed lane to lane. Work items reuse the pull plan's bins: THREAD and
-// GROUP16 rows take one group each (sixteen rows per workgroup), WAVE rows a wavefront (four
-// groups), BLOCK rows a whole workgroup, HUB rows fixed segments whose 64-wide partials a
-// one-workgroup finish kernel adds in segment order. The per-column L1 delta is reduced in
-// FP64 in a fixed order; the run stops when every column is below the tolerance. The solve is
-// captured once into a hipGraph and replayed.
+// The plain iteration of pageRank.c:942-1109 applied to up to 64 rank vectors at once, each with
+// its own restart vector. Contributions are stored vertex-major, W = 16, 32 or 64 per vertex, so
+// an in-edge gathers one contiguous run (128 bytes in BF16/FP16 and 256 in FP32 for 64 columns): a
+// group of W / 4 lanes (four columns per lane, 8-byte or 16-byte loads) reads it with one
+// coalesced load, and a group keeps the lines of 16 in-edges in flight at once, their source ids
+// fetched by coalesced loads and passed lane to lane. Work items reuse the pull plan's bins:
+// THREAD and GROUP16 rows take one group each, WAVE rows a wavefront, BLOCK rows a whole
+// workgroup, HUB rows fixed segments whose partials a one-workgroup finish kernel adds in segment
+// order. The per-column L1 delta is reduced in FP64 in a fixed order; the run stops when every
+// column is below the tolerance. A run of iterations is captured once into a hipGraph and
+// replayed until the run stops.
 #include <stdlib.h>
 #include <string.h>
 #include <time.h>
@@ -18,10 +18,9 @@
 #include "ag_internal.h"
 #include "ag_pull_kernel.h"
 
-#define PPR_W 64          // columns per vertex (fixed stride)
-#define PPR_GL 16         // lanes per group: one row's 64 columns, four per lane
-#define PPR_GROUPS (AG_WG / PPR_GL)
-#define PPR_FIN_GROUPS (AG_FIN_WG / PPR_GL)
+#define PPR_W 64          // most columns per vertex
+#define PPR_CH 16         // in-edges of a chunk: their contribution lines are in flight together
+#define PPR_REPLAY 16u    // iterations of the captured graph
 
 namespace {
 
@@ -41,13 +40,13 @@ struct PprConf {
 };
 
 struct PprArgs {
-    const void *c16[2];       // 16-bit contributions [N][64] (bf16 or fp16 bits)
-    const float *c32[2];      // f32 contributions [N][64]
-    float *rank;              // [N][64]
+    const void *c16[2];       // 16-bit contributions [N][W] (bf16 or fp16 bits)
+    const float *c32[2];      // f32 contributions [N][W]
+    float *rank;              // [N][W]
     const uint32_t *outdeg;
     const PprConf *conf;
-    float *hub_part;          // [n_segs][64]
-    double *part;             // [grid][64] per-workgroup column error partials
+    float *hub_part;          // [n_segs][W]
+    double *part;             // [grid][W] per-workgroup column error partials
     double *colerr;           // [64] last column errors
     double *hist;             // [max_iterations] max column error per iteration
     PrState *st;
@@ -113,64 +112,95 @@ __device__ __forceinline__ void add4(float4 &a, const float4 &b)
     a.w += b.w;
 }
 
-// This lane's source id in the first 16-edge chunk of group gi over in-edges [lo, hi)
-// (0 past hi).
-__device__ __forceinline__ uint32_t ppr_first_ids(const PullGeom &G, uint32_t lo, uint32_t hi,
-                                                  uint32_t gi, uint32_t q)
+// The kernels are built for W = 16, 32 and 64 columns per vertex, the least that holds the call's
+// columns: a group of W / 4 lanes (four columns each) owns a row, so a wavefront carries 16, 8 or 4
+// rows and gathers 32-, 64- or 128-byte lines (twice that in FP32). A call of few columns paid for
+// all 64 before: one column on RMAT-18 12.1 -> 4.8 ms a solve, RMAT-20 46 -> 14.5 ms (BF16), 32
+// columns 15.3 -> 7.6 and 60 -> 27 ms.
+template <uint32_t W>
+struct Ppr {
+    static constexpr uint32_t GL = W / 4u;                 // lanes per group
+    static constexpr uint32_t NG = AG_WG / GL;             // groups per workgroup
+    static constexpr uint32_t FG = AG_FIN_WG / GL;         // groups of the finish workgroup
+    static constexpr uint32_t NI = PPR_CH / GL;            // a lane's source ids of a chunk
+    struct Ids {
+        uint32_t v[NI];
+    };
+};
+
+// This lane's source ids of the 16-edge chunk at `base` of in-edges below hi (0 past hi): edge
+// u * GL + q of the chunk is lane q's u-th.
+template <uint32_t W>
+__device__ __forceinline__ typename Ppr<W>::Ids ppr_ids(const PullGeom &G, uint32_t base,
+                                                        uint32_t hi, uint32_t q)
 {
-    const uint32_t j = lo + gi * PPR_GL + q;
-    return j < hi ? __builtin_nontemporal_load(&G.src[j]) : 0u;
+    typename Ppr<W>::Ids s;
+#pragma unroll
+    for (uint32_t u = 0; u < Ppr<W>::NI; u++) {
+        const uint32_t j = base + u * Ppr<W>::GL + q;
+        s.v[u] = base < hi && j < hi ? __builtin_nontemporal_load(&G.src[j]) : 0u;
+    }
+    return s;
 }
 
 // Sum of columns 4q..4q+3 over the in-edges [lo, hi) owned by group gi of the ng groups that
 // share the row: the edges are cut into 16-edge chunks, chunk c belongs to group c % ng. A
-// chunk's source ids arrive in one coalesced load (one per lane; `sl` holds the first chunk's,
-// loaded by the caller) and are passed lane to lane, so every contribution line of the chunk
-// is in flight at once: 16 loads of 8 bytes per lane (16-bit storage) or two rounds of 8 loads
-// of 16 bytes (FP32); the next chunk's ids are loaded before them. Per lane the terms are added
-// in edge order into two accumulators (even and odd edges), combined at the end.
+// chunk's source ids arrive in coalesced loads (`sl` holds the first chunk's, loaded by the
+// caller) and are passed lane to lane, so every contribution line of the chunk is in flight at
+// once: 16 loads of 8 bytes per lane (16-bit storage) or two rounds of 8 loads of 16 bytes
+// (FP32); the next chunk's ids are loaded before them. Per lane the terms are added in edge
+// order into two accumulators (even and odd edges), combined at the end.
+template <uint32_t W>
 __device__ __forceinline__ float4 ppr_group_sum(const PullGeom &G, const PprArgs &A,
                                                 const Mode &m, uint32_t lo, uint32_t hi,
                                                 uint32_t gi, uint32_t ng, uint32_t q,
-                                                uint32_t sl)
+                                                typename Ppr<W>::Ids sl)
 {
+    constexpr uint32_t GL = Ppr<W>::GL;
     float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0;
     const uint2 *c16 = (const uint2 *)A.c16[m.rd];
     const float4 *c32 = (const float4 *)A.c32[m.rd];
-    const uint32_t stride = ng * PPR_GL;
-    for (uint32_t base = lo + gi * PPR_GL; base < hi; base += stride) {
-        const uint32_t cnt = hi - base < PPR_GL ? hi - base : PPR_GL;
-        const uint32_t nb = base + stride;
-        const uint32_t sl_next =
-            (nb < hi && nb + q < hi) ? __builtin_nontemporal_load(&G.src[nb + q]) : 0u;
+    const uint32_t stride = ng * PPR_CH;
+    for (uint32_t base = lo + gi * PPR_CH; base < hi; base += stride) {
+        const uint32_t cnt = hi - base < PPR_CH ? hi - base : PPR_CH;
+        const typename Ppr<W>::Ids next = ppr_ids<W>(G, base + stride, hi, q);
         if (m.r16) {
-            uint2 v[PPR_GL];
+            uint2 v[PPR_CH];
 #pragma unroll
-            for (uint32_t t = 0; t < PPR_GL; t++) {
-                const uint32_t sv = (uint32_t)__shfl((int)sl, (int)t, PPR_GL);
-                v[t] = t < cnt ? c16[(size_t)sv * PPR_GL + q] : make_uint2(0u, 0u);
+            for (uint32_t t = 0; t < PPR_CH; t++) {
+                const uint32_t sv = (uint32_t)__shfl((int)sl.v[t / GL], (int)(t % GL), (int)GL);
+                v[t] = t < cnt ? c16[(size_t)sv * GL + q] : make_uint2(0u, 0u);
             }
+            // one branch a chunk: the format chosen per value took RMAT-18 181 us an iteration
+            // in BF16 (64 columns), against 148
+            const auto add = [&](auto f16) {
 #pragma unroll
-            for (uint32_t t = 0; t < PPR_GL; t++) {
-                const float2 lo2 = unpack16(v[t].x, m.f16), hi2 = unpack16(v[t].y, m.f16);
-                add4((t & 1u) ? a1 : a0, make_float4(lo2.x, lo2.y, hi2.x, hi2.y));
-            }
+                for (uint32_t t = 0; t < PPR_CH; t++) {
+                    const float2 lo2 = unpack16(v[t].x, f16), hi2 = unpack16(v[t].y, f16);
+                    add4((t & 1u) ? a1 : a0, make_float4(lo2.x, lo2.y, hi2.x, hi2.y));
+                }
+            };
+            if (m.f16)
+                add(std::true_type());
+            else
+                add(std::false_type());
         } else {
 #pragma unroll
-            for (uint32_t h = 0; h < PPR_GL; h += PPR_GL / 2) {
-                float4 v[PPR_GL / 2];
+            for (uint32_t h = 0; h < PPR_CH; h += PPR_CH / 2) {
+                float4 v[PPR_CH / 2];
 #pragma unroll
-                for (uint32_t t = 0; t < PPR_GL / 2; t++) {
-                    const uint32_t sv = (uint32_t)__shfl((int)sl, (int)(h + t), PPR_GL);
-                    v[t] = h + t < cnt ? c32[(size_t)sv * PPR_GL + q]
+                for (uint32_t t = 0; t < PPR_CH / 2; t++) {
+                    const uint32_t sv = (uint32_t)__shfl((int)sl.v[(h + t) / GL],
+                                                         (int)((h + t) % GL), (int)GL);
+                    v[t] = h + t < cnt ? c32[(size_t)sv * GL + q]
                                        : make_float4(0.f, 0.f, 0.f, 0.f);
                 }
 #pragma unroll
-                for (uint32_t t = 0; t < PPR_GL / 2; t++)
+                for (uint32_t t = 0; t < PPR_CH / 2; t++)
                     add4((t & 1u) ? a1 : a0, v[t]);
             }
         }
-        sl = sl_next;
+        sl = next;
     }
     add4(a0, a1);
     return a0;
@@ -178,6 +208,7 @@ __device__ __forceinline__ float4 ppr_group_sum(const PullGeom &G, const PprArgs
 
 // Damping update of columns 4q..4q+3 of row v; each column's |delta| / N is accumulated in
 // err (FP64), the next contribution rank / out_degree stored in 16 bits or FP32.
+template <uint32_t W>
 __device__ __forceinline__ void ppr_finish(const PprArgs &A, const Mode &m, uint32_t v,
                                            uint32_t q, float4 sum, const uint32_t *seed,
                                            double *err)
@@ -194,7 +225,7 @@ __device__ __forceinline__ void ppr_finish(const PprArgs &A, const Mode &m, uint
         const float p = seed[c] == AG_PPR_UNIFORM ? A.base : (seed[c] == v ? A.basen : 0.0f);
         nw[c] = __fadd_rn(p, __fmul_rn(A.damp, sums[c]));
     }
-    float4 *rk = (float4 *)(A.rank + (size_t)v * PPR_W) + q;
+    float4 *rk = (float4 *)(A.rank + (size_t)v * W) + q;
     const float4 old = *rk;
     *rk = make_float4(nw[0], nw[1], nw[2], nw[3]);
     const float olds[4] = {old.x, old.y, old.z, old.w};
@@ -213,46 +244,48 @@ __device__ __forceinline__ void ppr_finish(const PprArgs &A, const Mode &m, uint
             for (int c = 0; c < 4; c++)
                 qv[c] = ldexpf(qv[c], -A.conf->f16_bias);
         }
-        ((uint2 *)A.c16[m.wr])[(size_t)v * PPR_GL + q] =
+        ((uint2 *)A.c16[m.wr])[(size_t)v * (W / 4u) + q] =
             make_uint2(pack16(qv[0], qv[1], m.f16), pack16(qv[2], qv[3], m.f16));
     }
     else
-        ((float4 *)A.c32[m.wr])[(size_t)v * PPR_GL + q] = make_float4(qv[0], qv[1], qv[2], qv[3]);
+        ((float4 *)A.c32[m.wr])[(size_t)v * (W / 4u) + q] = make_float4(qv[0], qv[1], qv[2], qv[3]);
 }
 
-// Column errors of one workgroup of NG groups: s_err[group][64] summed over groups in order.
-template <uint32_t NG>
+// Column errors of one workgroup of NG groups: s_err[group][W] summed over groups in order.
+template <uint32_t W, uint32_t NG>
 __device__ __forceinline__ void ppr_column_errors(const double *err, double *s_err, double *out)
 {
-    const uint32_t tid = threadIdx.x, q = tid % PPR_GL, gi = tid / PPR_GL;
+    const uint32_t tid = threadIdx.x, q = tid % (W / 4u), gi = tid / (W / 4u);
 #pragma unroll
     for (int c = 0; c < 4; c++)
-        s_err[gi * PPR_W + 4 * q + c] = err[c];
+        s_err[gi * W + 4 * q + c] = err[c];
     __syncthreads();
-    if (tid < PPR_W) {
+    if (tid < W) {
         double t = 0.0;
         for (uint32_t w = 0; w < NG; w++)
-            t += s_err[w * PPR_W + tid];
+            t += s_err[w * W + tid];
         out[tid] = t;
     }
     __syncthreads();
 }
 
 // One iteration's gather and update. Work items, heaviest first: hub segments and BLOCK rows
-// (16 groups on one row; partials combined in LDS in group order), WAVE rows (the four groups
-// of a wavefront on one row; combined by two lane exchanges), THREAD and GROUP16 rows (one
-// group per row, sixteen rows per workgroup).
-__global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
+// (every group of the workgroup on one row; partials combined in LDS in group order), WAVE rows
+// (the groups of a wavefront on one row; combined by lane exchanges), THREAD and GROUP16 rows
+// (one group per row).
+template <uint32_t W>
+__global__ __launch_bounds__(AG_WG, 4) void ppr_kernel(PullGeom G, PprArgs A)
 {
-    __shared__ float4 s_red[PPR_GROUPS * PPR_GL];
-    __shared__ double s_err[PPR_GROUPS * PPR_W];
-    __shared__ double s_tot[PPR_W];
+    constexpr uint32_t GL = Ppr<W>::GL, NG = Ppr<W>::NG;
+    __shared__ float4 s_red[NG * GL];
+    __shared__ double s_err[NG * W];
+    __shared__ double s_tot[W];
     if (*(volatile const uint32_t *)&A.st->done)
         return;
     const uint32_t iter = *(volatile const uint32_t *)&A.st->iter;
     const Mode m = ppr_mode(A, A.conf->storage, iter);
-    const uint32_t tid = threadIdx.x, q = tid % PPR_GL, gi = tid / PPR_GL;
-    const uint32_t wl = (tid % AG_WAVE) / PPR_GL;   // group inside its wavefront
+    const uint32_t tid = threadIdx.x, q = tid % GL, gi = tid / GL;
+    const uint32_t wl = (tid % AG_WAVE) / GL;   // group inside its wavefront
     uint32_t seed[4];
 #pragma unroll
     for (int c = 0; c < 4; c++)
@@ -261,7 +294,7 @@ __global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
     const uint32_t lite_rows = G.bin_row[AG_BIN_WAVE];    // THREAD + GROUP16 rows
     const uint32_t wave0 = G.bin_row[AG_BIN_WAVE], wave1 = G.bin_row[AG_BIN_WAVE + 1];
     const uint32_t nwave = (wave1 - wave0 + AG_WG / AG_WAVE - 1) / (AG_WG / AG_WAVE);
-    const uint32_t nlite = (lite_rows + PPR_GROUPS - 1) / PPR_GROUPS;
+    const uint32_t nlite = (lite_rows + NG - 1) / NG;
     const uint32_t nblock = G.bin_row[AG_BIN_BLOCK + 1] - G.bin_row[AG_BIN_BLOCK];
     const uint32_t nseg = G.slot_blk0[1] - G.slot_blk0[0];
     const uint32_t heavy = nseg + nblock;
@@ -280,17 +313,17 @@ __global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
                 lo = G.off[row];
                 hi = G.off[row + 1];
             }
-            s_red[gi * PPR_GL + q] = ppr_group_sum(G, A, m, lo, hi, gi, PPR_GROUPS, q,
-                                                   ppr_first_ids(G, lo, hi, gi, q));
+            s_red[gi * GL + q] = ppr_group_sum<W>(G, A, m, lo, hi, gi, NG, q,
+                                                   ppr_ids<W>(G, lo + gi * PPR_CH, hi, q));
             __syncthreads();
             if (gi == 0) {
                 float4 t = s_red[q];
-                for (uint32_t w = 1; w < PPR_GROUPS; w++)
-                    add4(t, s_red[w * PPR_GL + q]);
+                for (uint32_t w = 1; w < NG; w++)
+                    add4(t, s_red[w * GL + q]);
                 if (hub)
-                    ((float4 *)(A.hub_part + (size_t)it * PPR_W))[q] = t;
+                    ((float4 *)(A.hub_part + (size_t)it * W))[q] = t;
                 else
-                    ppr_finish(A, m, row, q, t, seed, err);
+                    ppr_finish<W>(A, m, row, q, t, seed, err);
             }
             __syncthreads();
         } else if (it < heavy + nwave) {
@@ -299,31 +332,32 @@ __global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
             float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
             if (valid) {
                 const uint32_t lo = G.off[row], hi = G.off[row + 1];
-                a = ppr_group_sum(G, A, m, lo, hi, wl, AG_WAVE / PPR_GL, q,
-                                  ppr_first_ids(G, lo, hi, wl, q));
+                a = ppr_group_sum<W>(G, A, m, lo, hi, wl, AG_WAVE / GL, q,
+                                  ppr_ids<W>(G, lo + wl * PPR_CH, hi, q));
             }
             // (g0 + g1) + (g2 + g3), the same value in every group (addition commutes)
 #pragma unroll
-            for (int msk = PPR_GL; msk < AG_WAVE; msk <<= 1) {
+            for (int msk = GL; msk < AG_WAVE; msk <<= 1) {
                 a.x += __shfl_xor(a.x, msk, AG_WAVE);
                 a.y += __shfl_xor(a.y, msk, AG_WAVE);
                 a.z += __shfl_xor(a.z, msk, AG_WAVE);
                 a.w += __shfl_xor(a.w, msk, AG_WAVE);
             }
             if (valid && wl == 0)
-                ppr_finish(A, m, row, q, a, seed, err);
+                ppr_finish<W>(A, m, row, q, a, seed, err);
         }
     }
     // THREAD and GROUP16 rows, a group each, two rows ahead: while row k is gathered, the
     // first source ids of row k + 1 and the offsets of row k + 2 are in flight
     {
-        const uint32_t step = gridDim.x * PPR_GROUPS;
-        uint32_t row = it < total ? (it - lite0) * PPR_GROUPS + gi : lite_rows;
-        uint32_t lo = 0, hi = 0, lo1 = 0, hi1 = 0, sl = 0;
+        const uint32_t step = gridDim.x * NG;
+        uint32_t row = it < total ? (it - lite0) * NG + gi : lite_rows;
+        uint32_t lo = 0, hi = 0, lo1 = 0, hi1 = 0;
+        typename Ppr<W>::Ids sl{};
         if (row < lite_rows) {
             lo = G.off[row];
             hi = G.off[row + 1];
-            sl = ppr_first_ids(G, lo, hi, 0, q);
+            sl = ppr_ids<W>(G, lo, hi, q);
         }
         if (row < lite_rows && row + step < lite_rows) {
             lo1 = G.off[row + step];
@@ -335,9 +369,9 @@ __global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
                 lo2 = G.off[row + 2 * step];
                 hi2 = G.off[row + 2 * step + 1];
             }
-            const uint32_t sl1 = ppr_first_ids(G, lo1, hi1, 0, q);
-            const float4 a = ppr_group_sum(G, A, m, lo, hi, 0, 1, q, sl);
-            ppr_finish(A, m, row, q, a, seed, err);
+            const typename Ppr<W>::Ids sl1 = ppr_ids<W>(G, lo1, hi1, q);
+            const float4 a = ppr_group_sum<W>(G, A, m, lo, hi, 0, 1, q, sl);
+            ppr_finish<W>(A, m, row, q, a, seed, err);
             lo = lo1;
             hi = hi1;
             sl = sl1;
@@ -345,42 +379,45 @@ __global__ __launch_bounds__(AG_WG) void ppr_kernel(PullGeom G, PprArgs A)
             hi1 = hi2;
         }
     }
-    ppr_column_errors<PPR_GROUPS>(err, s_err, s_tot);
-    if (tid < PPR_W)
-        A.part[(size_t)blockIdx.x * PPR_W + tid] = s_tot[tid];
+    ppr_column_errors<W, NG>(err, s_err, s_tot);
+    if (tid < W)
+        A.part[(size_t)blockIdx.x * W + tid] = s_tot[tid];
 }
 
 // Hub rows (their segment partials added in segment order), the column errors of the
 // iteration (fixed order) and the stop / refinement decisions. One workgroup.
+template <uint32_t W>
 __global__ __launch_bounds__(AG_FIN_WG) void ppr_finish_kernel(PullGeom G, PprArgs A)
 {
-    __shared__ double s_err[PPR_FIN_GROUPS * PPR_W];
-    __shared__ double s_tot[PPR_W];
+    constexpr uint32_t GL = Ppr<W>::GL, FG = Ppr<W>::FG;
+    __shared__ double s_err[FG * W];
+    __shared__ double s_tot[W];
     if (*(volatile const uint32_t *)&A.st->done)
         return;
     const PprConf &C = *A.conf;
     const uint32_t iter = *(volatile const uint32_t *)&A.st->iter;
     const Mode m = ppr_mode(A, C.storage, iter);
-    const uint32_t tid = threadIdx.x, q = tid % PPR_GL, gi = tid / PPR_GL;
+    const uint32_t tid = threadIdx.x, q = tid % GL, gi = tid / GL;
     uint32_t seed[4];
 #pragma unroll
     for (int c = 0; c < 4; c++)
         seed[c] = C.seed[4 * q + c];
     double err[4] = {0.0, 0.0, 0.0, 0.0};
-    for (uint32_t hub = gi; hub < G.n_hubs; hub += PPR_FIN_GROUPS) {
+    for (uint32_t hub = gi; hub < G.n_hubs; hub += FG) {
         const uint32_t s0 = G.hub_seg0[hub], s1 = G.hub_seg0[hub + 1];
-        float4 t = ((const float4 *)(A.hub_part + (size_t)s0 * PPR_W))[q];
+        float4 t = ((const float4 *)(A.hub_part + (size_t)s0 * W))[q];
         for (uint32_t sg = s0 + 1; sg < s1; sg++)
-            add4(t, ((const float4 *)(A.hub_part + (size_t)sg * PPR_W))[q]);
-        ppr_finish(A, m, G.bin_row[AG_BIN_HUB] + hub, q, t, seed, err);
+            add4(t, ((const float4 *)(A.hub_part + (size_t)sg * W))[q]);
+        ppr_finish<W>(A, m, G.bin_row[AG_BIN_HUB] + hub, q, t, seed, err);
     }
-    ppr_column_errors<PPR_FIN_GROUPS>(err, s_err, s_tot);
+    ppr_column_errors<W, FG>(err, s_err, s_tot);
     // the iteration kernel's per-workgroup column errors: lane (chunk j, column c) adds the
-    // workgroups of chunk j in order (8 loads in flight), then each column adds its hub term
+    // workgroups of chunk j in order (32 loads in flight; 8
+    // left this launch at 21 us with 2048 workgroups), then each column adds its hub term
     // and the chunks in chunk order -- a fixed order for any grid
     {
-        constexpr uint32_t NCH = AG_FIN_WG / PPR_W, U = 8;
-        const uint32_t c = tid % PPR_W, j = tid / PPR_W;
+        constexpr uint32_t NCH = AG_FIN_WG / W, U = 32;
+        const uint32_t c = tid % W, j = tid / W;
         const uint32_t len = (A.nparts + NCH - 1) / NCH;
         const uint32_t b0 = j * len, b1 = b0 + len < A.nparts ? b0 + len : A.nparts;
         double t = 0.0;
@@ -388,17 +425,17 @@ __global__ __launch_bounds__(AG_FIN_WG) void ppr_finish_kernel(PullGeom G, PprAr
             double v[U];
 #pragma unroll
             for (uint32_t u = 0; u < U; u++)
-                v[u] = b + u < b1 ? A.part[(size_t)(b + u) * PPR_W + c] : 0.0;
+                v[u] = b + u < b1 ? A.part[(size_t)(b + u) * W + c] : 0.0;
 #pragma unroll
             for (uint32_t u = 0; u < U; u++)
                 t += v[u];
         }
-        s_err[j * PPR_W + c] = t;   // s_err is free again (ppr_column_errors ends synced)
+        s_err[j * W + c] = t;   // s_err is free again (ppr_column_errors ends synced)
         __syncthreads();
-        if (tid < PPR_W) {
+        if (tid < W) {
             double tot = s_tot[tid];
             for (uint32_t q2 = 0; q2 < NCH; q2++)
-                tot += s_err[q2 * PPR_W + tid];
+                tot += s_err[q2 * W + tid];
             s_tot[tid] = tot;
         }
         __syncthreads();
@@ -437,6 +474,7 @@ __global__ __launch_bounds__(AG_FIN_WG) void ppr_finish_kernel(PullGeom G, PprAr
 // Start of a solve: every rank 1.0, contributions 1 / out_degree (0 for sinks) in the storage
 // of the first iteration, and the iteration state reset (thread 0; no other thread reads it
 // in this launch).
+template <uint32_t W>
 __global__ void ppr_init_kernel(PprArgs A)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;  // (vertex, lane)
@@ -451,9 +489,9 @@ __global__ void ppr_init_kernel(PprArgs A)
         st->best_err = 0.0;
         st->stall = 0;
     }
-    if (i >= (uint64_t)A.n * PPR_GL)
+    if (i >= (uint64_t)A.n * (W / 4u))
         return;
-    const uint32_t v = (uint32_t)(i / PPR_GL);
+    const uint32_t v = (uint32_t)(i / (W / 4u));
     ((float4 *)A.rank)[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     const uint32_t od = A.outdeg[v];
     const float c = od ? __fdiv_rn(1.0f, __uint2float_rn(od)) : 0.0f;
@@ -468,14 +506,14 @@ __global__ void ppr_init_kernel(PprArgs A)
     }
 }
 
-__global__ void ppr_out_kernel(uint32_t n, uint32_t k, const float *rank, const uint32_t *d2o,
+__global__ void ppr_out_kernel(uint32_t n, uint32_t k, uint32_t W, const float *rank, const uint32_t *d2o,
                                float nf, float *out)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (uint64_t)n * k)
         return;
     const uint32_t v = (uint32_t)(i / k), c = (uint32_t)(i % k);
-    out[(size_t)d2o[v] * k + c] = __fdiv_rn(rank[(size_t)v * PPR_W + c], nf);
+    out[(size_t)d2o[v] * k + c] = __fdiv_rn(rank[(size_t)v * W + c], nf);
 }
 
 } // namespace
@@ -491,13 +529,15 @@ struct ag_ppr_ws {
     double *part, *colerr, *hist;
     PrState *st;
     PprConf *conf;
-    PrState *st_host;          // pinned
+    PrState *st_host;          // pinned [2]
     PprConf *conf_host;        // pinned
     uint32_t *o2d;             // [n] host: device row of every vertex
     hipGraph_t graph;
     hipGraphExec_t exec;
-    uint32_t exec_maxit;       // iterations in the captured solve (0: none captured)
     uint32_t exec_grid;        // its iteration-kernel grid
+    uint32_t exec_width;       // and columns per vertex
+    uint32_t width;            // columns per vertex of this call: 16, 32 or 64
+    hipEvent_t ev[2];          // the state copies after the last two replays
 };
 
 void ag_ppr_free_ws(ag_dgraph *g)
@@ -519,6 +559,9 @@ void ag_ppr_free_ws(ag_dgraph *g)
         (void)hipHostFree(w->st_host);
     if (w->conf_host)
         (void)hipHostFree(w->conf_host);
+    for (hipEvent_t ev : w->ev)
+        if (ev)
+            (void)hipEventDestroy(ev);
     free(w->o2d);
     free(w);
     g->ppr = NULL;
@@ -544,7 +587,7 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
             w->o2d[g->h_d2o[r]] = r;
         // 16-lane groups with up to 16 contribution lines in flight per lane: as many
         // workgroups per CU as fit, up to 8
-        w->grid_max = ag_pull_grid(g, PPR_GROUPS * PPR_GL * 16u + PPR_GROUPS * PPR_W * 8u, 8u);
+        w->grid_max = ag_pull_grid(g, AG_WG * 16u + AG_WG * 4u * 8u, 8u);
         if (w->grid_max == 0)
             w->grid_max = 1;
         w->grid = w->grid_max;
@@ -560,7 +603,9 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
         AG_HIP(hipMalloc((void **)&w->colerr, PPR_W * sizeof(double)));
         AG_HIP(hipMalloc((void **)&w->st, sizeof(PrState)));
         AG_HIP(hipMalloc((void **)&w->conf, sizeof(PprConf)));
-        AG_HIP(hipHostMalloc((void **)&w->st_host, sizeof(PrState), hipHostMallocDefault));
+        AG_HIP(hipHostMalloc((void **)&w->st_host, 2 * sizeof(PrState), hipHostMallocDefault));
+        for (hipEvent_t &ev : w->ev)
+            AG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         AG_HIP(hipHostMalloc((void **)&w->conf_host, sizeof(PprConf), hipHostMallocDefault));
     }
     if (w->hist_cap < maxit) {
@@ -569,7 +614,6 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
             (void)hipGraphDestroy(w->graph);
             w->exec = NULL;
             w->graph = NULL;
-            w->exec_maxit = 0;
         }
         if (w->hist)
             AG_HIP(hipFree(w->hist));
@@ -609,10 +653,15 @@ static PprArgs ppr_args(const ag_dgraph *g, const ag_ppr_ws *w)
     return A;
 }
 
-static hipError_t ppr_enqueue_init(const ag_dgraph *g, const PprArgs &A, hipStream_t s)
+static hipError_t ppr_enqueue_init(const ag_dgraph *g, const ag_ppr_ws *w, const PprArgs &A,
+                                   hipStream_t s)
 {
-    const uint64_t tot = (uint64_t)g->n * PPR_GL;
-    ppr_init_kernel<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(A);
+    const uint32_t blocks = (uint32_t)(((uint64_t)g->n * (w->width / 4u) + 255u) / 256u);
+    switch (w->width) {
+    case 16: ppr_init_kernel<16><<<blocks, 256, 0, s>>>(A); break;
+    case 32: ppr_init_kernel<32><<<blocks, 256, 0, s>>>(A); break;
+    default: ppr_init_kernel<64><<<blocks, 256, 0, s>>>(A); break;
+    }
     return hipGetLastError();
 }
 
@@ -621,8 +670,20 @@ static hipError_t ppr_enqueue_iterations(const ag_dgraph *g, const ag_ppr_ws *w,
 {
     const PullGeom G = ag_make_geom(g);
     for (uint32_t i = 0; i < count; i++) {
-        ppr_kernel<<<w->grid, AG_WG, 0, s>>>(G, A);
-        ppr_finish_kernel<<<1, AG_FIN_WG, 0, s>>>(G, A);
+        switch (w->width) {
+        case 16:
+            ppr_kernel<16><<<w->grid, AG_WG, 0, s>>>(G, A);
+            ppr_finish_kernel<16><<<1, AG_FIN_WG, 0, s>>>(G, A);
+            break;
+        case 32:
+            ppr_kernel<32><<<w->grid, AG_WG, 0, s>>>(G, A);
+            ppr_finish_kernel<32><<<1, AG_FIN_WG, 0, s>>>(G, A);
+            break;
+        default:
+            ppr_kernel<64><<<w->grid, AG_WG, 0, s>>>(G, A);
+            ppr_finish_kernel<64><<<1, AG_FIN_WG, 0, s>>>(G, A);
+            break;
+        }
     }
     return hipGetLastError();
 }
@@ -639,11 +700,12 @@ extern "C" void ag_ppr_options_default(ag_ppr_options *o)
     o->use_hip_graph = 1;
 }
 
-// A solve is: the init launch, then max_iterations x (gather/update, finish); the finish
+// A solve is: the init launch, then up to max_iterations x (gather/update, finish); the finish
 // launch of the stopping iteration sets a device flag that turns every later launch into a
-// no-op. With use_hip_graph the whole solve is captured once per graph and iteration budget
-// and replayed with one hipGraphLaunch and one wait; otherwise it is queued eagerly, `chunk`
-// iterations between polls of the flag.
+// no-op. With use_hip_graph, PPR_REPLAY iterations are captured once per graph, width and grid
+// and replayed until a replay ends stopped (capturing all max_iterations paid for the no-op
+// launches past the stop: 230 of 300 iterations on RMAT-18, 1 of 15 ms); otherwise, and where
+// max_iterations is less, the iterations are queued eagerly, `chunk` between polls of the flag.
 extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
                            const ag_ppr_options *opts, float *ranks_out, double *col_error,
                            ag_ppr_result *res)
@@ -708,6 +770,7 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         }
         w->grid = grid ? grid : 1u;
     }
+    w->width = k <= 16u ? 16u : k <= 32u ? 32u : 64u;
     const PprArgs A = ppr_args(g, w);
     hipEvent_t e0 = NULL, e1 = NULL;
     hipError_t e = hipEventCreate(&e0);
@@ -715,21 +778,18 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         e = hipEventCreate(&e1);
     if (e == hipSuccess)
         e = hipEventRecord(e0, s);
-    if (e == hipSuccess && o.use_hip_graph) {
-        if (w->exec && (w->exec_maxit != maxit || w->exec_grid != w->grid)) {
+    if (e == hipSuccess && o.use_hip_graph && maxit >= PPR_REPLAY) {
+        if (w->exec && (w->exec_grid != w->grid || w->exec_width != w->width)) {
             (void)hipGraphExecDestroy(w->exec);
             (void)hipGraphDestroy(w->graph);
             w->exec = NULL;
             w->graph = NULL;
-            w->exec_maxit = 0;
         }
         if (!w->exec) {
             e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
-                hipError_t qe = ppr_enqueue_init(g, A, s);
-                if (qe == hipSuccess)
-                    qe = ppr_enqueue_iterations(g, w, A, maxit, s);
-                hipError_t ce = hipStreamEndCapture(s, &w->graph);
+                const hipError_t qe = ppr_enqueue_iterations(g, w, A, PPR_REPLAY, s);
+                const hipError_t ce = hipStreamEndCapture(s, &w->graph);
                 e = qe != hipSuccess ? qe : ce;
                 if (qe != hipSuccess && ce == hipSuccess) {
                     (void)hipGraphDestroy(w->graph);
@@ -739,19 +799,43 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
             if (e == hipSuccess)
                 e = hipGraphInstantiate(&w->exec, w->graph, NULL, NULL, 0);
             if (e == hipSuccess) {
-                w->exec_maxit = maxit;
                 w->exec_grid = w->grid;
+                w->exec_width = w->width;
             }
         }
         if (e == hipSuccess)
-            e = hipGraphLaunch(w->exec, s);
-        if (e == hipSuccess)
+            e = ppr_enqueue_init(g, w, A, s);
+        // replays, each followed by a copy of the state; the copy before the last is read while
+        // the last replay runs, so the device never waits for the host
+        bool stopped = false;
+        uint32_t done = 0;
+        for (uint32_t r = 0; e == hipSuccess && st == AG_OK && !stopped && done < maxit; r++) {
+            const uint32_t left = maxit - done;
+            if (left >= PPR_REPLAY)
+                e = hipGraphLaunch(w->exec, s);
+            else
+                e = ppr_enqueue_iterations(g, w, A, left, s);
+            done += left < PPR_REPLAY ? left : PPR_REPLAY;
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(&w->st_host[r & 1u], w->st, sizeof(PrState),
+                                   hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess)
+                e = hipEventRecord(w->ev[r & 1u], s);
+            if (e == hipSuccess && r > 0) {
+                st = ag_wait_event(g->dev, w->ev[(r & 1u) ^ 1u]);
+                stopped = st == AG_OK && w->st_host[(r & 1u) ^ 1u].done;
+            }
+        }
+        if (e == hipSuccess && st == AG_OK)
             e = hipEventRecord(e1, s);
-        if (e == hipSuccess)
+        if (e == hipSuccess && st == AG_OK)
             e = hipMemcpyAsync(w->st_host, w->st, sizeof(PrState), hipMemcpyDeviceToHost, s);
-        st = (e == hipSuccess) ? ag_wait_stream(g->dev) : ag_hip_fail(e, "PPR graph launch", __FILE__, __LINE__);
+        if (e != hipSuccess)
+            st = ag_hip_fail(e, "PPR graph launch", __FILE__, __LINE__);
+        else if (st == AG_OK)
+            st = ag_wait_stream(g->dev);
     } else if (e == hipSuccess) {
-        e = ppr_enqueue_init(g, A, s);
+        e = ppr_enqueue_init(g, w, A, s);
         const uint32_t chunk = o.chunk ? o.chunk : 8;
         uint32_t enq = 0;
         while (e == hipSuccess && st == AG_OK && enq < maxit) {
@@ -785,7 +869,7 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         // normalised ranks, original order; c32[1] is free as staging once the solve ended
         float *outd = w->c32[1];
         const uint64_t tot = (uint64_t)n * k;
-        ppr_out_kernel<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(n, k, w->rank, g->d2o,
+        ppr_out_kernel<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(n, k, w->width, w->rank, g->d2o,
                                                                      (float)n, outd);
         e = hipGetLastError();
         st = (e == hipSuccess) ? ag_copy_out(g->dev, ranks_out, outd, tot * sizeof(float))

@@ -184,7 +184,7 @@ static uint64_t now_ms(void)
 }
 
 // Wait for an event; bounded by the watchdog deadline when one is set.
-static int wait_event(ag_device *d, hipEvent_t ev)
+int ag_wait_event(ag_device *d, hipEvent_t ev)
 {
     if (d->run_timeout_ms == 0) {
         AG_HIP(hipEventSynchronize(ev));
@@ -215,7 +215,7 @@ int ag_wait_stream(ag_device *d)
     hipEvent_t ev;
     AG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     const hipError_t e = hipEventRecord(ev, d->stream);
-    const int st = e == hipSuccess ? wait_event(d, ev)
+    const int st = e == hipSuccess ? ag_wait_event(d, ev)
                                    : ag_hip_fail(e, "hipEventRecord", __FILE__, __LINE__);
     (void)hipEventDestroy(ev);
     return st;
@@ -265,7 +265,7 @@ static int stage_slot(ag_device *d, uint32_t *slot)
 {
     *slot = d->stage_next;
     d->stage_next = (d->stage_next + 1u) % AG_STAGE_SLOTS;
-    return (d->stage_used >> *slot & 1u) ? wait_event(d, d->stage_ev[*slot]) : AG_OK;
+    return (d->stage_used >> *slot & 1u) ? ag_wait_event(d, d->stage_ev[*slot]) : AG_OK;
 }
 
 int ag_copy_in(ag_device *d, void *dst, const void *host, size_t bytes)
@@ -322,7 +322,7 @@ int ag_copy_out(ag_device *d, void *host, const void *src, size_t bytes)
         if (st != AG_OK)
             break;
         const uint32_t k = slot[c % AG_STAGE_SLOTS];
-        st = wait_event(d, d->stage_ev[k]);
+        st = ag_wait_event(d, d->stage_ev[k]);
         if (st != AG_OK)
             break;
         const size_t o = c * AG_STAGE_BYTES;

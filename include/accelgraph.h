@@ -335,8 +335,8 @@ int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *x_q, uint64_t *y_q, uint32_
 /* Up to 64 PageRank columns pulled together: column c restarts at seeds[c] (an original vertex
  * id; AG_PPR_UNIFORM restarts uniformly, which is plain PageRank). Scaled units as the plain
  * path: the restart mass is (1 - Damp) * N, all of it on the seed; every column starts at 1.0.
- * Contributions are stored vertex-major, 64 per vertex (one 128-byte line in BF16/FP16), and
- * accumulated in FP32; with 16-bit storage the last iterations switch to FP32 contributions
+ * Contributions are stored vertex-major, 16, 32 or 64 per vertex (the least that holds k columns;
+ * 64: one 128-byte line in BF16/FP16), and accumulated in FP32; with 16-bit storage the last iterations switch to FP32 contributions
  * (refine_l1, as for ag_pr_options). The L1 delta of each column is reduced in FP64. */
 #define AG_PPR_MAX_COLS 64
 #define AG_PPR_UNIFORM 0xFFFFFFFFu
@@ -348,10 +348,9 @@ typedef struct ag_ppr_options {
     uint32_t storage;          /* AG_STORE_*                                                */
     double refine_l1;
     uint32_t chunk;            /* eager mode: iterations queued between polls (0 = auto)   */
-    uint32_t use_hip_graph;    /* 1 (default): the whole solve is one captured hipGraph,
-                                  replayed with one launch and one wait (captured once per
-                                  graph, max_iterations and grid; the buffers stay with the
-                                  graph)                                                   */
+    uint32_t use_hip_graph;    /* 1 (default): 16 iterations are captured once per graph, column
+                                  width and grid into a hipGraph and replayed until the run
+                                  stops (the buffers stay with the graph)                  */
     uint32_t wg_per_cu;        /* resident workgroups per CU of the iteration kernel (0 =
                                   as many as fit, up to 8)                                  */
 } ag_ppr_options;

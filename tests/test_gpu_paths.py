@@ -201,3 +201,33 @@ def test_sessions_reuse_parked_buffers(device):
     np.testing.assert_array_equal(
         rb, dg.pagerank(max_iterations=30, stop_rule=ag.STOP_NONE, kind=ag.KIND_FIXED32).ranks)
     dg.close()
+
+
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("storage", [ag.STORE_F32, ag.STORE_BF16, ag.STORE_F16])
+def test_ppr_widths(device, k, storage):
+    """The column widths the kernels are built for, at their ends: every column is the one a call
+    of 64 columns gives (up to the order of long rows' sums) and within the FP64 residual bound;
+    one graph serves calls of every width, captured and eager, of any iteration budget."""
+    g = graph_with_degrees(EDGE_DEGREES + [16385], seed=5)
+    dg = device.upload(g)
+    rng = np.random.default_rng(7)
+    seeds = rng.integers(0, g.n, 64).astype(np.uint32)
+    seeds[0] = ag.PPR_UNIFORM
+    kw = dict(max_iterations=200, l1_tolerance=1e-6, storage=storage)
+    wide, _, _ = dg.ppr(seeds, **kw)
+    ranks, err, res = dg.ppr(seeds[:k], **kw)
+    assert ranks.shape == (g.n, k) and res.executed < 200 and np.all(err <= 1e-6)
+    np.testing.assert_allclose(ranks, wide[:, :k], rtol=1e-4, atol=1e-9)
+    bound, _ = oracle.ppr_residual(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, seeds[:k], ranks)
+    assert np.all(bound / 0.15 <= 1e-5)
+    eager, _, re = dg.ppr(seeds[:k], use_hip_graph=0, **kw)
+    np.testing.assert_array_equal(eager.view(np.uint32), ranks.view(np.uint32))
+    assert re.executed == res.executed
+    for budget in (1, 16, 17, 31, 33):      # a replay's length, and not a multiple of it
+        a, _, ra = dg.ppr(seeds[:k], max_iterations=budget, stop_rule=ag.STOP_NONE, storage=storage)
+        b, _, rb = dg.ppr(seeds[:k], max_iterations=budget, stop_rule=ag.STOP_NONE, storage=storage,
+                          use_hip_graph=0)
+        assert ra.executed == rb.executed == budget
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+    dg.close()
