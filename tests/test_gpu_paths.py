@@ -231,3 +231,24 @@ def test_ppr_widths(device, k, storage):
         assert ra.executed == rb.executed == budget
         np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
     dg.close()
+
+
+@pytest.mark.parametrize("part_edges", [64, 4096, 16384])
+@pytest.mark.parametrize("heavy_deg", [8, 32, 5000])
+def test_batch_parts(device, part_edges, heavy_deg):
+    """Parts staged in LDS (up to 4096 in-edges) and larger ones, with rows at the ends of both and
+    graphs of a single row, no edge and many parts: every graph's run is its own single one."""
+    graphs = [graph_with_degrees(EDGE_DEGREES + [9000]), ag.Graph.from_edges([0], [1], n=2),
+              ag.Graph.from_edges([], [], n=5), ag.Graph.rmat(13),
+              graph_with_degrees([4097, 0, 4096, 1], n=5003)]
+    b = ag.Batch(device, graphs)
+    for maxit in (7, 100):
+        ranks, its, err, _ = b.pagerank(max_iterations=maxit, l1_tolerance=1e-6,
+                                        part_edges=part_edges, heavy_deg=heavy_deg)
+        assert np.all(np.isfinite(err)) and (maxit < 100 or np.all(err <= 1e-6))
+        for g, r, i in zip(graphs, ranks, its):
+            want = oracle.pagerank_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, init=1,
+                                        stop_rule=1, l1_tolerance=1e-6, max_iterations=maxit)
+            assert abs(int(i) - want.iterations) <= 1
+            assert np.abs(r - want.ranks).max() <= 1e-5
+    b.close()
