@@ -17,15 +17,16 @@ void ag_par_copy(void *dst, const void *src, size_t bytes)
         memcpy(dst, src, bytes);
         return;
     }
-    int nt = omp_get_max_threads();
-    if (nt > 8)
-        nt = 8;
-    #pragma omp parallel num_threads(nt)
+    /* the whole team enters, so that the regions around this one (the planner's) find their
+     * threads again: a smaller team ends the others, and starting them took 3 ms of an upload */
+    #pragma omp parallel
     {
-        const size_t t = (size_t)omp_get_thread_num(), n = (size_t)omp_get_num_threads();
+        const size_t t = (size_t)omp_get_thread_num(), all = (size_t)omp_get_num_threads();
+        const size_t n = all < 8 ? all : 8;
         const size_t part = ((bytes + n - 1) / n + 4095) & ~(size_t)4095;
-        const size_t lo = t * part < bytes ? t * part : bytes;
+        const size_t lo = t < n && t * part < bytes ? t * part : bytes;
         const size_t hi = lo + part < bytes ? lo + part : bytes;
-        memcpy((char *)dst + lo, (const char *)src + lo, hi - lo);
+        if (hi > lo)
+            memcpy((char *)dst + lo, (const char *)src + lo, hi - lo);
     }
 }
