@@ -926,7 +926,7 @@ __global__ __launch_bounds__(AG_WG) void pr_ddf_cmb_kernel(BlockGeom B, PrCtl C,
 // only serial work: its ids and contributions are loaded a chunk ahead, and the chain itself
 // takes one instruction per in-edge (16-lane rows: a DPP broadcast folded into the add; 64-lane
 // rows: a lane read and an add; a workgroup's rows: LDS values, staged by all its lanes).
-// Bound by those chains and the gathers. RMAT-19 (8 M in-edges): 75 us an iteration, where
+// Bound by those chains and the gathers. RMAT-19 (8 M in-edges): 67 us an iteration, where
 // the worklists took 370 (nearly every vertex stays listed until the end of a run, so marking
 // the out-neighbours, 16 lanes along a hub's 30 K out-edges, cost more than it saved).
 

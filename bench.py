@@ -642,9 +642,9 @@ def main() -> int:
                                 ("pr_f32_hot_kernel (hot source segments gathered from LDS) + "
                                  if info.hot_segments else "") +
                                 "pr_f32_blk_kernel (source-blocked gather) + "
-                                "pr_f32_cmb_kernel (combine + update) + pr_f32_finish"
+                                "pr_f32_cmb_kernel (combine + update)"
                                 if info.src_block_bits else
-                                "one iteration = pr_f32_kernel + pr_f32_finish"),
+                                "one iteration = pr_f32_kernel"),
                      "src_block_bits": info.src_block_bits,
                      "hot_segments": info.hot_segments,
                      "hot_edge_fraction": round(info.hot_edges / max(m, 1), 4),
