@@ -846,8 +846,9 @@ __global__ __launch_bounds__(AG_FIN_WG) void pr_int_hubs(PullGeom G, PrCtl C, Pr
 // neighbour carries the fact in its sign bit (contributions are never negative otherwise), so
 // the gather reads no extra byte. This equals the worklist form exactly: an unlisted vertex's
 // in-neighbours kept their contributions since its previous evaluation, so its sum and |delta|
-// repeat -- 0 if it took the new rank then, below epsilon if it did not -- and it neither
-// moves nor counts towards the error. Sums are ordered as in the FP32 pull.
+// repeat -- 0 if it took the new rank then, below epsilon if it did not. It neither moves nor
+// counts towards the error or the active vertices (with epsilon 0 its |delta| of 0 would). Sums
+// are ordered as in the FP32 pull.
 struct PrDdPol {
     using Acc = DdAcc;
     const float *cin;     // signed contributions of this iteration
@@ -868,9 +869,10 @@ struct PrDdPol {
         const float nw = __fadd_rn(base, __fmul_rn(damp, acc.s));
         float rk = __builtin_nontemporal_load(&rank[r]);
         const double e = (double)fabsf(__fsub_rn(nw, rk));
-        if (all_listed || acc.f > 0.0f)
+        const bool listed = all_listed || acc.f > 0.0f;
+        if (listed)
             red.err += e;
-        const bool upd = e >= eps;
+        const bool upd = listed && e >= eps;
         if (upd) {
             rk = nw;
             __builtin_nontemporal_store(nw, &rank[r]);

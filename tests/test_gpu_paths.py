@@ -48,6 +48,41 @@ def test_data_driven_row_classes(device, init):
     dg.close()
 
 
+def acyclic_graphs():
+    """A chain, and edges from lower to higher vertices with some in-degrees above a tile's lane
+    and wavefront rows."""
+    chain = np.arange(49)
+    yield ag.Graph.from_edges(chain, chain + 1, n=50)
+    rng = np.random.default_rng(17)
+    n = 3000
+    s, d = rng.integers(0, n, (2, 9 * n))
+    keep = s < d
+    big = np.arange(2500)
+    yield ag.Graph.from_edges(np.concatenate([s[keep], big]),
+                              np.concatenate([d[keep], np.full(big.size, n - 3)]), n=n)
+
+
+@pytest.mark.parametrize("plan", [{}, dict(src_block_bits=8)])
+@pytest.mark.parametrize("which", [0, 1])
+def test_data_driven_epsilon_zero(device, which, plan):
+    """Epsilon 0 updates every listed vertex, and only those: on an acyclic graph the lists run
+    empty and the run stops, with the active counts of the oracle and of explicit worklists."""
+    g = list(acyclic_graphs())[which]
+    dg = device.upload(g, params=ag.plan_params(**plan))
+    kw = dict(direction=ag.DIR_DATA_DRIVEN, max_iterations=200, epsilon=0.0, scaled=True)
+    ref = oracle.pagerank_dd_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, g.edges_idx,
+                                  g.out_degree, g.fwd_dest, max_iterations=200, epsilon=0.0)
+    assert ref.executed < 200 and ref.hist_active[-1] == 0
+    start = np.full(g.n, np.float32(1) - np.float32(0.85), np.float32)
+    for run in (dg.pagerank(**kw), dg.pagerank(init_ranks=start, **kw)):
+        assert (run.iterations, run.executed) == (ref.iterations, ref.executed)
+        np.testing.assert_array_equal(run.hist_active, ref.hist_active)
+        # two orders of a sum of d positive terms: 2 d 2^-24 at most, per rank on a path
+        np.testing.assert_allclose(run.scaled, ref.scaled,
+                                   rtol=2 * 2.0 ** -24 * float(g.in_degree.max() + ref.executed))
+    dg.close()
+
+
 @pytest.mark.parametrize("degree", [8193, 12288, 12289, 18000])
 def test_data_driven_long_rows(device, degree):
     """Rows above 8192 in-edges take one fixed tree in both forms of the data-driven pull."""
