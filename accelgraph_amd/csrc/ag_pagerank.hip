@@ -1079,9 +1079,11 @@ __device__ __forceinline__ DdAcc dd_wg_row(const uint32_t *src, const float *c, 
     return DdAcc(s, f ? 1.0f : 0.0f);
 }
 
-// Work items, heaviest first: BLOCK and HUB rows (a workgroup each), WAVE rows (a wavefront
-// each), GROUP16 rows (16 lanes each), THREAD tiles (a lane per row, from LDS).
-__global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF32Args A)
+// Work items, heaviest first: the rows from r_big on (a workgroup each: the first bin whose rows
+// may have more than AG_DD_SEQ_MAX in-edges, BLOCK at the latest), WAVE rows (a wavefront each),
+// GROUP16 rows (16 lanes each), THREAD tiles (a lane per row, from LDS).
+__global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF32Args A,
+                                                       uint32_t r_big)
 {
     __shared__ float s_vals[AG_TILE_NNZ_MAX];
     __shared__ float s_wave[AG_WG / AG_WAVE];
@@ -1092,8 +1094,8 @@ __global__ __launch_bounds__(AG_WG) void pr_dds_kernel(PullGeom G, PrCtl C, PrF3
     Red red{};
     const PrDdPol p = dd_policy(C.it, A);
     const uint32_t tid = threadIdx.x;
-    const uint32_t r_grp = G.bin_row[AG_BIN_GROUP16], r_wav = G.bin_row[AG_BIN_WAVE];
-    const uint32_t r_big = G.bin_row[AG_BIN_BLOCK], r_end = G.bin_row[AG_NBINS];
+    const uint32_t r_grp = G.bin_row[AG_BIN_GROUP16], r_end = G.bin_row[AG_NBINS];
+    const uint32_t r_wav = min(G.bin_row[AG_BIN_WAVE], r_big);
     const uint32_t n_big = r_end - r_big;
     const uint32_t n_wav = n_big + (r_big - r_wav + AG_WG / AG_WAVE - 1u) / (AG_WG / AG_WAVE);
     const uint32_t n_grp = n_wav + (r_wav - r_grp + AG_WG / 16u - 1u) / (AG_WG / 16u);
@@ -1910,7 +1912,10 @@ static int pr_launch_iteration(ag_pr_session *s, bool pending)
     }
     if (s->o.direction == AG_DIR_DATA_DRIVEN && !s->dd_queue[0]) {
         C.nparts = ag_pull_grid(g, AG_TILE_NNZ_MAX * 4u);
-        pr_dds_kernel<<<C.nparts, block, 0, stream>>>(G, C, A);
+        const int big = g->params.group16_max_deg > AG_DD_SEQ_MAX ? AG_BIN_GROUP16
+                        : g->params.wave_max_deg > AG_DD_SEQ_MAX  ? AG_BIN_WAVE
+                                                                  : AG_BIN_BLOCK;
+        pr_dds_kernel<<<C.nparts, block, 0, stream>>>(G, C, A, g->bin_row[big]);
         s->nparts = C.nparts;
         AG_HIP(hipGetLastError());
         return AG_OK;

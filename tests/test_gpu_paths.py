@@ -96,6 +96,28 @@ def test_data_driven_long_rows(device, degree):
     dg.close()
 
 
+@pytest.mark.parametrize("plan", [dict(wave_max_deg=20000, block_max_deg=20000),
+                                  dict(group16_max_deg=20000, wave_max_deg=20000,
+                                       block_max_deg=30000)])
+@pytest.mark.parametrize("degree", [8192, 8193, 18000])
+def test_data_driven_long_rows_of_lower_bins(device, plan, degree):
+    """Where a row is summed in edge order or in the tree depends on its in-degree alone, not on
+    the bin that the plan puts it in: both forms agree, and rows up to 8192 with the oracle."""
+    g = graph_with_degrees([degree, 200, 17, 5000])
+    dg = device.upload(g, params=ag.plan_params(**plan))
+    kw = dict(direction=ag.DIR_DATA_DRIVEN, max_iterations=60, epsilon=1e-5, scaled=True)
+    run = dg.pagerank(init=ag.INIT_UNIFORM, **kw)
+    lists = dg.pagerank(init_ranks=np.ones(g.n, np.float32), **kw)
+    np.testing.assert_array_equal(run.scaled.view(np.uint32), lists.scaled.view(np.uint32))
+    np.testing.assert_array_equal(run.hist_active, lists.hist_active)
+    if degree <= 8192:
+        ref = oracle.pagerank_dd_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, g.edges_idx,
+                                      g.out_degree, g.fwd_dest, init=1, max_iterations=60,
+                                      epsilon=1e-5)
+        np.testing.assert_array_equal(run.scaled.view(np.uint32), ref.scaled.view(np.uint32))
+    dg.close()
+
+
 TILE_PLANS = {"default": {}, "few-workgroups": dict(wg_per_cu=1), "small-tiles": dict(tile_nnz=64),
               # rows above 64 in-edges in the thread bin: still one lane, in stream order
               "long-lanes": dict(thread_max_deg=200, group16_max_deg=300),
