@@ -107,6 +107,7 @@ struct PullGeom {
     uint32_t n_rt;
     uint32_t n_heavy;        // items of slot_blk0 before the row tiles (hub segments, block rows)
     uint32_t lane_max;       // rows of a tile up to this in-degree are summed by one lane
+    uint32_t seq_max;        // and up to this one in stream order
     uint32_t n;
     uint32_t n_hubs;
     uint32_t seq_hubs;       // plan in reference order: a hub row is one segment, added by one

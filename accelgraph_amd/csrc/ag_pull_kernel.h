@@ -381,17 +381,19 @@ struct TopTab {
 
 // ---------------------------------------------------------------- row tiles
 //
-// The regular schedule hands the rows of the bins up to G.rt_row1 to the workgroups as tiles of
-// consecutive rows (at most AG_TILE_NNZ_MAX in-edges, see ag_row_tiles), whatever their bin: a
-// tile's ids and then its values are gathered with up to 16 loads in flight a lane and staged in
-// LDS, rows of at most lane_max in-edges are summed by one lane in stream order, longer ones by a
-// wavefront, and every row is finished by a lane of its own, so the loads and stores of the
-// update are coalesced. The next tile's ids, and this tile's row bounds and update operands, are
+// The regular schedule hands the rows of the lower bins (all whose rows fit a tile) to the
+// workgroups as tiles of consecutive rows (G.rt, at most AG_TILE_NNZ_MAX in-edges, see
+// cut_row_tiles), whatever their bin: a tile's ids and then its values are gathered with up to 16
+// loads in flight a lane and staged in LDS. Rows of at most seq_max in-edges (the thread bin's) are
+// summed by one lane in stream order, rows of at most lane_max by one lane in lane_tree's order,
+// longer ones by a wavefront in strided_sum's, and every row is finished by a lane of its own, so
+// the loads and stores of the update are coalesced. The next tile's ids, and this tile's row bounds and update operands, are
 // in flight while the values arrive: a tile costs one dependent round of loads.
 // A group of lanes per row, four gathers in flight each and a chain of four dependent loads a
-// row (offsets, ids, values, update operands), left the chip waiting. SpMV before -> with row
-// tiles: RMAT-16 9.4 -> 7.0 us, RMAT-18 28 -> 22, RMAT-20 102 -> 78 (0.2 T in-edges/s, the L2
-// request rate that also bounds the blocked pass 1), Erdos-Renyi 300 K rows 29.5 -> 25.
+// row (offsets, ids, values, update operands), left the chip waiting. A SpMV before -> with row
+// tiles: RMAT-16 7.9 -> 7.6 us, RMAT-18 27.8 -> 22.2, RMAT-20 99 -> 82 (0.2 T in-edges/s, the rate
+// of the blocked pass 1), Erdos-Renyi 300 K rows of 16 in-edges 29.2 -> 25.3, of 40 64.5 -> 56.4.
+// lane_tree against a chain of additions takes 0.3 to 0.7 us of these (RMAT-20 1.5).
 
 struct RowTile {
     uint32_t r0, r1, e0, e1;
@@ -440,6 +442,40 @@ __device__ __forceinline__ Acc lane_sum(const Acc *s_vals, uint32_t b, uint32_t 
     for (; q < e; q++)
         acc = acc + s_vals[q];
     return acc;
+}
+
+// A row's values v[0, d), d <= 64, by one lane. FP32: the order of a group of 16 lanes that take
+// the values in turn with four accumulators each and combine in a tree (6 additions a value at
+// most, against d - 1 in a chain: 1.7 to 2.7 times less rms error for 20 to 64 equal terms), every
+// value in flight at once. Integer sums are exact in any order.
+template <typename Acc>
+__device__ __forceinline__ Acc lane_tree(const Acc *v, uint32_t d)
+{
+    if constexpr (!std::is_floating_point_v<Acc>) {
+        return lane_sum(v, 0u, d);
+    } else {
+        static_assert(AG_LANE_MAX <= 64u, "four values a lane of the group");
+        Acc t[16];
+#pragma unroll
+        for (uint32_t l = 0; l < 16u; l++)
+            t[l] = l < d ? v[l] : Acc(0);
+#pragma unroll
+        for (uint32_t l = 0; l < 16u; l++)
+            t[l] = t[l] + (16u + l < d ? v[16u + l] : Acc(0));
+        if (d > 32u) {
+#pragma unroll
+            for (uint32_t l = 0; l < 16u; l++)
+                t[l] = t[l] + ((32u + l < d ? v[32u + l] : Acc(0)) +
+                               (48u + l < d ? v[48u + l] : Acc(0)));
+        }
+#pragma unroll
+        for (uint32_t m = 8u; m >= 1u; m >>= 1)
+#pragma unroll
+            for (uint32_t l = 0; l < 8u; l++)
+                if (l < m)
+                    t[l] = t[l] + t[l + m];
+        return t[0] + Acc(0);   // a sum of -0 terms is +0, as where zeros start it
+    }
 }
 
 // A workgroup's tile, with its ids and per-edge data loaded (or on their way), and the next one.
@@ -540,7 +576,9 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, P &pol, Red &r
                 L.lng[wave * AG_LONG_MAX + nl +
                       __builtin_popcountll(mask & ((1ull << lane) - 1ull))] = r;
             else if (r < cur.r1)
-                pol.finish(r, lane_sum(L.vals, b - cur.e0, e - cur.e0), red, pre);
+                pol.finish(r, e - b > G.seq_max ? lane_tree(L.vals + (b - cur.e0), e - b)
+                                                : lane_sum(L.vals, b - cur.e0, e - cur.e0),
+                           red, pre);
             nl += (uint32_t)__builtin_popcountll(mask);
             r = rn;
             b = bn;
@@ -568,10 +606,18 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, P &pol, Red &r
             for (uint32_t k = wave; k < c3; k += AG_WG / AG_WAVE) {
                 const uint32_t row = row_of(k);
                 const uint32_t lo = G.off[row] - cur.e0, hi = G.off[row + 1] - cur.e0;
-                Acc acc = Acc(0);
-                for (uint32_t q = lo + lane; q < hi; q += AG_WAVE)
-                    acc = acc + L.vals[q];
-                acc = group_reduce<Acc, AG_WAVE>(acc);
+                // four accumulators a lane, as strided_sum
+                Acc a[AG_UNROLL];
+#pragma unroll
+                for (int u = 0; u < AG_UNROLL; u++)
+                    a[u] = Acc(0);
+                for (uint32_t q = lo + lane; q < hi; q += AG_UNROLL * AG_WAVE) {
+#pragma unroll
+                    for (int u = 0; u < AG_UNROLL; u++)
+                        if (q + u * AG_WAVE < hi)
+                            a[u] = a[u] + L.vals[q + u * AG_WAVE];
+                }
+                const Acc acc = group_reduce<Acc, AG_WAVE>((a[0] + a[1]) + (a[2] + a[3]));
                 if (lane == 0)
                     L.lsum[k] = acc;
             }

@@ -392,6 +392,7 @@ PullGeom ag_make_geom(const ag_dgraph *g)
     G.n_rt = g->n_rt;
     G.n_heavy = g->n_heavy;
     G.lane_max = g->params.thread_max_deg > AG_LANE_MAX ? g->params.thread_max_deg : AG_LANE_MAX;
+    G.seq_max = g->params.thread_max_deg;
     G.n = g->n;
     G.n_hubs = g->n_hubs;
     G.seq_hubs = g->params.fp32_order == AG_ORDER_REFERENCE ? 1u : 0u;

@@ -130,8 +130,8 @@ TILE_PLANS = {"default": {}, "few-workgroups": dict(wg_per_cu=1), "small-tiles":
 @pytest.mark.parametrize("n", [20011, 700_001])
 def test_row_tiles(device, pname, n):
     """The regular schedule's row tiles at the ends of the row classes, of a tile's in-edges and
-    rows and with as many rounds as one workgroup per CU needs: fixed point exact, FP32 rows
-    summed by one lane equal to the sequential sum, the others within a reordered sum's bound."""
+    rows and with as many rounds as one workgroup per CU needs: fixed point exact, FP32 rows of
+    the thread bin equal to the sequential sum, the others within a reordered sum's bound."""
     degrees = EDGE_DEGREES + [4095, 6000, 6001, 9000, 16384, 16385]
     degrees = [d for d in degrees if d < n - len(degrees)]
     g = graph_with_degrees(degrees, n)
@@ -146,15 +146,50 @@ def test_row_tiles(device, pname, n):
     x = rng.random(n, dtype=np.float32)
     y, _ = dg.spmv(x)
     ref = oracle.spmv_f32(g.inv_idx, g.in_degree, g.inv_src, None, x)
-    lane = g.in_degree <= max(64, p.get("thread_max_deg", 0))
-    if pname not in ("wide-groups",):
-        np.testing.assert_array_equal(y[lane].view(np.uint32), ref[lane].view(np.uint32))
+    lane = g.in_degree <= p.get("thread_max_deg", 16)
+    np.testing.assert_array_equal(y[lane].view(np.uint32), ref[lane].view(np.uint32))
     d = g.in_degree.astype(np.float64)
     assert np.all(np.abs(y.astype(np.float64) - ref) <= 2 * d * 2.0 ** -24 * np.abs(ref))
     run = dg.pagerank(kind=ag.KIND_FIXED32, max_iterations=6, stop_rule=ag.STOP_NONE)
     want = oracle.pagerank_pull(g.out_degree, g.inv_idx, g.in_degree, g.inv_src, kind=32,
                                 max_iterations=6, stop_rule=2)
     np.testing.assert_array_equal(run.ranks.view(np.uint32), want.ranks.view(np.uint32))
+    dg.close()
+
+
+def lanes_sum(v, width):
+    """v added by `width` lanes in turn, four accumulators each, then a tree over the lanes."""
+    a = np.zeros((4, width), np.float32)
+    for k, i in enumerate(range(0, v.size, width)):
+        part = v[i:i + width]
+        a[k % 4, :part.size] += part
+    t = (a[0] + a[1]) + (a[2] + a[3])
+    while t.size > 1:
+        t = t[:t.size // 2] + t[t.size // 2:]
+    return t[0]
+
+
+@pytest.mark.parametrize("negative", [False, True])
+def test_row_tile_sums(device, negative):
+    """FP32 rows of a tile above the thread bin keep the partial sums that 16 lanes (up to 64
+    in-edges) or a wavefront with four accumulators a lane give them, bit for bit: no longer chain
+    of additions, and so no larger error. All values negative zero sum to zero."""
+    degrees = list(range(17, 130)) + [192, 193, 255, 256, 257, 511, 512, 513, 2047, 2048]
+    g = graph_with_degrees(degrees)
+    dg = device.upload(g, params=ag.plan_params(src_block_bits=ag.SRC_BLOCK_OFF))
+    x = np.random.default_rng(23).random(g.n, dtype=np.float32)
+    if negative:
+        x = -x
+    y, _ = dg.spmv(x)
+    s, _ = dg.spmv_push(x)
+    terms = x * np.float32(0.0001)
+    for r, d in enumerate(degrees):
+        row = g.inv_src[g.inv_idx[r]:g.inv_idx[r] + g.in_degree[r]]
+        want = lanes_sum(terms[row], 16 if d <= 64 else 64)
+        assert y[r].view(np.uint32) == want.view(np.uint32), d
+        assert s[r].view(np.uint32) == want.view(np.uint32), d
+    zeros, _ = dg.spmv(np.full(g.n, -0.0, np.float32))
+    assert not np.any(zeros[:len(degrees)].view(np.uint32))
     dg.close()
 
 
