@@ -345,6 +345,7 @@ static void drop_capture(ag_batch *b)
     b->exec_maxit = 0;
 }
 
+// Leaves the batch without a layout: the next call builds one (part_edges is never 0).
 static void free_layout(ag_batch *b)
 {
     void *p[] = {b->d_parts, b->d_gpart, b->d_heavy, b->d_perr, b->d_pact};
@@ -354,6 +355,12 @@ static void free_layout(ag_batch *b)
     b->d_parts = NULL;
     b->d_gpart = b->d_heavy = b->d_pact = NULL;
     b->d_perr = NULL;
+    b->part_edges = b->heavy_deg = 0u;
+    b->a.parts = NULL;
+    b->a.gpart = b->a.heavy = NULL;
+    b->a.perr = NULL;
+    b->a.pact = NULL;
+    b->a.nparts = 0u;
 }
 
 extern "C" int ag_batch_free(ag_batch *b)

@@ -1,0 +1,61 @@
+"""The host side of the device layer (csrc/) on a HIP runtime of host memory (tests/fake/hip_fake.c,
+preloaded): what an allocation that fails leaves behind, and what the next call then does. Kernels
+do nothing there, so no result is looked at, only statuses, allocations and copies."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+HEAD = """
+import ctypes as C, numpy as np
+import accelgraph_amd as ag
+fake = C.CDLL(None)
+fake.fake_limit.argtypes = [C.c_size_t]
+fake.fake_held.restype = fake.fake_copied.restype = C.c_size_t
+dev = ag.Device(0)
+
+def status(f):
+    try:
+        f()
+    except ag.AGError as e:
+        return e.status
+    return 0
+"""
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake_hip") / "libhip_fake.so"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "fake", "hip_fake.c"), "-o", str(so)], check=True)
+    return so
+
+
+def run(fake_hip, body):
+    preload = ":".join(filter(None, [str(fake_hip), os.environ.get("LD_PRELOAD")]))
+    env = dict(os.environ, LD_PRELOAD=preload, OMP_NUM_THREADS="2", PYTHONPATH=ROOT)
+    res = subprocess.run([sys.executable, "-c", HEAD + textwrap.dedent(body)], env=env, cwd=ROOT,
+                         stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=120)
+    assert res.returncode == 0, res.stderr[-3000:]
+
+
+@pytest.mark.parametrize("fail", range(5))
+def test_batch_layout_rebuilt_after_a_failure(fake_hip, fail):
+    """A new part layout that does not fit leaves none: the next call, with the options of the
+    layout before, builds it again instead of running on freed parts."""
+    run(fake_hip, f"""
+    b = ag.Batch(dev, [ag.Graph.rmat(8, seed=s) for s in (1, 2)])
+    b.pagerank(max_iterations=3)
+    fake.fake_fail_in({fail})
+    assert status(lambda: b.pagerank(max_iterations=3, part_edges=64, heavy_deg=8)) == ag._abi.AG_ERR_OOM
+    fake.fake_fail_in(-1)
+    before = fake.fake_mallocs()
+    b.pagerank(max_iterations=3)
+    assert fake.fake_mallocs() - before == 5
+    b.close()
+    assert fake.fake_live() == 0
+    """)
