@@ -567,8 +567,41 @@ void ag_ppr_free_ws(ag_dgraph *g)
     g->ppr = NULL;
 }
 
-// Allocates the workspace on first use; grows the history (dropping the captured solve) when a
-// call asks for more iterations than it holds.
+static int ppr_allocate(ag_dgraph *g, ag_ppr_ws *w)
+{
+    w->o2d = (uint32_t *)malloc((size_t)g->n * sizeof(uint32_t));
+    if (!w->o2d)
+        return ag_set_error(AG_ERR_OOM, "host allocation failed");
+    w->n = g->n;
+    for (uint32_t r = 0; r < g->n; r++)
+        w->o2d[g->h_d2o[r]] = r;
+    // 16-lane groups with up to 16 contribution lines in flight per lane: as many
+    // workgroups per CU as fit, up to 8
+    w->grid_max = ag_pull_grid(g, AG_WG * 16u + AG_WG * 4u * 8u, 8u);
+    if (w->grid_max == 0)
+        w->grid_max = 1;
+    w->grid = w->grid_max;
+    const size_t nv = (size_t)g->n * PPR_W;
+    AG_HIP(hipMalloc((void **)&w->rank, nv * sizeof(float)));
+    AG_HIP(hipMalloc((void **)&w->c32[0], nv * sizeof(float)));
+    AG_HIP(hipMalloc((void **)&w->c32[1], nv * sizeof(float)));
+    AG_HIP(hipMalloc(&w->c16[0], nv * 2));
+    AG_HIP(hipMalloc(&w->c16[1], nv * 2));
+    AG_HIP(hipMalloc((void **)&w->hub_part,
+                     (size_t)(g->n_segs ? g->n_segs : 1) * PPR_W * sizeof(float)));
+    AG_HIP(hipMalloc((void **)&w->part, (size_t)w->grid_max * PPR_W * sizeof(double)));
+    AG_HIP(hipMalloc((void **)&w->colerr, PPR_W * sizeof(double)));
+    AG_HIP(hipMalloc((void **)&w->st, sizeof(PrState)));
+    AG_HIP(hipMalloc((void **)&w->conf, sizeof(PprConf)));
+    AG_HIP(hipHostMalloc((void **)&w->st_host, 2 * sizeof(PrState), hipHostMallocDefault));
+    for (hipEvent_t &ev : w->ev)
+        AG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    AG_HIP(hipHostMalloc((void **)&w->conf_host, sizeof(PprConf), hipHostMallocDefault));
+    return AG_OK;
+}
+
+// Allocates the workspace on first use (whole, or none); grows the history (dropping the captured
+// solve) when a call asks for more iterations than it holds.
 static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
 {
     ag_ppr_ws *w = g->ppr;
@@ -576,37 +609,12 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
         w = (ag_ppr_ws *)calloc(1, sizeof(ag_ppr_ws));
         if (!w)
             return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        w->o2d = (uint32_t *)malloc((size_t)g->n * sizeof(uint32_t));
-        if (!w->o2d) {
-            free(w);
-            return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        }
         g->ppr = w;
-        w->n = g->n;
-        for (uint32_t r = 0; r < g->n; r++)
-            w->o2d[g->h_d2o[r]] = r;
-        // 16-lane groups with up to 16 contribution lines in flight per lane: as many
-        // workgroups per CU as fit, up to 8
-        w->grid_max = ag_pull_grid(g, AG_WG * 16u + AG_WG * 4u * 8u, 8u);
-        if (w->grid_max == 0)
-            w->grid_max = 1;
-        w->grid = w->grid_max;
-        const size_t nv = (size_t)g->n * PPR_W;
-        AG_HIP(hipMalloc(&w->rank, nv * sizeof(float)));
-        AG_HIP(hipMalloc((void **)&w->c32[0], nv * sizeof(float)));
-        AG_HIP(hipMalloc((void **)&w->c32[1], nv * sizeof(float)));
-        AG_HIP(hipMalloc(&w->c16[0], nv * 2));
-        AG_HIP(hipMalloc(&w->c16[1], nv * 2));
-        AG_HIP(hipMalloc((void **)&w->hub_part,
-                         (size_t)(g->n_segs ? g->n_segs : 1) * PPR_W * sizeof(float)));
-        AG_HIP(hipMalloc((void **)&w->part, (size_t)w->grid_max * PPR_W * sizeof(double)));
-        AG_HIP(hipMalloc((void **)&w->colerr, PPR_W * sizeof(double)));
-        AG_HIP(hipMalloc((void **)&w->st, sizeof(PrState)));
-        AG_HIP(hipMalloc((void **)&w->conf, sizeof(PprConf)));
-        AG_HIP(hipHostMalloc((void **)&w->st_host, 2 * sizeof(PrState), hipHostMallocDefault));
-        for (hipEvent_t &ev : w->ev)
-            AG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        AG_HIP(hipHostMalloc((void **)&w->conf_host, sizeof(PprConf), hipHostMallocDefault));
+        const int st = ppr_allocate(g, w);
+        if (st != AG_OK) {
+            ag_ppr_free_ws(g);
+            return st;
+        }
     }
     if (w->hist_cap < maxit) {
         if (w->exec) {

@@ -59,3 +59,24 @@ def test_batch_layout_rebuilt_after_a_failure(fake_hip, fail):
     b.close()
     assert fake.fake_live() == 0
     """)
+
+
+@pytest.mark.parametrize("kind", ["device", "pinned"])
+def test_ppr_workspace_whole_or_none(fake_hip, kind):
+    """A PPR workspace that does not fit is given back whole, whichever allocation fails, and the
+    next call allocates it."""
+    run(fake_hip, f"""
+    g = ag.Graph.rmat(8)
+    dg = dev.upload(g)
+    seeds = np.arange(3, dtype=np.uint32)
+    fail = fake.fake_fail_in if "{kind}" == "device" else fake.fake_fail_host_in
+    kept = fake.fake_live()
+    for n in range(10 if "{kind}" == "device" else 2):
+        fail(n)
+        assert status(lambda: dg.ppr(seeds, max_iterations=20)) == ag._abi.AG_ERR_OOM
+        assert fake.fake_live() == kept
+    fail(-1)
+    dg.ppr(seeds, max_iterations=20)
+    dg.close()
+    assert fake.fake_live() == 0
+    """)
