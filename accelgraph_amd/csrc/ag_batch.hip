@@ -392,7 +392,7 @@ template <typename T>
 static int balloc(ag_batch *b, T **p, size_t count, const T *src)
 {
     size_t bytes = (count ? count : 1) * sizeof(T);
-    AG_HIP(hipMalloc((void **)p, bytes));
+    AG_HIP(ag_dev_malloc(b->dev, p, bytes));
     b->allocs[b->nalloc++] = *p;
     if (src && count)
         AG_HIP(hipMemcpyAsync(*p, src, count * sizeof(T), hipMemcpyHostToDevice, b->dev->stream));
@@ -473,11 +473,11 @@ static int build_layout(ag_batch *b, uint32_t part_edges, uint32_t heavy_deg)
     free_layout(b);
     int st = AG_OK;
     hipStream_t s = b->dev->stream;
-    hipError_t e = hipMalloc((void **)&b->d_parts, (np ? np : 1) * sizeof(BatchPart));
-    if (e == hipSuccess) e = hipMalloc((void **)&b->d_gpart, (size_t)G * 2 * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b->d_heavy, (nh ? nh : 1) * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&b->d_perr, (np ? np : 1) * 2 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **)&b->d_pact, (np ? np : 1) * 2 * sizeof(uint32_t));
+    hipError_t e = ag_dev_malloc(b->dev, &b->d_parts, (np ? np : 1) * sizeof(BatchPart));
+    if (e == hipSuccess) e = ag_dev_malloc(b->dev, &b->d_gpart, (size_t)G * 2 * sizeof(uint32_t));
+    if (e == hipSuccess) e = ag_dev_malloc(b->dev, &b->d_heavy, (nh ? nh : 1) * sizeof(uint32_t));
+    if (e == hipSuccess) e = ag_dev_malloc(b->dev, &b->d_perr, (np ? np : 1) * 2 * sizeof(double));
+    if (e == hipSuccess) e = ag_dev_malloc(b->dev, &b->d_pact, (np ? np : 1) * 2 * sizeof(uint32_t));
     if (e == hipSuccess && np)
         e = hipMemcpyAsync(b->d_parts, parts, np * sizeof(BatchPart), hipMemcpyHostToDevice, s);
     if (e == hipSuccess)

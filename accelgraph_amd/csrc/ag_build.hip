@@ -285,13 +285,14 @@ struct Pool {
     void *p[24];
     int k;
     int status;
+    ag_device *dev;
     template <typename T>
     T *get(size_t count)
     {
         if (status != AG_OK)
             return NULL;
         void *q = NULL;
-        hipError_t e = hipMalloc(&q, (count ? count : 1) * sizeof(T));
+        hipError_t e = ag_dev_malloc(dev, &q, (count ? count : 1) * sizeof(T));
         if (e != hipSuccess) {
             status = ag_hip_fail(e, "graph build allocation", __FILE__, __LINE__);
             return NULL;
@@ -312,7 +313,7 @@ int device_max(ag_device *dev, uint64_t m, const T *a, const T *b, T *out)
 {
     const uint32_t nb = 1024;
     T *part = NULL;
-    AG_HIP(hipMalloc((void **)&part, nb * sizeof(T)));
+    AG_HIP(ag_dev_malloc(dev, &part, nb * sizeof(T)));
     T host[1024];
     max_kernel<T><<<nb, BUILD_WG, 0, dev->stream>>>(m, a, b, part);
     hipError_t e = hipGetLastError();
@@ -337,7 +338,7 @@ int sort_pairs(ag_device *dev, uint64_t m, uint64_t *key, uint64_t *key2, uint32
     AG_HIP(rocprim::radix_sort_pairs(nullptr, tmp, key, key2, val, val2, (size_t)m, 0u, end_bit,
                                      dev->stream));
     void *t = NULL;
-    AG_HIP(hipMalloc(&t, tmp ? tmp : 8));
+    AG_HIP(ag_dev_malloc(dev, &t, tmp ? tmp : 8));
     hipError_t e = rocprim::radix_sort_pairs(t, tmp, key, key2, val, val2, (size_t)m, 0u, end_bit,
                                              dev->stream);
     int st = (e == hipSuccess) ? ag_wait_stream(dev) : ag_hip_fail(e, "radix sort", __FILE__, __LINE__);
@@ -351,7 +352,7 @@ int exclusive_scan_u32(ag_device *dev, uint64_t m, const uint32_t *in, uint32_t 
     AG_HIP(rocprim::exclusive_scan(nullptr, tmp, in, out, 0u, (size_t)m, rocprim::plus<uint32_t>(),
                                    dev->stream));
     void *t = NULL;
-    AG_HIP(hipMalloc(&t, tmp ? tmp : 8));
+    AG_HIP(ag_dev_malloc(dev, &t, tmp ? tmp : 8));
     hipError_t e = rocprim::exclusive_scan(t, tmp, in, out, 0u, (size_t)m,
                                            rocprim::plus<uint32_t>(), dev->stream);
     int st = (e == hipSuccess) ? ag_wait_stream(dev) : ag_hip_fail(e, "scan", __FILE__, __LINE__);
@@ -374,6 +375,7 @@ int build_on_device(ag_device *dev, uint32_t n, uint64_t m, const uint32_t *src,
     const uint32_t end_bit = 2u * shift;
     Pool P;
     P.k = 0;
+    P.dev = dev;
     P.status = AG_OK;
     uint32_t mm = 0;
     uint32_t *fs = NULL, *fd = NULL;
@@ -384,6 +386,7 @@ int build_on_device(ag_device *dev, uint32_t n, uint64_t m, const uint32_t *src,
         // sort temporaries (T) are released before the inverse pass
         Pool T;
         T.k = 0;
+        T.dev = dev;
         T.status = AG_OK;
         uint64_t *key = T.get<uint64_t>(m), *key2 = T.get<uint64_t>(m);
         uint32_t *val = T.get<uint32_t>(m), *val2 = T.get<uint32_t>(m);
@@ -590,11 +593,12 @@ int ag_graph_forward(ag_dgraph *g)
     const uint32_t n = g->n, m = g->m;
     uint32_t *off = NULL, *fdst = NULL;
     Pool T{};
+    T.dev = dev;
     T.status = AG_OK;
     int st = AG_OK;
-    hipError_t e = hipMalloc((void **)&off, ((size_t)n + 1) * sizeof(uint32_t));
+    hipError_t e = ag_dev_malloc(dev, &off, ((size_t)n + 1) * sizeof(uint32_t));
     if (e == hipSuccess)
-        e = hipMalloc((void **)&fdst, (size_t)(m ? m : 1) * sizeof(uint32_t));
+        e = ag_dev_malloc(dev, &fdst, (size_t)(m ? m : 1) * sizeof(uint32_t));
     if (e != hipSuccess)
         st = ag_hip_fail(e, "forward CSR allocation", __FILE__, __LINE__);
     uint32_t *row = T.get<uint32_t>(m);
@@ -615,7 +619,7 @@ int ag_graph_forward(ag_dgraph *g)
                                           bits_for(n), dev->stream);
         void *t = NULL;
         if (e == hipSuccess)
-            e = hipMalloc(&t, tmp ? tmp : 8);
+            e = ag_dev_malloc(dev, &t, tmp ? tmp : 8);
         if (e == hipSuccess)
             e = rocprim::radix_sort_pairs(t, tmp, g->src, fsrc, idx, sidx, (size_t)m, 0u,
                                           bits_for(n), dev->stream);
@@ -668,7 +672,7 @@ extern "C" int ag_generate_rmat_edges(ag_device *dev, uint32_t scale, uint64_t m
         return st;
     AG_HIP(hipSetDevice(dev->ordinal));
     uint32_t *d = NULL;
-    AG_HIP(hipMalloc((void **)&d, m * 2 * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(dev, &d, m * 2 * sizeof(uint32_t)));
     st = generate_device(dev, m, seed, scale, f, d, d + m);
     hipError_t e = hipSuccess;
     if (st == AG_OK)
@@ -690,7 +694,7 @@ extern "C" int ag_generate_er_edges(ag_device *dev, uint32_t n, uint64_t m, uint
         return AG_OK;
     AG_HIP(hipSetDevice(dev->ordinal));
     uint32_t *d = NULL;
-    AG_HIP(hipMalloc((void **)&d, m * 2 * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(dev, &d, m * 2 * sizeof(uint32_t)));
     int st = generate_device(dev, m, seed, 2u, ErEdge{n}, d, d + m);
     hipError_t e = hipSuccess;
     if (st == AG_OK)
@@ -713,7 +717,7 @@ extern "C" int ag_graph_csr_build(ag_device *dev, uint32_t n, uint64_t m, const 
     AG_HIP(hipSetDevice(dev->ordinal));
     uint32_t *d = NULL;
     float *dw = NULL;
-    AG_HIP(hipMalloc((void **)&d, (m ? m : 1) * 2 * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(dev, &d, (m ? m : 1) * 2 * sizeof(uint32_t)));
     int st = AG_OK;
     hipError_t e = hipSuccess;
     if (m) {
@@ -721,7 +725,7 @@ extern "C" int ag_graph_csr_build(ag_device *dev, uint32_t n, uint64_t m, const 
         if (e == hipSuccess)
             e = hipMemcpyAsync(d + m, dst, m * 4, hipMemcpyHostToDevice, dev->stream);
         if (e == hipSuccess && weight) {
-            e = hipMalloc((void **)&dw, m * sizeof(float));
+            e = ag_dev_malloc(dev, &dw, m * sizeof(float));
             if (e == hipSuccess)
                 e = hipMemcpyAsync(dw, weight, m * 4, hipMemcpyHostToDevice, dev->stream);
         }
@@ -760,7 +764,7 @@ extern "C" int ag_graph_csr_generate_rmat(ag_device *dev, uint32_t scale, uint32
         return ag_set_error(AG_ERR_INVALID, "more than 2^32 - 1 edges");
     AG_HIP(hipSetDevice(dev->ordinal));
     uint32_t *d = NULL;
-    AG_HIP(hipMalloc((void **)&d, (m ? m : 1) * 2 * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(dev, &d, (m ? m : 1) * 2 * sizeof(uint32_t)));
     st = generate_device(dev, m, seed, scale, f, d, d + m);
     if (st == AG_OK)
         st = build_on_device(dev, 1u << scale, m, d, d + m, NULL, simplify, out);
@@ -776,7 +780,7 @@ extern "C" int ag_graph_csr_generate_er(ag_device *dev, uint32_t n, uint64_t m, 
     *out = NULL;
     AG_HIP(hipSetDevice(dev->ordinal));
     uint32_t *d = NULL;
-    AG_HIP(hipMalloc((void **)&d, (m ? m : 1) * 2 * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(dev, &d, (m ? m : 1) * 2 * sizeof(uint32_t)));
     int st = generate_device(dev, m, seed, 2u, ErEdge{n}, d, d + m);
     if (st == AG_OK)
         st = build_on_device(dev, n, m, d, d + m, NULL, simplify, out);

@@ -18,7 +18,8 @@ struct ag_device {
     hipStream_t stream;
     uint64_t run_timeout_ms;
     uint32_t poll_us;
-    uint32_t live_graphs;   // graphs uploaded on this device and not yet freed
+    uint32_t live_graphs;   // graphs and batches on this device, not yet freed
+    struct ag_dgraph *graphs;   // list of the uploaded graphs (ag_dgraph::next)
     uint32_t num_cus;       // compute units (persistent-grid sizing)
     void *scratch;          // this device's copy of the ag_spmv_pull_noalloc scratch array
     // pinned ring of the staged transfers (ag_copy_in / ag_copy_out), allocated on first use
@@ -31,7 +32,8 @@ struct ag_device {
 
 // Buffers that ended sessions of a graph hand back for the next one to take (every PageRank call
 // begins and ends a session): at most AG_PARK_BYTES of device memory, one pinned block and one
-// set of events. Freed with the graph, or when an allocation fails.
+// set of events. Freed with the graph, or by ag_dev_malloc when memory runs out; counted in the
+// graph's device bytes meanwhile.
 #define AG_PARK_BLOCKS 8u
 #define AG_PARK_BYTES ((size_t)1 << 30)
 #define AG_PIN_BYTES ((size_t)64 << 10)
@@ -47,6 +49,7 @@ struct ag_parked {
 // Device-resident graph: the plan arrays in HBM plus launch geometry.
 struct ag_dgraph {
     ag_device *dev;
+    ag_dgraph *next;     // of the device's list
     ag_plan_params params;
     uint32_t n, m;
     uint32_t bin_row[AG_NBINS + 1];
@@ -230,6 +233,14 @@ int ag_copy_in(ag_device *dev, void *dst, const void *host, size_t bytes);
 int ag_copy_out(ag_device *dev, void *host, const void *src, size_t bytes);
 // Frees the parked buffers of a graph.
 void ag_parked_free(ag_dgraph *g);
+// hipMalloc for every allocation of the library: when device memory runs out, the parked buffers of
+// all the device's graphs are freed and it tries once more. Returns a hipError_t.
+hipError_t ag_dev_malloc_bytes(ag_device *dev, void **p, size_t bytes);
+template <typename T>
+static inline hipError_t ag_dev_malloc(ag_device *dev, T **p, size_t bytes)
+{
+    return ag_dev_malloc_bytes(dev, (void **)p, bytes);
+}
 
 #define AG_HIP(call)                                                   \
     do {                                                               \

@@ -490,9 +490,9 @@ static int mlp_grow(ag_mlp *m, uint32_t S)
     m->y = NULL;
     m->perm = NULL;
     m->cap = 0;
-    AG_HIP(hipMalloc((void **)&m->X, (size_t)S * MLP_FSTRIDE * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&m->y, (size_t)S * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&m->perm, (size_t)S * sizeof(uint32_t)));
+    AG_HIP(ag_dev_malloc(m->dev, &m->X, (size_t)S * MLP_FSTRIDE * sizeof(float)));
+    AG_HIP(ag_dev_malloc(m->dev, &m->y, (size_t)S * sizeof(float)));
+    AG_HIP(ag_dev_malloc(m->dev, &m->perm, (size_t)S * sizeof(uint32_t)));
     m->cap = S;
     return AG_OK;
 }
@@ -514,8 +514,8 @@ static int mlp_part(ag_mlp *m, uint32_t grid)
     m->part = NULL;
     m->loss_part = NULL;
     m->part_cap = 0;
-    AG_HIP(hipMalloc((void **)&m->part, need * P_COUNT * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&m->loss_part, need * sizeof(double)));
+    AG_HIP(ag_dev_malloc(m->dev, &m->part, need * P_COUNT * sizeof(float)));
+    AG_HIP(ag_dev_malloc(m->dev, &m->loss_part, need * sizeof(double)));
     m->part_cap = need;
     return AG_OK;
 }
@@ -529,7 +529,7 @@ static int mlp_upload(ag_mlp *m, const float *X, const float *y, uint32_t S)
     hipStream_t s = m->dev->stream;
     // stage X[S][5] in the perm+y area is too small; use a temporary
     float *tmp = NULL;
-    AG_HIP(hipMalloc((void **)&tmp, (size_t)S * MLP_NF * sizeof(float)));
+    AG_HIP(ag_dev_malloc(m->dev, &tmp, (size_t)S * MLP_NF * sizeof(float)));
     hipError_t e = hipMemcpyAsync(tmp, X, (size_t)S * MLP_NF * sizeof(float), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         pack_features_kernel<<<(S + 255) / 256, 256, 0, s>>>(S, tmp, m->X);
@@ -576,10 +576,10 @@ extern "C" int ag_mlp_create(ag_device *dev, uint32_t seed, ag_mlp **out)
         h[P_W2 + k] = (float)(rnd() * sqrt(6.0 / MLP_H));
     for (int k = 0; k < MLP_H; k++)
         h[P_W3 + k] = (float)(rnd() * sqrt(3.0 / MLP_H));
-    hipError_t e = hipMalloc((void **)&m->p, P_COUNT * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&m->m1, P_COUNT * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&m->m2, P_COUNT * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&m->grad, P_COUNT * sizeof(float));
+    hipError_t e = ag_dev_malloc(m->dev, &m->p, P_COUNT * sizeof(float));
+    if (e == hipSuccess) e = ag_dev_malloc(m->dev, &m->m1, P_COUNT * sizeof(float));
+    if (e == hipSuccess) e = ag_dev_malloc(m->dev, &m->m2, P_COUNT * sizeof(float));
+    if (e == hipSuccess) e = ag_dev_malloc(m->dev, &m->grad, P_COUNT * sizeof(float));
     if (e == hipSuccess) e = hipMemcpy(m->p, h, P_COUNT * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(m->m1, 0, P_COUNT * sizeof(float));
     if (e == hipSuccess) e = hipMemset(m->m2, 0, P_COUNT * sizeof(float));
@@ -817,10 +817,10 @@ static int warm_scratch(ag_dgraph *g, float **feat, float **r1, float **r2, floa
 {
     const size_t n = g->n ? g->n : 1;
     const size_t nblk = (n + AG_WG - 1) / AG_WG;
-    AG_HIP(hipMalloc((void **)feat, n * MLP_FSTRIDE * sizeof(float)));
-    AG_HIP(hipMalloc((void **)r1, n * sizeof(float)));
-    AG_HIP(hipMalloc((void **)r2, n * sizeof(float)));
-    AG_HIP(hipMalloc((void **)pred, n * sizeof(float) + (2 * nblk + 2) * sizeof(double) + 16));
+    AG_HIP(ag_dev_malloc(g->dev, feat, n * MLP_FSTRIDE * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, r1, n * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, r2, n * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, pred, n * sizeof(float) + (2 * nblk + 2) * sizeof(double) + 16));
     return AG_OK;
 }
 

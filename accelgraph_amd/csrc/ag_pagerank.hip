@@ -1549,13 +1549,7 @@ static int salloc(ag_pr_session *s, void **p, size_t bytes)
         P.dev[best] = P.dev[P.n_dev];
         P.bytes[best] = P.bytes[P.n_dev];
     } else {
-        hipError_t e = hipMalloc(p, bytes);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            ag_parked_free(s->g);
-            e = hipMalloc(p, bytes);
-        }
-        AG_HIP(e);
+        AG_HIP(ag_dev_malloc(s->g->dev, p, bytes));
         s->blk_bytes[s->n_blk] = bytes;
     }
     s->blk[s->n_blk++] = *p;

@@ -582,17 +582,17 @@ static int ppr_allocate(ag_dgraph *g, ag_ppr_ws *w)
         w->grid_max = 1;
     w->grid = w->grid_max;
     const size_t nv = (size_t)g->n * PPR_W;
-    AG_HIP(hipMalloc((void **)&w->rank, nv * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&w->c32[0], nv * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&w->c32[1], nv * sizeof(float)));
-    AG_HIP(hipMalloc(&w->c16[0], nv * 2));
-    AG_HIP(hipMalloc(&w->c16[1], nv * 2));
-    AG_HIP(hipMalloc((void **)&w->hub_part,
+    AG_HIP(ag_dev_malloc(g->dev, &w->rank, nv * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->c32[0], nv * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->c32[1], nv * sizeof(float)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->c16[0], nv * 2));
+    AG_HIP(ag_dev_malloc(g->dev, &w->c16[1], nv * 2));
+    AG_HIP(ag_dev_malloc(g->dev, &w->hub_part,
                      (size_t)(g->n_segs ? g->n_segs : 1) * PPR_W * sizeof(float)));
-    AG_HIP(hipMalloc((void **)&w->part, (size_t)w->grid_max * PPR_W * sizeof(double)));
-    AG_HIP(hipMalloc((void **)&w->colerr, PPR_W * sizeof(double)));
-    AG_HIP(hipMalloc((void **)&w->st, sizeof(PrState)));
-    AG_HIP(hipMalloc((void **)&w->conf, sizeof(PprConf)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->part, (size_t)w->grid_max * PPR_W * sizeof(double)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->colerr, PPR_W * sizeof(double)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->st, sizeof(PrState)));
+    AG_HIP(ag_dev_malloc(g->dev, &w->conf, sizeof(PprConf)));
     AG_HIP(hipHostMalloc((void **)&w->st_host, 2 * sizeof(PrState), hipHostMallocDefault));
     for (hipEvent_t &ev : w->ev)
         AG_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -628,7 +628,7 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
         w->hist = NULL;
         w->hist_cap = 0;
         const uint32_t cap = maxit > 512u ? maxit : 512u;
-        AG_HIP(hipMalloc((void **)&w->hist, (size_t)cap * sizeof(double)));
+        AG_HIP(ag_dev_malloc(g->dev, &w->hist, (size_t)cap * sizeof(double)));
         w->hist_cap = cap;
     }
     *out = w;

@@ -221,6 +221,20 @@ int ag_wait_stream(ag_device *d)
     return st;
 }
 
+// ------------------------------------------------------------------ device memory
+
+hipError_t ag_dev_malloc_bytes(ag_device *dev, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        for (ag_dgraph *g = dev->graphs; g; g = g->next)
+            ag_parked_free(g);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 // ------------------------------------------------------------------ staged transfers
 //
 // Callers' vectors are ordinary (pageable) memory, which the runtime moves through megabyte
@@ -346,7 +360,7 @@ template <typename T>
 static int dev_upload(ag_dgraph *g, T **dst, const T *src, size_t count)
 {
     size_t bytes = (count ? count : 1) * sizeof(T);
-    AG_HIP(hipMalloc((void **)dst, bytes));
+    AG_HIP(ag_dev_malloc(g->dev, dst, bytes));
     g->device_bytes += bytes;
     if (count)
         AG_HIP(hipMemcpyAsync(*dst, src, count * sizeof(T), hipMemcpyHostToDevice, g->dev->stream));
@@ -359,6 +373,11 @@ extern "C" int ag_graph_free(ag_dgraph *g)
         return AG_OK;
     (void)hipSetDevice(g->dev->ordinal);
     (void)hipStreamSynchronize(g->dev->stream);
+    for (ag_dgraph **q = &g->dev->graphs; *q; q = &(*q)->next)
+        if (*q == g) {
+            *q = g->next;
+            break;
+        }
     ag_ppr_free_ws(g);
     ag_parked_free(g);
     void *ptrs[] = {g->d2o, g->off, g->src, g->w, g->wq, g->outdeg, g->tile_row, g->rt, g->seg_row,
@@ -554,8 +573,8 @@ int ag_ensure_vec(ag_dgraph *g, size_t bytes)
         AG_HIP(hipFree(g->vec_b));
     g->vec_a = g->vec_b = NULL;
     g->vec_bytes = 0;
-    AG_HIP(hipMalloc(&g->vec_a, bytes));
-    AG_HIP(hipMalloc(&g->vec_b, bytes));
+    AG_HIP(ag_dev_malloc(g->dev, &g->vec_a, bytes));
+    AG_HIP(ag_dev_malloc(g->dev, &g->vec_b, bytes));
     g->vec_bytes = bytes;
     return AG_OK;
 }
@@ -580,6 +599,8 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
         return ag_set_error(AG_ERR_OOM, "host allocation failed");
     }
     g->dev = dev;
+    g->next = dev->graphs;
+    dev->graphs = g;
     dev->live_graphs++;
     g->params = plan.params;
     g->n = plan.n;
@@ -594,12 +615,7 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
     g->n_segs = plan.n_segs;
 
     hipError_t he = hipSetDevice(dev->ordinal);
-    if (he != hipSuccess) {
-        ag_plan_free(&plan);
-        free(g);
-        return ag_hip_fail(he, "hipSetDevice", __FILE__, __LINE__);
-    }
-    st = AG_OK;
+    st = he == hipSuccess ? AG_OK : ag_hip_fail(he, "hipSetDevice", __FILE__, __LINE__);
     if (st == AG_OK) {
         g->h_d2o = (uint32_t *)malloc((size_t)(plan.n ? plan.n : 1) * sizeof(uint32_t));
         if (!g->h_d2o)
@@ -622,7 +638,7 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
     if (st == AG_OK) st = dev_upload(g, &g->hub_seg0, plan.hub_seg0, (size_t)plan.n_hubs + 1);
     if (st == AG_OK) {
         size_t pb = (size_t)(plan.n_segs ? plan.n_segs : 1) * sizeof(uint64_t);
-        he = hipMalloc((void **)&g->hub_part, pb);
+        he = ag_dev_malloc(dev, &g->hub_part, pb);
         if (he != hipSuccess)
             st = ag_hip_fail(he, "hub scratch allocation", __FILE__, __LINE__);
         g->device_bytes += pb;
@@ -656,7 +672,7 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
         if (st == AG_OK && B.sorted) st = dev_upload(g, &g->blk.tbase, B.tbase, B.n_items);
         if (st == AG_OK) {
             size_t pb = (size_t)(B.nv ? B.nv : 1) * sizeof(uint64_t);
-            he = hipMalloc((void **)&g->vpart, pb);
+            he = ag_dev_malloc(dev, &g->vpart, pb);
             if (he != hipSuccess)
                 st = ag_hip_fail(he, "partial-sum allocation", __FILE__, __LINE__);
             g->device_bytes += pb;
@@ -674,7 +690,7 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
             g->bdyn = !reg && (order == AG_TILES_TICKET ||
                                (order == AG_TILES_AUTO && 2ull * B.nv >= B.mb));
             const size_t tb = 2 * AG_NXCD * sizeof(uint32_t);
-            he = hipMalloc((void **)&g->btick, tb);
+            he = ag_dev_malloc(dev, &g->btick, tb);
             if (he == hipSuccess)
                 he = hipMemsetAsync(g->btick, 0, tb, dev->stream);
             if (he != hipSuccess)
@@ -715,7 +731,7 @@ extern "C" int ag_graph_set_fixed_weights(ag_dgraph *g, const uint32_t *inv_edge
     }
     hipError_t e = hipSetDevice(g->dev->ordinal);
     if (e == hipSuccess && !g->wq) {
-        e = hipMalloc((void **)&g->wq, (size_t)(g->m ? g->m : 1) * sizeof(uint32_t));
+        e = ag_dev_malloc(g->dev, &g->wq, (size_t)(g->m ? g->m : 1) * sizeof(uint32_t));
         if (e == hipSuccess)
             g->device_bytes += (size_t)g->m * sizeof(uint32_t);
     }
@@ -746,6 +762,8 @@ extern "C" int ag_graph_get_info(const ag_dgraph *g, ag_graph_info *info)
     info->num_segments = g->n_segs;
     info->has_weights = g->w != NULL;
     info->device_bytes = g->device_bytes;
+    for (uint32_t i = 0; i < g->parked.n_dev; i++)
+        info->device_bytes += g->parked.bytes[i];
     info->params = g->params;
     info->src_block_bits = g->blk.bits;
     info->src_blocks = g->blk.nblocks;
@@ -779,8 +797,8 @@ extern "C" int ag_device_copy_bandwidth(ag_device *dev, uint64_t bytes, uint32_t
     AG_HIP(hipSetDevice(dev->ordinal));
     const uint64_t n16 = bytes / 16;
     ag_u32x4 *a = NULL, *b = NULL;
-    AG_HIP(hipMalloc((void **)&a, n16 * 16));
-    hipError_t e = hipMalloc((void **)&b, n16 * 16);
+    AG_HIP(ag_dev_malloc(dev, &a, n16 * 16));
+    hipError_t e = ag_dev_malloc(dev, &b, n16 * 16);
     hipEvent_t e0 = NULL, e1 = NULL;
     if (e == hipSuccess)
         e = hipMemsetAsync(a, 1, n16 * 16, dev->stream);
@@ -873,8 +891,8 @@ extern "C" int ag_fixed_encode(ag_device *dev, uint32_t bits, const float *in, u
     AG_HIP(hipSetDevice(dev->ordinal));
     float *din = NULL;
     uint64_t *dout = NULL;
-    AG_HIP(hipMalloc((void **)&din, (size_t)n * sizeof(float)));
-    hipError_t e = hipMalloc((void **)&dout, (size_t)n * sizeof(uint64_t));
+    AG_HIP(ag_dev_malloc(dev, &din, (size_t)n * sizeof(float)));
+    hipError_t e = ag_dev_malloc(dev, &dout, (size_t)n * sizeof(uint64_t));
     if (e == hipSuccess)
         e = hipMemcpyAsync(din, in, (size_t)n * sizeof(float), hipMemcpyHostToDevice, dev->stream);
     if (e == hipSuccess) {
@@ -900,8 +918,8 @@ extern "C" int ag_fixed_decode(ag_device *dev, uint32_t bits, const uint64_t *in
     AG_HIP(hipSetDevice(dev->ordinal));
     uint64_t *din = NULL;
     double *dout = NULL;
-    AG_HIP(hipMalloc((void **)&din, (size_t)n * sizeof(uint64_t)));
-    hipError_t e = hipMalloc((void **)&dout, (size_t)n * sizeof(double));
+    AG_HIP(ag_dev_malloc(dev, &din, (size_t)n * sizeof(uint64_t)));
+    hipError_t e = ag_dev_malloc(dev, &dout, (size_t)n * sizeof(double));
     if (e == hipSuccess)
         e = hipMemcpyAsync(din, in, (size_t)n * sizeof(uint64_t), hipMemcpyHostToDevice, dev->stream);
     if (e == hipSuccess) {

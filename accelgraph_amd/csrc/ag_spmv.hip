@@ -404,7 +404,7 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
         return st;
     hipStream_t stream = g->dev->stream;
     if (g->w && !g->wq && g->m) {
-        AG_HIP(hipMalloc((void **)&g->wq, (size_t)g->m * sizeof(uint32_t)));
+        AG_HIP(ag_dev_malloc(g->dev, &g->wq, (size_t)g->m * sizeof(uint32_t)));
         g->device_bytes += (size_t)g->m * sizeof(uint32_t);
         quantize_weights_kernel<<<(g->m + AG_WG - 1) / AG_WG, AG_WG, 0, stream>>>(g->m, g->w, g->wq);
         AG_HIP(hipGetLastError());
@@ -413,7 +413,7 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
     // the caller exist only in regular order, so such a graph keeps the regular schedule.
     const bool blocked = g->blk.bits && !g->wq_user;
     if (blocked && g->w && !g->vwq && g->blk.mb) {
-        AG_HIP(hipMalloc((void **)&g->vwq, (size_t)g->blk.mb * sizeof(uint32_t)));
+        AG_HIP(ag_dev_malloc(g->dev, &g->vwq, (size_t)g->blk.mb * sizeof(uint32_t)));
         g->device_bytes += (size_t)g->blk.mb * sizeof(uint32_t);
         quantize_weights_kernel<<<(g->blk.mb + AG_WG - 1) / AG_WG, AG_WG, 0, stream>>>(
             g->blk.mb, g->blk.vw, g->vwq);

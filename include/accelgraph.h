@@ -169,7 +169,7 @@ typedef struct ag_graph_info {
     uint32_t num_tiles;
     uint32_t num_segments;
     uint32_t has_weights;
-    uint64_t device_bytes;
+    uint64_t device_bytes;     /* of HBM held, buffers kept for the next session among them */
     ag_plan_params params;
     uint32_t src_block_bits;   /* blocking in effect (0: none)                          */
     uint32_t src_blocks;       /* source blocks                                         */

@@ -26,15 +26,18 @@ int fake_copies(void) { return copies; }
 size_t fake_held(void) { return held; }
 size_t fake_copied(void) { size_t c = peak_copy; peak_copy = 0; return c; }
 void fake_limit(size_t bytes) { limit = bytes; }
-void fake_fail_in(int n) { fail_in = n; }            /* the n-th device allocation from now */
-void fake_fail_host_in(int n) { fail_host_in = n; }  /* the n-th pinned one */
+/* after n more device allocations, or pinned ones, every one fails (-1: none does) */
+void fake_fail_in(int n) { fail_in = n; }
+void fake_fail_host_in(int n) { fail_host_in = n; }
 
 int hipMalloc(void **p, size_t bytes)
 {
     mallocs++;
     *p = NULL;
-    if ((fail_in >= 0 && fail_in-- == 0) || held + bytes > limit)
+    if (fail_in == 0 || held + bytes > limit)
         return ERR_OOM;
+    if (fail_in > 0)
+        fail_in--;
     for (int i = 0; i < 4096; i++)
         if (!blocks[i].p) {
             *p = blocks[i].p = calloc(1, bytes ? bytes : 1);
@@ -67,8 +70,10 @@ int hipHostMalloc(void **p, size_t bytes, unsigned flags)
 {
     (void)flags;
     *p = NULL;
-    if (fail_host_in >= 0 && fail_host_in-- == 0)
+    if (fail_host_in == 0)
         return ERR_OOM;
+    if (fail_host_in > 0)
+        fail_host_in--;
     *p = calloc(1, bytes ? bytes : 1);
     return *p ? OK : ERR_OOM;
 }

@@ -80,3 +80,30 @@ def test_ppr_workspace_whole_or_none(fake_hip, kind):
     dg.close()
     assert fake.fake_live() == 0
     """)
+
+
+@pytest.mark.parametrize("op", [
+    "dev.upload(ag.Graph.rmat(9)).close()", "small.gather(np.ones(small.n, np.uint64), ag.GATHER_U64)",
+    "small.ppr(np.arange(2, dtype=np.uint32), max_iterations=5)", "small.spmv_fixed(np.ones(small.n, np.uint32))",
+    "small.pagerank(max_iterations=3)", "small.features()",
+    "ag.Batch(dev, [ag.Graph.rmat(8)]).close()", "dev.fixed_encode(32, np.ones(1000, np.float32))"])
+def test_parked_buffers_given_back(fake_hip, op):
+    """Buffers that a graph keeps for its next session are counted in its device bytes and given back
+    to whatever finds the memory full, another graph's calls among them."""
+    run(fake_hip, f"""
+    dg, tiny = dev.upload(ag.Graph.rmat(14)), ag.Graph.rmat(6)
+    tiny.set_weights(np.ones(tiny.m, np.float32))
+    small = dev.upload(tiny, weights=True)
+    held = fake.fake_held()
+    bare = dg.info().device_bytes
+    dg.pagerank(max_iterations=3)
+    parked = dg.info().device_bytes - bare
+    assert parked >= 3 * 4 * dg.n and fake.fake_held() >= held + parked
+    fake.fake_limit(fake.fake_held())
+    assert status(lambda: {op}) == 0
+    assert dg.info().device_bytes == bare
+    fake.fake_limit(fake.fake_held())          # nothing left to give back
+    assert status(lambda: dev.upload(ag.Graph.rmat(14))) == ag._abi.AG_ERR_OOM
+    fake.fake_limit(1 << 40)
+    dg.pagerank(max_iterations=3)
+    """)
