@@ -486,6 +486,8 @@ static int build_layout(ag_batch *b, uint32_t part_edges, uint32_t heavy_deg)
         e = hipMemcpyAsync(b->d_heavy, heavy, nh * sizeof(uint32_t), hipMemcpyHostToDevice, s);
     st = (e == hipSuccess) ? ag_wait_stream(b->dev)   // the host arrays must outlive the copies
                            : ag_hip_fail(e, "batch layout upload", __FILE__, __LINE__);
+    if (st != AG_OK)
+        (void)hipStreamSynchronize(s);
     free(parts);
     free(gpart);
     free(heavy);
@@ -624,6 +626,8 @@ extern "C" int ag_batch_upload(ag_device *dev, uint32_t G, const uint32_t *vert_
     }
     if (st == AG_OK)
         st = ag_wait_stream(dev);  // host staging buffers must outlive the copies
+    if (st != AG_OK)
+        (void)hipStreamSynchronize(dev->stream);
     free(hsrc);
     if (st == AG_OK) {
         memset(&b->a, 0, sizeof(b->a));

@@ -698,9 +698,11 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
             g->device_bytes += tb;
         }
     }
-    // the host plan arrays must outlive the asynchronous copies
+    // the host plan arrays must outlive the asynchronous copies, also those before a failure
     if (st == AG_OK)
         st = ag_wait_stream(dev);
+    if (st != AG_OK)
+        (void)hipStreamSynchronize(dev->stream);
     ag_plan_free(&plan);
     if (st != AG_OK) {
         ag_graph_free(g);
@@ -740,6 +742,8 @@ extern "C" int ag_graph_set_fixed_weights(ag_dgraph *g, const uint32_t *inv_edge
                            g->dev->stream);
     int st = (e == hipSuccess) ? ag_wait_stream(g->dev)
                                : ag_hip_fail(e, "fixed weight upload", __FILE__, __LINE__);
+    if (st != AG_OK)
+        (void)hipStreamSynchronize(g->dev->stream);   // buf must outlive its copy
     free(buf);
     if (st == AG_OK)
         g->wq_user = 1;

@@ -3,7 +3,6 @@
  * side of the device layer (csrc/ .hip files) runs without a GPU: allocations are host memory, copies are
  * memcpy, kernels do nothing. Device allocations are counted and can be made to fail.
  */
-#define _GNU_SOURCE
 #include <stddef.h>
 #include <stdint.h>
 #include <stdlib.h>
@@ -16,11 +15,14 @@ static struct block {
     size_t bytes;
 } blocks[4096];
 static size_t held, limit = (size_t)-1, peak_copy;
+static int pending;   /* copies queued since the last wait */
+static int early;     /* plans freed under them */
 static int mallocs, live, captures, copies, fail_in = -1, fail_host_in = -1;
 
 /* what the tests read and set */
 int fake_mallocs(void) { return mallocs; }
 int fake_live(void) { return live; }
+int fake_early_frees(void) { return early; }
 int fake_captures(void) { return captures; }
 int fake_copies(void) { return copies; }
 size_t fake_held(void) { return held; }
@@ -95,6 +97,7 @@ int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; return copy(d,
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st)
 {
     (void)k; (void)st;
+    pending++;
     return copy(d, s, n);
 }
 int hipMemset(void *d, int v, size_t n) { memset(d, v, n); return OK; }
@@ -124,7 +127,7 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int b, s
 static int handle(void **h) { *h = malloc(1); return *h ? OK : ERR_OOM; }
 int hipStreamCreateWithFlags(void **s, unsigned f) { (void)f; return handle(s); }
 int hipStreamDestroy(void *s) { free(s); return OK; }
-int hipStreamSynchronize(void *s) { (void)s; return OK; }
+int hipStreamSynchronize(void *s) { (void)s; pending = 0; return OK; }
 int hipEventCreate(void **e) { return handle(e); }
 int hipEventCreateWithFlags(void **e, unsigned f) { (void)f; return handle(e); }
 int hipEventDestroy(void *e) { free(e); return OK; }
@@ -171,3 +174,12 @@ void **__hipRegisterFatBinary(const void *d)
 void __hipUnregisterFatBinary(void **h) { (void)h; }
 void __hipRegisterFunction(void) {}
 void __hipRegisterVar(void) {}
+
+/* in front of the library's own: counts the plans freed while a copy may still read them */
+static void (*own_plan_free)(void *);
+void fake_plan_free_is(void (*own)(void *)) { own_plan_free = own; }
+void ag_plan_free(void *plan)
+{
+    early += pending != 0;
+    own_plan_free(plan);
+}

@@ -16,6 +16,7 @@ import accelgraph_amd as ag
 fake = C.CDLL(None)
 fake.fake_limit.argtypes = [C.c_size_t]
 fake.fake_held.restype = fake.fake_copied.restype = C.c_size_t
+fake.fake_plan_free_is(C.CDLL(ag._abi.LIB_PATH).ag_plan_free)
 dev = ag.Device(0)
 
 def status(f):
@@ -106,4 +107,16 @@ def test_parked_buffers_given_back(fake_hip, op):
     assert status(lambda: dev.upload(ag.Graph.rmat(14))) == ag._abi.AG_ERR_OOM
     fake.fake_limit(1 << 40)
     dg.pagerank(max_iterations=3)
+    """)
+
+
+@pytest.mark.parametrize("fail", [1, 4, 9, 20])
+def test_failed_upload_waits_for_its_copies(fake_hip, fail):
+    """An upload that runs out of memory half way waits for the copies already queued before it
+    frees the host arrays that they read."""
+    run(fake_hip, f"""
+    fake.fake_fail_in({fail})
+    st = status(lambda: dev.upload(ag.Graph.rmat(9), params=ag.plan_params(src_block_bits=8)))
+    assert st == ag._abi.AG_ERR_OOM
+    assert fake.fake_early_frees() == 0 and fake.fake_live() == 0
     """)
