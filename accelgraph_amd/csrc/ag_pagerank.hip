@@ -210,38 +210,54 @@ __device__ __forceinline__ void block_sum_all(double &e, uint32_t &a)
     }
 }
 
+// The previous iteration's partials: four a lane loaded ahead, then their sums over the workgroup,
+// the same in every lane and in the same order whichever kernel closes the iteration.
+struct PrPartials {
+    double e[4];
+    uint32_t a[4];
+
+    __device__ __forceinline__ PrPartials(const PrCtl &C, bool pending)
+    {
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t i = threadIdx.x + u * AG_WG;
+            const bool in = pending && i < C.nparts;
+            e[u] = in ? C.prev_err[i] : 0.0;
+            a[u] = in ? C.prev_act[i] : 0u;
+        }
+    }
+    __device__ __forceinline__ void sums(const PrCtl &C, double &E, uint32_t &A) const
+    {
+        E = (e[0] + e[1]) + (e[2] + e[3]);
+        A = (a[0] + a[1]) + (a[2] + a[3]);
+        for (uint32_t i = threadIdx.x + 4u * AG_WG; i < C.nparts; i += AG_WG) {
+            E += C.prev_err[i];
+            A += C.prev_act[i];
+        }
+        block_sum_all<AG_WG>(E, A);
+    }
+};
+
 // First step of an iteration's first kernel, in two halves: the constructor loads the state and
 // (up to four a lane) the previous iteration's partials, the call makes S the state with every
 // earlier iteration closed. False when the run has stopped (the same in every workgroup).
 struct PrAhead {
     PrRun S;
-    double e[4];
-    uint32_t a[4];
+    PrPartials prev;
     bool run;
 
-    __device__ __forceinline__ explicit PrAhead(const PrCtl &C) : run(false)
+    __device__ __forceinline__ explicit PrAhead(const PrCtl &C)
+        : S(pr_load(&C.st[C.it & 1u])), prev(C, C.pending), run(false)
     {
-        S = pr_load(&C.st[C.it & 1u]);
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; u++) {
-            const uint32_t i = threadIdx.x + u * AG_WG;
-            const bool in = C.pending && i < C.nparts;
-            e[u] = in ? C.prev_err[i] : 0.0;
-            a[u] = in ? C.prev_act[i] : 0u;
-        }
     }
     __device__ __forceinline__ bool operator()(const PrCtl &C)
     {
         const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
         const bool was_done = S.done != 0u;
         if (!was_done && C.pending) {
-            double E = (e[0] + e[1]) + (e[2] + e[3]);
-            uint32_t A = (a[0] + a[1]) + (a[2] + a[3]);
-            for (uint32_t i = threadIdx.x + 4u * AG_WG; i < C.nparts; i += AG_WG) {
-                E += C.prev_err[i];
-                A += C.prev_act[i];
-            }
-            block_sum_all<AG_WG>(E, A);
+            double E;
+            uint32_t A;
+            prev.sums(C, E, A);
             pr_control(C, S, C.it - 1u, E, A, writer);
         }
         if (writer) {
@@ -279,13 +295,9 @@ __global__ __launch_bounds__(AG_WG) void pr_close_kernel(PrCtl C)
     PrRun S = pr_load(&C.st[C.it & 1u]);
     if (S.done)
         return;
-    double E = 0.0;
-    uint32_t A = 0u;
-    for (uint32_t i = threadIdx.x; i < C.nparts; i += AG_WG) {
-        E += C.prev_err[i];
-        A += C.prev_act[i];
-    }
-    block_sum_all<AG_WG>(E, A);
+    double E;
+    uint32_t A;
+    PrPartials(C, true).sums(C, E, A);
     if (threadIdx.x == 0) {
         pr_control(C, S, C.it - 1u, E, A, true);
         pr_save(&C.st[C.it & 1u], S);

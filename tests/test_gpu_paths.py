@@ -246,6 +246,29 @@ def test_steps_of_any_length(device, plan, run):
     dg.close()
 
 
+# the data-driven pull of an unblocked plan runs a start of one's own on worklists, whose order varies
+@pytest.mark.parametrize("plan,run", [(p, r) for p in ({}, dict(src_block_bits=13))
+                                      for r in range(len(STEP_RUNS))
+                                      if p or "direction" not in STEP_RUNS[r]])
+def test_steps_close_in_one_order(device, plan, run):
+    """An iteration of more than two partials a lane (512 workgroups) has the same error to the last
+    bit whether the next launch or the step's end closes it, so no stop depends on the steps. One
+    huge start value on a vertex without out-edges makes its workgroup's partial so large that the
+    others are fractions of its last bit, where the order of a sum shows."""
+    g = ag.Graph.rmat(17)
+    dg = device.upload(g, params=ag.plan_params(**plan))
+    rng = np.random.default_rng(31)
+    for sink in rng.choice(np.flatnonzero(g.out_degree == 0), 6, replace=False):
+        for e in range(56, 64):
+            start = rng.random(g.n, dtype=np.float32)
+            start[sink] = 2.0 ** e
+            kw = dict(max_iterations=3, stop_rule=ag.STOP_NONE, init_ranks=start, **STEP_RUNS[run])
+            a, b = dg.pagerank(chunk=1, **kw), dg.pagerank(chunk=3, **kw)
+            np.testing.assert_array_equal(a.hist_err.view(np.uint64), b.hist_err.view(np.uint64))
+            np.testing.assert_array_equal(a.hist_active, b.hist_active)
+    dg.close()
+
+
 @pytest.mark.parametrize("n", [1, 1000, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 4 * (1 << 20) + 3,
                                5 * (1 << 20) + 7])
 def test_staged_transfers(device, n):
