@@ -2107,7 +2107,8 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
     if (!s || !rows)
         return ag_set_error(AG_ERR_INVALID, "null argument");
     AG_HIP(hipSetDevice(s->g->dev->ordinal));
-    // short histories come with the state, in one transfer to the session's pinned block
+    // short histories come with the state, in one transfer to the session's pinned block; of longer
+    // ones (more than about 2300 iterations) the rows of the executed iterations alone
     const size_t all = s->hist_bytes, head = 256u;
     const bool with_state = all + head <= AG_PIN_BYTES;
     if (with_state)
@@ -2123,37 +2124,35 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
     *rows = k;
     if (k == 0)
         return AG_OK;
-    char *buf = NULL;
-    if (!with_state) {
-        buf = (char *)malloc(all);
-        if (!buf)
-            return ag_set_error(AG_ERR_OOM, "host allocation failed");
-        st = ag_copy_out(s->g->dev, buf, s->hist_err, all);
-        if (st != AG_OK) {
-            free(buf);
-            return st;
-        }
-    }
-    const char *h = with_state ? (const char *)s->pin + head : buf;
-    const double *he = (const double *)h;
-    const uint64_t *ht = (const uint64_t *)(h + ((const char *)s->hist_t - (const char *)s->hist_err));
-    const uint32_t *ha = (const uint32_t *)(h + ((const char *)s->hist_act - (const char *)s->hist_err));
+    const char *h = (const char *)s->pin + head;
+    // rows of one history array: out of the pinned block, or straight from the device
+    const auto take = [&](void *dst, const void *src, size_t bytes) {
+        if (!with_state)
+            return ag_copy_out(s->g->dev, dst, src, bytes);
+        memcpy(dst, h + ((const char *)src - (const char *)s->hist_err), bytes);
+        return (int)AG_OK;
+    };
     if (active)
-        memcpy(active, ha, (size_t)k * sizeof(uint32_t));
-    if (error)
-        memcpy(error, he, (size_t)k * sizeof(double));
-    if (iter_ms) {
+        st = take(active, s->hist_act, (size_t)k * sizeof(uint32_t));
+    if (st == AG_OK && error)
+        st = take(error, s->hist_err, (size_t)k * sizeof(double));
+    if (st == AG_OK && iter_ms) {
         int khz = 0;   // the device clock ticks at a constant rate
-        const hipError_t e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate,
-                                                   s->g->dev->ordinal);
-        if (e != hipSuccess)
-            st = ag_hip_fail(e, "hipDeviceGetAttribute(clock rate)", __FILE__, __LINE__);
+        uint64_t *t = NULL;
+        if (s->o.record_history) {
+            t = (uint64_t *)malloc((size_t)k * 16u);
+            if (!t)
+                return ag_set_error(AG_ERR_OOM, "host allocation failed");
+            st = take(t, s->hist_t, (size_t)k * 16u);
+            const hipError_t e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate,
+                                                       s->g->dev->ordinal);
+            if (st == AG_OK && e != hipSuccess)
+                st = ag_hip_fail(e, "hipDeviceGetAttribute(clock rate)", __FILE__, __LINE__);
+        }
         for (uint32_t i = 0; i < k; i++)
-            iter_ms[i] = s->o.record_history && khz > 0
-                             ? (float)((double)(ht[2 * i + 1] - ht[2 * i]) / (double)khz)
-                             : 0.0f;
+            iter_ms[i] = khz > 0 ? (float)((double)(t[2 * i + 1] - t[2 * i]) / (double)khz) : 0.0f;
+        free(t);
     }
-    free(buf);
     return st;
 }
 

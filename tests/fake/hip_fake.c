@@ -14,7 +14,8 @@ static struct block {
     void *p;
     size_t bytes;
 } blocks[4096];
-static size_t held, limit = (size_t)-1, peak_copy;
+static size_t held, limit = (size_t)-1, copied;
+static uint32_t fill;  /* every word of the next device allocation */
 static int pending;   /* copies queued since the last wait */
 static int early;     /* plans freed under them */
 static int mallocs, live, captures, copies, fail_in = -1, fail_host_in = -1;
@@ -26,7 +27,8 @@ int fake_early_frees(void) { return early; }
 int fake_captures(void) { return captures; }
 int fake_copies(void) { return copies; }
 size_t fake_held(void) { return held; }
-size_t fake_copied(void) { size_t c = peak_copy; peak_copy = 0; return c; }
+size_t fake_copied(void) { size_t c = copied; copied = 0; return c; }   /* since the last call */
+void fake_fill(uint32_t word) { fill = word; }
 void fake_limit(size_t bytes) { limit = bytes; }
 /* after n more device allocations, or pinned ones, every one fails (-1: none does) */
 void fake_fail_in(int n) { fail_in = n; }
@@ -45,6 +47,9 @@ int hipMalloc(void **p, size_t bytes)
             *p = blocks[i].p = calloc(1, bytes ? bytes : 1);
             if (!*p)
                 return ERR_OOM;
+            for (size_t w = 0; fill && w < bytes / 4; w++)
+                ((uint32_t *)*p)[w] = fill;
+            fill = 0;
             blocks[i].bytes = bytes;
             held += bytes;
             live++;
@@ -89,7 +94,7 @@ int hipHostFree(void *p)
 static int copy(void *d, const void *s, size_t n)
 {
     copies++;
-    peak_copy += n;
+    copied += n;
     memcpy(d, s, n);
     return OK;
 }

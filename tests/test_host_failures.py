@@ -120,3 +120,21 @@ def test_failed_upload_waits_for_its_copies(fake_hip, fail):
     assert st == ag._abi.AG_ERR_OOM
     assert fake.fake_early_frees() == 0 and fake.fake_live() == 0
     """)
+
+
+@pytest.mark.parametrize("max_iterations", [2000, 2400, 1000000])
+def test_history_moves_executed_rows(fake_hip, max_iterations):
+    """The history of a run that may take a million iterations is read for those it took: at most
+    the 64 KB of a session's pinned block beside the rows themselves."""
+    run(fake_hip, f"""
+    dg = dev.upload(ag.Graph.rmat(6))
+    fake.fake_fill(5)      # the state says that 6 iterations ran
+    s = dg.session(max_iterations={max_iterations}, record_history=1)
+    s.step(5)
+    rows = C.c_uint32(0)
+    act, err, ms = (C.c_uint32 * 5)(), (C.c_double * 5)(), (C.c_float * 5)()
+    fake.fake_copied()
+    assert ag.lib().ag_pr_history(s._s, 5, act, err, ms, C.byref(rows)) == 0
+    assert rows.value == 5 and list(act) == [5] * 5
+    assert fake.fake_copied() <= 66000
+    """)
