@@ -785,7 +785,8 @@ extern "C" int ag_batch_pagerank(ag_batch *b, const ag_batch_options *opts, floa
             st = ag_hip_fail(he, "batch results", __FILE__, __LINE__);
     }
     if (st == AG_OK && ranks_out)
-        st = ag_copy_out(b->dev, ranks_out, b->a.out, (size_t)b->total_n * sizeof(float));
+        st = ag_copy_out(b->dev, ranks_out, b->a.out, (size_t)b->total_n * sizeof(float),
+                         (size_t)b->total_n * sizeof(float));
     if (st == AG_OK && (!ranks_out || b->total_n == 0))
         st = ag_wait_stream(b->dev);
     if (st == AG_OK && iterations)

@@ -226,11 +226,12 @@ int ag_set_error(int status, const char *fmt, ...);
 int ag_hip_fail(hipError_t e, const char *what, const char *file, int line);
 int ag_wait_stream(ag_device *dev);
 int ag_wait_event(ag_device *dev, hipEvent_t ev);
-// Host -> device copy on the device's stream, through the pinned ring: `host` may be reused on
-// return. Memory that is pinned already is copied straight (then it may not, before a wait).
-int ag_copy_in(ag_device *dev, void *dst, const void *host, size_t bytes);
+// Host -> device copy on the device's stream, straight for small vectors and memory that the runtime
+// knows (pinned memory may not be reused before a wait), else through the pinned ring. `largest`:
+// bytes of the largest vector that the call moves, in or out (its vectors go the same way).
+int ag_copy_in(ag_device *dev, void *dst, const void *host, size_t bytes, size_t largest);
 // Device -> host copy after the work on the device's stream; done on return.
-int ag_copy_out(ag_device *dev, void *host, const void *src, size_t bytes);
+int ag_copy_out(ag_device *dev, void *host, const void *src, size_t bytes, size_t largest);
 // Frees the parked buffers of a graph.
 void ag_parked_free(ag_dgraph *g);
 // hipMalloc for every allocation of the library: when device memory runs out, the parked buffers of

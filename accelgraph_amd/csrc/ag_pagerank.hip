@@ -1758,7 +1758,8 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     }
     if (o.init == AG_INIT_USER && n) {
         AG_TRY(salloc(s, (void **)&s->user, (size_t)n * sizeof(float)));
-        AG_TRY(ag_copy_in(g->dev, s->user, o.init_ranks, (size_t)n * sizeof(float)));
+        AG_TRY(ag_copy_in(g->dev, s->user, o.init_ranks, (size_t)n * sizeof(float),
+                          (size_t)n * sizeof(float)));
     }
     if (n) {
         void *c0 = (kc == 1 || kc == 2) ? s->c16[0] : s->c[0];
@@ -2128,7 +2129,7 @@ extern "C" int ag_pr_history(ag_pr_session *s, uint32_t cap, uint32_t *active, d
     // rows of one history array: out of the pinned block, or straight from the device
     const auto take = [&](void *dst, const void *src, size_t bytes) {
         if (!with_state)
-            return ag_copy_out(s->g->dev, dst, src, bytes);
+            return ag_copy_out(s->g->dev, dst, src, bytes, bytes);
         memcpy(dst, h + ((const char *)src - (const char *)s->hist_err), bytes);
         return (int)AG_OK;
     };
@@ -2170,7 +2171,8 @@ extern "C" int ag_pr_read_scaled(ag_pr_session *s, float *scaled_out)
     scaled_copy_kernel<<<(g->n + AG_WG - 1) / AG_WG, AG_WG, 0, g->dev->stream>>>(
         g->n, s->rank, g->d2o, (float *)g->vec_a);
     AG_HIP(hipGetLastError());
-    return ag_copy_out(g->dev, scaled_out, g->vec_a, (size_t)g->n * sizeof(float));
+    return ag_copy_out(g->dev, scaled_out, g->vec_a, (size_t)g->n * sizeof(float),
+                       (size_t)g->n * sizeof(float));
 }
 
 extern "C" int ag_pr_end(ag_pr_session *s, float *ranks_out, ag_pr_result *res)
@@ -2205,7 +2207,8 @@ extern "C" int ag_pr_end(ag_pr_session *s, float *ranks_out, ag_pr_result *res)
         if (e != hipSuccess)
             st = ag_hip_fail(e, "finalize", __FILE__, __LINE__);
         if (st == AG_OK && ranks_out)
-            st = ag_copy_out(g->dev, ranks_out, g->vec_a, (size_t)g->n * sizeof(float));
+            st = ag_copy_out(g->dev, ranks_out, g->vec_a, (size_t)g->n * sizeof(float),
+                             (size_t)g->n * sizeof(float));
     }
     if (st == AG_OK && (!ranks_out || !g->n))
         st = ag_wait_stream(g->dev);

@@ -880,10 +880,11 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         ppr_out_kernel<<<(uint32_t)((tot + 255) / 256), 256, 0, s>>>(n, k, w->width, w->rank, g->d2o,
                                                                      (float)n, outd);
         e = hipGetLastError();
-        st = (e == hipSuccess) ? ag_copy_out(g->dev, ranks_out, outd, tot * sizeof(float))
+        const size_t ob = tot * sizeof(float), eb = (size_t)k * sizeof(double);
+        st = (e == hipSuccess) ? ag_copy_out(g->dev, ranks_out, outd, ob, ob)
                                : ag_hip_fail(e, "PPR output", __FILE__, __LINE__);
         if (st == AG_OK && col_error)
-            st = ag_copy_out(g->dev, col_error, w->colerr, (size_t)k * sizeof(double));
+            st = ag_copy_out(g->dev, col_error, w->colerr, eb, eb);
     }
     if (e0)
         (void)hipEventDestroy(e0);

@@ -242,6 +242,15 @@ hipError_t ag_dev_malloc_bytes(ag_device *dev, void **p, size_t bytes)
 // 20-iteration RMAT-25 call. Here chunks of 4 MB go through a pinned ring kept by the device,
 // the link ahead of (or behind) the copies of eight cores: 16 MB each way 1.9 -> 1.1 ms, 134 MB
 // out 14 -> 5 ms. Chunks of 1 MB were slower (1.4 ms; every chunk pays its launch and wait).
+// Vectors of a call go straight while the larger of its vectors is below 1 MB: the ring's second
+// copy, event and wait cost more than they save. A SpMV call (x in, y out; straight / ring, us) of
+// 64 KB each way 50 / 60, 256 KB 66 / 83, 400 KB 78 / 93, 800 KB 114 / 118, 1 MB 149 / 133; 256 KB
+// in and 512 KB out 81 / 95, 460 and 920 KB 107 / 117, 512 KB and 1 MB 132 / 125. One vector
+// straight and the other through the ring was slower than either (600 KB: 127). Results of at most
+// 16 KB leave through the ring, for which the link has a faster path out of pinned memory (16 KB
+// each way 41, straight 43 to 56).
+#define AG_STRAIGHT_BELOW ((size_t)1 << 20)
+#define AG_PINNED_OUT ((size_t)16 << 10)
 
 static int stage_open(ag_device *d)
 {
@@ -282,11 +291,11 @@ static int stage_slot(ag_device *d, uint32_t *slot)
     return (d->stage_used >> *slot & 1u) ? ag_wait_event(d, d->stage_ev[*slot]) : AG_OK;
 }
 
-int ag_copy_in(ag_device *d, void *dst, const void *host, size_t bytes)
+int ag_copy_in(ag_device *d, void *dst, const void *host, size_t bytes, size_t largest)
 {
     if (bytes == 0)
         return AG_OK;
-    if (is_known(host)) {
+    if (largest < AG_STRAIGHT_BELOW || is_known(host)) {
         AG_HIP(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, d->stream));
         return AG_OK;
     }
@@ -306,11 +315,11 @@ int ag_copy_in(ag_device *d, void *dst, const void *host, size_t bytes)
     return st;
 }
 
-int ag_copy_out(ag_device *d, void *host, const void *src, size_t bytes)
+int ag_copy_out(ag_device *d, void *host, const void *src, size_t bytes, size_t largest)
 {
     if (bytes == 0)
         return AG_OK;
-    if (is_known(host)) {
+    if ((largest < AG_STRAIGHT_BELOW && bytes > AG_PINNED_OUT) || is_known(host)) {
         AG_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, d->stream));
         return ag_wait_stream(d);
     }

@@ -300,7 +300,7 @@ static int spmv_f32_device(ag_dgraph *g, const float *x, float *y, float *xo, fl
     const size_t nb = (size_t)n * sizeof(float);
     int st = AG_OK;
     if (staged)
-        st = ag_copy_in(g->dev, xo, x, nb);
+        st = ag_copy_in(g->dev, xo, x, nb, nb);
     else
         AG_HIP(hipMemcpyAsync(xo, x, nb, hipMemcpyHostToDevice, stream));
     if (st != AG_OK)
@@ -323,7 +323,7 @@ static int spmv_f32_device(ag_dgraph *g, const float *x, float *y, float *xo, fl
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, yo);
     AG_HIP(hipGetLastError());
     if (staged) {
-        st = ag_copy_out(g->dev, y, yo, nb);
+        st = ag_copy_out(g->dev, y, yo, nb, nb);
     } else {
         AG_HIP(hipMemcpyAsync(y, yo, nb, hipMemcpyDeviceToHost, stream));
         st = ag_wait_stream(g->dev);
@@ -424,7 +424,8 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
     uint32_t *xd = (uint32_t *)g->vec_b;
     uint64_t *yd = (uint64_t *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    st = ag_copy_in(g->dev, xo, xq, (size_t)n * sizeof(uint32_t));
+    const size_t yb = (size_t)n * sizeof(uint64_t);
+    st = ag_copy_in(g->dev, xo, xq, (size_t)n * sizeof(uint32_t), yb);
     if (st != AG_OK)
         return st;
     permute_in_kernel<uint32_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
@@ -444,7 +445,7 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, yo);
     AG_HIP(hipGetLastError());
-    st = ag_copy_out(g->dev, yq, yo, (size_t)n * sizeof(uint64_t));
+    st = ag_copy_out(g->dev, yq, yo, yb, yb);
     return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
@@ -480,7 +481,8 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     float *xd = (float *)g->vec_b;
     float *yd = (float *)((char *)g->vec_b + (size_t)n * sizeof(float));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    st = ag_copy_in(g->dev, xo, x, (size_t)n * sizeof(float));
+    const size_t nb = (size_t)n * sizeof(float);
+    st = ag_copy_in(g->dev, xo, x, nb, nb);
     if (st != AG_OK)
         return st;
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
@@ -493,7 +495,7 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
         return st;
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
     AG_HIP(hipGetLastError());
-    st = ag_copy_out(g->dev, y, xo, (size_t)n * sizeof(float));
+    st = ag_copy_out(g->dev, y, xo, nb, nb);
     return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
@@ -516,7 +518,8 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     uint64_t *xd = (uint64_t *)g->vec_b;
     uint64_t *yd = (uint64_t *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    st = ag_copy_in(g->dev, xo, xq, (size_t)n * sizeof(uint64_t));
+    const size_t nb = (size_t)n * sizeof(uint64_t);
+    st = ag_copy_in(g->dev, xo, xq, nb, nb);
     if (st != AG_OK)
         return st;
     permute_in_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
@@ -530,7 +533,7 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
     AG_HIP(hipGetLastError());
-    st = ag_copy_out(g->dev, yq, xo, (size_t)n * sizeof(uint64_t));
+    st = ag_copy_out(g->dev, yq, xo, nb, nb);
     return st == AG_OK ? timed_ms(g, reps, avg_ms) : st;
 }
 
@@ -547,7 +550,8 @@ static int gather_typed(ag_dgraph *g, const void *values, void *out)
     VT *vd = (VT *)g->vec_b;
     A *ad = (A *)((char *)g->vec_b + (size_t)n * sizeof(uint64_t));
     const uint32_t blk = (n + AG_WG - 1) / AG_WG;
-    st = ag_copy_in(g->dev, vo, values, (size_t)n * sizeof(VT));
+    const size_t ob = (size_t)n * sizeof(A);   // no smaller than the values
+    st = ag_copy_in(g->dev, vo, values, (size_t)n * sizeof(VT), ob);
     if (st != AG_OK)
         return st;
     permute_in_kernel<VT><<<blk, AG_WG, 0, stream>>>(n, vo, g->d2o, vd);
@@ -557,7 +561,7 @@ static int gather_typed(ag_dgraph *g, const void *values, void *out)
         return st;
     permute_out_kernel<A><<<blk, AG_WG, 0, stream>>>(n, ad, g->d2o, ao);
     AG_HIP(hipGetLastError());
-    return ag_copy_out(g->dev, out, ao, (size_t)n * sizeof(A));
+    return ag_copy_out(g->dev, out, ao, ob, ob);
 }
 
 extern "C" int ag_pull_gather(ag_dgraph *g, uint32_t type, const void *values, void *out)

@@ -288,6 +288,29 @@ def test_staged_transfers(device, n):
     dg.close()
 
 
+@pytest.mark.parametrize("kb", [16, 1024])
+@pytest.mark.parametrize("more", [-1, 0, 1])
+def test_transfers_at_the_ring_sizes(device, kb, more):
+    """Vectors at the sizes where a result leaves the pinned ring (16 KB) and where both ways take it
+    (1 MB), of 4- and 8-byte values and of both at once, the ways taking turns."""
+    for width in (4, 8):
+        n = kb * 1024 // width + more
+        chain = np.arange(n - 1, dtype=np.uint32)
+        dg = device.upload(ag.Graph.from_edges(chain, chain + 1, n=n))
+        rng = np.random.default_rng(n)
+        for _ in range(2):
+            v = rng.random(n, dtype=np.float32)
+            want = np.concatenate([np.zeros(1, np.float32), v[:-1]])
+            np.testing.assert_array_equal(dg.gather(v, ag.GATHER_F32), want)
+            u = rng.integers(0, 1 << 32, n, dtype=np.uint32)
+            np.testing.assert_array_equal(dg.gather(u, ag.GATHER_U32),
+                                          np.concatenate([[0], u[:-1]]).astype(np.uint64))
+            q = rng.integers(0, 1 << 62, n, dtype=np.uint64)
+            np.testing.assert_array_equal(dg.gather(q, ag.GATHER_U64),
+                                          np.concatenate([np.zeros(1, np.uint64), q[:-1]]))
+        dg.close()
+
+
 def test_sessions_reuse_parked_buffers(device):
     """Sessions of different kinds, lengths and overlapping lifetimes on one graph take the buffers
     that earlier ones left: the results are those of a fresh graph."""

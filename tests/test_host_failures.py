@@ -138,3 +138,16 @@ def test_history_moves_executed_rows(fake_hip, max_iterations):
     assert rows.value == 5 and list(act) == [5] * 5
     assert fake.fake_copied() <= 66000
     """)
+
+
+def test_small_vectors_go_straight(fake_hip):
+    """A SpMV on a small graph moves its two vectors in a copy each and allocates no pinned ring."""
+    run(fake_hip, """
+    dg = dev.upload(ag.Graph.rmat(14))
+    fake.fake_fail_host_in(0)
+    x = np.ones(dg.n, np.float32)
+    dg.spmv(x)
+    before = fake.fake_copies()
+    dg.spmv(x)
+    assert fake.fake_copies() - before == 2
+    """)
