@@ -252,24 +252,28 @@ hipError_t ag_dev_malloc_bytes(ag_device *dev, void **p, size_t bytes)
 #define AG_STRAIGHT_BELOW ((size_t)1 << 20)
 #define AG_PINNED_OUT ((size_t)16 << 10)
 
-static int stage_open(ag_device *d)
+// Whether the device has its ring, allocated on first use. Without pinned memory for it transfers
+// go straight.
+static bool stage_open(ag_device *d)
 {
     if (d->stage)
-        return AG_OK;
+        return true;
     char *p = NULL;
-    AG_HIP(hipHostMalloc((void **)&p, AG_STAGE_SLOTS * AG_STAGE_BYTES, hipHostMallocDefault));
-    for (uint32_t i = 0; i < AG_STAGE_SLOTS; i++) {
-        const hipError_t e = hipEventCreateWithFlags(&d->stage_ev[i], hipEventDisableTiming);
-        if (e != hipSuccess) {
-            while (i-- > 0)
-                (void)hipEventDestroy(d->stage_ev[i]);
+    hipError_t e = hipHostMalloc((void **)&p, AG_STAGE_SLOTS * AG_STAGE_BYTES, hipHostMallocDefault);
+    uint32_t i = 0;
+    for (; e == hipSuccess && i < AG_STAGE_SLOTS; i++)
+        e = hipEventCreateWithFlags(&d->stage_ev[i], hipEventDisableTiming);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // no later launch reports it
+        for (uint32_t k = 0; k + 1u < i; k++)   // the last one is the one that failed
+            (void)hipEventDestroy(d->stage_ev[k]);
+        if (p)
             (void)hipHostFree(p);
-            return ag_hip_fail(e, "hipEventCreate", __FILE__, __LINE__);
-        }
+        return false;
     }
     d->stage = p;
     d->stage_used = d->stage_next = 0u;
-    return AG_OK;
+    return true;
 }
 
 // Whether the runtime knows this memory (pinned, managed or a GPU's): it then copies it straight.
@@ -295,11 +299,11 @@ int ag_copy_in(ag_device *d, void *dst, const void *host, size_t bytes, size_t l
 {
     if (bytes == 0)
         return AG_OK;
-    if (largest < AG_STRAIGHT_BELOW || is_known(host)) {
+    if (largest < AG_STRAIGHT_BELOW || is_known(host) || !stage_open(d)) {
         AG_HIP(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, d->stream));
         return AG_OK;
     }
-    int st = stage_open(d);
+    int st = AG_OK;
     for (size_t o = 0; st == AG_OK && o < bytes; o += AG_STAGE_BYTES) {
         const size_t len = bytes - o < AG_STAGE_BYTES ? bytes - o : AG_STAGE_BYTES;
         uint32_t k = 0;
@@ -319,11 +323,12 @@ int ag_copy_out(ag_device *d, void *host, const void *src, size_t bytes, size_t 
 {
     if (bytes == 0)
         return AG_OK;
-    if ((largest < AG_STRAIGHT_BELOW && bytes > AG_PINNED_OUT) || is_known(host)) {
+    if ((largest < AG_STRAIGHT_BELOW && bytes > AG_PINNED_OUT) || is_known(host) ||
+        !stage_open(d)) {
         AG_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, d->stream));
         return ag_wait_stream(d);
     }
-    int st = stage_open(d);
+    int st = AG_OK;
     const size_t chunks = (bytes + AG_STAGE_BYTES - 1) / AG_STAGE_BYTES;
     uint32_t slot[AG_STAGE_SLOTS];
     size_t sent = 0;

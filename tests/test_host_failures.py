@@ -151,3 +151,20 @@ def test_small_vectors_go_straight(fake_hip):
     dg.spmv(x)
     assert fake.fake_copies() - before == 2
     """)
+
+
+@pytest.mark.parametrize("scale", [6, 19])
+def test_transfers_without_a_ring(fake_hip, scale):
+    """Without pinned memory for the ring the transfers that use it, tiny results and large vectors,
+    go straight; the ring is made once there is memory again."""
+    run(fake_hip, f"""
+    dg = dev.upload(ag.Graph.rmat({scale}, 2))
+    x = np.ones(dg.n, np.float32)
+    for n in (0, -1, -1):
+        fake.fake_fail_host_in(n)
+        assert status(lambda: dg.spmv(x)) == 0
+    s = dg.session(max_iterations=3)
+    s.step(1)
+    fake.fake_fail_host_in(0)
+    s.end()
+    """)
