@@ -532,13 +532,26 @@ struct ag_ppr_ws {
     PrState *st_host;          // pinned [2]
     PprConf *conf_host;        // pinned
     uint32_t *o2d;             // [n] host: device row of every vertex
-    hipGraph_t graph;
-    hipGraphExec_t exec;
-    uint32_t exec_grid;        // its iteration-kernel grid
-    uint32_t exec_width;       // and columns per vertex
+    // the captured iterations of each column width, kept so that calls of different widths can
+    // take turns
+    struct {
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+        uint32_t grid;         // its iteration-kernel grid
+    } cap[3];
     uint32_t width;            // columns per vertex of this call: 16, 32 or 64
     hipEvent_t ev[2];          // the state copies after the last two replays
 };
+
+static void ppr_drop_capture(ag_ppr_ws *w, uint32_t i)
+{
+    if (w->cap[i].exec)
+        (void)hipGraphExecDestroy(w->cap[i].exec);
+    if (w->cap[i].graph)
+        (void)hipGraphDestroy(w->cap[i].graph);
+    w->cap[i].exec = NULL;
+    w->cap[i].graph = NULL;
+}
 
 void ag_ppr_free_ws(ag_dgraph *g)
 {
@@ -546,10 +559,8 @@ void ag_ppr_free_ws(ag_dgraph *g)
     if (!w)
         return;
     (void)hipStreamSynchronize(g->dev->stream);
-    if (w->exec)
-        (void)hipGraphExecDestroy(w->exec);
-    if (w->graph)
-        (void)hipGraphDestroy(w->graph);
+    for (uint32_t i = 0; i < 3u; i++)
+        ppr_drop_capture(w, i);
     void *ptrs[] = {w->c16[0], w->c16[1], w->c32[0], w->c32[1], w->rank, w->hub_part, w->part,
                     w->colerr, w->hist, w->st, w->conf};
     for (void *p : ptrs)
@@ -601,7 +612,7 @@ static int ppr_allocate(ag_dgraph *g, ag_ppr_ws *w)
 }
 
 // Allocates the workspace on first use (whole, or none); grows the history (dropping the captured
-// solve) when a call asks for more iterations than it holds.
+// iterations) when a call asks for more iterations than it holds.
 static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
 {
     ag_ppr_ws *w = g->ppr;
@@ -617,12 +628,8 @@ static int ppr_workspace(ag_dgraph *g, uint32_t maxit, ag_ppr_ws **out)
         }
     }
     if (w->hist_cap < maxit) {
-        if (w->exec) {
-            (void)hipGraphExecDestroy(w->exec);
-            (void)hipGraphDestroy(w->graph);
-            w->exec = NULL;
-            w->graph = NULL;
-        }
+        for (uint32_t i = 0; i < 3u; i++)
+            ppr_drop_capture(w, i);
         if (w->hist)
             AG_HIP(hipFree(w->hist));
         w->hist = NULL;
@@ -787,29 +794,23 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
     if (e == hipSuccess)
         e = hipEventRecord(e0, s);
     if (e == hipSuccess && o.use_hip_graph && maxit >= PPR_REPLAY) {
-        if (w->exec && (w->exec_grid != w->grid || w->exec_width != w->width)) {
-            (void)hipGraphExecDestroy(w->exec);
-            (void)hipGraphDestroy(w->graph);
-            w->exec = NULL;
-            w->graph = NULL;
-        }
-        if (!w->exec) {
+        const uint32_t ci = w->width == 16u ? 0u : w->width == 32u ? 1u : 2u;
+        auto &cap = w->cap[ci];
+        if (cap.exec && cap.grid != w->grid)
+            ppr_drop_capture(w, ci);
+        if (!cap.exec) {
             e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
                 const hipError_t qe = ppr_enqueue_iterations(g, w, A, PPR_REPLAY, s);
-                const hipError_t ce = hipStreamEndCapture(s, &w->graph);
+                const hipError_t ce = hipStreamEndCapture(s, &cap.graph);
                 e = qe != hipSuccess ? qe : ce;
-                if (qe != hipSuccess && ce == hipSuccess) {
-                    (void)hipGraphDestroy(w->graph);
-                    w->graph = NULL;
-                }
             }
             if (e == hipSuccess)
-                e = hipGraphInstantiate(&w->exec, w->graph, NULL, NULL, 0);
-            if (e == hipSuccess) {
-                w->exec_grid = w->grid;
-                w->exec_width = w->width;
-            }
+                e = hipGraphInstantiate(&cap.exec, cap.graph, NULL, NULL, 0);
+            if (e == hipSuccess)
+                cap.grid = w->grid;
+            else
+                ppr_drop_capture(w, ci);
         }
         if (e == hipSuccess)
             e = ppr_enqueue_init(g, w, A, s);
@@ -820,7 +821,7 @@ extern "C" int ag_ppr_pull(ag_dgraph *g, uint32_t k, const uint32_t *seeds,
         for (uint32_t r = 0; e == hipSuccess && st == AG_OK && !stopped && done < maxit; r++) {
             const uint32_t left = maxit - done;
             if (left >= PPR_REPLAY)
-                e = hipGraphLaunch(w->exec, s);
+                e = hipGraphLaunch(cap.exec, s);
             else
                 e = ppr_enqueue_iterations(g, w, A, left, s);
             done += left < PPR_REPLAY ? left : PPR_REPLAY;

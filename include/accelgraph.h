@@ -336,8 +336,9 @@ int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *x_q, uint64_t *y_q, uint32_
  * id; AG_PPR_UNIFORM restarts uniformly, which is plain PageRank). Scaled units as the plain
  * path: the restart mass is (1 - Damp) * N, all of it on the seed; every column starts at 1.0.
  * Contributions are stored vertex-major, 16, 32 or 64 per vertex (the least that holds k columns;
- * 64: one 128-byte line in BF16/FP16), and accumulated in FP32; with 16-bit storage the last iterations switch to FP32 contributions
- * (refine_l1, as for ag_pr_options). The L1 delta of each column is reduced in FP64. */
+ * 64: one 128-byte line in BF16/FP16), and accumulated in FP32; with 16-bit storage the last
+ * iterations switch to FP32 contributions (refine_l1, as for ag_pr_options). The L1 delta of each
+ * column is reduced in FP64. */
 #define AG_PPR_MAX_COLS 64
 #define AG_PPR_UNIFORM 0xFFFFFFFFu
 

@@ -168,3 +168,18 @@ def test_transfers_without_a_ring(fake_hip, scale):
     fake.fake_fail_host_in(0)
     s.end()
     """)
+
+
+def test_ppr_widths_take_turns(fake_hip):
+    """Calls that alternate between 1, 20 and 64 columns capture each width's iterations once."""
+    run(fake_hip, """
+    dg = dev.upload(ag.Graph.rmat(7))
+    for _ in range(3):
+        for k in (1, 64, 20):
+            dg.ppr(np.arange(k, dtype=np.uint32), max_iterations=40)
+    assert fake.fake_captures() == 3
+    dg.ppr(np.arange(5, dtype=np.uint32), max_iterations=40, wg_per_cu=1)     # another grid
+    dg.ppr(np.arange(5, dtype=np.uint32), max_iterations=600)                 # a longer history
+    dg.close()
+    assert fake.fake_live() == 0
+    """)
