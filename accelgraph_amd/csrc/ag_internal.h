@@ -169,7 +169,8 @@ uint32_t ag_tile_grid(const ag_dgraph *g, uint32_t lds_bytes);
 // Device-side iteration state of a PageRank session.
 struct PrState {
     uint32_t iter;          // iterations executed so far
-    uint32_t done;          // set by the last block of the stopping iteration
+    uint32_t done;          // set when the stopping iteration is closed (the next launch's opening
+                            // step, or the closing kernel at a step's end)
     uint32_t stop_iter;     // index of the stopping iteration
     int32_t refine_iter;    // first iteration that writes f32 contributions (-1: none yet)
     uint32_t last_active;

@@ -941,8 +941,9 @@ __global__ __launch_bounds__(AG_WG) void pr_ddf_cmb_kernel(BlockGeom B, PrCtl C,
 // takes one instruction per in-edge (16-lane rows: a DPP broadcast folded into the add; 64-lane
 // rows: a lane read and an add; a workgroup's rows: LDS values, staged by all its lanes).
 // Bound by those chains and the gathers. RMAT-19 (8 M in-edges): 67 us an iteration, where
-// the worklists took 370 (nearly every vertex stays listed until the end of a run, so marking
-// the out-neighbours, 16 lanes along a hub's 30 K out-edges, cost more than it saved).
+// the worklists took 370 (on RMAT graphs the listed vertices hold nearly all in-edges until the end
+// of a run, and marking the out-neighbours, 16 lanes along a hub's 30 K out-edges, cost more than
+// the rest saved).
 
 // rows up to this in-degree are summed in edge order; longer rows in a lane-strided tree
 #define AG_DD_SEQ_MAX 8192u
@@ -1660,8 +1661,13 @@ extern "C" int ag_pr_begin(ag_dgraph *g, const ag_pr_options *opts, ag_pr_sessio
     // contribution is >= +0, i.e. from a start vector without negative entries, -0 or NaN
     // (ranks stay positive from there); other user starts keep explicit worklists. So do all
     // user starts on unblocked plans: a restart from nearly converged ranks lists few vertices
-    // after its first iteration, which an iteration over every row cannot use (from the
-    // built-in starts nearly every vertex stays listed until the end of the run).
+    // after its first iteration, which an iteration over every row cannot use. From the built-in
+    // starts an iteration over every row is the faster one also where the lists shorten early,
+    // since four launches and the marks cost a listed vertex more than it costs here. A call to
+    // epsilon 1e-4, full pull / worklists (ms): RMAT-16 3.3 / 35.5, RMAT-20 11.9 / 57.9,
+    // Erdos-Renyi 1 M vertices 5.5 / 10.5, grids with a third of the edges removed (active
+    // vertices 52 to 60% on average) of 490 K 1.4 / 4.3 and 1.96 M 3.2 / 11.4, a binary tree of
+    // 1 M 0.5 / 1.5, a chain of 1 M 0.9 / 5.5.
     bool dd_lists = o.direction == AG_DIR_DATA_DRIVEN && g->blk.bits == 0 &&
                     o.init == AG_INIT_USER;
     if (o.direction == AG_DIR_DATA_DRIVEN && !dd_lists && o.init == AG_INIT_USER &&

@@ -1,4 +1,4 @@
-// ag_ppr.hip -- 64-column personalised PageRank pull.
+// ag_ppr.hip -- personalised PageRank pull of up to 64 columns.
 //
 // The plain iteration of pageRank.c:942-1109 applied to up to 64 rank vectors at once, each with
 // its own restart vector. Contributions are stored vertex-major, W = 16, 32 or 64 per vertex, so
@@ -9,8 +9,8 @@
 // THREAD and GROUP16 rows take one group each, WAVE rows a wavefront, BLOCK rows a whole
 // workgroup, HUB rows fixed segments whose partials a one-workgroup finish kernel adds in segment
 // order. The per-column L1 delta is reduced in FP64 in a fixed order; the run stops when every
-// column is below the tolerance. A run of iterations is captured once into a hipGraph and
-// replayed until the run stops.
+// column is below the tolerance. A run of iterations is captured once per column width into a
+// hipGraph and replayed until the solve stops.
 #include <stdlib.h>
 #include <string.h>
 #include <time.h>
