@@ -214,14 +214,15 @@ struct Gather {
 
 } // namespace
 
-// Launches of one pull policy `reps` times between the device's two timing events (read by
-// timed_ms once the call has waited).
+// Launches of one pull policy `reps` times, where `timed` between the device's two timing events
+// (read by timed_ms once the call has waited).
 template <class P>
-static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps)
+static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps, bool timed)
 {
     hipStream_t stream = g->dev->stream;
     PullGeom G = ag_make_geom(g);
-    AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
+    if (timed)
+        AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
     const uint32_t grid = ag_tile_grid(g, AG_TILE_NNZ_MAX * (uint32_t)sizeof(typename P::Acc));
     for (uint32_t i = 0; i < reps && g->total_blocks; i++) {
         pull_kernel<P><<<grid, AG_WG, 0, stream>>>(G, pol);
@@ -229,7 +230,8 @@ static int run_pull(ag_dgraph *g, const P &pol, uint32_t reps)
             pull_finish_kernel<P><<<1, AG_FIN_WG, 0, stream>>>(G, pol);
     }
     AG_HIP(hipGetLastError());
-    AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
+    if (timed)
+        AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
     return AG_OK;
 }
 
@@ -266,7 +268,7 @@ static bool spmv_hot_launch(const ag_dgraph *g, const BlockGeom &B,
 // regular order (unblocked rows); the hot pass (FP32), pass 1 then the combine pass per
 // repetition.
 template <class P>
-static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps)
+static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps, bool timed)
 {
     hipStream_t stream = g->dev->stream;
     const PullGeom U = ag_make_unblocked_geom(g);
@@ -275,7 +277,8 @@ static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t rep
     static const uint32_t res1 = ag_resident_per_cu(pull_blocked_kernel<P, P>);
     static const uint32_t res2 = ag_resident_per_cu(pull_combine_kernel<P>);
     const uint32_t g1 = ag_blocked_grid(g, res1, 4u), g2 = ag_blocked_grid(g, res2, 8u);
-    AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
+    if (timed)
+        AG_HIP(hipEventRecord(g->dev->time_ev[0], stream));
     for (uint32_t i = 0; i < reps; i++) {
         if (spmv_hot_launch(g, B, pv, stream))
             ag_block_geom_skip_hot(g, B1);
@@ -283,7 +286,8 @@ static int run_pull_blocked(ag_dgraph *g, const P &pv, const P &pu, uint32_t rep
         pull_combine_kernel<P><<<g2, AG_WG, 0, stream>>>(B, pu);
     }
     AG_HIP(hipGetLastError());
-    AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
+    if (timed)
+        AG_HIP(hipEventRecord(g->dev->time_ev[1], stream));
     return AG_OK;
 }
 
@@ -309,14 +313,14 @@ static int spmv_f32_device(ag_dgraph *g, const float *x, float *y, float *xo, fl
     AG_HIP(hipGetLastError());
     if (g->blk.bits && g->w)
         st = run_pull_blocked(g, SpmvF32Pol<true>{xd, g->blk.vw, yd},
-                              SpmvF32Pol<true>{xd, g->w, yd}, reps);
+                              SpmvF32Pol<true>{xd, g->w, yd}, reps, avg_ms != NULL);
     else if (g->blk.bits)
         st = run_pull_blocked(g, SpmvF32Pol<false>{xd, NULL, yd}, SpmvF32Pol<false>{xd, NULL, yd},
-                              reps);
+                              reps, avg_ms != NULL);
     else if (g->w)
-        st = run_pull(g, SpmvF32Pol<true>{xd, g->w, yd}, reps);
+        st = run_pull(g, SpmvF32Pol<true>{xd, g->w, yd}, reps, avg_ms != NULL);
     else
-        st = run_pull(g, SpmvF32Pol<false>{xd, NULL, yd}, reps);
+        st = run_pull(g, SpmvF32Pol<false>{xd, NULL, yd}, reps, avg_ms != NULL);
     if (st != AG_OK)
         return st;
     float *yo = (yd == xo) ? xd : xo;   // y in original order
@@ -433,14 +437,14 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
     const uint32_t wc = host_fixed32(0.0001f);
     if (blocked && g->wq)
         st = run_pull_blocked(g, SpmvFixPol<true>{xd, g->vwq, 0u, yd},
-                              SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps);
+                              SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps, avg_ms != NULL);
     else if (blocked)
         st = run_pull_blocked(g, SpmvFixPol<false>{xd, NULL, wc, yd},
-                              SpmvFixPol<false>{xd, NULL, wc, yd}, reps);
+                              SpmvFixPol<false>{xd, NULL, wc, yd}, reps, avg_ms != NULL);
     else if (g->wq)
-        st = run_pull(g, SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps);
+        st = run_pull(g, SpmvFixPol<true>{xd, g->wq, 0u, yd}, reps, avg_ms != NULL);
     else
-        st = run_pull(g, SpmvFixPol<false>{xd, NULL, wc, yd}, reps);
+        st = run_pull(g, SpmvFixPol<false>{xd, NULL, wc, yd}, reps, avg_ms != NULL);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, yo);
@@ -452,15 +456,14 @@ extern "C" int ag_spmv_pull_fixed(ag_dgraph *g, const uint32_t *xq, uint64_t *yq
 // Clears y and runs `reps` accumulating passes: pv reads per-edge data in virtual-row order, pu
 // in regular order.
 template <class P>
-static int run_push(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps)
+static int run_push(ag_dgraph *g, const P &pv, const P &pu, uint32_t reps, bool timed)
 {
     const uint32_t words = (uint32_t)(sizeof(*pu.y) / 4u) * g->n;
     const uint32_t zb = (words + AG_WG - 1) / AG_WG;
     zero_u32_kernel<<<zb < 4096u ? zb : 4096u, AG_WG, 0, g->dev->stream>>>((uint32_t *)pu.y,
                                                                            words);
     AG_HIP(hipGetLastError());
-    return g->blk.bits ? run_pull_blocked(g, pv, pu, reps)
-                       : run_pull(g, pu, reps);
+    return g->blk.bits ? run_pull_blocked(g, pv, pu, reps, timed) : run_pull(g, pu, reps, timed);
 }
 
 extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t reps, double *avg_ms)
@@ -488,9 +491,9 @@ extern "C" int ag_spmv_push(ag_dgraph *g, const float *x, float *y, uint32_t rep
     permute_in_kernel<float><<<blk, AG_WG, 0, stream>>>(n, xo, g->d2o, xd);
     AG_HIP(hipGetLastError());
     st = g->w ? run_push(g, SpmvPushPol<true>{{yd}, {}, {xd, g->blk.vw, NULL}},
-                         SpmvPushPol<true>{{yd}, {}, {xd, g->w, NULL}}, reps)
+                         SpmvPushPol<true>{{yd}, {}, {xd, g->w, NULL}}, reps, avg_ms != NULL)
               : run_push(g, SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}},
-                         SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}}, reps);
+                         SpmvPushPol<false>{{yd}, {}, {xd, NULL, NULL}}, reps, avg_ms != NULL);
     if (st != AG_OK)
         return st;
     permute_out_kernel<float><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
@@ -526,9 +529,9 @@ extern "C" int ag_spmv_push_fixed(ag_dgraph *g, const uint64_t *xq, uint64_t *yq
     AG_HIP(hipGetLastError());
     const uint64_t wc = DoubleToFixed64((double)0.0001f);   // SPMV.c:1080
     st = g->w ? run_push(g, SpmvPushFixPol<true>{{yd}, {}, xd, g->blk.vw, 0u},
-                         SpmvPushFixPol<true>{{yd}, {}, xd, g->w, 0u}, reps)
+                         SpmvPushFixPol<true>{{yd}, {}, xd, g->w, 0u}, reps, avg_ms != NULL)
               : run_push(g, SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc},
-                         SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc}, reps);
+                         SpmvPushFixPol<false>{{yd}, {}, xd, NULL, wc}, reps, avg_ms != NULL);
     if (st != AG_OK)
         return st;
     permute_out_kernel<uint64_t><<<blk, AG_WG, 0, stream>>>(n, yd, g->d2o, xo);
@@ -556,7 +559,7 @@ static int gather_typed(ag_dgraph *g, const void *values, void *out)
         return st;
     permute_in_kernel<VT><<<blk, AG_WG, 0, stream>>>(n, vo, g->d2o, vd);
     AG_HIP(hipGetLastError());
-    st = run_pull(g, Gather<VT, A>{vd, ad}, 1);
+    st = run_pull(g, Gather<VT, A>{vd, ad}, 1, false);
     if (st != AG_OK)
         return st;
     permute_out_kernel<A><<<blk, AG_WG, 0, stream>>>(n, ad, g->d2o, ao);
