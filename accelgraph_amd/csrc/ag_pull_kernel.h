@@ -844,17 +844,30 @@ static_assert(AG_TILE_NNZ_MAX <= AG_TILE_UNROLL * AG_WG,
               "a lane holds all of its ids of a sorted tile at once");
 
 // The packed ids and per-edge data of a sorted tile, AG_TILE_UNROLL per lane: the whole tile.
+// Predicated loads where sums have 4 bytes. Where they have 8 (the integer kinds and the
+// data-driven pull) the compiler made the kernels wait for each of the first three of those before
+// the next, so there lanes past the tile read its first id, which nothing uses (an item without
+// ids: the array's first), and the loads need no branch. RMAT-25 iteration, predicated / not:
+// fixed 64 and 32 3.15 / 3.05 and 2.64 / 2.51 ms, quantised 16 and 8 2.52 / 2.36 and 2.35 / 2.18,
+// data-driven 2.73 / 2.59, but FP32 2.274 / 2.303.
 template <class P>
 __device__ __forceinline__ void load_sorted_ids(const uint32_t *vsp, const P &pol,
                                                 const SortedTile &t,
                                                 uint32_t (&w)[AG_TILE_UNROLL],
                                                 typename EdgeOf<P>::T (&ed)[AG_TILE_UNROLL])
 {
+    const uint32_t e0 = t.nnz ? t.e0 : 0u;
 #pragma unroll
     for (int u = 0; u < AG_TILE_UNROLL; u++) {
         const uint32_t kk = threadIdx.x + u * AG_WG;
-        w[u] = kk < t.nnz ? ld_stream(&vsp[t.e0 + kk]) : 0u;
-        ed[u] = kk < t.nnz ? EdgeOf<P>::load(pol, t.e0 + kk) : typename EdgeOf<P>::T{};
+        if constexpr (sizeof(typename P::Acc) > 4u) {
+            const uint32_t j = e0 + (kk < t.nnz ? kk : 0u);
+            w[u] = ld_stream(&vsp[j]);
+            ed[u] = EdgeOf<P>::load(pol, j);
+        } else {
+            w[u] = kk < t.nnz ? ld_stream(&vsp[t.e0 + kk]) : 0u;
+            ed[u] = kk < t.nnz ? EdgeOf<P>::load(pol, t.e0 + kk) : typename EdgeOf<P>::T{};
+        }
     }
 }
 
