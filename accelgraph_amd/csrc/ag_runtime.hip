@@ -13,7 +13,6 @@
 #include <time.h>
 #include <unistd.h>
 
-#include <algorithm>
 #include <new>
 #include <vector>
 
@@ -527,12 +526,41 @@ uint32_t ag_tile_grid(const ag_dgraph *g, uint32_t lds_bytes)
     return grid < items ? grid : items;
 }
 
+// The largest e in (r, last] with off[e] <= lim, r + 1 if there is none: searched outwards from
+// r + guess, the rows of the tile before (rows are ordered by degree class).
+static uint32_t tile_end(const uint32_t *off, uint32_t r, uint32_t last, uint64_t lim,
+                         uint32_t guess)
+{
+    if (off[last] <= lim)
+        return last;
+    uint32_t lo = r, hi = last, step = 4u;   // off[lo] <= lim < off[hi]
+    const uint32_t p = guess < last - r ? r + guess : r;
+    if (p > r && off[p] <= lim) {
+        for (lo = p; hi - lo > step && off[lo + step] <= lim; step *= 2u)
+            lo += step;
+        hi = hi - lo > step ? lo + step : hi;
+    } else if (p > r) {
+        for (hi = p; hi - lo > step && off[hi - step] > lim; step *= 2u)
+            hi -= step;
+        lo = hi - lo > step ? hi - step : lo;
+    }
+    while (hi - lo > 1u) {
+        const uint32_t mid = lo + (hi - lo) / 2u;
+        if (off[mid] <= lim)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo > r ? lo : r + 1u;
+}
+
 // Cuts the rows of the bins whose rows fit a tile into row tiles. A tile holds
 // at most `nnz` in-edges (one row may hold more, up to AG_TILE_NNZ_MAX) and `rows` rows: as few
 // as let the resident workgroups finish in as many rounds as full tiles would need, so that
 // small graphs still give every CU work (RMAT-12: 256 in-edges a tile) and the last round is
-// not nearly empty.
-static int cut_row_tiles(ag_dgraph *g, const uint32_t *off, std::vector<uint4> &rt)
+// not nearly empty. Source-blocked plans, whose sums by the regular schedule are few, take full
+// tiles at once. On the host: RMAT-22 2 ms (5 with a search of every tile's whole range).
+static int cut_row_tiles(ag_dgraph *g, const uint32_t *off, bool blocked, std::vector<uint4> &rt)
 {
     const ag_plan_params &q = g->params;
     // bins are ordered by degree: the first bin whose rows may exceed a tile ends the tiles
@@ -548,21 +576,20 @@ static int cut_row_tiles(ag_dgraph *g, const uint32_t *off, std::vector<uint4> &
     const uint64_t rounds = (items + slots - 1) / slots;
     try {
         const uint64_t budget = slots * rounds, room = budget - g->n_heavy;
-        uint64_t nnz = (m1 + room - 1u) / room;   // items covers n_heavy: room > 0
+        // items covers n_heavy: room > 0
+        uint64_t nnz = blocked ? q.tile_nnz : (m1 + room - 1u) / room;
         for (nnz = nnz < AG_WG ? AG_WG : nnz;; nnz += nnz / 8u) {
             nnz = nnz < q.tile_nnz ? nnz : q.tile_nnz;
             const uint32_t rows = q.tile_rows < nnz ? q.tile_rows
                                                     : nnz < AG_WG ? AG_WG : (uint32_t)nnz;
             const bool last_try = nnz == q.tile_nnz;
             rt.clear();
-            uint32_t r = 0;
+            uint32_t r = 0, guess = 0;
             while (r < row1 && (last_try || rt.size() + g->n_heavy < budget)) {
                 const uint32_t last = row1 - r < rows ? row1 : r + rows;
-                // the last row end within nnz in-edges (off is their prefix sum), a row at least
-                const uint64_t lim = (uint64_t)off[r] + nnz;
-                uint32_t e = (uint32_t)(std::upper_bound(off + r + 1, off + last + 1, lim) - off);
-                e = e - 1u > r ? e - 1u : r + 1u;
+                const uint32_t e = tile_end(off, r, last, (uint64_t)off[r] + nnz, guess);
                 rt.push_back(make_uint4(r, e, off[r], off[e]));
+                guess = e - r;
                 r = e;
             }
             if (r >= row1)
@@ -644,7 +671,7 @@ extern "C" int ag_graph_upload(ag_device *dev, uint32_t n, uint32_t m, const uin
     if (st == AG_OK) st = dev_upload(g, &g->outdeg, plan.outdeg, plan.n);
     if (st == AG_OK) st = dev_upload(g, &g->tile_row, plan.tile_row, (size_t)plan.n_tiles + 1);
     std::vector<uint4> rt;   // outlives its copy: freed after the wait below
-    if (st == AG_OK) st = cut_row_tiles(g, plan.off, rt);
+    if (st == AG_OK) st = cut_row_tiles(g, plan.off, plan.blk.bits != 0u, rt);
     if (st == AG_OK) st = dev_upload(g, &g->rt, rt.data(), rt.size());
     if (st == AG_OK) st = dev_upload(g, &g->seg_row, plan.seg_row, plan.n_segs);
     if (st == AG_OK) st = dev_upload(g, &g->seg_lo, plan.seg_lo, plan.n_segs);
