@@ -391,9 +391,10 @@ struct TopTab {
 // in flight while the values arrive: a tile costs one dependent round of loads.
 // A group of lanes per row, four gathers in flight each and a chain of four dependent loads a
 // row (offsets, ids, values, update operands), left the chip waiting. A SpMV before -> with row
-// tiles: RMAT-16 7.9 -> 7.6 us, RMAT-18 27.8 -> 22.2, RMAT-20 99 -> 82 (0.2 T in-edges/s, the rate
-// of the blocked pass 1), Erdos-Renyi 300 K rows of 16 in-edges 29.2 -> 25.3, of 40 64.5 -> 56.4.
-// lane_tree against a chain of additions takes 0.3 to 0.7 us of these (RMAT-20 1.5).
+// tiles: RMAT-16 7.9 -> 7.1 us, RMAT-18 27.4 -> 21.6, RMAT-20 98 -> 81.6 (0.2 T in-edges/s from
+// 0.146 T L2 requests/s; the blocked pass 1 makes 0.19), Erdos-Renyi 300 K rows of 16 in-edges
+// 29.3 -> 24.9, of 40 64.4 -> 55.5. A product on a few hundred rows takes longer, 2.6 -> 3.5 us (3
+// rows): the unrolled rounds of loads are there to fetch whether a tile fills them or not.
 
 struct RowTile {
     uint32_t r0, r1, e0, e1;
@@ -401,14 +402,14 @@ struct RowTile {
 
 template <class P>
 struct TileLds {
-    typename P::Acc *vals;                     // [AG_TILE_NNZ_MAX]
+    typename P::Acc *vals;                     // [AG_TILE_NNZ_MAX + AG_LANE_MAX] (lane_tree)
     typename P::Acc *lsum;                     // [AG_LONG_MAX] sums of the long rows
     uint32_t *lng;                             // [AG_WG / AG_WAVE][AG_LONG_MAX] each wavefront's
     uint32_t *cnt;                             // [AG_WG / AG_WAVE]
 };
 
 #define AG_TILE_LDS(P, T)                                             \
-    __shared__ typename P::Acc T##_vals[AG_TILE_NNZ_MAX];             \
+    __shared__ typename P::Acc T##_vals[AG_TILE_NNZ_MAX + AG_LANE_MAX]; \
     __shared__ typename P::Acc T##_lsum[AG_LONG_MAX];                 \
     __shared__ uint32_t T##_lng[AG_WG / AG_WAVE * AG_LONG_MAX];       \
     __shared__ uint32_t T##_cnt[AG_WG / AG_WAVE];                     \
@@ -444,38 +445,75 @@ __device__ __forceinline__ Acc lane_sum(const Acc *s_vals, uint32_t b, uint32_t 
     return acc;
 }
 
-// A row's values v[0, d), d <= 64, by one lane. FP32: the order of a group of 16 lanes that take
+// An FP32 row's values v[0, d), d <= 64, by one lane, in the order of a group of 16 lanes that take
 // the values in turn with four accumulators each and combine in a tree (6 additions a value at
-// most, against d - 1 in a chain: 1.7 to 2.7 times less rms error for 20 to 64 equal terms), every
-// value in flight at once. Integer sums are exact in any order.
-template <typename Acc>
-__device__ __forceinline__ Acc lane_tree(const Acc *v, uint32_t d)
+// most, against d - 1 in a chain: 1.7 to 2.7 times less rms error for 20 to 64 equal terms). Every
+// value is read, the ones past the row (the tile's LDS has room for them) dropped: with a branch a
+// value the sum took 0.5 us a tile more.
+__device__ __forceinline__ float lane_tree(const float *v, uint32_t d)
 {
-    if constexpr (!std::is_floating_point_v<Acc>) {
-        return lane_sum(v, 0u, d);
-    } else {
-        static_assert(AG_LANE_MAX <= 64u, "four values a lane of the group");
-        Acc t[16];
+    static_assert(AG_LANE_MAX <= 64u, "four values a lane of the group");
+    const auto at = [&](uint32_t i) {
+        const float x = v[i];
+        return i < d ? x : 0.0f;
+    };
+    float t[16];
+#pragma unroll
+    for (uint32_t l = 0; l < 16u; l++)
+        t[l] = at(l) + at(16u + l);
+    if (d > 32u) {
 #pragma unroll
         for (uint32_t l = 0; l < 16u; l++)
-            t[l] = l < d ? v[l] : Acc(0);
-#pragma unroll
-        for (uint32_t l = 0; l < 16u; l++)
-            t[l] = t[l] + (16u + l < d ? v[16u + l] : Acc(0));
-        if (d > 32u) {
-#pragma unroll
-            for (uint32_t l = 0; l < 16u; l++)
-                t[l] = t[l] + ((32u + l < d ? v[32u + l] : Acc(0)) +
-                               (48u + l < d ? v[48u + l] : Acc(0)));
-        }
-#pragma unroll
-        for (uint32_t m = 8u; m >= 1u; m >>= 1)
-#pragma unroll
-            for (uint32_t l = 0; l < 8u; l++)
-                if (l < m)
-                    t[l] = t[l] + t[l + m];
-        return t[0] + Acc(0);   // a sum of -0 terms is +0, as where zeros start it
+            t[l] = t[l] + (at(32u + l) + at(48u + l));
     }
+#pragma unroll
+    for (uint32_t m = 8u; m >= 1u; m >>= 1)
+#pragma unroll
+        for (uint32_t l = 0; l < 8u; l++)
+            if (l < m)
+                t[l] = t[l] + t[l + m];
+    return t[0] + 0.0f;   // a sum of -0 terms is +0, as where zeros start it
+}
+
+// A row of a tile by one lane: integer sums, exact in any order, and rows of the thread bin in
+// element order, other FP32 rows by lane_tree.
+__device__ __forceinline__ float tile_row_sum(const float *s_vals, uint32_t b, uint32_t e,
+                                              uint32_t seq_max)
+{
+    return e - b > seq_max ? lane_tree(s_vals + b, e - b) : lane_sum(s_vals, b, e);
+}
+__device__ __forceinline__ uint64_t tile_row_sum(const uint64_t *s_vals, uint32_t b, uint32_t e,
+                                                 uint32_t)
+{
+    return lane_sum(s_vals, b, e);
+}
+
+// This lane's values v[q], v[q + 64], ... below hi: integers one after another, FP32 in four
+// accumulators that take turns, as strided_sum.
+__device__ __forceinline__ uint64_t lane_strided(const uint64_t *v, uint32_t q, uint32_t hi)
+{
+    uint64_t a = 0;
+    for (; q < hi; q += AG_WAVE)
+        a = a + v[q];
+    return a;
+}
+__device__ __forceinline__ float lane_strided(const float *v, uint32_t q, uint32_t hi)
+{
+    static_assert(AG_UNROLL == 4, "four accumulators");
+    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+    for (; q + 3u * AG_WAVE < hi; q += 4u * AG_WAVE) {
+        a0 = a0 + v[q];
+        a1 = a1 + v[q + AG_WAVE];
+        a2 = a2 + v[q + 2u * AG_WAVE];
+        a3 = a3 + v[q + 3u * AG_WAVE];
+    }
+    if (q < hi)
+        a0 = a0 + v[q];
+    if (q + AG_WAVE < hi)
+        a1 = a1 + v[q + AG_WAVE];
+    if (q + 2u * AG_WAVE < hi)
+        a2 = a2 + v[q + 2u * AG_WAVE];
+    return (a0 + a1) + (a2 + a3);
 }
 
 // A workgroup's tile, with its ids and per-edge data loaded (or on their way), and the next one.
@@ -576,9 +614,7 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, P &pol, Red &r
                 L.lng[wave * AG_LONG_MAX + nl +
                       __builtin_popcountll(mask & ((1ull << lane) - 1ull))] = r;
             else if (r < cur.r1)
-                pol.finish(r, e - b > G.seq_max ? lane_tree(L.vals + (b - cur.e0), e - b)
-                                                : lane_sum(L.vals, b - cur.e0, e - cur.e0),
-                           red, pre);
+                pol.finish(r, tile_row_sum(L.vals, b - cur.e0, e - cur.e0, G.seq_max), red, pre);
             nl += (uint32_t)__builtin_popcountll(mask);
             r = rn;
             b = bn;
@@ -606,18 +642,7 @@ __device__ __forceinline__ void pull_row_tiles(const PullGeom &G, P &pol, Red &r
             for (uint32_t k = wave; k < c3; k += AG_WG / AG_WAVE) {
                 const uint32_t row = row_of(k);
                 const uint32_t lo = G.off[row] - cur.e0, hi = G.off[row + 1] - cur.e0;
-                // four accumulators a lane, as strided_sum
-                Acc a[AG_UNROLL];
-#pragma unroll
-                for (int u = 0; u < AG_UNROLL; u++)
-                    a[u] = Acc(0);
-                for (uint32_t q = lo + lane; q < hi; q += AG_UNROLL * AG_WAVE) {
-#pragma unroll
-                    for (int u = 0; u < AG_UNROLL; u++)
-                        if (q + u * AG_WAVE < hi)
-                            a[u] = a[u] + L.vals[q + u * AG_WAVE];
-                }
-                const Acc acc = group_reduce<Acc, AG_WAVE>((a[0] + a[1]) + (a[2] + a[3]));
+                const Acc acc = group_reduce<Acc, AG_WAVE>(lane_strided(L.vals, lo + lane, hi));
                 if (lane == 0)
                     L.lsum[k] = acc;
             }
