@@ -4,13 +4,13 @@
 // row with more is a part by itself) and at most AG_BATCH_PART_ROWS rows; the parts of the
 // largest graphs come first. One iteration of pageRank.c:942-1109 for every graph still
 // iterating is two launches:
-//   batch_part_kernel   every part of every unstopped graph: its values gathered into LDS with
-//                       16 loads in flight a lane, then light rows (<= heavy_deg in-edges)
-//                       summed by one lane in the reference's stream order, heavy rows by a
+//   batch_part_kernel   every part of every unstopped graph: its ids loaded (16 in flight a
+//                       lane), its values gathered into LDS, then light rows (<= heavy_deg
+//                       in-edges) summed by one lane in the reference's stream order, heavy rows by a
 //                       wavefront (four strided accumulators, fixed tree); the fused damping
 //                       update and next contribution; the part's FP64 L1 and active partial
 //                       (fixed-order workgroup reduction). A lane reading its row's ids and then
-//                       its values, four in flight, made 48 graphs of scale 10 to 15 take 3.26
+//                       its values, four ids at a time, made 48 graphs of scale 10 to 15 take 3.26
 //                       ms to L1 1e-6, against 2.50 with this and the finish by wavefronts
 //   batch_fin_kernel    per graph: its parts' partials in a fixed order, the stop rule
 //                       (active count or L1), the iteration count, the graph's done flag

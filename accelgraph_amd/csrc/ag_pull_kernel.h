@@ -138,8 +138,7 @@ struct NoPre {
 
 // Per-edge data (SpMV weights) that a tile loads with its source ids, a tile ahead of the gathers
 // that multiply by it: P::Edge, P::edge_pre(j) and P::edge_at(s, data) of policies that have any.
-// Loaded with the gathers instead, the weights took the place of gathers in flight: weighted
-// SpMV RMAT-22 422 us, RMAT-20 122, Erdos-Renyi 300 K 39; a tile ahead 307, 99 and 29.
+// Loaded with the gathers instead, the weights added a wait to each of them: weighted SpMV RMAT-22 422 us, RMAT-20 122, Erdos-Renyi 300 K 39; a tile ahead 307, 99 and 29.
 template <class P, class = void>
 struct EdgeOf {
     using T = NoPre;
@@ -176,17 +175,19 @@ static_assert(AG_TILE_NNZ_MAX / (AG_LANE_MAX + 1u) < AG_LONG_MAX,
 // (2.43 / 4.34 ms; 60 VGPRs, the same occupancy)
 #define AG_CMB_UNROLL 8
 #define AG_CMB_UNROLL_4B 4
-// source-id loads (then gathers) in flight per lane in an LDS tile: 16 covers a full tile
-// (AG_TILE_NNZ_MAX / AG_WG) in one round. Measured on RMAT-25 / ER-25 pass 1: 2 / 4 / 8 / 16
-// gave 2.96 / 2.76 / 2.63 / 2.57 ms and 5.11 / 4.63 / 4.52 / 4.43 ms per iteration
+// Source-id loads in flight per lane in an LDS tile: 16 covers a full tile (AG_TILE_NNZ_MAX /
+// AG_WG) in one round. Measured on RMAT-25 / ER-25 pass 1: 2 / 4 / 8 / 16 gave 2.96 / 2.76 / 2.63 /
+// 2.57 ms and 5.11 / 4.63 / 4.52 / 4.43 ms per iteration. The gathers of the round go one after
+// another: each is predicated together with the use of its value (an LDS store, an addition), and
+// the compiled code waits for it there, so a lane has one gather in flight, a wavefront up to 64
+// lines, and the wavefronts of a CU overlap theirs.
 #define AG_TILE_UNROLL 16
 
 // Lane-strided partial sum of in-edges lo, lo+S, ... < hi. Each round issues the source-id
-// loads of U elements, then their gathers, all predicated, so a lane has up to U independent
-// gathers in flight and a short row costs one round trip, not one per element. Four accumulators
+// loads of U elements, all in flight, then their gathers one by one (above). Four accumulators
 // take the elements in turn and combine in a fixed tree, whatever U is. Workgroup rows take 16
-// loads a lane (4096 in-edges a round, as an LDS
-// tile): RMAT-18 SpMV 25.4 -> 22.1 us, RMAT-20 81.7 -> 77.9 us against 4.
+// loads a lane (4096 in-edges a round, as an LDS tile): RMAT-18 SpMV 25.4 -> 22.1 us, RMAT-20
+// 81.7 -> 77.9 us against 4.
 template <class P, uint32_t S, int U = AG_UNROLL>
 __device__ __forceinline__ typename P::Acc strided_sum(const PullGeom &G, const P &pol,
                                                         uint32_t lo, uint32_t hi)
@@ -383,14 +384,14 @@ struct TopTab {
 //
 // The regular schedule hands the rows of the lower bins (all whose rows fit a tile) to the
 // workgroups as tiles of consecutive rows (G.rt, at most AG_TILE_NNZ_MAX in-edges, see
-// cut_row_tiles), whatever their bin: a tile's ids and then its values are gathered with up to 16
-// loads in flight a lane and staged in LDS. Rows of at most seq_max in-edges (the thread bin's) are
+// cut_row_tiles), whatever their bin: a tile's ids arrive with up to 16 loads in flight a lane, its
+// values are gathered (one after another a lane) and staged in LDS. Rows of at most seq_max in-edges (the thread bin's) are
 // summed by one lane in stream order, rows of at most lane_max by one lane in lane_tree's order,
 // longer ones by a wavefront in strided_sum's, and every row is finished by a lane of its own, so
-// the loads and stores of the update are coalesced. The next tile's ids, and this tile's row bounds and update operands, are
-// in flight while the values arrive: a tile costs one dependent round of loads.
-// A group of lanes per row, four gathers in flight each and a chain of four dependent loads a
-// row (offsets, ids, values, update operands), left the chip waiting. A SpMV before -> with row
+// the loads and stores of the update are coalesced. The next tile's ids load while this one is
+// summed, its row bounds and update operands beside the gathers.
+// A group of lanes per row, with a chain of four dependent loads a row (offsets, ids, values,
+// update operands), left the chip waiting. A SpMV before -> with row
 // tiles: RMAT-16 7.9 -> 7.1 us, RMAT-18 27.4 -> 21.6, RMAT-20 98 -> 81.6 (0.2 T in-edges/s from
 // 0.146 T L2 requests/s; the blocked pass 1 makes 0.19), Erdos-Renyi 300 K rows of 16 in-edges
 // 29.3 -> 24.9, of 40 64.4 -> 55.5. A product on a few hundred rows takes longer, 2.6 -> 3.5 us (3
@@ -703,7 +704,7 @@ struct CombPol {
 };
 
 // Gathers in-edges [e0, e0 + nnz) (nnz <= AG_TILE_NNZ_MAX) into s_vals with coalesced
-// source-id reads, AG_TILE_UNROLL loads then gathers in flight per lane.
+// source-id reads, AG_TILE_UNROLL of those loads in flight per lane, then the gathers.
 template <class P, class TT = NoTop>
 __device__ __forceinline__ void stage_edges(const uint32_t *src, uint32_t e0, uint32_t nnz,
                                             const P &pol, typename P::Acc *s_vals,
