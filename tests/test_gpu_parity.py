@@ -546,11 +546,10 @@ def test_pagerank_data_driven_user_starts(device, rmat16):
 
 
 def test_push_bin_shapes(device):
-    """The push's bins (ranges of at most 4096 destination rows and 2^17 in-edges; a heavier
-    row is a bin by itself) on a graph that reaches every case: two hub rows above 2^17
-    in-edges, a run of rows without in-edges, a 240 K-row chain (bins cut at 4096 rows) and a
-    vertex count that is not a multiple of 4096. Fixed point bit-exact with the pull oracle,
-    FP32 within the FP32 bar; SpMV push likewise."""
+    """The push direction, which runs the pull's kernels, on a graph with two hub rows above 2^17
+    in-edges, a run of rows without in-edges, a 240 K-row chain and a vertex count that is not
+    a multiple of 4096. Fixed point bit-exact with the pull oracle, FP32 within the FP32 bar;
+    SpMV push likewise."""
     say("push bins: hub rows, empty rows, long chain")
     n = 250_003
     hub0 = np.arange(1, 200_001, dtype=np.uint32)
